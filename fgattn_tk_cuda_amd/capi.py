@@ -46,6 +46,8 @@ _SIGNATURES = {
     "spattn_maxq_denom_blockmax": (_c_int, [_c_void_p] * 5 + [_c_int] * 5 + [_c_float, _c_void_p]),
     "spattn_fullattn_maxq_denom_blockmax": (_c_int, [_c_void_p] * 7 + [_c_int] * 5 + [_c_float, _c_void_p]),
     "spattn_blockmax_to_blocklists": (_c_int, [_c_void_p] * 6 + [_c_float] + [_c_int] * 6 + [_c_float, _c_int, _c_void_p]),
+    "spattn_blockmax_to_packedmask": (_c_int, [_c_void_p] * 6 + [_c_float] + [_c_int] * 6 + [_c_float, _c_void_p]),
+    "spattn_packedmask_to_indexmask_filled": (_c_int, [_c_void_p] * 3 + [_c_int] * 5 + [_c_void_p]),
     "spattn_booleanmask_128_blocks": (_c_int, [_c_void_p, _c_float, _c_int] + [_c_void_p] * 6 + [_c_int] * 6 + [_c_float, _c_void_p]),
     "spattn_booleanmask_packed_blocks": (_c_int, [_c_void_p, _c_float, _c_int, _c_int] + [_c_void_p] * 6 + [_c_int] * 6 + [_c_float, _c_void_p]),
     "spattn_pack_mask": (_c_int, [_c_void_p] * 2 + [_c_int] * 4 + [_c_void_p]),
@@ -368,6 +370,21 @@ def blockmax_to_blocklists(blk_indices, blk_counts, blockmax, max_q, denom, thre
                                                 scale, MB, _stream(stream)))
 
 
+def blockmax_to_packedmask(packed, blockmax, max_q, denom, q, k, threshold, *, kv_len=0, scale=0.0, stream=None):
+    """The bits of booleanmask_packed (qblk = 128) from the block maxima of a statistics sweep: only the pairs of
+    32-row group and 64-key block that can hold a passing key are multiplied."""
+    B, H, S, D = _bhsd(q)
+    if packed.dim() != 4 or tuple(packed.shape[:3]) != (B, H, (S + 127) // 128):
+        raise ValueError("packed must be uint8 [B,H,ceil(S/128),mask_stride/8]")
+    if tuple(k.shape) != (B, H, S, D):
+        raise ValueError("k must match q")
+    _need_padded(max_q, denom, B, H, S)
+    _need_blockmax(blockmax, B, H, S)
+    _check(load().spattn_blockmax_to_packedmask(_ptr(packed, torch.uint8), _ptr(blockmax, bf16), _ptr(max_q, f32),
+                                                _ptr(denom, f32), _ptr(q, bf16), _ptr(k, bf16), float(threshold),
+                                                int(packed.shape[3]) * 8, B, H, S, D, kv_len, scale, _stream(stream)))
+
+
 def pack_mask(packed, booleanmask, *, stream=None):
     """packed: uint8 [B,H,SB,mask_stride/8]; bit (c & 7) of byte c >> 3 is set where booleanmask[..., c] > 0."""
     if booleanmask.dim() != 4:
@@ -378,16 +395,18 @@ def pack_mask(packed, booleanmask, *, stream=None):
     _check(load().spattn_pack_mask(_ptr(packed, torch.uint8), _ptr(booleanmask, i32), B, H, SB, MS, _stream(stream)))
 
 
-def packedmask_to_indexmask(kv_indices, kv_num_indices, packed, seq, *, stream=None):
-    """Index lists straight from a bit-packed mask (uint8 [B,H,SB,mask_stride/8])."""
+def packedmask_to_indexmask(kv_indices, kv_num_indices, packed, seq, *, fill_tail=False, stream=None):
+    """Index lists straight from a bit-packed mask (uint8 [B,H,SB,mask_stride/8]); with fill_tail the entries
+    behind a count are written with mask_stride."""
     if packed.dim() != 4:
         raise ValueError("packed must be [B,H,SB,mask_stride/8]")
     B, H, SB, MB = (int(x) for x in packed.shape)
     MS = MB * 8
     if tuple(kv_indices.shape) != (B, H, SB, MS) or kv_num_indices.numel() != B * H * SB:
         raise ValueError("kv_indices / kv_num_indices do not match the packed mask")
-    _check(load().spattn_packedmask_to_indexmask(_ptr(kv_indices, i32), _ptr(kv_num_indices, i32),
-                                                 _ptr(packed, torch.uint8), B, H, int(seq), SB, MS, _stream(stream)))
+    fn = load().spattn_packedmask_to_indexmask_filled if fill_tail else load().spattn_packedmask_to_indexmask
+    _check(fn(_ptr(kv_indices, i32), _ptr(kv_num_indices, i32), _ptr(packed, torch.uint8), B, H, int(seq), SB, MS,
+              _stream(stream)))
 
 
 def qk_topkmask_indices(kv_indices, kv_num_indices, score, qmean, q, k, select_k, *, blocksz=128, kv_len=0,

@@ -87,7 +87,7 @@ constexpr int kBitFlush = 1024;
 
 __global__ __launch_bounds__(256) void packed_to_indexmask_kernel(int* __restrict__ kv_indices, int* __restrict__ kv_num,
                                                                   const uint32_t* __restrict__ packed, int rows,
-                                                                  int mask_stride, int kv_len) {
+                                                                  int mask_stride, int kv_len, int fill_tail) {
   constexpr int QN = kBitRing;
   constexpr int FL = kBitFlush;
   static_assert(FL + 1024 <= QN && FL % 256 == 0, "one sub-step must fit next to a pending flush");
@@ -156,16 +156,22 @@ __global__ __launch_bounds__(256) void packed_to_indexmask_kernel(int* __restric
     for (; head < tail; head += 64)
       if (head + lane < tail) dst[head + lane] = q[(head + lane) & (QN - 1)];
     if (lane == 0) kv_num[row] = tail;
+    if (fill_tail) {   // mask_stride behind the count: whole lines from the next 16-byte boundary on
+      const int v0 = (tail + 3) & ~3;
+      if (lane < v0 - tail) dst[tail + lane] = mask_stride;
+      const i32x4 f = {mask_stride, mask_stride, mask_stride, mask_stride};
+      for (int i = v0 + 4 * lane; i < mask_stride; i += 256) *reinterpret_cast<i32x4*>(dst + i) = f;
+    }
   }
 }
 
 hipError_t run_packed_to_indexmask(int* kv_indices, int* kv_num, const uint32_t* packed, int rows, int mask_stride,
-                                   int kv_len, hipStream_t stream) {
+                                   int kv_len, bool fill_tail, hipStream_t stream) {
   if (rows <= 0) return hipSuccess;
   int grid = (rows + 3) / 4;
   if (grid > 2048) grid = 2048;
   hipLaunchKernelGGL(packed_to_indexmask_kernel, dim3(grid), dim3(256), 0, stream, kv_indices, kv_num, packed, rows,
-                     mask_stride, kv_len);
+                     mask_stride, kv_len, fill_tail ? 1 : 0);
   return hipGetLastError();
 }
 

@@ -163,6 +163,20 @@ int spattn_blockmax_to_blocklists(int* blk_indices, int* blk_counts, void* block
                                                      max_blocks, as_stream(stream)));
 }
 
+int spattn_blockmax_to_packedmask(void* packed, const void* blockmax, const float* max_q, const float* denom, const void* q,
+                                  const void* k, float threshold, int mask_stride, int B, int H, int S, int D, int kv_len,
+                                  float scale, void* stream) {
+  if (int st = check_qkv(q, k, B, H, S, D)) return done(st);
+  if (!packed || !blockmax || !max_q || !denom) return done(SPATTN_ERR_NULL);
+  if (misaligned(packed) || misaligned(blockmax)) return done(SPATTN_ERR_ALIGN);
+  const int kv = (kv_len <= 0 || kv_len > S) ? S : kv_len;
+  if (mask_stride <= 0 || mask_stride % 128 != 0 || mask_stride < kv) return done(SPATTN_ERR_STRIDE);
+  const float sc = scale > 0.f ? scale : 1.0f / sqrtf((float)D);
+  return from_hip(spattn::run_blockmax_votes(static_cast<uint32_t*>(packed), static_cast<const uint16_t*>(blockmax), max_q,
+                                             denom, static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k),
+                                             threshold, mask_stride, B * H, S, D, kv, spattn::kLog2e * sc, as_stream(stream)));
+}
+
 int spattn_booleanmask_128(int* booleanmask, float threshold, int mask_stride, const float* max_q, const float* denom,
                            const void* q, const void* k, int B, int H, int S, int D, int kv_len, float scale,
                            void* stream) {
@@ -266,14 +280,26 @@ int spattn_pack_mask(void* packed, const int* booleanmask, int B, int H, int seq
                                         as_stream(stream)));
 }
 
-int spattn_packedmask_to_indexmask(int* kv_indices, int* num_kv_indices, const void* packed, int B, int H, int seq,
-                                   int seqblocks, int mask_stride, void* stream) {
+namespace {
+int packed_to_lists(int* kv_indices, int* num_kv_indices, const void* packed, int B, int H, int seq, int seqblocks,
+                    int mask_stride, bool fill_tail, void* stream) {
   if (!kv_indices || !num_kv_indices || !packed) return done(SPATTN_ERR_NULL);
   if (B <= 0 || H <= 0 || seqblocks <= 0 || seq < 0) return done(SPATTN_ERR_SHAPE);
   if (mask_stride <= 0 || mask_stride % 128 != 0) return done(SPATTN_ERR_STRIDE);
   if (misaligned(kv_indices) || misaligned(packed)) return done(SPATTN_ERR_ALIGN);
   return from_hip(spattn::run_packed_to_indexmask(kv_indices, num_kv_indices, static_cast<const uint32_t*>(packed),
-                                                  B * H * seqblocks, mask_stride, seq, as_stream(stream)));
+                                                  B * H * seqblocks, mask_stride, seq, fill_tail, as_stream(stream)));
+}
+}  // namespace
+
+int spattn_packedmask_to_indexmask(int* kv_indices, int* num_kv_indices, const void* packed, int B, int H, int seq,
+                                   int seqblocks, int mask_stride, void* stream) {
+  return packed_to_lists(kv_indices, num_kv_indices, packed, B, H, seq, seqblocks, mask_stride, false, stream);
+}
+
+int spattn_packedmask_to_indexmask_filled(int* kv_indices, int* num_kv_indices, const void* packed, int B, int H, int seq,
+                                          int seqblocks, int mask_stride, void* stream) {
+  return packed_to_lists(kv_indices, num_kv_indices, packed, B, H, seq, seqblocks, mask_stride, true, stream);
 }
 
 int spattn_qk_topkmask_indices(int* kv_indices, int* num_kv_indices, void* score, void* qmean, const void* q,

@@ -99,6 +99,18 @@ __device__ __forceinline__ float pair_sum(float x) {
   return a + b;
 }
 
+// Inclusive prefix sum over the 64 lanes (fields packed in x must not carry into each other).
+__device__ __forceinline__ uint32_t lane_scan(uint32_t x) {
+  int v = (int)x;
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);   // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);   // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);   // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+  return (uint32_t)v;
+}
+
 // WGs are dealt to the 8 XCDs round-robin by launch order; give each XCD one
 // contiguous range of logical work ids so that neighbouring q-blocks of a head
 // share that XCD's L2.

@@ -25,7 +25,7 @@ hipError_t run_all_index(int* kv_indices, int* kv_num, int rows, int mask_stride
 // bitmask_kernels.hip
 hipError_t run_pack_mask(uint32_t* packed, const int* mask, int rows, int mask_stride, hipStream_t stream);
 hipError_t run_packed_to_indexmask(int* kv_indices, int* kv_num, const uint32_t* packed, int rows, int mask_stride,
-                                   int kv_len, hipStream_t stream);
+                                   int kv_len, bool fill_tail, hipStream_t stream);
 
 // blocklist_kernels.hip
 hipError_t run_packed_to_blocklists(int* blk_indices, int* blk_counts, unsigned char* blockmask, const uint32_t* packed,
@@ -36,6 +36,11 @@ hipError_t run_votes_to_blocklists(int* blk_indices, int* blk_counts, unsigned c
 hipError_t run_blockmax_to_blocklists(int* blk_indices, int* blk_counts, unsigned char* blockmask, const uint16_t* blockmax,
                                       const float* max_q, const float* denom, float thresh, float sf, int qblk,
                                       int heads_total, int S, int kv_len, int max_blocks, hipStream_t stream);
+
+// votes_kernels.hip
+hipError_t run_blockmax_votes(uint32_t* bits, const uint16_t* blockmax, const float* max_q, const float* denom,
+                              const uint16_t* q, const uint16_t* k, float thresh, int mask_stride, int HB, int S, int D,
+                              int kv_len, float sf, hipStream_t stream);
 
 // topk_kernels.hip
 hipError_t run_topk_mask(int* kv_indices, int* kv_num, uint16_t* score, uint16_t* qmean, const uint16_t* q,

@@ -400,18 +400,6 @@ __device__ __forceinline__ uint32_t dot2_u16(uint32_t flags, uint32_t weights, u
   typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
   return __builtin_amdgcn_udot2(__builtin_bit_cast(u16x2, flags), __builtin_bit_cast(u16x2, weights), acc, false);
 }
-// Inclusive prefix sum over the 64 lanes (fields packed in x must not carry into each other).
-__device__ __forceinline__ uint32_t lane_scan(uint32_t x) {
-  int v = (int)x;
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);   // row_shr:2
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);   // row_shr:4
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);   // row_shr:8
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
-  return (uint32_t)v;
-}
-
 // find_bin on plain counts with the bins dealt to the lanes from the top (lane l holds bins
 // 255 - 4l .. 252 - 4l): the sum over the bins at and above a lane's own is then an inclusive
 // prefix sum over the lanes, six DPP adds instead of six cross-lane reads through LDS.

@@ -383,6 +383,29 @@ void blockmax_to_blocklists(torch::Tensor blk_idx, torch::Tensor blk_cnt, OptTen
                "blockmax_to_blocklists");
 }
 
+// The threshold sweep over the (32-row group, 64-key block) pairs whose block maxima say that they can hold a
+// passing key: packed uint8 [B,H,ceil(S/128),mask_stride/8], bit for bit booleanmask_packed at qblk = 128.
+void blockmax_to_packedmask(torch::Tensor packed, torch::Tensor blockmax, torch::Tensor o_max_q, torch::Tensor o_denom,
+                            torch::Tensor q, torch::Tensor k, double threshold, double scale, int64_t kv_len) {
+  check_bhsd(q, "q", q);
+  check_bhsd(k, "k", q);
+  check_aux(packed, "packed", at::kByte, q);
+  check_aux(o_max_q, "o_max_q", at::kFloat, q);
+  check_aux(o_denom, "o_denom", at::kFloat, q);
+  const int64_t B = q.size(0), H = q.size(1), S = q.size(2), SB = (S + 127) / 128;
+  TORCH_CHECK(packed.dim() == 4 && packed.size(0) == B && packed.size(1) == H && packed.size(2) == SB,
+              "packed must be [B,H,ceil(S/128),mask_stride/8]");
+  const int64_t need = B * H * padded128(S);
+  TORCH_CHECK(o_max_q.numel() == need && o_denom.numel() == need, "o_max_q / o_denom must be [B,H,1,128*ceil(S/128)]");
+  check_blockmax(blockmax, q, B, H, S);
+  const DeviceGuard guard(q.device());
+  check_status(spattn_blockmax_to_packedmask(packed.data_ptr(), blockmax.data_ptr(), o_max_q.data_ptr<float>(),
+                                             o_denom.data_ptr<float>(), q.data_ptr(), k.data_ptr(), (float)threshold,
+                                             (int)packed.size(3) * 8, (int)B, (int)H, (int)S, (int)q.size(3),
+                                             checked_kv_len(kv_len, q), (float)scale, cur_stream()),
+               "blockmax_to_packedmask");
+}
+
 void booleanmask_128_ex(torch::Tensor booleanmask, torch::Tensor o_max_q, torch::Tensor o_denom, torch::Tensor q,
                         torch::Tensor k, double threshold, double scale, int64_t kv_len) {
   check_bhsd(q, "q", q);
@@ -569,7 +592,8 @@ void pack_mask(torch::Tensor packed, torch::Tensor booleanmask) {
                "pack_mask");
 }
 
-void packedmask_to_indexmask(torch::Tensor kv_indices, torch::Tensor kv_numindices, torch::Tensor packed, int64_t seq) {
+static void packedmask_to_lists(torch::Tensor& kv_indices, torch::Tensor& kv_numindices, torch::Tensor& packed, int64_t seq,
+                                bool fill_tail) {
   TORCH_CHECK(packed.is_cuda() && packed.scalar_type() == at::kByte && packed.is_contiguous() && packed.dim() == 4,
               "packed must be a contiguous uint8 device tensor [B,H,SB,mask_stride/8]");
   check_aux(kv_indices, "kv_indices", at::kInt, packed);
@@ -581,10 +605,19 @@ void packedmask_to_indexmask(torch::Tensor kv_indices, torch::Tensor kv_numindic
               "kv_numindices must have B*H*SB entries");
   TORCH_CHECK(seq >= 0, "seq must not be negative");
   const DeviceGuard guard(packed.device());
-  check_status(spattn_packedmask_to_indexmask(kv_indices.data_ptr<int>(), kv_numindices.data_ptr<int>(), packed.data_ptr(),
-                                              (int)packed.size(0), (int)packed.size(1), (int)seq, (int)packed.size(2),
-                                              (int)packed.size(3) * 8, cur_stream()),
+  auto* const run = fill_tail ? spattn_packedmask_to_indexmask_filled : spattn_packedmask_to_indexmask;
+  check_status(run(kv_indices.data_ptr<int>(), kv_numindices.data_ptr<int>(), packed.data_ptr(), (int)packed.size(0),
+                   (int)packed.size(1), (int)seq, (int)packed.size(2), (int)packed.size(3) * 8, cur_stream()),
                "packedmask_to_indexmask");
+}
+
+void packedmask_to_indexmask(torch::Tensor kv_indices, torch::Tensor kv_numindices, torch::Tensor packed, int64_t seq) {
+  packedmask_to_lists(kv_indices, kv_numindices, packed, seq, false);
+}
+
+// The same with the entries behind a count written with mask_stride, the fill of the reference's lists.
+void packedmask_to_indexmask_filled(torch::Tensor kv_indices, torch::Tensor kv_numindices, torch::Tensor packed, int64_t seq) {
+  packedmask_to_lists(kv_indices, kv_numindices, packed, seq, true);
 }
 
 // The top-k mask generator of the reference's Python layer (python/spattn/mask_utils.py:389-417)
@@ -647,6 +680,9 @@ void noop_md_bm(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torc
 void noop_bm_lists(torch::Tensor, torch::Tensor, OptTensor, torch::Tensor, torch::Tensor, torch::Tensor, double, int64_t, int64_t,
                    int64_t, double, int64_t) {}
 
+void noop_bm_packed(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, double, double,
+                    int64_t) {}
+
 TORCH_LIBRARY_FRAGMENT(cuda_attn, m) {
   m.def("full_attn(Tensor(a!) o, Tensor q, Tensor k, Tensor v) -> ()");
   m.def("all_index_mask(Tensor(a!) kv_indices, Tensor(b!) kv_num_indices, int batch, int heads, int seqblocks, int seq) -> ()");
@@ -674,6 +710,8 @@ TORCH_LIBRARY_FRAGMENT(cuda_attn, m) {
   m.def("fullattn_maxq_denom_blockmax(Tensor(a!) o, Tensor(b!) o_max_q, Tensor(c!) o_denom, Tensor(d!) blockmax, Tensor q, Tensor k, Tensor v, float scale, int kv_len) -> ()");
   m.def("maxq_denom_blockmax(Tensor(a!) o_max_q, Tensor(b!) o_denom, Tensor(c!) blockmax, Tensor q, Tensor k, float scale, int kv_len) -> ()");
   m.def("blockmax_to_blocklists(Tensor(a!) blk_idx, Tensor(b!) blk_cnt, Tensor(c!)? blockmask, Tensor blockmax, Tensor o_max_q, Tensor o_denom, float threshold, int seq, int head_dim, int qblk, float scale, int kv_len) -> ()");
+  m.def("blockmax_to_packedmask(Tensor(a!) packed, Tensor blockmax, Tensor o_max_q, Tensor o_denom, Tensor q, Tensor k, float threshold, float scale, int kv_len) -> ()");
+  m.def("packedmask_to_indexmask_filled(Tensor(a!) kv_indices, Tensor(b!) kv_numindices, Tensor packed, int seq) -> ()");
 }
 
 TORCH_LIBRARY_IMPL(cuda_attn, Meta, m) {
@@ -702,6 +740,8 @@ TORCH_LIBRARY_IMPL(cuda_attn, Meta, m) {
   m.impl("fullattn_maxq_denom_blockmax", noop_fmd_bm);
   m.impl("maxq_denom_blockmax", noop_md_bm);
   m.impl("blockmax_to_blocklists", noop_bm_lists);
+  m.impl("blockmax_to_packedmask", noop_bm_packed);
+  m.impl("packedmask_to_indexmask_filled", noop_b2i);
 }
 
 // The CUDA dispatch key serves HIP tensors on PyTorch-ROCm.
@@ -731,6 +771,8 @@ TORCH_LIBRARY_IMPL(cuda_attn, CUDA, m) {
   m.impl("fullattn_maxq_denom_blockmax", fullattn_maxq_denom_blockmax);
   m.impl("maxq_denom_blockmax", maxq_denom_blockmax);
   m.impl("blockmax_to_blocklists", blockmax_to_blocklists);
+  m.impl("blockmax_to_packedmask", blockmax_to_packedmask);
+  m.impl("packedmask_to_indexmask_filled", packedmask_to_indexmask_filled);
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -759,4 +801,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fullattn_maxq_denom_blockmax", &fullattn_maxq_denom_blockmax, "fullattn_maxq_denom + per-block row maxima");
   m.def("maxq_denom_blockmax", &maxq_denom_blockmax, "maxq_denom + per-block row maxima");
   m.def("blockmax_to_blocklists", &blockmax_to_blocklists, "block maxima -> KV-block lists");
+  m.def("blockmax_to_packedmask", &blockmax_to_packedmask, "threshold sweep over what the block maxima leave, bit-packed");
+  m.def("packedmask_to_indexmask_filled", &packedmask_to_indexmask_filled, "packedmask_to_indexmask with the tail filled");
 }

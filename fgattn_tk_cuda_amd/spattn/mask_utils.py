@@ -279,16 +279,18 @@ def pack_votes_cuda(booleanmask):
     return packed
 
 
-def packedmask_to_indexmask_cuda(packed, seq=None):
+def packedmask_to_indexmask_cuda(packed, seq=None, fill_tail=True):
     """Index lists and counts straight from a bit-packed mask; equals
-    ``bitmask_to_indexmask_cuda(unpack(packed), seq)``."""
+    ``bitmask_to_indexmask_cuda(unpack(packed), seq)``.  ``fill_tail=False`` leaves the entries behind a count
+    unwritten (a caller that hands the lists to ``sp_attn`` and drops them)."""
     B, H, SB, MB = packed.shape
     MS = MB * 8
     if seq is None:
         seq = MS
-    kv_indices = torch.full((B, H, SB, MS), MS, dtype=torch.int32, device=packed.device)
-    num_kv_indices = torch.zeros((B, H, SB), dtype=torch.int32, device=packed.device)
-    spattn_interface.packedmask_to_indexmask(kv_indices, num_kv_indices, packed.contiguous(), seq)
+    kv_indices = torch.empty((B, H, SB, MS), dtype=torch.int32, device=packed.device)
+    num_kv_indices = torch.empty((B, H, SB), dtype=torch.int32, device=packed.device)
+    decode = spattn_interface.packedmask_to_indexmask_filled if fill_tail else spattn_interface.packedmask_to_indexmask
+    decode(kv_indices, num_kv_indices, packed.contiguous(), seq)
     return kv_indices, num_kv_indices
 
 
@@ -298,12 +300,23 @@ def qk_indexmask_from_maxq_denom_cuda(max_q, denom, q, k, thresh, blocksz=128):
     return bitmask_to_indexmask_cuda(booleanmask, q.shape[2])
 
 
-def qk_indexmask_cuda(q, k, thresh, blocksz=128):
-    """Statistics -> vote mask -> index lists (python/spattn/mask_utils.py:306-334)."""
+def qk_indexmask_cuda(q, k, thresh, blocksz=128, onepass=None, fill_tail=True):
+    """Key lists from the threshold mask (python/spattn/mask_utils.py:306-334): statistics with block maxima,
+    then the lists from those; or, where the maxima of one head are too large (``head_groups``) or with
+    ``onepass=False``, the reference's statistics -> vote mask -> index lists.  The same lists either way.
+    ``fill_tail=False`` leaves the entries behind a count unwritten (a caller that hands the lists to
+    ``sp_attn`` and drops them)."""
     assert blocksz == BLOCKSZ
+    groups = head_groups(q, onepass)
     max_q, denom = _stats_buffers(q)
-    spattn_interface.maxq_denom(max_q, denom, q.contiguous(), k.contiguous())
-    return qk_indexmask_from_maxq_denom_cuda(max_q, denom, q, k, thresh, blocksz)
+    if groups is None:
+        spattn_interface.maxq_denom(max_q, denom, q.contiguous(), k.contiguous())
+        return qk_indexmask_from_maxq_denom_cuda(max_q, denom, q, k, thresh, blocksz)
+
+    def sweep(lo, hi, blockmax, q_, k_, max_q_, denom_):
+        spattn_interface.maxq_denom_blockmax(max_q_, denom_, blockmax, q_, k_, 0.0, 0)
+
+    return packedmask_to_indexmask_cuda(packedmask_by_groups(groups, sweep, q, k, max_q, denom, thresh), q.shape[2], fill_tail)
 
 
 def qblock_order_cuda(counts):
@@ -400,6 +413,42 @@ def use_onepass(q, onepass=None, budget_bytes=None):
     return blockmax_bytes(q) <= budget
 
 
+def head_groups(q, onepass=None, budget_bytes=None):
+    """Ranges [(lo, hi), ...] over the B*H heads whose block maxima a one-sweep refresh holds at a time, or
+    None for the reference's two full sweeps.  Everything at once where ``use_onepass`` says so; above the
+    budget, near-equal groups whose buffer takes at most half of it (every group reuses the one buffer, and
+    what else the refresh holds stays small against it); None where not even one head fits that, or with
+    onepass=False."""
+    B, H = int(q.shape[0]), int(q.shape[1])
+    if use_onepass(q, onepass, budget_bytes):
+        return [(0, B * H)]
+    if onepass is not None:
+        return None
+    budget = BLOCKMAX_BUDGET_BYTES if budget_bytes is None else int(budget_bytes)
+    fit = (budget // 2) // (blockmax_bytes(q) // (B * H))
+    if fit < 1:
+        return None
+    n = -(-B * H // fit)
+    return [(B * H * i // n, B * H * (i + 1) // n) for i in range(n)]
+
+
+def packedmask_by_groups(groups, sweep, q, k, max_q, denom, thresh):
+    """The bit-packed threshold mask (per 128 rows) of a one-sweep refresh.  ``sweep(lo, hi, blockmax, q, k,
+    max_q, denom)`` runs the statistics sweep with block maxima over heads lo..hi-1 (its tensors are views of
+    those heads); the bits of the group follow from the maxima, whose buffer the next group reuses."""
+    B, H, S, D = q.shape
+    n, sp = B * H, max_q.shape[3]
+    packed = torch.empty((B, H, sp // BLOCKSZ, sp // 8), dtype=torch.uint8, device=q.device)
+    heads = [t.contiguous().view(1, n, *t.shape[2:]) for t in (q, k, max_q, denom, packed)]
+    blockmax = torch.empty((1, max(hi - lo for lo, hi in groups), sp // KVBLK, sp), dtype=torch.bfloat16, device=q.device)
+    for lo, hi in groups:
+        qs, ks, ms, ds, ps = (t[:, lo:hi] for t in heads)
+        bm = blockmax[:, : hi - lo]
+        sweep(lo, hi, bm, qs, ks, ms, ds)
+        spattn_interface.blockmax_to_packedmask(ps, bm, ms, ds, qs, ks, thresh, 0.0, 0)
+    return packed
+
+
 def blockmax_buffer(q):
     """bf16 [B,H,Sp/64,Sp] for the per-(row, key block) score maxima of a statistics sweep (the
     sweep rounds them toward +inf)."""
@@ -462,18 +511,22 @@ def qk_bitmask_from_blockmax_cuda(blockmax, max_q, denom, q, k, thresh, blocksz=
 
 
 def qk_packedmask_from_blockmax_cuda(blockmax, max_q, denom, q, k, thresh, qblk=128, kv_len=0):
-    """The same votes as bits (qk_packedmask_from_maxq_denom_cuda over the blocks that can hold a key)."""
+    """The same votes as bits (qk_packedmask_from_maxq_denom_cuda over what can hold a key: pairs of 32 rows and
+    64 keys for bits per 128 rows, key blocks for bits per 64 rows)."""
     B, H, S, D = q.shape
-    blk_idx, blk_cnt = _blocks_that_can_hold_a_key(blockmax, max_q, denom, thresh, S, D, kv_len)
+    max_q, denom, q, k = max_q.contiguous(), denom.contiguous(), q.contiguous(), k.contiguous()
     packed = torch.empty((B, H, (S + qblk - 1) // qblk, max_q.shape[3] // 8), dtype=torch.uint8, device=q.device)
-    spattn_interface.booleanmask_packed_blocks(packed, max_q.contiguous(), denom.contiguous(), q.contiguous(), k.contiguous(),
-                                               blk_idx, blk_cnt, thresh, qblk, 0.0, kv_len)
+    if qblk == 128:
+        spattn_interface.blockmax_to_packedmask(packed, blockmax, max_q, denom, q, k, thresh, 0.0, kv_len)
+    else:
+        blk_idx, blk_cnt = _blocks_that_can_hold_a_key(blockmax, max_q, denom, thresh, S, D, kv_len)
+        spattn_interface.booleanmask_packed_blocks(packed, max_q, denom, q, k, blk_idx, blk_cnt, thresh, qblk, 0.0, kv_len)
     return packed
 
 
 def qk_indexmask_from_blockmax_cuda(blockmax, max_q, denom, q, k, thresh, blocksz=128, kv_len=0):
-    """Key lists (the reference's form) from the block maxima: blocks that can hold a key, the sweep over
-    those blocks with its votes as bits, the key lists decoded from the bits."""
+    """Key lists (the reference's form) from the block maxima: the threshold sweep over what can hold a key
+    with its votes as bits, the key lists decoded from the bits."""
     packed = qk_packedmask_from_blockmax_cuda(blockmax, max_q, denom, q, k, thresh, blocksz, kv_len)
     return packedmask_to_indexmask_cuda(packed, kv_len or q.shape[2])
 

@@ -81,8 +81,10 @@ def attn_topkmask_cuda(query, key, value, current_layer=None, ditrun=None, *args
 
 
 def attn_computed_with_sparse_mask_cuda(query, key, value, *args, **kwargs):
-    """Threshold pre-pass on the device, then sparse attention (:62-70)."""
-    kv_indices, kv_num_indices = mask_utils.qk_indexmask_cuda(query, key, kwargs["thresh"], blocksz=kwargs["blocksz"])
+    """Threshold pre-pass on the device, then sparse attention (:62-70).  The lists do not leave the call:
+    what lies behind their counts is not written."""
+    kv_indices, kv_num_indices = mask_utils.qk_indexmask_cuda(query, key, kwargs["thresh"], blocksz=kwargs["blocksz"],
+                                                              fill_tail=False)
     return _sparse(query, key, value, kv_indices, kv_num_indices)
 
 
@@ -103,18 +105,34 @@ def sparse_attn_from_cache_cuda(query, key, value, *args, **kwargs):
 def cached_attn_cuda(query, key, value, current_layer, ditrun, *args, **kwargs):
     """On the steps that refresh the cache: dense attention with statistics, then the mask
     pre-pass; on every other step: sparse attention from the cached lists (:95-114).
-    Where the buffer for it fits the budget, the refresh step sweeps Q K^T once in full instead of
-    twice: the dense pass also writes the score maximum of every row over every 64-key block (bf16,
-    S*S/32 bytes per head, freed on return) and the threshold sweep then runs over the key blocks that
-    can hold a key only; the lists are the same.  ``onepass=True`` / ``False`` forces one route
-    (False: the reference's two full sweeps, no extra buffer); by default the route is the one-sweep
-    one when the buffer is at most ``blockmax_budget_bytes`` (default
-    ``mask_utils.BLOCKMAX_BUDGET_BYTES``, 2 GiB)."""
+    The refresh step sweeps Q K^T once in full instead of twice: the dense pass also writes the score
+    maximum of every row over every 64-key block (bf16, S*S/32 bytes per head, freed on return) and the
+    votes are then taken over the pairs of row group and key block that can hold a key only; the lists are
+    the same.  ``onepass=True`` / ``False`` forces one route (True: all heads at once; False: the
+    reference's two full sweeps, no extra buffer); by default all heads go at once when the buffer is at
+    most ``blockmax_budget_bytes`` (default ``mask_utils.BLOCKMAX_BUDGET_BYTES``, 2 GiB), else in groups of
+    heads whose buffer takes at most half of that, and in two sweeps where one head's does not
+    (``mask_utils.head_groups``)."""
     mask_cache = kwargs["mask_cache"]
     if mask_cache.run_fullattn(ditrun):
-        if mask_utils.use_onepass(query, kwargs.get("onepass"), kwargs.get("blockmax_budget_bytes")):
-            # the dense pass also writes the block maxima; the threshold sweep then runs over the key
-            # blocks that can hold a key only
+        route = kwargs.get("onepass"), kwargs.get("blockmax_budget_bytes")
+        groups = mask_utils.head_groups(query, *route) if kwargs["blocksz"] == mask_utils.BLOCKSZ else None
+        if groups is not None:
+            # the dense pass also writes the block maxima; the votes are then taken over the (row group,
+            # key block) pairs that can hold a key only
+            query, key, value = _c(query, key, value)
+            out = _out_like(query)
+            max_q, denom = mask_utils._stats_buffers(query)
+            B, H, S, D = query.shape
+            o_, v_ = out.view(1, B * H, S, D), value.view(1, B * H, S, D)
+
+            def sweep(lo, hi, blockmax, qs, ks, ms, ds):
+                spattn_interface.fullattn_maxq_denom_blockmax(o_[:, lo:hi], ms, ds, blockmax, qs, ks, v_[:, lo:hi], 0.0, 0)
+
+            packed = mask_utils.packedmask_by_groups(groups, sweep, query, key, max_q, denom, kwargs["thresh"])
+            kv_indices, kv_num_indices = mask_utils.packedmask_to_indexmask_cuda(packed, S)
+        elif mask_utils.use_onepass(query, *route):
+            # lists per 64 rows
             out = _out_like(query)
             max_q, denom = mask_utils._stats_buffers(query)
             blockmax = mask_utils.blockmax_buffer(query)

@@ -208,6 +208,19 @@ int spattn_booleanmask_packed_blocks(void* packed, float threshold, int mask_str
                                      const int* blk_counts, int max_blocks, int batch, int heads, int seq, int D,
                                      int kv_len, float scale, void* stream);
 
+/* The threshold sweep behind a statistics sweep with block maxima: blockmax
+ * ([batch,heads,Sp/64,Sp] of spattn_maxq_denom_blockmax / spattn_fullattn_maxq_denom_blockmax) says which
+ * pairs of a 32-row group and a 64-key block can hold a passing key; only those are multiplied.  packed as
+ * in spattn_booleanmask_packed at qblk = 128, bit for bit what that full sweep writes.  max_q, denom, scale
+ * and kv_len must be those of the statistics sweep; mask_stride a multiple of 128 not below the kv length. */
+int spattn_blockmax_to_packedmask(void* packed, const void* blockmax, const float* max_q, const float* denom, const void* q,
+                                  const void* k, float threshold, int mask_stride, int batch, int heads, int seq, int D,
+                                  int kv_len, float scale, void* stream);
+/* spattn_packedmask_to_indexmask that also writes mask_stride into the entries behind a count (what the
+ * reference's caller prefills, python/spattn/mask_utils.py:298). */
+int spattn_packedmask_to_indexmask_filled(int* kv_indices, int* num_kv_indices, const void* packed, int batch, int heads,
+                                          int seq, int seqblocks, int mask_stride, void* stream);
+
 /* Top-k mask generator (python/spattn/mask_utils.py:389-417, qk_topkmask_indices): per
  * q-block of `blocksz` rows the select_k keys c < kv_len (0 = seq) with the largest
  * (block mean of q / sqrt(D)) . k[c], every step rounded to bf16 as the reference's bf16 torch

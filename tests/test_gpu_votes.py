@@ -1,0 +1,66 @@
+"""GPU: blockmax_to_packedmask (the threshold sweep over what the block maxima leave) against the full sweep
+(booleanmask_packed, pinned to the oracle elsewhere), bit for bit, at the edges of its tiles: 32-row groups,
+128-row q-blocks, 64-key blocks, the 64 pieces of 32 keys that a wave's words go out in, and the key chunks of
+20480 (d = 128) and 32768 (d = 64) keys; and the key lists decoded with their tails filled."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D,S,kv_len,x", [
+    (64, 1, 0, 0.5), (128, 33, 0, 2), (64, 64, 63, 2), (128, 129, 65, 2), (64, 200, 1, 0.5), (128, 300, 0, 1e-6), (64, 300, 0, 1e6),
+    (64, 8193, 0, 16), (128, 8256, 8191, 32), (64, 8300, 0, 1e-6), (128, 20480, 0, 32), (128, 20545, 0, 16), (64, 32768, 32700, 64),
+    (64, 32900, 0, 32), (128, 20490, 0, 1e-6), (64, 100, 20, 1e-6), (128, 8224, 8220, 1e-6),
+])
+def test_votes_from_block_maxima(dev, D, S, kv_len, x):
+    from fgattn_tk_cuda_amd.spattn import mask_utils as mu
+
+    print("case blockmax_to_packedmask", D, S, kv_len, x, flush=True)
+    ops = torch.ops.cuda_attn
+    H = 2
+    g = torch.Generator(device=dev).manual_seed(S + D)
+    q, k = (torch.randn((1, H, S, D), generator=g, device=dev) +
+            torch.randn((1, H, (S + 63) // 64, D), generator=g, device=dev).repeat_interleave(64, dim=2)[:, :, :S] for _ in range(2))
+    q, k = q.to(torch.bfloat16).contiguous(), k.to(torch.bfloat16).contiguous()
+    thresh = x / (kv_len or S)
+    max_q, denom = mu._stats_buffers(q)
+    blockmax = mu.blockmax_buffer(q).fill_(float("nan"))     # blocks without a key stay unwritten and unread
+    ops.maxq_denom_blockmax(max_q, denom, blockmax, q, k, 0.0, kv_len)
+    want = mu.qk_packedmask_from_maxq_denom_cuda(max_q, denom, q, k, thresh, 128, kv_len)
+    got = torch.full_like(want, 0x5a)
+    ops.blockmax_to_packedmask(got, blockmax, max_q, denom, q, k, thresh, 0.0, kv_len)
+    assert torch.equal(got, want)
+    idx, num = (torch.full((1, H, want.shape[2], n), -7, dtype=torch.int32, device=dev) for n in (want.shape[3] * 8, 1))
+    ops.packedmask_to_indexmask(idx, num, got, kv_len or S)
+    filled, num2 = mu.packedmask_to_indexmask_cuda(got, kv_len or S)
+    assert torch.equal(num.view(-1), num2.view(-1))
+    tail = torch.arange(idx.shape[3], device=dev) >= num
+    assert torch.equal(filled.masked_fill(tail, -7), idx) and bool((filled[tail] == idx.shape[3]).all())
+    if x < 1e-3:                                              # a threshold below every weight keeps every key there is
+        assert int(num.sum()) == (kv_len or S) * num.numel()
+    with pytest.raises(RuntimeError):
+        ops.blockmax_to_packedmask(got, blockmax[:, :1].contiguous(), max_q, denom, q, k, thresh, 0.0, kv_len)
+
+
+@pytest.mark.parametrize("S,D", [(700, 64), (1300, 128)])
+def test_refresh_in_groups_of_heads(dev, S, D):
+    """cached_attn_cuda and qk_indexmask_cuda with a budget that holds some heads' block maxima only: output,
+    lists and counts equal those of all heads at once and of the two full sweeps."""
+    from fgattn_tk_cuda_amd.spattn import mask_utils as mu, sparseattn_functionals as fn
+
+    print("case head groups", S, D, flush=True)
+    B, H = 2, 3
+    g = torch.Generator(device=dev).manual_seed(S)
+    q, k, v = (torch.randn((B, H, S, D), generator=g, device=dev).to(torch.bfloat16) for _ in range(3))
+    per_head = mu.blockmax_bytes(q) // (B * H)
+    got = []
+    for kw in (dict(onepass=True), dict(onepass=False), dict(blockmax_budget_bytes=4 * per_head), dict(blockmax_budget_bytes=2 * per_head),
+               dict(blockmax_budget_bytes=per_head)):
+        cache = mu.NaiveMaskCache([0])
+        out = fn.cached_attn_cuda(q, k, v, 0, 0, thresh=4.0 / S, blocksz=128, mask_cache=cache, **kw)
+        got.append((out,) + tuple(cache.get_mask_from_cache(0)))
+    for other in got[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(got[0], other))
+    one, two = mu.qk_indexmask_cuda(q, k, 4.0 / S), mu.qk_indexmask_cuda(q, k, 4.0 / S, onepass=False)
+    assert torch.equal(one[0], two[0]) and torch.equal(one[1], two[1]) and 0 < float(two[1].float().mean()) < S
