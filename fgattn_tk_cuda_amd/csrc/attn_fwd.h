@@ -62,14 +62,14 @@ struct AttnCfg {
   static constexpr int kLoadsPerTile = kTileBytes / 1024 / 4;   // per wave
 };
 
-// Waves per SIMD the register allocation aims at.  Two everywhere (256 registers), except for block lists at
-// d = 64 with 128-row q-blocks: that instantiation fits 168 registers with a handful of spills outside the
-// tile loop, its 40 KB ring lets three workgroups share a CU, and it is bound by the vector ALU, which a
-// third wave keeps fed (measured side by side on one board: -7 %; the dense and token-list forms of the same
-// shape need 40-50 spills for it and lose).
+// Waves per SIMD the register allocation aims at.  Two (256 registers), except at d = 64 with 128-row q-blocks,
+// where 168 registers are enough for dense attention and block lists with a handful of spills outside the tile
+// loop: the 40 KB ring lets three workgroups share a CU, and these kernels are bound by the vector ALU, which a
+// third wave keeps fed (side by side: block lists -7 %, dense 16 x 16384 1.203 -> 1.178 ms, with statistics 1.253 ->
+// 1.222 ms).  Token lists of that shape need 184 registers and spill in the loop for it (0.72 -> 0.83 ms).
 template <int D, int QBLK, int MODE>
 constexpr int attn_waves_per_simd() {
-  return (D == 64 && QBLK == 128 && MODE == KV_BLOCKS) ? 3 : 2;
+  return (D == 64 && QBLK == 128 && MODE != KV_TOKENS) ? 3 : 2;
 }
 
 template <int D, int QBLK, int MODE, bool HAS_V, bool STATS>
@@ -354,11 +354,10 @@ void attn_fwd_kernel(const AttnParams p) {
 
   // Per-lane LDS addresses inside slot 0; slot, score block and k-step offsets are added
   // as constants (instruction immediates in the unrolled loop).
-  // A operand of QK^T, k-step t, score block 0.  K_XOR (d=128 with 128-row q-blocks, where the
-  // registers do not reach and two Q operands were reloaded from scratch on every tile, each
-  // reload waiting for every tile copy in flight): only the address of k-step 0 is kept, that
-  // of k-step t is the same with t XORed into chunk bits 1-3.
-  constexpr bool K_XOR = (D == 128 && QBLK == 128);
+  // A operand of QK^T, k-step t, score block 0.  K_XOR (the forms held to 168 registers): only the address of
+  // k-step 0 is kept, that of k-step t is the same with t XORed into chunk bits 1-3 (at d = 128, where the
+  // registers reach, keeping all of them is 1 % faster).
+  constexpr bool K_XOR = (QBLK == 128 && HAS_V && D == 64 && MODE != KV_TOKENS);
   lds_cptr k_lo[K_XOR ? 1 : NT];
   {
     const int krow = ksub * KW + ln;
@@ -398,33 +397,31 @@ void attn_fwd_kernel(const AttnParams p) {
   // Keys of tile `it` that do not exist get -inf.  Accumulator register 4j+i of block mb
   // is key ksub*KW + 32mb + 8j + 4g + i of the tile.
   auto mask_tile = [&](int desc, int desc_hi, f32x16 (&s)[NMB]) {
+    bool some;                 // wave-uniform: some key of the tile does not exist
+    unsigned long long m;      // bit c: key c of the tile exists
     if constexpr (MODE == KV_TOKENS) {
-      if ((desc & desc_hi) != -1) {   // wave-uniform: some key of the tile does not exist
-        const unsigned long long m = ((unsigned long long)(unsigned)desc_hi << 32) | (unsigned)desc;
-        const unsigned long long mine = m >> (ksub * KW + 4 * g);   // bit c: this lane's key c
-#pragma unroll
-        for (int mb = 0; mb < NMB; ++mb)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int c = 32 * mb + 8 * (r >> 2) + (r & 3);
-            if (!((mine >> c) & 1)) s[mb][r] = kNegInf;
-          }
-      }
+      some = (desc & desc_hi) != -1;
+      m = ((unsigned long long)(unsigned)desc_hi << 32) | (unsigned)desc;
     } else {
       const int keys = desc >> 24;
-      if (keys < 64) {
-        // existing keys are tile rows lo .. hi-1 (wave-uniform)
-        const int lo = kv_short ? 0 : 64 - keys;
-        const int hi = kv_short ? keys : 64;
-        const int kb = ksub * KW + 4 * g;    // this lane's first key
+      some = keys < 64;
+      // existing keys are the last of the tile, of a sequence shorter than a tile the first
+      const unsigned long long ones = (1ull << (keys & 63)) - 1ull;
+      m = kv_short ? ones : ones << ((64 - keys) & 63);
+    }
+    if (some) {
+      // Bit tests against constants: comparisons of key numbers kept one register per score alive through
+      // the whole loop, 30 of the dense and block-list forms (without them the sweeps are 4-6 % faster, the
+      // d = 128 forms no longer spill, and the d = 64 forms have room for a third wave).
+      unsigned long long mine = m >> (ksub * KW + 4 * g);   // bit c: this lane's key c
+      asm volatile("" : "+v"(mine));
 #pragma unroll
-        for (int mb = 0; mb < NMB; ++mb)
+      for (int mb = 0; mb < NMB; ++mb)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int c = 32 * mb + 8 * (r >> 2) + (r & 3);
-            if (kb < lo - c || kb >= hi - c) s[mb][r] = kNegInf;
-          }
-      }
+        for (int r = 0; r < 16; ++r) {
+          const int c = 32 * mb + 8 * (r >> 2) + (r & 3);
+          if (!((mine >> c) & 1)) s[mb][r] = kNegInf;
+        }
     }
   };
   // Row max of a score tile in NP pieces (so that they can be placed between multiplies),
@@ -517,11 +514,12 @@ void attn_fwd_kernel(const AttnParams p) {
     l_run += l_tile;
   };
 
-  // V^T operands of one 16-key step (PV group gi = 2mb + h), double-buffered over groups; where
-  // the registers do not reach (K_XOR) one buffer, the operand of block db refilled for the
-  // next group as soon as its multiply of this group has been issued.
+  // V^T operands of one 16-key step (PV group gi = 2mb + h), double-buffered over groups; with
+  // 128-row q-blocks where registers are short one buffer, the operand of block db refilled for the next
+  // group as soon as its multiply of this group has been issued (two buffers: at d = 128 sixteen registers
+  // more and 0.2-0.6 % slower, at d = 64 spills in the loop and 0.8 % slower).
   constexpr int NG = 2 * NMB;
-  constexpr int VB = K_XOR ? 1 : 2;
+  constexpr int VB = (QBLK == 128 && (D == 128 || (LAZY_MAX && MODE != KV_TOKENS))) ? 1 : 2;
   u32x2 va[HAS_V ? VB : 1][HAS_V ? NDB : 1][2];
   auto v_read_db = [&](uint32_t vofs, int gi, int db) {
     if constexpr (HAS_V) {
@@ -538,9 +536,11 @@ void attn_fwd_kernel(const AttnParams p) {
     for (int db = 0; db < (HAS_V ? NDB : 0); ++db) v_read_db(vofs, gi, db);
   };
 
-  // s_out^T = K Q^T from the K tile at ring offset kofs (bytes), one 32-key block at a
-  // time.  WITH_SM: the softmax of s_in is interleaved, one MFMA then the vector-ALU work of
-  // 16/NT score registers.  tl: a tile copy whose parts are issued between the multiplies
+  // s_out^T = K Q^T from the K tile at ring offset kofs (bytes).  The score blocks of 32 keys advance together,
+  // k-step by k-step: neighbouring multiplies share their Q operand and never wait for each other's result
+  // (block after block: dense d = 64 1.7 %, d = 128 0.4-0.7 %, the sweeps 1.5 % slower).  WITH_SM: the softmax
+  // of s_in is interleaved, one MFMA then the vector-ALU work of 16/NT score registers.  tl: a tile copy whose
+  // parts are issued between the multiplies
   // if `live` (in one burst they queue behind the other waves' copies and stall this wave).
   // EARLY_V: the V^T operands of the first PV group are requested before the last multiply,
   // so that PV does not start by waiting for LDS.
@@ -552,61 +552,65 @@ void attn_fwd_kernel(const AttnParams p) {
     constexpr int EPM = 16 / NT;
     constexpr int MPP = NT / 4;   // SPLIT_SM: multiplies per pair of score registers 8-15
     const float base = base_eff;
+    // Multiply m: k-step m / NMB of score block m % NMB - neighbours share their Q operand.
+    constexpr int NM = NMB * NT;
+    u32x4 ka[NT];
+    auto k_reads = [&](int m0, int m1) {
 #pragma unroll
-    for (int mb = 0; mb < NMB; ++mb) {
-      u32x4 ka[NT];
-      auto k_reads = [&](int t0, int t1) {
-#pragma unroll
-        for (int t = t0; t < t1; ++t) {
-          if constexpr (K_XOR) {
-            const uint32_t a0 = k_cur ^ (uint32_t)(t << 5);
-            ka[t] = *(SPATTN_LDS const u32x4*)((lds_cptr)(uintptr_t)a0 + kofs + mb * 32 * ROWB);
-          } else {
-            ka[t] = *(SPATTN_LDS const u32x4*)(k_lo[t] + kofs + mb * 32 * ROWB);
-          }
+      for (int m = m0; m < m1; ++m) {
+        const int t = m / NMB, mb = m % NMB;
+        if constexpr (K_XOR) {
+          const uint32_t a0 = k_cur ^ (uint32_t)(t << 5);
+          ka[m % NT] = *(SPATTN_LDS const u32x4*)((lds_cptr)(uintptr_t)a0 + kofs + mb * 32 * ROWB);
+        } else {
+          ka[m % NT] = *(SPATTN_LDS const u32x4*)(k_lo[t] + kofs + mb * 32 * ROWB);
         }
-        __builtin_amdgcn_sched_barrier(0);
-      };
-      // the operands arrive in two batches, to bound the registers they hold
-      k_reads(0, NT / 2);
-      const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      auto steps = [&](int t0, int t1) {
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    auto steps = [&](int m0, int m1) {
 #pragma unroll
-        for (int t = t0; t < t1; ++t) {
-          s_out[mb] = mfma32(ka[t], qf[t], t == 0 ? zero : s_out[mb]);
-          if constexpr (WITH_SM && SPLIT_SM) {
-            if (t % MPP == 0) softmax_chunk(s_in, base, mb, 8 + 2 * (t / MPP), 2, par_in);
-          } else if constexpr (WITH_SM) {
-            softmax_chunk(s_in, base, mb, t * EPM, EPM, par_in);
-          }
-          if (tl != nullptr && live) {
-            constexpr int STEP = (NMB * NT) / LPT;
-            const int m = mb * NT + t;
-            if (m % STEP == STEP - 1) load_part(*tl, m / STEP);
-          }
+      for (int m = m0; m < m1; ++m) {
+        const int t = m / NMB, mb = m % NMB;
+        s_out[mb] = mfma32(ka[m % NT], qf[t], t == 0 ? zero : s_out[mb]);
+        if constexpr (WITH_SM && SPLIT_SM) {
+          if (m % MPP == 0) softmax_chunk(s_in, base, (m / MPP) / 4, 8 + 2 * ((m / MPP) % 4), 2, par_in);
+        } else if constexpr (WITH_SM) {
+          softmax_chunk(s_in, base, m / NT, (m % NT) * EPM, EPM, par_in);
         }
-        if constexpr (WITH_SM) {
+        if (tl != nullptr && live) {
+          constexpr int STEP = NM / LPT;
+          if (m % STEP == STEP - 1) load_part(*tl, m / STEP);
+        }
+      }
+      if constexpr (WITH_SM) {
 #pragma unroll
-          for (int t = t0; t < t1; ++t) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);            // one MFMA
-            // its share of the softmax: seven instructions per pair of score registers
-            if constexpr (!SPLIT_SM) __builtin_amdgcn_sched_group_barrier(0x002, EPM * 7 / 2, 0);
-            else if constexpr (MPP == 1) __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
-            else if (t % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
-            else __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
-          }
+        for (int m = m0; m < m1; ++m) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);            // one MFMA
+          // its share of the softmax: seven instructions per pair of score registers
+          if constexpr (!SPLIT_SM) __builtin_amdgcn_sched_group_barrier(0x002, EPM * 7 / 2, 0);
+          else if constexpr (MPP == 1) __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
+          else if (m % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+          else __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
         }
-        __builtin_amdgcn_sched_barrier(0);
-      };
-      steps(0, NT / 4);
-      k_reads(NT / 2, NT);
-      if (EARLY_V && mb == NMB - 1) {
-        steps(NT / 4, NT - kEarly);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    // the operands arrive in batches of NT / 2, each requested NT / 4 multiplies ahead
+    k_reads(0, NT / 2);
+    steps(0, NT / 4);
+#pragma unroll
+    for (int b = 1; b < 2 * NMB; ++b) {
+      k_reads(b * NT / 2, (b + 1) * NT / 2);
+      const int m0 = b * NT / 2 - NT / 4, m1 = b + 1 < 2 * NMB ? m0 + NT / 2 : NM;
+      if (EARLY_V && b + 1 == 2 * NMB) {
+        steps(m0, m1 - kEarly);
         v_reads(vofs, 0);
         __builtin_amdgcn_sched_barrier(0);
-        steps(NT - kEarly, NT);
+        steps(m1 - kEarly, m1);
       } else {
-        steps(NT / 4, NT);
+        steps(m0, m1);
       }
     }
     if constexpr (WITH_SM) pin_softmax(par_in, SPLIT_SM ? 1 : 2);
