@@ -75,88 +75,79 @@ hipError_t run_pack_mask(uint32_t* packed, const int* mask, int rows, int mask_s
 // ------------------------------------------------------------------------------------
 // packed bits -> index lists, the fused form of unpack + booleanmask_to_indexmask
 // (include/mask_utils.cuh:273-302 for the compaction): per row the keys c < kv_len whose
-// bit is set, ascending, then the caller's fill; counts exact.
-// One wave per row.  A step takes 1 KB of bits (8192 keys, one 16-byte load per lane, the
-// next step in flight) into a wave-private LDS stage and walks it in eight sub-steps of
-// 1024 keys: lane l owns the 16 keys 16 l .. 16 l + 15 of the sub-step, a wave prefix sum of
-// the lanes' popcounts (five ballots) gives its place in the output, and it appends its keys to the same
-// kind of ring that compact_kernel uses, written out 4 KB at a time.
-// ------------------------------------------------------------------------------------
-constexpr int kBitRing = 2048;    // ints; a sub-step appends at most 1024 to fewer than kBitFlush pending
-constexpr int kBitFlush = 1024;
-
+// bit is set, ascending, counts exact; what lies behind the count is left to the caller or written
+// with mask_stride (FILL).
+// One wave per row, 2048 keys per step: a lane owns the 32 keys of one word (the words of the next four
+// steps are in flight), a lane scan of the popcounts gives its place, it writes its keys into the wave's
+// stage in LDS, and the stage leaves as consecutive words.
+// What bounds it: without the fill the instructions of the bit loop, as many rounds as the fullest lane has
+// keys.  32 keys per lane, four rounds between two branches and no ring bookkeeping: 71 us at 40 x 32760 rows
+// (8.5 % of the keys, in runs; 42 MB read, 114 MB written), where 16 keys per lane and 4 KB bursts through a
+// ring took 104.  With the fill the 1.34 GB of the lists, 0.28 ms (a plain fill of that size: 0.20 ms; the
+// four waves filling one row after the other, staggered starts, 128-byte aligned or non-temporal stores:
+// no faster).
+template <bool FILL>
 __global__ __launch_bounds__(256) void packed_to_indexmask_kernel(int* __restrict__ kv_indices, int* __restrict__ kv_num,
                                                                   const uint32_t* __restrict__ packed, int rows,
-                                                                  int mask_stride, int kv_len, int fill_tail) {
-  constexpr int QN = kBitRing;
-  constexpr int FL = kBitFlush;
-  static_assert(FL + 1024 <= QN && FL % 256 == 0, "one sub-step must fit next to a pending flush");
-  __shared__ __attribute__((aligned(16))) int ring[4][QN];
-  __shared__ __attribute__((aligned(16))) uint16_t stage[4][512];   // 1 KB of bits per wave
+                                                                  int mask_stride, int kv_len) {
+  constexpr int U = 4;   // steps whose words are in flight
+  __shared__ int stage_all[4][2048 + 64];   // and a slot per lane for the rounds in which it has no key left
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  int* q = ring[wave];
-  uint16_t* st = stage[wave];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int* const stage = stage_all[wave];
   const int lim = kv_len < mask_stride ? kv_len : mask_stride;
-  const int vec_per_row = mask_stride >> 7;            // 16-byte vectors (128 keys) per row
-  const int nstep = (lim + 8191) >> 13;                // steps that contain keys below lim
+  const int words = mask_stride >> 5;
+  const int nstep = (lim + 2047) >> 11;
 
   for (int row = blockIdx.x * 4 + wave; row < rows; row += gridDim.x * 4) {
-    const u32x4* __restrict__ src = reinterpret_cast<const u32x4*>(packed + (size_t)row * (mask_stride >> 5));
+    const uint32_t* __restrict__ src = packed + (size_t)row * words;
     int* __restrict__ dst = kv_indices + (size_t)row * mask_stride;
-    int tail = 0, head = 0;
-    auto load = [&](int c) -> u32x4 {
-      const int v = c * 64 + lane;
-      const u32x4 z = {0, 0, 0, 0};
-      return (v < vec_per_row) ? src[v] : z;
+    int tail = 0;
+    auto load = [&](int c) -> uint32_t {
+      const int w = c * 64 + lane;
+      return w < words ? src[w] : 0u;
     };
-    u32x4 cur = {0, 0, 0, 0}, nxt = {0, 0, 0, 0};
-    if (nstep > 0) cur = load(0);
-    for (int c = 0; c < nstep; ++c) {
-      if (c + 1 < nstep) nxt = load(c + 1);
-      *reinterpret_cast<u32x4*>(st + 8 * lane) = cur;   // keys 128 l .. 128 l + 127 of the step
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll 1
-      for (int s = 0; s < 8; ++s) {
-        const int key0 = c * 8192 + s * 1024 + 16 * lane;   // first key of this lane
-        if (c * 8192 + s * 1024 >= lim) break;               // wave-uniform
-        uint32_t bits = st[s * 64 + lane];
-        const int valid = lim - key0;                        // keys of this lane below lim
-        if (valid < 16) bits = valid <= 0 ? 0u : (bits & ((1u << valid) - 1u));
-        // exclusive prefix sum of the lanes' counts (0..16) without any exchange: one ballot per
-        // bit of the count, weighted by its place
-        const int cnt = __popc(bits);
-        int before = 0, total = 0;
+    uint32_t next[U];
 #pragma unroll
-        for (int w = 0; w < 5; ++w) {
-          const unsigned long long m = __ballot((cnt >> w) & 1);
-          before += (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0)) << w;
-          total += __popcll(m) << w;
-        }
-        int pos = tail + before;
-        while (bits) {
-          const int b = __builtin_ctz(bits);
-          q[pos & (QN - 1)] = key0 + b;
-          ++pos;
-          bits &= bits - 1;
-        }
-        tail += total;
-        if (tail - head >= FL) {
+    for (int u = 0; u < U; ++u) next[u] = load(u);
+    for (int c0 = 0; c0 < nstep; c0 += U) {
+      uint32_t cur[U];
 #pragma unroll
-          for (int w = 0; w < FL / 256; ++w)
-            *reinterpret_cast<i32x4*>(dst + head + w * 256 + 4 * lane) =
-                *reinterpret_cast<const i32x4*>(q + ((head + w * 256 + 4 * lane) & (QN - 1)));
-          head += FL;
-        }
+      for (int u = 0; u < U; ++u) cur[u] = next[u];
+      if (c0 + U < nstep) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) next[u] = load(c0 + U + u);
       }
-      __builtin_amdgcn_wave_barrier();
-      cur = nxt;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int key0 = ((c0 + u) * 64 + lane) * 32;   // first key of this lane
+        const int left = lim - key0;                     // its keys below lim
+        uint32_t bits = cur[u];
+        if (left < 32) bits = left <= 0 ? 0u : (bits & ((1u << left) - 1u));
+        if (__ballot(bits != 0) == 0) continue;          // wave-uniform
+        const int own = __popc(bits);
+        const int incl = (int)lane_scan((uint32_t)own);
+        const int total = __builtin_amdgcn_readlane(incl, 63);
+        // four rounds between two branches; a lane without a key left writes its spare slot
+        int at = incl - own;
+        do {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            stage[bits ? at : 2048 + lane] = key0 + __builtin_ctz(bits);
+            bits &= bits - 1;
+            ++at;
+          }
+        } while (__ballot(bits != 0) != 0);
+        // the stage is the wave's own: its LDS operations are executed in order
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        for (int i = lane; i < total; i += 64) dst[tail + i] = stage[i];
+        __builtin_amdgcn_wave_barrier();
+        tail += total;
+      }
     }
-    for (; head < tail; head += 64)
-      if (head + lane < tail) dst[head + lane] = q[(head + lane) & (QN - 1)];
     if (lane == 0) kv_num[row] = tail;
-    if (fill_tail) {   // mask_stride behind the count: whole lines from the next 16-byte boundary on
+    if constexpr (FILL) {   // whole lines from the next 16-byte boundary on
       const int v0 = (tail + 3) & ~3;
       if (lane < v0 - tail) dst[tail + lane] = mask_stride;
       const i32x4 f = {mask_stride, mask_stride, mask_stride, mask_stride};
@@ -169,9 +160,13 @@ hipError_t run_packed_to_indexmask(int* kv_indices, int* kv_num, const uint32_t*
                                    int kv_len, bool fill_tail, hipStream_t stream) {
   if (rows <= 0) return hipSuccess;
   int grid = (rows + 3) / 4;
-  if (grid > 2048) grid = 2048;
-  hipLaunchKernelGGL(packed_to_indexmask_kernel, dim3(grid), dim3(256), 0, stream, kv_indices, kv_num, packed, rows,
-                     mask_stride, kv_len, fill_tail ? 1 : 0);
+  if (grid > 65536) grid = 65536;
+  if (fill_tail)
+    hipLaunchKernelGGL(packed_to_indexmask_kernel<true>, dim3(grid), dim3(256), 0, stream, kv_indices, kv_num, packed, rows,
+                       mask_stride, kv_len);
+  else
+    hipLaunchKernelGGL(packed_to_indexmask_kernel<false>, dim3(grid), dim3(256), 0, stream, kv_indices, kv_num, packed, rows,
+                       mask_stride, kv_len);
   return hipGetLastError();
 }
 

@@ -120,6 +120,11 @@ class BitMaskCache:
         mask, seq_len = self.cache[layer]
         return bitmask_to_indexmask_cuda(mask, seq_len)
 
+    def lists_for_attention(self, layer):
+        """The lists of get_mask_from_cache for a caller that hands them to ``sp_attn`` and drops them: what lies
+        behind the counts may be left unwritten."""
+        return self.get_mask_from_cache(layer)
+
     def update_cache(self, layer, bytemask, seq_len):
         self.cache[layer] = (bytemask, seq_len)
 
@@ -134,6 +139,12 @@ class CompressedBitMaskCache(BitMaskCache):
         if packed.is_cuda and packed.dim() == 4:
             return packedmask_to_indexmask_cuda(packed, seq_len)
         return bitmask_to_indexmask_cuda(unpack(packed).to(torch.int32), seq_len)
+
+    def lists_for_attention(self, layer):
+        packed, seq_len = self.cache[layer]
+        if type(self) is CompressedBitMaskCache and packed.is_cuda and packed.dim() == 4:
+            return packedmask_to_indexmask_cuda(packed, seq_len, fill_tail=False)
+        return self.get_mask_from_cache(layer)   # a subclass may keep something else
 
     def update_cache(self, layer, bitmask, seq_len):
         if bitmask.is_cuda and bitmask.dim() == 4 and bitmask.dtype == torch.int32 and bitmask.shape[-1] % 128 == 0:

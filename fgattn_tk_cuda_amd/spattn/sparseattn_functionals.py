@@ -191,7 +191,8 @@ def bitmaskcached_attn_cuda(query, key, value, current_layer, ditrun, *args, **k
         bitmask = mask_utils.qk_bitmask_from_maxq_denom_cuda(max_q, denom, query, key, kwargs["thresh"], blocksz=kwargs["blocksz"])
         mask_cache.update_cache(current_layer, bitmask, query.shape[2])
         return out
-    kv_indices, kv_num_indices = mask_cache.get_mask_from_cache(current_layer)
+    lists = getattr(mask_cache, "lists_for_attention", mask_cache.get_mask_from_cache)
+    kv_indices, kv_num_indices = lists(current_layer)
     return _sparse(query, key, value, kv_indices, kv_num_indices)
 
 
