@@ -35,6 +35,7 @@ _SIGNATURES = {
     "spattn_sp_attn_blocks_balanced": (_c_int, [_c_void_p] * 7 + [_c_int] * 7 + [_c_float, _c_void_p]),
     "spattn_init": (_c_int, []),
     "spattn_qblock_order": (_c_int, [_c_void_p] * 2 + [_c_int, _c_void_p]),
+    "spattn_qblock_schedule": (_c_int, [_c_void_p] * 2 + [_c_int, _c_int, _c_void_p]),
     "spattn_all_index_mask": (_c_int, [_c_void_p] * 2 + [_c_int] * 5 + [_c_void_p]),
     "spattn_fullattn_maxq_denom": (_c_int, [_c_void_p] * 6 + [_c_int] * 5 + [_c_float, _c_void_p]),
     "spattn_maxq_denom": (_c_int, [_c_void_p] * 4 + [_c_int] * 5 + [_c_float, _c_void_p]),
@@ -383,6 +384,14 @@ def blockmax_to_packedmask(packed, blockmax, max_q, denom, q, k, threshold, *, k
     _check(load().spattn_blockmax_to_packedmask(_ptr(packed, torch.uint8), _ptr(blockmax, bf16), _ptr(max_q, f32),
                                                 _ptr(denom, f32), _ptr(q, bf16), _ptr(k, bf16), float(threshold),
                                                 int(packed.shape[3]) * 8, B, H, S, D, kv_len, scale, _stream(stream)))
+
+
+def qblock_schedule(order, counts, per_head, *, stream=None):
+    """order int32 [n]: a work order that keeps an XCD on one head at a time, longest lists first inside it;
+    per_head: q-blocks per head."""
+    if order.numel() != counts.numel():
+        raise ValueError("order must have one entry per count")
+    _check(load().spattn_qblock_schedule(_ptr(order, i32), _ptr(counts, i32), int(counts.numel()), int(per_head), _stream(stream)))
 
 
 def pack_mask(packed, booleanmask, *, stream=None):

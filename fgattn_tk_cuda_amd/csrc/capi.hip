@@ -326,6 +326,12 @@ int spattn_qblock_order(int* order, const int* counts, int n, void* stream) {
   return from_hip(spattn::run_qblock_order(order, counts, n, as_stream(stream)));
 }
 
+int spattn_qblock_schedule(int* order, const int* counts, int n, int per_head, void* stream) {
+  if (!order || !counts) return done(SPATTN_ERR_NULL);
+  if (n <= 0 || per_head <= 0) return done(SPATTN_ERR_SHAPE);
+  return from_hip(spattn::run_qblock_schedule(order, counts, n, per_head, as_stream(stream)));
+}
+
 int spattn_sp_attn_ordered(void* o, float* lse, const void* q, const void* k, const void* v, const int* kv_indices,
                            const int* num_kv_indices, const int* order, int mask_stride, int qblk, int B, int H, int S,
                            int D, int kv_len, float scale, void* stream) {

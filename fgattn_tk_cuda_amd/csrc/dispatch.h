@@ -49,5 +49,6 @@ hipError_t run_topk_mask(int* kv_indices, int* kv_num, uint16_t* score, uint16_t
 
 // order_kernels.hip
 hipError_t run_qblock_order(int* order, const int* counts, int n, hipStream_t stream);
+hipError_t run_qblock_schedule(int* order, const int* counts, int n, int per_head, hipStream_t stream);
 
 }  // namespace spattn

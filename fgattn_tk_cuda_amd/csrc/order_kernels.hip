@@ -114,6 +114,170 @@ __global__ __launch_bounds__(kOrderThreads) void qblock_order_kernel(int* __rest
   });
 }
 
+// ------------------------------------------------------------------------------------
+// The same purpose with an eye on L2.  Sorted over all heads, the q-blocks that an XCD works on at a time come
+// from every head, and the key rows they gather share nothing: the sort costs more than the balance gives.
+// Workgroups go to the XCDs round robin, so position 8 k + x of an order is the k-th workgroup of XCD x.  Every
+// XCD keeps its contiguous share of the q-blocks, in index order by windows of whole heads (at least kWindow
+// q-blocks), and inside a window the longest lists go first: one head at a time stays in its L2, lists of like
+// length walk the keys in step, and the last window still ends balanced.  Attention in ms, sorted over
+// everything / in index order / this: threshold lists 12 x 32760 x 128 0.582 / 0.575 / 0.559, 40 heads 2.00 /
+// 1.93 / 1.87, 24 x 32760 x 64 0.696 / 0.685 / 0.671; Zipf lists 8 x 65536 x 128 4.39 / 5.40 / 4.25, 32 x 16384 x
+// 128 0.661 / 0.585 / 0.502, 32 x 4096 x 128 0.101 / 0.081 / 0.074.
+// Two exceptions, decided on the counts: where the longest list is more than kTail of the work of one of an
+// XCD's 64 workgroup slots, a late window would end with it alone, and the share is one window (Zipf lists
+// 24 x 20000 x 64, 0.5 of a slot's work: 0.389 instead of 0.417 ms); and where the shares differ by more than
+// kSkew, the sort over everything balances the XCDs (shares within 1.09 of each other still gain by the windows).
+// The kernel takes 7 us for 6144 q-blocks (qblock_order_kernel: 20; classes of a sixteenth of an octave: no gain).
+// One workgroup per XCD, a wave per window; classes of an eighth of an octave over the seven octaves below the
+// longest list, stable, so the order is a function of the counts alone.
+// ------------------------------------------------------------------------------------
+constexpr int kXcds = 8;
+constexpr int kSlotsPerXcd = 64;
+constexpr int kWindow = 192;
+constexpr float kTail = 0.3f;
+constexpr float kSkew = 1.1f;
+constexpr int kSchedSub = 3;
+constexpr int kSchedOctaves = 7;
+constexpr int kSchedClasses = (kSchedOctaves << kSchedSub) + 4;   // a multiple of 4: a lane reads its table entries 16 bytes at a time
+
+// 0 holds the longest lists; top: floor(log2) of the longest of all
+__device__ __forceinline__ int schedule_class(int c, int top) {
+  if (c <= 0) return kSchedClasses - 1;
+  const int lg = 31 - __builtin_clz((unsigned)c);
+  const int below = lg >= kSchedSub ? ((c >> (lg - kSchedSub)) & ((1 << kSchedSub) - 1))
+                                    : ((c << (kSchedSub - lg)) & ((1 << kSchedSub) - 1));
+  const int cls = ((top - lg) << kSchedSub) + ((1 << kSchedSub) - 1 - below);
+  return cls < kSchedClasses - 2 ? cls : kSchedClasses - 2;
+}
+
+__global__ __launch_bounds__(256) void qblock_schedule_kernel(int* __restrict__ order, const int* __restrict__ counts, int n,
+                                                              int per_head) {
+  __shared__ __attribute__((aligned(16))) int tables[4][kSchedClasses * 64];   // [wave][class][lane]
+  __shared__ float share_l[kXcds];
+  __shared__ int longest_l[4];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int x = blockIdx.x;
+  const int per = n / kXcds;
+
+  // the work of every XCD's share and the longest list; a wave takes two shares
+  {
+    int longest = 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int y = 2 * wave + h;
+      float sum = 0.f;
+      for (int i = y * per + lane; i < (y + 1) * per; i += 512) {
+        int c[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) c[u] = i + 64 * u < (y + 1) * per ? counts[i + 64 * u] : 0;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          sum += (float)c[u];
+          longest = c[u] > longest ? c[u] : longest;
+        }
+      }
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+      if (lane == 0) share_l[y] = sum;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const int o = __shfl_xor(longest, off, 64);
+      longest = o > longest ? o : longest;
+    }
+    if (lane == 0) longest_l[wave] = longest;
+  }
+  __syncthreads();
+  float total = 0.f, most = 0.f;
+#pragma unroll
+  for (int y = 0; y < kXcds; ++y) {
+    total += share_l[y];
+    most = share_l[y] > most ? share_l[y] : most;
+  }
+  int longest = longest_l[0];
+#pragma unroll
+  for (int w = 1; w < 4; ++w) longest = longest_l[w] > longest ? longest_l[w] : longest;
+  const int top = 31 - __builtin_clz((unsigned)(longest > 0 ? longest : 1));
+  const bool global = most * kXcds > kSkew * total;
+  const bool one_window = (float)longest * kSlotsPerXcd > kTail * share_l[x];
+  int* const table = tables[wave];
+
+  // Stable counting sort of q-blocks a .. b-1 by class, one wave; the entry of rank r goes to
+  // order[first + r * step].  A lane owns a contiguous segment.  A wave's LDS operations execute in order.
+  auto sort = [&](int a, int b, int first, int step) {
+    auto settle = [] {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    };
+    for (int i = 4 * lane; i < kSchedClasses * 64; i += 256) {
+      const i32x4 z = {0, 0, 0, 0};
+      *reinterpret_cast<i32x4*>(table + i) = z;
+    }
+    const int seg = (b - a + 63) / 64;
+    const int i0 = a + lane * seg < b ? a + lane * seg : b;
+    const int i1 = i0 + seg < b ? i0 + seg : b;
+    settle();
+    for (int i = i0; i < i1; ++i) table[schedule_class(counts[i], top) * 64 + lane] += 1;
+    settle();
+    // exclusive prefix sum in storage order (class-major, lane-minor): lane l scans kSchedClasses entries from
+    // l * kSchedClasses on
+    int sum = 0;
+    i32x4* const own = reinterpret_cast<i32x4*>(table + lane * kSchedClasses);
+#pragma unroll
+    for (int j = 0; j < kSchedClasses / 4; ++j) {
+      const i32x4 v = own[j];
+      sum += v[0] + v[1] + v[2] + v[3];
+    }
+    int run = (int)lane_scan((uint32_t)sum) - sum;
+#pragma unroll
+    for (int j = 0; j < kSchedClasses / 4; ++j) {
+      const i32x4 v = own[j];
+      i32x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        o[e] = run;
+        run += v[e];
+      }
+      own[j] = o;
+    }
+    settle();
+    for (int i = i0; i < i1; ++i) {
+      const int slot = schedule_class(counts[i], top) * 64 + lane;
+      const int r = table[slot];
+      order[(size_t)first + (size_t)r * step] = i;
+      table[slot] = r + 1;
+    }
+    settle();
+  };
+
+  if (global) {
+    if (x == 0 && wave == 0) sort(0, n, 0, 1);
+    return;
+  }
+  const int end = (x + 1) * per;
+  int turn = 0;
+  for (int a = x * per; a < end; ++turn) {
+    int b = end;
+    if (!one_window) {
+      b = (a / per_head + 1) * per_head;
+      if (b - a < kWindow) b += (kWindow - (b - a) + per_head - 1) / per_head * per_head;
+      b = b < end ? b : end;
+    }
+    if ((turn & 3) == wave) sort(a, b, (a - x * per) * kXcds + x, kXcds);
+    a = b;
+  }
+  if (x == 0)
+    for (int i = per * kXcds + (int)threadIdx.x; i < n; i += 256) order[i] = i;
+}
+
+hipError_t run_qblock_schedule(int* order, const int* counts, int n, int per_head, hipStream_t stream) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(qblock_schedule_kernel, dim3(kXcds), dim3(256), 0, stream, order, counts, n, per_head);
+  return hipGetLastError();
+}
+
 hipError_t run_qblock_order(int* order, const int* counts, int n, hipStream_t stream) {
   if (n <= 0) return hipSuccess;
   hipLaunchKernelGGL(qblock_order_kernel, dim3(1), dim3(kOrderThreads), 0, stream, order, counts, n);

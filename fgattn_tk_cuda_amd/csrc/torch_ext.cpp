@@ -144,6 +144,18 @@ static void check_sp_attn_args(torch::Tensor& o, torch::Tensor& q, torch::Tensor
   TORCH_CHECK(kv_num_indices.numel() == q.size(0) * q.size(1) * kv_indices.size(2), "kv_num_indices must have B*H*SB entries");
 }
 
+// The work order for counts of per_head q-blocks per head.  Below kScheduleMin q-blocks all of them are resident
+// at once and the plain longest-first order does.
+constexpr int64_t kScheduleMin = 512;
+
+static void schedule_into(torch::Tensor& order, const torch::Tensor& counts, int64_t per_head, void* stream) {
+  const int n = (int)counts.numel();
+  int* const o = order.data_ptr<int>();
+  const int* const c = counts.data_ptr<int>();
+  check_status(n < kScheduleMin ? spattn_qblock_order(o, c, n, stream) : spattn_qblock_schedule(o, c, n, (int)per_head, stream),
+               "work order");
+}
+
 // Work orders of the reference-named sp_attn, which has no argument to pass one in.  One entry per
 // (device, stream, address and size of the counts tensor); the entry remembers the version counter
 // of the counts it was computed from.  A call that finds its entry with the same version launches
@@ -173,14 +185,11 @@ static int64_t counts_version(const torch::Tensor& t) {
 // The work order for these counts on the current stream; computes it if the cache has none.
 // Returns the tensor that owns the buffer (kept alive by the cache or, when the cache is full or
 // the stream is being captured into a graph, by the caller for the length of the call).
-static torch::Tensor cached_qblock_order(const torch::Tensor& counts) {
+static torch::Tensor cached_qblock_order(const torch::Tensor& counts, int64_t per_head) {
   const int dev = (int)counts.device().index();
   void* stream = cur_stream();
   const int64_t ver = counts_version(counts);
-  auto compute = [&](torch::Tensor& order) {
-    check_status(spattn_qblock_order(order.data_ptr<int>(), counts.data_ptr<int>(), (int)counts.numel(), stream),
-                 "sp_attn (work order)");
-  };
+  auto compute = [&](torch::Tensor& order) { schedule_into(order, counts, per_head, stream); };
   const bool capturing =
       c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
   std::lock_guard<std::mutex> lock(g_order_mu);
@@ -208,7 +217,7 @@ void sp_attn(torch::Tensor o, torch::Tensor q, torch::Tensor k, torch::Tensor v,
   // workgroups longest list first (lists within a factor of two of each other keep the default
   // order).  The order is computed when the counts tensor is first seen or has been written to
   // since (its version counter); every other call is the attention launch alone.
-  const torch::Tensor order = cached_qblock_order(kv_num_indices);
+  const torch::Tensor order = cached_qblock_order(kv_num_indices, kv_indices.size(2));
   sp_attn_impl(o, c10::nullopt, q, k, v, kv_indices, kv_num_indices, order.data_ptr<int>(), 0.0, 0);
 }
 
@@ -265,6 +274,17 @@ void qblock_order(torch::Tensor order, torch::Tensor counts) {
   const DeviceGuard guard(counts.device());
   check_status(spattn_qblock_order(order.data_ptr<int>(), counts.data_ptr<int>(), (int)counts.numel(), cur_stream()),
                "qblock_order");
+}
+
+// order int32 [n] <- a work order for counts of per_head q-blocks per head.
+void qblock_schedule(torch::Tensor order, torch::Tensor counts, int64_t per_head) {
+  TORCH_CHECK(counts.is_cuda() && counts.scalar_type() == at::kInt && counts.is_contiguous(),
+              "counts must be a contiguous int32 device tensor");
+  check_aux(order, "order", at::kInt, counts);
+  TORCH_CHECK(order.numel() == counts.numel() && counts.numel() > 0, "order must have one entry per count");
+  TORCH_CHECK(per_head > 0, "per_head must be positive");
+  const DeviceGuard guard(counts.device());
+  schedule_into(order, counts, per_head, cur_stream());
 }
 
 void fullattn_maxq_denom_ex(torch::Tensor o, torch::Tensor o_max_q, torch::Tensor o_denom, torch::Tensor q,
@@ -658,6 +678,7 @@ void noop6(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Te
 void noop_mask(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, double) {}
 void noop_b2i(torch::Tensor, torch::Tensor, torch::Tensor, int64_t) {}
 void noop2(torch::Tensor, torch::Tensor) {}
+void noop_schedule(torch::Tensor, torch::Tensor, int64_t) {}
 void noop_topk(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, int64_t, int64_t) {}
 void noop_full_ex(torch::Tensor, OptTensor, torch::Tensor, torch::Tensor, torch::Tensor, double, int64_t) {}
 void noop_sp_ex(torch::Tensor, OptTensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, OptTensor,
@@ -705,6 +726,7 @@ TORCH_LIBRARY_FRAGMENT(cuda_attn, m) {
   m.def("packedmask_to_blocklists(Tensor(a!) blk_idx, Tensor(b!) blk_cnt, Tensor(c!)? blockmask, Tensor packed, int seq) -> ()");
   m.def("booleanmask_to_blocklists(Tensor(a!) blk_idx, Tensor(b!) blk_cnt, Tensor(c!)? blockmask, Tensor booleanmask, int seq) -> ()");
   m.def("qblock_order(Tensor(a!) order, Tensor counts) -> ()");
+  m.def("qblock_schedule(Tensor(a!) order, Tensor counts, int per_head) -> ()");
   m.def("booleanmask_128_blocks(Tensor(a!) booleanmask, Tensor o_max_q, Tensor o_denom, Tensor q, Tensor k, Tensor blk_idx, Tensor blk_cnt, float threshold, float scale, int kv_len) -> ()");
   m.def("booleanmask_packed_blocks(Tensor(a!) packed, Tensor o_max_q, Tensor o_denom, Tensor q, Tensor k, Tensor blk_idx, Tensor blk_cnt, float threshold, int qblk, float scale, int kv_len) -> ()");
   m.def("fullattn_maxq_denom_blockmax(Tensor(a!) o, Tensor(b!) o_max_q, Tensor(c!) o_denom, Tensor(d!) blockmax, Tensor q, Tensor k, Tensor v, float scale, int kv_len) -> ()");
@@ -735,6 +757,7 @@ TORCH_LIBRARY_IMPL(cuda_attn, Meta, m) {
   m.impl("packedmask_to_blocklists", noop_blocklists);
   m.impl("booleanmask_to_blocklists", noop_blocklists);
   m.impl("qblock_order", noop2);
+  m.impl("qblock_schedule", noop_schedule);
   m.impl("booleanmask_128_blocks", noop_mask_blocks);
   m.impl("booleanmask_packed_blocks", noop_mask_packed_blocks);
   m.impl("fullattn_maxq_denom_blockmax", noop_fmd_bm);
@@ -766,6 +789,7 @@ TORCH_LIBRARY_IMPL(cuda_attn, CUDA, m) {
   m.impl("packedmask_to_blocklists", packedmask_to_blocklists);
   m.impl("booleanmask_to_blocklists", booleanmask_to_blocklists);
   m.impl("qblock_order", qblock_order);
+  m.impl("qblock_schedule", qblock_schedule);
   m.impl("booleanmask_128_blocks", booleanmask_128_blocks);
   m.impl("booleanmask_packed_blocks", booleanmask_packed_blocks);
   m.impl("fullattn_maxq_denom_blockmax", fullattn_maxq_denom_blockmax);
@@ -795,6 +819,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("booleanmask_packed", &booleanmask_packed, "threshold sweep, bit-packed result");
   m.def("packedmask_to_blocklists", &packedmask_to_blocklists, "bit-packed mask -> KV-block lists");
   m.def("booleanmask_to_blocklists", &booleanmask_to_blocklists, "vote mask -> KV-block lists");
+  m.def("qblock_schedule", &qblock_schedule, "work order by windows of heads, longest list first inside");
   m.def("qblock_order", &qblock_order, "work order, longest list first");
   m.def("booleanmask_128_blocks", &booleanmask_128_blocks, "threshold sweep over listed key blocks, int32 votes");
   m.def("booleanmask_packed_blocks", &booleanmask_packed_blocks, "threshold sweep over listed key blocks, bit-packed");

@@ -331,10 +331,12 @@ def qk_indexmask_cuda(q, k, thresh, blocksz=128, onepass=None, fill_tail=True):
 
 
 def qblock_order_cuda(counts):
-    """int32 [counts.numel()]: the q-blocks longest list first (the schedule of the list-driven
-    attention operators); lists within a factor of two of each other keep the default order."""
+    """int32 [counts.numel()]: the schedule of the list-driven attention operators for counts [B,H,SB].  From 512
+    q-blocks on every XCD works through its share by windows of whole heads, longest lists first inside a
+    window (``qblock_schedule``); below, where all q-blocks are resident at once, longest list first with lists
+    within a factor of two of each other in the default order (``qblock_order``)."""
     order = torch.empty((counts.numel(),), dtype=torch.int32, device=counts.device)
-    spattn_interface.qblock_order(order, counts.contiguous())
+    spattn_interface.qblock_schedule(order, counts.contiguous(), counts.shape[-1])
     return order
 
 

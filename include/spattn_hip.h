@@ -245,6 +245,11 @@ int spattn_qk_topkmask_indices(int* kv_indices, int* num_kv_indices, void* score
  * (nothing is read or written for it), a q-block that no entry names keeps whatever o held, and
  * a q-block named twice is computed twice. */
 int spattn_qblock_order(int* order, const int* counts, int n, void* stream);
+/* A work order for large sets of lists that also keeps an XCD on one head at a time: every XCD its contiguous
+ * share of the q-blocks by windows of whole heads (per_head q-blocks each, ceil(seq / qblk)), longest lists first
+ * inside a window; sorted over everything where the shares differ in work by more than a tenth.  A function of
+ * the counts alone, a permutation of 0..n-1, for the same order arguments. */
+int spattn_qblock_schedule(int* order, const int* counts, int n, int per_head, void* stream);
 int spattn_sp_attn_ordered(void* o, float* lse, const void* q, const void* k, const void* v, const int* kv_indices,
                            const int* num_kv_indices, const int* order, int mask_stride, int qblk, int batch, int heads,
                            int seq, int D, int kv_len, float scale, void* stream);
