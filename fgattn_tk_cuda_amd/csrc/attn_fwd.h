@@ -62,6 +62,13 @@ struct AttnCfg {
   static constexpr int kLoadsPerTile = kTileBytes / 1024 / 4;   // per wave
 };
 
+// LDS of one workgroup.  Statistics over 64-row q-blocks: the two waves that share the rows of a tile also exchange
+// its row maxima, for the block maxima (two tiles x 64 rows, behind the ring).
+template <int D, int QBLK, int MODE, bool HAS_V, bool STATS>
+constexpr int attn_lds_bytes() {
+  return AttnCfg<D, MODE, HAS_V>::kTotal + ((STATS && QBLK == 64) ? 2 * 64 * 4 : 0);
+}
+
 // Waves per SIMD the register allocation aims at.  Two (256 registers), except at d = 64 with 128-row q-blocks,
 // where 168 registers are enough for dense attention and block lists with a handful of spills outside the tile
 // loop: the 40 KB ring lets three workgroups share a CU, and these kernels are bound by the vector ALU, which a
@@ -437,10 +444,26 @@ void attn_fwd_kernel(const AttnParams p) {
   // for them per key block (blockmax[J][row], raw like max_q): the threshold test of the mask
   // pre-pass, softmax(r, c) > tau, holds for some key of block J exactly when the block's maximum
   // passes it, so these S x S/64 numbers replace the second score sweep for block-level masks.
+  constexpr bool BLOCKMAX = STATS && MODE == KV_DENSE;
+  float* const bm_xchg = reinterpret_cast<float*>(smem + Cfg::kTotal);   // KSPLIT == 2
+  float bm_own = kNegInf;
+  auto blockmax_merge = [&](int tile) {   // behind the barrier that follows the maxima of this tile
+    if constexpr (BLOCKMAX && KSPLIT == 2) {
+      if (p.blockmax != nullptr && ksub == 0 && g == 0)
+        p.blockmax[((size_t)bh * (p.Sp >> 6) + tile) * p.Sp + qrow] =
+            bf16_round_up(max_raw(bm_own, bm_xchg[(tile & 1) * 64 + 32 * qsub + ln]));
+    }
+  };
   auto stat_finish = [&](float mloc, int tile) -> float {
     mloc = pair_max(mloc);
-    if constexpr (STATS && KSPLIT == 1 && MODE == KV_DENSE) {
+    if constexpr (BLOCKMAX && KSPLIT == 1) {
       if (p.blockmax != nullptr && g == 0) p.blockmax[((size_t)bh * (p.Sp >> 6) + tile) * p.Sp + qrow] = bf16_round_up(mloc);
+    }
+    if constexpr (BLOCKMAX && KSPLIT == 2) {
+      // the wave with the upper keys hands its maxima over; they are read behind the next barrier, and a slot is
+      // written again two barriers later
+      if (ksub == 1) bm_xchg[(tile & 1) * 64 + 32 * qsub + ln] = mloc;
+      else bm_own = mloc;
     }
     m_true = max_raw(m_true, mloc);
     return mloc * p.sf;
@@ -696,6 +719,7 @@ void attn_fwd_kernel(const AttnParams p) {
       ids_resolve(it + NK, idr[(KC + NK) % 6], idw[(KC + NK) % 6], idh[(KC + NK) % 6]);
     }
     __syncthreads();
+    blockmax_merge(it);
     v_addr_refresh();
     // what the copies of V(it+1) and K(it+NK) are prepared from, and the key mask of tile it+1
     const int d_v = (MODE == KV_TOKENS) ? idr[(KC + 1) % 6] : idw[(KC + 1) % 6];
@@ -829,6 +853,7 @@ void attn_fwd_kernel(const AttnParams p) {
     for (int t = 0; t < NT; ++t) asm volatile("" ::"v"(qf[t]));
   }
   __syncthreads();   // every wave is done with the ring
+  if (ntiles > 0) blockmax_merge(ntiles - 1);
 
   // ---- combine the two 32-lane halves, then the two key halves -------------------
   float l_tot = pair_sum(l_run);
@@ -931,21 +956,21 @@ void attn_fwd_kernel(const AttnParams p) {
 // does it beforehand through spattn_init).
 template <int D, int QBLK, int MODE, bool HAS_V, bool STATS>
 inline hipError_t prepare_attn_fwd() {
-  using Cfg = AttnCfg<D, MODE, HAS_V>;
   static bool attr_set[kMaxDevices] = {};
-  return raise_lds_limit(reinterpret_cast<const void*>(attn_fwd_kernel<D, QBLK, MODE, HAS_V, STATS>), Cfg::kTotal, attr_set);
+  return raise_lds_limit(reinterpret_cast<const void*>(attn_fwd_kernel<D, QBLK, MODE, HAS_V, STATS>),
+                         attn_lds_bytes<D, QBLK, MODE, HAS_V, STATS>(), attr_set);
 }
 
 // Host launcher; returns hipError_t of the launch.
 template <int D, int QBLK, int MODE, bool HAS_V, bool STATS>
 inline hipError_t launch_attn_fwd(const AttnParams& p, hipStream_t stream) {
-  using Cfg = AttnCfg<D, MODE, HAS_V>;
   auto kern = attn_fwd_kernel<D, QBLK, MODE, HAS_V, STATS>;
   const hipError_t ea = prepare_attn_fwd<D, QBLK, MODE, HAS_V, STATS>();
   if (ea != hipSuccess) return ea;
   const int total = p.nqblk * p.H * p.B;
   if (total <= 0) return hipSuccess;
-  hipLaunchKernelGGL(kern, dim3(total), dim3(256), Cfg::kTotal, stream, p);
+  constexpr int kLds = attn_lds_bytes<D, QBLK, MODE, HAS_V, STATS>();
+  hipLaunchKernelGGL(kern, dim3(total), dim3(256), kLds, stream, p);
   return hipGetLastError();
 }
 
