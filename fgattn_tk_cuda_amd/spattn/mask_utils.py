@@ -403,8 +403,8 @@ def qk_blocklists_cuda(q, k, thresh, qblk=128, kv_len=0):
 
 # Largest block-maxima buffer the one-sweep routes allocate without being told to (bytes).  The
 # buffer takes 2 * Sp * Sp / 64 bytes per head: 0.81 GB at (1,24,32768), 1.5 GB at (1,12,75648),
-# 4.3 GB at (1,24,75904), 7.2 GB at (1,40,75648).  Above the budget the callers fall back to the
-# reference's two full sweeps, which need no such buffer.
+# 4.3 GB at (1,24,75904), 7.2 GB at (1,40,75648).  Above the budget the callers go through groups of
+# heads (head_groups).
 BLOCKMAX_BUDGET_BYTES = 2 << 30
 
 
@@ -445,20 +445,20 @@ def head_groups(q, onepass=None, budget_bytes=None):
     return [(B * H * i // n, B * H * (i + 1) // n) for i in range(n)]
 
 
-def packedmask_by_groups(groups, sweep, q, k, max_q, denom, thresh):
-    """The bit-packed threshold mask (per 128 rows) of a one-sweep refresh.  ``sweep(lo, hi, blockmax, q, k,
+def packedmask_by_groups(groups, sweep, q, k, max_q, denom, thresh, qblk=BLOCKSZ):
+    """The bit-packed threshold mask (per qblk rows) of a one-sweep refresh.  ``sweep(lo, hi, blockmax, q, k,
     max_q, denom)`` runs the statistics sweep with block maxima over heads lo..hi-1 (its tensors are views of
     those heads); the bits of the group follow from the maxima, whose buffer the next group reuses."""
     B, H, S, D = q.shape
     n, sp = B * H, max_q.shape[3]
-    packed = torch.empty((B, H, sp // BLOCKSZ, sp // 8), dtype=torch.uint8, device=q.device)
+    packed = torch.empty((B, H, (S + qblk - 1) // qblk, sp // 8), dtype=torch.uint8, device=q.device)
     heads = [t.contiguous().view(1, n, *t.shape[2:]) for t in (q, k, max_q, denom, packed)]
     blockmax = torch.empty((1, max(hi - lo for lo, hi in groups), sp // KVBLK, sp), dtype=torch.bfloat16, device=q.device)
     for lo, hi in groups:
         qs, ks, ms, ds, ps = (t[:, lo:hi] for t in heads)
         bm = blockmax[:, : hi - lo]
         sweep(lo, hi, bm, qs, ks, ms, ds)
-        spattn_interface.blockmax_to_packedmask(ps, bm, ms, ds, qs, ks, thresh, 0.0, 0)
+        _packedmask_from_blockmax(ps, bm, ms, ds, qs, ks, thresh, qblk, 0)
     return packed
 
 
@@ -523,17 +523,21 @@ def qk_bitmask_from_blockmax_cuda(blockmax, max_q, denom, q, k, thresh, blocksz=
     return mask
 
 
+def _packedmask_from_blockmax(packed, blockmax, max_q, denom, q, k, thresh, qblk, kv_len):
+    if qblk == 128:
+        spattn_interface.blockmax_to_packedmask(packed, blockmax, max_q, denom, q, k, thresh, 0.0, kv_len)
+    else:
+        blk_idx, blk_cnt = _blocks_that_can_hold_a_key(blockmax, max_q, denom, thresh, q.shape[2], q.shape[3], kv_len)
+        spattn_interface.booleanmask_packed_blocks(packed, max_q, denom, q, k, blk_idx, blk_cnt, thresh, qblk, 0.0, kv_len)
+
+
 def qk_packedmask_from_blockmax_cuda(blockmax, max_q, denom, q, k, thresh, qblk=128, kv_len=0):
     """The same votes as bits (qk_packedmask_from_maxq_denom_cuda over what can hold a key: pairs of 32 rows and
     64 keys for bits per 128 rows, key blocks for bits per 64 rows)."""
     B, H, S, D = q.shape
-    max_q, denom, q, k = max_q.contiguous(), denom.contiguous(), q.contiguous(), k.contiguous()
     packed = torch.empty((B, H, (S + qblk - 1) // qblk, max_q.shape[3] // 8), dtype=torch.uint8, device=q.device)
-    if qblk == 128:
-        spattn_interface.blockmax_to_packedmask(packed, blockmax, max_q, denom, q, k, thresh, 0.0, kv_len)
-    else:
-        blk_idx, blk_cnt = _blocks_that_can_hold_a_key(blockmax, max_q, denom, thresh, S, D, kv_len)
-        spattn_interface.booleanmask_packed_blocks(packed, max_q, denom, q, k, blk_idx, blk_cnt, thresh, qblk, 0.0, kv_len)
+    _packedmask_from_blockmax(packed, blockmax, max_q.contiguous(), denom.contiguous(), q.contiguous(), k.contiguous(), thresh,
+                              qblk, kv_len)
     return packed
 
 

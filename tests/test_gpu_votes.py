@@ -64,3 +64,24 @@ def test_refresh_in_groups_of_heads(dev, S, D):
         assert all(torch.equal(a, b) for a, b in zip(got[0], other))
     one, two = mu.qk_indexmask_cuda(q, k, 4.0 / S), mu.qk_indexmask_cuda(q, k, 4.0 / S, onepass=False)
     assert torch.equal(one[0], two[0]) and torch.equal(one[1], two[1]) and 0 < float(two[1].float().mean()) < S
+
+
+@pytest.mark.parametrize("S,D,qblk", [(700, 64, 64), (1300, 128, 64), (1300, 64, 128), (65, 128, 128)])
+def test_block_refresh_in_groups_of_heads(dev, S, D, qblk):
+    """blockcached_attn_cuda above its budget: output, lists and counts equal those of the two full sweeps."""
+    from fgattn_tk_cuda_amd.spattn import mask_utils as mu, sparseattn_functionals as fn
+
+    print("case block lists by head groups", S, D, qblk, flush=True)
+    B, H = 2, 3
+    g = torch.Generator(device=dev).manual_seed(S + qblk)
+    q, k, v = (torch.randn((B, H, S, D), generator=g, device=dev).to(torch.bfloat16) for _ in range(3))
+    per_head = mu.blockmax_bytes(q) // (B * H)
+    got = []
+    for kw in (dict(onepass=False), dict(blockmax_budget_bytes=4 * per_head), dict(blockmax_budget_bytes=2 * per_head),
+               dict(blockmax_budget_bytes=per_head)):
+        cache = mu.BlockListCache([0])
+        out = fn.blockcached_attn_cuda(q, k, v, 0, 0, thresh=8.0 / S, qblk=qblk, mask_cache=cache, **kw)
+        got.append((out,) + tuple(cache.get_mask_from_cache(0)))
+    for other in got[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(got[0], other))
+    assert int(got[0][2].sum()) > 0
