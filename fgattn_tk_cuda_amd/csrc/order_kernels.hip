@@ -199,7 +199,10 @@ __global__ __launch_bounds__(256) void qblock_schedule_kernel(int* __restrict__ 
   int longest = longest_l[0];
 #pragma unroll
   for (int w = 1; w < 4; ++w) longest = longest_l[w] > longest ? longest_l[w] : longest;
-  const int top = 31 - __builtin_clz((unsigned)(longest > 0 ? longest : 1));
+  // the sort over everything also classes the up to seven q-blocks behind the shares
+  int longest_all = longest;
+  for (int i = kXcds * per; i < n; ++i) longest_all = counts[i] > longest_all ? counts[i] : longest_all;
+  const int top = 31 - __builtin_clz((unsigned)(longest_all > 0 ? longest_all : 1));
   const bool global = most * kXcds > kSkew * total;
   const bool one_window = (float)longest * kSlotsPerXcd > kTail * share_l[x];
   int* const table = tables[wave];

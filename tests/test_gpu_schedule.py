@@ -1,6 +1,7 @@
 """GPU: qblock_schedule, the work order by windows of whole heads, against its definition on the host, entry for
 entry, at the edges: fewer entries than XCDs, shares that end inside a head, one window per share (a list longer
-than a third of a slot's work), shares of very different work (the sort over everything), empty lists."""
+than a third of a slot's work), shares of very different work (the sort over everything), empty lists, the longest list
+behind the shares."""
 import numpy as np
 import pytest
 import torch
@@ -45,12 +46,15 @@ def _schedule(counts, per_head):
 
 
 @pytest.mark.parametrize("n,per_head,kind", [(5, 5, "even"), (8, 3, "even"), (3072, 256, "near"), (3072, 256, "zipf"), (10240, 256, "near"),
-                                              (4728, 591, "near"), (2000, 64, "near"), (4096, 512, "skewed"), (70007, 9001, "near"), (1000, 7, "zeros")])
+                                              (4728, 591, "near"), (2000, 64, "near"), (4096, 512, "skewed"), (70007, 9001, "near"), (1000, 7, "zeros"),
+                                              (1003, 59, "last"), (1007, 53, "skewed_last")])
 def test_schedule_equals_its_definition(dev, n, per_head, kind):
     print("case schedule", n, per_head, kind, flush=True)
     rng = np.random.default_rng(n)
     counts = {"even": np.full(n, 26), "near": rng.integers(1700, 3600, size=n), "zipf": np.minimum(rng.zipf(1.2, size=n), 1024),
-              "skewed": np.where(np.arange(n) < n // 8, 5000, 300) + rng.integers(0, 200, size=n), "zeros": rng.integers(0, 2, size=n) * 9}[kind]
+              "skewed": np.where(np.arange(n) < n // 8, 5000, 300) + rng.integers(0, 200, size=n), "zeros": rng.integers(0, 2, size=n) * 9,
+              "last": np.where(np.arange(n) == n - 1, 60000, 300),
+              "skewed_last": np.where(np.arange(n) == n - 1, 60000, np.where(np.arange(n) < n // 8, 5000, 300))}[kind]
     counts = counts.astype(np.int32)
     c = torch.from_numpy(counts).to(dev)
     order = torch.full((n,), -1, dtype=torch.int32, device=dev)
