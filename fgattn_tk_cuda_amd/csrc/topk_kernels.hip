@@ -368,8 +368,11 @@ __global__ __launch_bounds__(256) void topk_select_kernel(int* __restrict__ kv_i
 constexpr int kRegThreads = 512;
 constexpr int kRegSlots = 32;
 constexpr int kRegSlotShift = 5;
-constexpr int kRegMaxVpl = 18;
-constexpr int kRegMaxKeys = kRegThreads * kRegMaxVpl * 8;   // 73728
+// The longest rows that the register form takes.  The library's longest sequence, 75600 keys, needs 19 vectors per
+// lane (191 registers, no spills): 12 x 75600 x 128 with 8 % of the keys 1619 -> 1121 us for means, scores (496) and
+// selection against the select that reads its row three times.
+constexpr int kRegMaxVpl = 19;
+constexpr int kRegMaxKeys = kRegThreads * kRegMaxVpl * 8;   // 77824
 
 __device__ __forceinline__ uint32_t pk_sub_sat_u16(uint32_t a, uint32_t b) {
   uint32_t d;
@@ -586,11 +589,13 @@ __global__ __launch_bounds__(kRegThreads) __attribute__((amdgpu_waves_per_eu(VPL
     __syncthreads();
     int out_pos = 0, eq_seen = 0;
     {
-      uint32_t before = 0;
+      // added up apart: seven waves of 19 vectors per lane hold more than 65535 keys
 #pragma unroll
-      for (int u = 0; u < kRegThreads / 64 - 1; ++u) before += u < wave ? wave_cnt[u] : 0u;
-      out_pos = (int)(before & 0xffffu);
-      eq_seen = (int)(before >> 16);
+      for (int u = 0; u < kRegThreads / 64 - 1; ++u) {
+        const uint32_t c = u < wave ? wave_cnt[u] : 0u;
+        out_pos += (int)(c & 0xffffu);
+        eq_seen += (int)(c >> 16);
+      }
     }
     out_pos += eq_seen < r ? eq_seen : r;
     if (wave_total >> 16) {
@@ -689,6 +694,7 @@ hipError_t run_topk_mask(int* kv_indices, int* kv_num, uint16_t* score, uint16_t
     SPATTN_TOPK_REG(8);
     SPATTN_TOPK_REG(12);
     SPATTN_TOPK_REG(18);
+    SPATTN_TOPK_REG(19);
 #undef SPATTN_TOPK_REG
   }
   int grid = (rows + 3) / 4;

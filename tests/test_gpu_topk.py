@@ -99,6 +99,22 @@ def test_topk_rows_longer_than_the_register_path(dev):
     assert np.array_equal(kvi[0, 0, rows, :select_k], want_sel)
 
 
+@pytest.mark.parametrize("S,select_k,ties", [(73729, 5900, False), (75600, 6048, False), (77824, 77000, False), (77823, 77822, True),
+                                             (77825, 300, False)])
+def test_topk_longest_rows_of_the_register_path(dev, S, select_k, ties):
+    """19 vectors per lane, more keys ahead of the last wave than 16 bits count: above the threshold, and all of
+    them equal (the lowest keys win); one key more takes the select that re-reads its row."""
+    print("case topk longest register rows", S, select_k, ties, flush=True)
+    q, k, _ = wl.randn_qkv(1, 1, S, 64, seed=S)
+    if ties:
+        k = torch.ones_like(k)
+    kvi, kvn, score, _, fill = _run(dev, q, k, select_k, 128)
+    rows = [0, 300, orc.ceil_div(S, 128) - 1]
+    assert np.all(kvn == select_k)
+    assert np.array_equal(kvi[0, 0, rows, :select_k], orc.topk_select(score[0, 0, rows, :S], select_k))
+    assert np.all(kvi[0, 0, :, select_k:] == fill)
+
+
 def test_topk_select_ties_and_wide_rows(dev):
     """Constant keys give equal scores everywhere: the lowest keys win; a second head with
     two score levels checks the boundary between the levels."""
