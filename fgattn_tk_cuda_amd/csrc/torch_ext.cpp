@@ -12,6 +12,7 @@
 #include <ATen/hip/HIPGraphsUtils.cuh>
 #include <torch/extension.h>
 
+#include <algorithm>
 #include <mutex>
 #include <vector>
 
@@ -78,6 +79,9 @@ int checked_kv_len(int64_t kv_len, const torch::Tensor& q) {
 
 }  // namespace
 
+// Work orders that sp_attn keeps for these counts are computed again (defined with them, below).
+static void counts_written(const torch::Tensor& counts);
+
 void full_attn_ex(torch::Tensor o, OptTensor lse, torch::Tensor q, torch::Tensor k, torch::Tensor v, double scale,
                   int64_t kv_len) {
   check_bhsd(q, "q", q);
@@ -108,6 +112,7 @@ void all_index_mask(torch::Tensor kv_indices, torch::Tensor kv_num_indices, int6
   check_status(spattn_all_index_mask(kv_indices.data_ptr<int>(), kv_num_indices.data_ptr<int>(), (int)batch, (int)heads,
                                      (int)seqblocks, (int)seq, (int)kv_indices.size(3), cur_stream()),
                "all_index_mask");
+  counts_written(kv_num_indices);
 }
 
 // Token lists.  order: the work order of spattn_qblock_order for these counts, or none.
@@ -144,6 +149,10 @@ static void check_sp_attn_args(torch::Tensor& o, torch::Tensor& q, torch::Tensor
   TORCH_CHECK(kv_num_indices.numel() == q.size(0) * q.size(1) * kv_indices.size(2), "kv_num_indices must have B*H*SB entries");
 }
 
+// Up to one q-block per CU there is nothing to balance, and every workgroup would only wait for its entry: token
+// lists 8 x 4096 x 128 14.8 us without an order, 15.9 with; 4 x 2048 x 128 9.3 / 9.2 (heads of equal density),
+// 10.1 / 10.6 (very different ones).
+constexpr int64_t kNoOrder = 256;
 // The work order for counts of per_head q-blocks per head.  Below kScheduleMin q-blocks all of them are resident
 // at once and the plain longest-first order does.
 constexpr int64_t kScheduleMin = 512;
@@ -156,20 +165,24 @@ static void schedule_into(torch::Tensor& order, const torch::Tensor& counts, int
                "work order");
 }
 
-// Work orders of the reference-named sp_attn, which has no argument to pass one in.  One entry per
-// (device, stream, address and size of the counts tensor); the entry remembers the version counter
-// of the counts it was computed from.  A call that finds its entry with the same version launches
-// the attention kernel and nothing else; a new version recomputes the order into the entry's buffer
-// (same stream, so launches that still read it are ahead in stream order); only the first sight of a
-// counts tensor allocates.  Buffers are never freed or handed to another key, so a launch recorded
-// into a graph keeps a valid pointer.  Any permutation of the q-blocks gives the same result: an
-// entry that outlived its counts tensor (same address, size and version by coincidence) can cost
-// balance, never correctness.
+// Work orders of the reference-named sp_attn, which has no argument to pass one in.  An entry belongs to a
+// device, a stream and a counts tensor, which it recognises by its storage (a weak reference: a tensor that
+// was freed is never taken for another one at the same address), place in it, size and q-blocks per head.  A
+// call that finds its entry launches the attention kernel and nothing else.  The order is computed again, into
+// the entry's buffer, when the counts were written to since: their version counter says so, and the operators
+// of this file that write counts, which do not move that counter, mark the entries themselves
+// (counts_written).  Launches that still read the buffer are ahead in stream order.  An entry goes when its
+// counts do.  A call under stream capture computes its order inside the graph: a replay may run on another
+// stream than the next call that writes an entry's buffer, and its counts may be written by the graph.
+// What is left undetected, writes through raw pointers, by a replayed graph, or by torch to inference tensors, which have
+// no version counter, costs balance: any permutation of the q-blocks gives the same result.
 struct OrderEntry {
   int device;
   void* stream;
+  c10::weak_intrusive_ptr<c10::StorageImpl> storage;
   const void* counts;
   int64_t numel;
+  int64_t per_head;
   int64_t version;
   torch::Tensor order;
 };
@@ -177,9 +190,17 @@ static std::mutex g_order_mu;
 // never destroyed: the tensors must not be released after the HIP runtime has shut down at process exit
 static std::vector<OrderEntry>& g_orders = *new std::vector<OrderEntry>();
 constexpr size_t kMaxOrderEntries = 1024;
+constexpr int64_t kWritten = -1;   // version of an entry whose counts an operator of this file has written
 
 static int64_t counts_version(const torch::Tensor& t) {
   return t.is_inference() ? 0 : (int64_t)t._version();
+}
+
+static void counts_written(const torch::Tensor& counts) {
+  const c10::StorageImpl* st = counts.storage().unsafeGetStorageImpl();
+  std::lock_guard<std::mutex> lock(g_order_mu);
+  for (auto& e : g_orders)
+    if (e.storage._unsafe_get_target() == st) e.version = kWritten;
 }
 
 // The work order for these counts on the current stream; computes it if the cache has none.
@@ -188,13 +209,20 @@ static int64_t counts_version(const torch::Tensor& t) {
 static torch::Tensor cached_qblock_order(const torch::Tensor& counts, int64_t per_head) {
   const int dev = (int)counts.device().index();
   void* stream = cur_stream();
-  const int64_t ver = counts_version(counts);
   auto compute = [&](torch::Tensor& order) { schedule_into(order, counts, per_head, stream); };
-  const bool capturing =
-      c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
+  if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) {
+    torch::Tensor order = torch::empty({counts.numel()}, counts.options());
+    compute(order);
+    return order;
+  }
+  const int64_t ver = counts_version(counts);
+  const c10::StorageImpl* st = counts.storage().unsafeGetStorageImpl();
   std::lock_guard<std::mutex> lock(g_order_mu);
+  g_orders.erase(std::remove_if(g_orders.begin(), g_orders.end(), [](const OrderEntry& e) { return e.storage.expired(); }),
+                 g_orders.end());
   for (auto& e : g_orders) {
-    if (e.device == dev && e.stream == stream && e.counts == counts.data_ptr() && e.numel == counts.numel()) {
+    if (e.device == dev && e.stream == stream && e.storage._unsafe_get_target() == st && e.counts == counts.data_ptr() &&
+        e.numel == counts.numel() && e.per_head == per_head) {
       if (e.version != ver) {
         compute(e.order);
         e.version = ver;
@@ -204,21 +232,36 @@ static torch::Tensor cached_qblock_order(const torch::Tensor& counts, int64_t pe
   }
   torch::Tensor order = torch::empty({counts.numel()}, counts.options());
   compute(order);
-  if (!capturing && g_orders.size() < kMaxOrderEntries)
-    g_orders.push_back(OrderEntry{dev, stream, counts.data_ptr(), counts.numel(), ver, order});
+  if (g_orders.size() < kMaxOrderEntries)
+    g_orders.push_back(OrderEntry{dev, stream, counts.storage().getWeakStorageImpl(), counts.data_ptr(), counts.numel(), per_head, ver,
+                                  order});
   return order;
+}
+
+// The order that sp_attn takes for these counts now, on the current stream; none up to kNoOrder q-blocks.
+static OptTensor sp_attn_work_order(const torch::Tensor& counts, int64_t per_head) {
+  if (counts.numel() <= kNoOrder) return c10::nullopt;
+  return cached_qblock_order(counts, per_head);
+}
+
+OptTensor work_order_of(torch::Tensor counts, int64_t per_head) {
+  TORCH_CHECK(counts.is_cuda() && counts.scalar_type() == at::kInt && counts.is_contiguous(),
+              "counts must be a contiguous int32 device tensor");
+  TORCH_CHECK(per_head > 0, "per_head must be positive");
+  const DeviceGuard guard(counts.device());
+  return sp_attn_work_order(counts, per_head);
 }
 
 void sp_attn(torch::Tensor o, torch::Tensor q, torch::Tensor k, torch::Tensor v, torch::Tensor kv_indices,
              torch::Tensor kv_num_indices) {
   check_sp_attn_args(o, q, k, v, kv_indices, kv_num_indices);
   const DeviceGuard guard(q.device());
-  // Threshold masks give lists of very different lengths: the q-blocks are handed to the
-  // workgroups longest list first (lists within a factor of two of each other keep the default
-  // order).  The order is computed when the counts tensor is first seen or has been written to
-  // since (its version counter); every other call is the attention launch alone.
-  const torch::Tensor order = cached_qblock_order(kv_num_indices, kv_indices.size(2));
-  sp_attn_impl(o, c10::nullopt, q, k, v, kv_indices, kv_num_indices, order.data_ptr<int>(), 0.0, 0);
+  // Threshold masks give lists of very different lengths: the q-blocks are handed to the workgroups in a work
+  // order, computed when the counts tensor is first seen or has been written to since; every other call is the
+  // attention launch alone.
+  const OptTensor order = sp_attn_work_order(kv_num_indices, kv_indices.size(2));
+  sp_attn_impl(o, c10::nullopt, q, k, v, kv_indices, kv_num_indices, order.has_value() ? order->data_ptr<int>() : nullptr, 0.0,
+               0);
 }
 
 // sp_attn with an optional log-sum-exp output, an optional precomputed work order (none: the
@@ -593,6 +636,7 @@ void booleanmask_to_indexmask(torch::Tensor kv_indices, torch::Tensor kv_numindi
                                                booleanmask.data_ptr<int>(), (int)booleanmask.size(0), (int)booleanmask.size(1),
                                                (int)seq, (int)booleanmask.size(2), (int)booleanmask.size(3), cur_stream()),
                "booleanmask_to_indexmask");
+  counts_written(kv_numindices);
 }
 
 // Two operators beyond the reference's seven, for its bit-packed mask cache
@@ -629,6 +673,7 @@ static void packedmask_to_lists(torch::Tensor& kv_indices, torch::Tensor& kv_num
   check_status(run(kv_indices.data_ptr<int>(), kv_numindices.data_ptr<int>(), packed.data_ptr(), (int)packed.size(0),
                    (int)packed.size(1), (int)seq, (int)packed.size(2), (int)packed.size(3) * 8, cur_stream()),
                "packedmask_to_indexmask");
+  counts_written(kv_numindices);
 }
 
 void packedmask_to_indexmask(torch::Tensor kv_indices, torch::Tensor kv_numindices, torch::Tensor packed, int64_t seq) {
@@ -669,6 +714,7 @@ void qk_topkmask_indices(torch::Tensor kv_indices, torch::Tensor kv_numindices, 
                                           (int)blocksz, 0, (int)select_k, (int)score.size(3), (int)kv_indices.size(3),
                                           cur_stream()),
                "qk_topkmask_indices");
+  counts_written(kv_numindices);
 }
 
 // Meta kernels: shapes only, nothing to compute (all ops mutate their arguments in place).
@@ -821,6 +867,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("booleanmask_to_blocklists", &booleanmask_to_blocklists, "vote mask -> KV-block lists");
   m.def("qblock_schedule", &qblock_schedule, "work order by windows of heads, longest list first inside");
   m.def("qblock_order", &qblock_order, "work order, longest list first");
+  m.def("work_order_of", &work_order_of, "the work order that sp_attn takes for these counts, or None");
   m.def("booleanmask_128_blocks", &booleanmask_128_blocks, "threshold sweep over listed key blocks, int32 votes");
   m.def("booleanmask_packed_blocks", &booleanmask_packed_blocks, "threshold sweep over listed key blocks, bit-packed");
   m.def("fullattn_maxq_denom_blockmax", &fullattn_maxq_denom_blockmax, "fullattn_maxq_denom + per-block row maxima");

@@ -1,0 +1,57 @@
+"""GPU: the work order that sp_attn keeps for a counts tensor is that tensor's own: not that of an earlier one whose
+storage was freed and handed out again, not that of other q-blocks per head, and not one from before the counts were
+written, by torch or by an operator of the library."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+N = 640   # q-blocks: more than one per CU, fewer than that have no order
+
+
+def _fresh(ops, counts, per_head):
+    order = torch.empty((counts.numel(),), dtype=torch.int32, device=counts.device)
+    ops.qblock_schedule(order, counts, per_head)
+    return order
+
+
+def _counts(dev, seed):
+    return torch.randint(1, 4000, (1, 8, N // 8), generator=torch.Generator().manual_seed(seed), dtype=torch.int32).to(dev)
+
+
+def test_order_follows_the_counts(dev):
+    from fgattn_tk_cuda_amd.spattn import cuda_attn, mask_utils as mu
+
+    print("case sp_attn order follows the counts", flush=True)
+    ops = torch.ops.cuda_attn
+    want, ptrs = [], []
+    for seed in (1, 2):                                   # the second tensor takes the storage that the first one freed
+        c = _counts(dev, seed)
+        ptrs.append(c.data_ptr())
+        want.append(_fresh(ops, c, N // 8))
+        assert torch.equal(cuda_attn.work_order_of(c, N // 8), want[-1])
+        if seed == 1:
+            del c
+    assert ptrs[0] == ptrs[1] and not torch.equal(*want)
+    assert cuda_attn.work_order_of(c, N // 8).data_ptr() == cuda_attn.work_order_of(c, N // 8).data_ptr()   # kept
+    one_head = cuda_attn.work_order_of(c, N)
+    assert torch.equal(one_head, _fresh(ops, c, N)) and torch.equal(cuda_attn.work_order_of(c, N // 8), want[1])
+    c.copy_(_counts(dev, 3))                              # written by torch
+    assert torch.equal(cuda_attn.work_order_of(c, N // 8), _fresh(ops, c, N // 8))
+    # written by an operator of the library
+    S = 128 * (N // 8)
+    packed = mu.pack(torch.rand((1, 8, N // 8, S), generator=torch.Generator().manual_seed(4)) <
+                     torch.rand((1, 8, N // 8, 1), generator=torch.Generator().manual_seed(5))).to(dev)
+    lists = torch.empty((1, 8, N // 8, S), dtype=torch.int32, device=dev)
+    before = _fresh(ops, c, N // 8)
+    ops.packedmask_to_indexmask(lists, c, packed, S)
+    after = _fresh(ops, c, N // 8)
+    assert not torch.equal(before, after) and torch.equal(cuda_attn.work_order_of(c, N // 8), after)
+
+
+def test_no_order_up_to_one_qblock_per_cu(dev):
+    from fgattn_tk_cuda_amd.spattn import cuda_attn
+
+    print("case sp_attn without an order", flush=True)
+    c = _counts(dev, 6).view(-1)
+    assert cuda_attn.work_order_of(c[:256].contiguous(), 32) is None and cuda_attn.work_order_of(c[:257].contiguous(), 257) is not None
