@@ -55,3 +55,31 @@ def test_no_order_up_to_one_qblock_per_cu(dev):
     print("case sp_attn without an order", flush=True)
     c = _counts(dev, 6).view(-1)
     assert cuda_attn.work_order_of(c[:256].contiguous(), 32) is None and cuda_attn.work_order_of(c[:257].contiguous(), 257) is not None
+
+
+@pytest.mark.parametrize("H,ordered", [(31, False), (32, True)])
+def test_lists_used_once_take_their_own_order(dev, monkeypatch, H, ordered):
+    """Masks derived on every call: from 2048 q-blocks on each call orders its own counts, below none does, and the
+    output is that of the lists in index order."""
+    from fgattn_tk_cuda_amd.spattn import mask_utils as mu, sparseattn_functionals as fn
+
+    print("case lists used once", H, flush=True)
+    S, D, seen = 8192, 64, []
+    order_of = mu.qblock_order_cuda
+    monkeypatch.setattr(mu, "qblock_order_cuda", lambda c: (seen.append(c.clone()), order_of(c))[1])
+    cache = mu.CompressedBitMaskCache([0])
+    for seed in (1, 2):
+        g = torch.Generator(device=dev).manual_seed(seed)
+        q, k, v = (torch.randn((1, H, S, D), generator=g, device=dev).to(torch.bfloat16) for _ in range(3))
+        lists, counts = mu.qk_indexmask_cuda(q, k, 8.0 / S)
+        want = torch.empty_like(q)
+        torch.ops.cuda_attn.sp_attn_ex(want, None, q, k, v, lists, counts, None, 0.0, 0)
+        fn.bitmaskcached_attn_cuda(q, k, v, 0, 0, thresh=8.0 / S, blocksz=128, mask_cache=cache)
+        for call in (lambda: fn.attn_computed_with_sparse_mask_cuda(q, k, v, thresh=8.0 / S, blocksz=128),
+                     lambda: fn.bitmaskcached_attn_cuda(q, k, v, 0, 1, thresh=8.0 / S, blocksz=128, mask_cache=cache)):
+            seen.clear()
+            assert torch.equal(call(), want)
+            assert len(seen) == int(ordered) and all(torch.equal(c, counts) for c in seen)
+    seen.clear()
+    fn.attn_topkmask_cuda(q, k, v, select_k=100, blocksz=128)
+    assert not seen                                       # lists of equal length
