@@ -450,6 +450,8 @@ def packedmask_by_groups(groups, sweep, q, k, max_q, denom, thresh, qblk=BLOCKSZ
     max_q, denom)`` runs the statistics sweep with block maxima over heads lo..hi-1 (its tensors are views of
     those heads); the bits of the group follow from the maxima, whose buffer the next group reuses."""
     B, H, S, D = q.shape
+    # the operators see views over all heads: what they refuse of the whole tensors is refused here
+    torch._check(k.shape == q.shape, lambda: "k must have the shape of q")
     n, sp = B * H, max_q.shape[3]
     packed = torch.empty((B, H, (S + qblk - 1) // qblk, sp // 8), dtype=torch.uint8, device=q.device)
     heads = [t.contiguous().view(1, n, *t.shape[2:]) for t in (q, k, max_q, denom, packed)]

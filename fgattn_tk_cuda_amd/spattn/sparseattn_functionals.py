@@ -118,6 +118,7 @@ def sparse_attn_from_cache_cuda(query, key, value, *args, **kwargs):
 def _dense_and_packedmask(query, key, value, groups, thresh, qblk):
     """Dense attention that also writes the block maxima, and the bit-packed threshold mask per qblk rows taken
     over what can hold a key only, by groups of heads (``mask_utils.head_groups``)."""
+    torch._check(value.shape == query.shape, lambda: "v must have the shape of q")
     query, key, value = _c(query, key, value)
     out = _out_like(query)
     max_q, denom = mask_utils._stats_buffers(query)

@@ -1,4 +1,5 @@
 """Host logic of the one-sweep refresh in groups of heads."""
+import pytest
 import torch
 
 
@@ -13,3 +14,20 @@ def test_head_groups_cover_all_heads_within_half_the_budget():
     assert max(sizes) * per_head <= mu.BLOCKMAX_BUDGET_BYTES // 2 and max(sizes) - min(sizes) <= 1
     assert mu.head_groups(q, True) == [(0, 40)] and mu.head_groups(q, False) is None
     assert mu.head_groups(q, None, 40 * per_head) == [(0, 40)] and mu.head_groups(q, None, per_head) is None
+
+
+@pytest.mark.parametrize("bad", ["k", "v"])
+@pytest.mark.parametrize("shape", [(3, 2, 300, 64), (2, 3, 64, 300), (1, 6, 300, 64), (2, 3, 600, 32)])
+def test_other_shapes_of_as_many_numbers_are_refused(bad, shape):
+    """The refreshes hand the operators views over all heads: k and v of another shape are refused all the same."""
+    from fgattn_tk_cuda_amd.spattn import mask_utils as mu, sparseattn_functionals as fn
+
+    t = {n: torch.empty(shape if n == bad else (2, 3, 300, 64), dtype=torch.bfloat16, device="meta") for n in "qkv"}
+    args = t["q"], t["k"], t["v"], 0, 0
+    with pytest.raises(RuntimeError, match=bad + " must have the shape of q"):
+        fn.cached_attn_cuda(*args, thresh=0.01, blocksz=128, mask_cache=mu.NaiveMaskCache([0]))
+    with pytest.raises(RuntimeError, match=bad + " must have the shape of q"):
+        fn.blockcached_attn_cuda(*args, thresh=0.01, mask_cache=mu.BlockListCache([0]), blockmax_budget_bytes=2 * mu.blockmax_bytes(t["q"]) // 6)
+    if bad == "k":
+        with pytest.raises(RuntimeError, match="k must have the shape of q"):
+            mu.qk_indexmask_cuda(t["q"], t["k"], 0.01)
