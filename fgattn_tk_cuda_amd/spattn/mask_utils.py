@@ -311,14 +311,15 @@ def qk_indexmask_from_maxq_denom_cuda(max_q, denom, q, k, thresh, blocksz=128):
     return bitmask_to_indexmask_cuda(booleanmask, q.shape[2])
 
 
-def qk_indexmask_cuda(q, k, thresh, blocksz=128, onepass=None, fill_tail=True):
+def qk_indexmask_cuda(q, k, thresh, blocksz=128, onepass=None, fill_tail=True, budget_bytes=None):
     """Key lists from the threshold mask (python/spattn/mask_utils.py:306-334): statistics with block maxima,
-    then the lists from those; or, where the maxima of one head are too large (``head_groups``) or with
-    ``onepass=False``, the reference's statistics -> vote mask -> index lists.  The same lists either way.
+    then the lists from those; or, where the maxima of one head are too large for ``budget_bytes``
+    (``head_groups``) or with ``onepass=False``, the reference's statistics -> vote mask -> index lists.  The
+    same lists either way.
     ``fill_tail=False`` leaves the entries behind a count unwritten (a caller that hands the lists to
     ``sp_attn`` and drops them)."""
     assert blocksz == BLOCKSZ
-    groups = head_groups(q, onepass)
+    groups = head_groups(q, onepass, budget_bytes)
     max_q, denom = _stats_buffers(q)
     if groups is None:
         spattn_interface.maxq_denom(max_q, denom, q.contiguous(), k.contiguous())

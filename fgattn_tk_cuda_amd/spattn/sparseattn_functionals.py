@@ -95,9 +95,11 @@ def attn_topkmask_cuda(query, key, value, current_layer=None, ditrun=None, *args
 
 def attn_computed_with_sparse_mask_cuda(query, key, value, *args, **kwargs):
     """Threshold pre-pass on the device, then sparse attention (:62-70).  The lists do not leave the call:
-    what lies behind their counts is not written."""
+    what lies behind their counts is not written.  ``onepass`` and ``blockmax_budget_bytes`` as in
+    ``cached_attn_cuda``."""
     kv_indices, kv_num_indices = mask_utils.qk_indexmask_cuda(query, key, kwargs["thresh"], blocksz=kwargs["blocksz"],
-                                                              fill_tail=False)
+                                                              onepass=kwargs.get("onepass"), fill_tail=False,
+                                                              budget_bytes=kwargs.get("blockmax_budget_bytes"))
     return _sparse_once(query, key, value, kv_indices, kv_num_indices)
 
 

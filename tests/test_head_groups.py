@@ -31,3 +31,22 @@ def test_other_shapes_of_as_many_numbers_are_refused(bad, shape):
     if bad == "k":
         with pytest.raises(RuntimeError, match="k must have the shape of q"):
             mu.qk_indexmask_cuda(t["q"], t["k"], 0.01)
+
+
+def test_masks_of_every_step_keep_to_the_callers_route_and_budget(monkeypatch):
+    """attn_computed_with_sparse_mask_cuda takes the routes that its keywords name, as the refreshes do."""
+    from fgattn_tk_cuda_amd.spattn import mask_utils as mu, sparseattn_functionals as fn
+
+    q = torch.empty((2, 3, 300, 64), dtype=torch.bfloat16, device="meta")
+    per_head, seen = mu.blockmax_bytes(q) // 6, []
+    by_groups = mu.packedmask_by_groups
+    monkeypatch.setattr(mu, "packedmask_by_groups", lambda groups, *a: (seen.append(groups), by_groups(groups, *a))[1])
+
+    def groups(**kw):
+        seen.clear()
+        fn.attn_computed_with_sparse_mask_cuda(q, q, q, thresh=0.01, blocksz=128, **kw)
+        return list(seen)
+
+    assert groups() == groups(onepass=True) == groups(blockmax_budget_bytes=6 * per_head) == [[(0, 6)]]
+    assert groups(blockmax_budget_bytes=4 * per_head) == [[(0, 2), (2, 4), (4, 6)]]
+    assert groups(onepass=False) == groups(blockmax_budget_bytes=per_head) == []
