@@ -46,6 +46,8 @@ _SIGNATURES = {
     "spattn_booleanmask_to_blocklists": (_c_int, [_c_void_p] * 4 + [_c_int] * 6 + [_c_void_p]),
     "spattn_maxq_denom_blockmax": (_c_int, [_c_void_p] * 5 + [_c_int] * 5 + [_c_float, _c_void_p]),
     "spattn_fullattn_maxq_denom_blockmax": (_c_int, [_c_void_p] * 7 + [_c_int] * 5 + [_c_float, _c_void_p]),
+    "spattn_maxq_denom_blockmax_of": (_c_int, [_c_void_p] * 5 + [_c_int] * 5 + [_c_float, _c_int, _c_void_p]),
+    "spattn_fullattn_maxq_denom_blockmax_of": (_c_int, [_c_void_p] * 7 + [_c_int] * 5 + [_c_float, _c_int, _c_void_p]),
     "spattn_blockmax_to_blocklists": (_c_int, [_c_void_p] * 6 + [_c_float] + [_c_int] * 6 + [_c_float, _c_int, _c_void_p]),
     "spattn_blockmax_to_packedmask": (_c_int, [_c_void_p] * 6 + [_c_float] + [_c_int] * 6 + [_c_float, _c_void_p]),
     "spattn_packedmask_to_indexmask_filled": (_c_int, [_c_void_p] * 3 + [_c_int] * 5 + [_c_void_p]),
@@ -332,24 +334,25 @@ def _need_blockmax(blockmax, B, H, S):
         raise ValueError("blockmax must be bf16 [B,H,%d,%d]" % (sp // 64, sp))
 
 
-def maxq_denom_blockmax(max_q, denom, blockmax, q, k, *, kv_len=0, scale=0.0, stream=None):
+def maxq_denom_blockmax(max_q, denom, blockmax, q, k, *, kv_len=0, scale=0.0, of_heads=0, stream=None):
     """maxq_denom that also writes blockmax bf16 [B,H,Sp/64,Sp] (rounded toward +inf): [J][r] = max of q[r].k[c] over the keys c < kv_len
-    of 64-key block J (blocks without such a key are left as they are)."""
+    of 64-key block J (blocks without such a key are left as they are).  of_heads: B*H of the computation that the call is
+    a part of (0: it is the whole); the results are the same bits as in one call over all of those heads."""
     B, H, S, D = _bhsd(q)
     _need_padded(max_q, denom, B, H, S)
     _need_blockmax(blockmax, B, H, S)
-    _check(load().spattn_maxq_denom_blockmax(_ptr(max_q, f32), _ptr(denom, f32), _ptr(blockmax, bf16), _ptr(q, bf16),
-                                             _ptr(k, bf16), B, H, S, D, kv_len, scale, _stream(stream)))
+    _check(load().spattn_maxq_denom_blockmax_of(_ptr(max_q, f32), _ptr(denom, f32), _ptr(blockmax, bf16), _ptr(q, bf16),
+                                                _ptr(k, bf16), B, H, S, D, kv_len, scale, int(of_heads), _stream(stream)))
 
 
-def fullattn_maxq_denom_blockmax(o, max_q, denom, blockmax, q, k, v, *, kv_len=0, scale=0.0, stream=None):
-    """fullattn_maxq_denom with the blockmax output of maxq_denom_blockmax."""
+def fullattn_maxq_denom_blockmax(o, max_q, denom, blockmax, q, k, v, *, kv_len=0, scale=0.0, of_heads=0, stream=None):
+    """fullattn_maxq_denom with the blockmax output (and the of_heads) of maxq_denom_blockmax."""
     B, H, S, D = _bhsd(q)
     _need_padded(max_q, denom, B, H, S)
     _need_blockmax(blockmax, B, H, S)
-    _check(load().spattn_fullattn_maxq_denom_blockmax(_ptr(o, bf16), _ptr(max_q, f32), _ptr(denom, f32),
-                                                      _ptr(blockmax, bf16), _ptr(q, bf16), _ptr(k, bf16), _ptr(v, bf16),
-                                                      B, H, S, D, kv_len, scale, _stream(stream)))
+    _check(load().spattn_fullattn_maxq_denom_blockmax_of(_ptr(o, bf16), _ptr(max_q, f32), _ptr(denom, f32),
+                                                         _ptr(blockmax, bf16), _ptr(q, bf16), _ptr(k, bf16), _ptr(v, bf16),
+                                                         B, H, S, D, kv_len, scale, int(of_heads), _stream(stream)))
 
 
 def blockmax_to_blocklists(blk_indices, blk_counts, blockmax, max_q, denom, threshold, seq, D, *, qblk=128,

@@ -14,30 +14,32 @@ namespace spattn {
 //   (24 x 1536 27.0 -> 23.5 us), with statistics 1.02-1.07x, statistics only 1.02-1.12x.  At 256 and 512 keys that
 //   is 0.92-1.08x, behind 768 q-blocks 0.88-0.93x (64 x 1000 21.9 -> 24.3 us).  d = 128 loses 0.81-0.99x (with
 //   statistics 0.65-0.83x, its LDS allows one workgroup per CU) from the second q-block per CU on.
-static bool small_launch(const AttnParams& p, int D) {
+// The two forms add the row sums and outputs of a row in another order: a launch over some heads of a computation
+// goes by all of its heads, so that a row's denominator, and with it a key at a threshold, does not depend on the split.
+static bool small_launch(const AttnParams& p, int D, int heads) {
   constexpr int kCus = 256;
-  const long long n64 = (long long)p.B * p.H * ((p.S + 63) / 64);
+  const long long n64 = (long long)(heads > 0 ? heads : p.B * p.H) * ((p.S + 63) / 64);
   return n64 <= kCus || (D == 64 && p.kv_len >= 768 && n64 <= 3 * kCus);
 }
 
 template <int D, bool HAS_V, bool STATS>
-static hipError_t run(const AttnParams& p, hipStream_t stream) {
-  if (!small_launch(p, D)) return launch_attn_fwd<D, 128, KV_DENSE, HAS_V, STATS>(p, stream);
+static hipError_t run(const AttnParams& p, int heads, hipStream_t stream) {
+  if (!small_launch(p, D, heads)) return launch_attn_fwd<D, 128, KV_DENSE, HAS_V, STATS>(p, stream);
   AttnParams p64 = p;
   // the statistics cover the rows up to Sp
   p64.nqblk = (STATS ? p.Sp : p.S + 63) / 64;
   return launch_attn_fwd<D, 64, KV_DENSE, HAS_V, STATS>(p64, stream);
 }
 
-hipError_t run_attn_dense(const AttnParams& p, int D, bool has_v, bool stats, hipStream_t stream) {
+hipError_t run_attn_dense(const AttnParams& p, int D, bool has_v, bool stats, hipStream_t stream, int heads) {
   if (D == 128) {
-    if (has_v && !stats) return run<128, true, false>(p, stream);
-    if (has_v && stats) return run<128, true, true>(p, stream);
-    if (!has_v && stats) return run<128, false, true>(p, stream);
+    if (has_v && !stats) return run<128, true, false>(p, heads, stream);
+    if (has_v && stats) return run<128, true, true>(p, heads, stream);
+    if (!has_v && stats) return run<128, false, true>(p, heads, stream);
   } else if (D == 64) {
-    if (has_v && !stats) return run<64, true, false>(p, stream);
-    if (has_v && stats) return run<64, true, true>(p, stream);
-    if (!has_v && stats) return run<64, false, true>(p, stream);
+    if (has_v && !stats) return run<64, true, false>(p, heads, stream);
+    if (has_v && stats) return run<64, true, true>(p, heads, stream);
+    if (!has_v && stats) return run<64, false, true>(p, heads, stream);
   }
   return hipErrorInvalidValue;
 }

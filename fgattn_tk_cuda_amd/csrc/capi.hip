@@ -126,25 +126,38 @@ int spattn_maxq_denom(float* max_q, float* denom, const void* q, const void* k, 
 
 int spattn_fullattn_maxq_denom_blockmax(void* o, float* max_q, float* denom, void* blockmax, const void* q, const void* k,
                                         const void* v, int B, int H, int S, int D, int kv_len, float scale, void* stream) {
+  return spattn_fullattn_maxq_denom_blockmax_of(o, max_q, denom, blockmax, q, k, v, B, H, S, D, kv_len, scale, 0, stream);
+}
+
+int spattn_fullattn_maxq_denom_blockmax_of(void* o, float* max_q, float* denom, void* blockmax, const void* q, const void* k,
+                                           const void* v, int B, int H, int S, int D, int kv_len, float scale, int of_heads,
+                                           void* stream) {
   if (int st = check_qkv(q, k, B, H, S, D)) return done(st);
+  if (of_heads != 0 && of_heads < B * H) return done(SPATTN_ERR_SHAPE);
   if (!o || !v || !max_q || !denom || !blockmax) return done(SPATTN_ERR_NULL);
   if (misaligned(o) || misaligned(v)) return done(SPATTN_ERR_ALIGN);
   spattn::AttnParams p = base_params(q, k, v, o, B, H, S, D, kv_len, scale, 128);
   p.max_q = max_q;
   p.denom = denom;
   p.blockmax = static_cast<uint16_t*>(blockmax);
-  return from_hip(spattn::run_attn_dense(p, D, true, true, as_stream(stream)));
+  return from_hip(spattn::run_attn_dense(p, D, true, true, as_stream(stream), of_heads));
 }
 
 int spattn_maxq_denom_blockmax(float* max_q, float* denom, void* blockmax, const void* q, const void* k, int B, int H,
                                int S, int D, int kv_len, float scale, void* stream) {
+  return spattn_maxq_denom_blockmax_of(max_q, denom, blockmax, q, k, B, H, S, D, kv_len, scale, 0, stream);
+}
+
+int spattn_maxq_denom_blockmax_of(float* max_q, float* denom, void* blockmax, const void* q, const void* k, int B, int H,
+                                  int S, int D, int kv_len, float scale, int of_heads, void* stream) {
   if (int st = check_qkv(q, k, B, H, S, D)) return done(st);
+  if (of_heads != 0 && of_heads < B * H) return done(SPATTN_ERR_SHAPE);
   if (!max_q || !denom || !blockmax) return done(SPATTN_ERR_NULL);
   spattn::AttnParams p = base_params(q, k, nullptr, nullptr, B, H, S, D, kv_len, scale, 128);
   p.max_q = max_q;
   p.denom = denom;
   p.blockmax = static_cast<uint16_t*>(blockmax);
-  return from_hip(spattn::run_attn_dense(p, D, false, true, as_stream(stream)));
+  return from_hip(spattn::run_attn_dense(p, D, false, true, as_stream(stream), of_heads));
 }
 
 int spattn_blockmax_to_blocklists(int* blk_indices, int* blk_counts, void* blockmask, const void* blockmax,

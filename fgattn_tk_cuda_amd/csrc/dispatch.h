@@ -7,7 +7,8 @@ namespace spattn {
 // attn_inst_tokens.hip / attn_inst_blocks.hip / attn_inst_dense.hip
 hipError_t run_attn_tokens(const AttnParams& p, int D, int qblk, hipStream_t stream);
 hipError_t run_attn_blocks(const AttnParams& p, int D, int qblk, hipStream_t stream);
-hipError_t run_attn_dense(const AttnParams& p, int D, bool has_v, bool stats, hipStream_t stream);
+// heads: of the whole computation where the launch is a part of one, 0: those of the launch
+hipError_t run_attn_dense(const AttnParams& p, int D, bool has_v, bool stats, hipStream_t stream, int heads = 0);
 // every instantiation's dynamic-LDS limit on the current device (idempotent)
 hipError_t prepare_attn_tokens();
 hipError_t prepare_attn_blocks();

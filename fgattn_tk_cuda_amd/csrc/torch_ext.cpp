@@ -380,8 +380,15 @@ void check_blockmax(const torch::Tensor& blockmax, const torch::Tensor& q_like, 
   TORCH_CHECK(blockmax.numel() == B * H * (sp / 64) * sp, "blockmax must be bf16 [B,H,Sp/64,Sp] with Sp = 128*ceil(S/128)");
 }
 
-void fullattn_maxq_denom_blockmax(torch::Tensor o, torch::Tensor o_max_q, torch::Tensor o_denom, torch::Tensor blockmax,
-                                  torch::Tensor q, torch::Tensor k, torch::Tensor v, double scale, int64_t kv_len) {
+// of_heads: B*H of the computation that these heads are a part of (0: the call is the whole).
+int checked_of_heads(int64_t of_heads, const torch::Tensor& q) {
+  TORCH_CHECK(of_heads == 0 || (of_heads >= q.size(0) * q.size(1) && of_heads <= INT32_MAX), "of_heads must be 0 or at least B*H");
+  return (int)of_heads;
+}
+
+void fullattn_maxq_denom_blockmax_of(torch::Tensor o, torch::Tensor o_max_q, torch::Tensor o_denom, torch::Tensor blockmax,
+                                     torch::Tensor q, torch::Tensor k, torch::Tensor v, double scale, int64_t kv_len,
+                                     int64_t of_heads) {
   check_bhsd(q, "q", q);
   check_bhsd(k, "k", q);
   check_bhsd(v, "v", q);
@@ -392,15 +399,21 @@ void fullattn_maxq_denom_blockmax(torch::Tensor o, torch::Tensor o_max_q, torch:
   TORCH_CHECK(o_max_q.numel() == need && o_denom.numel() == need, "o_max_q / o_denom must be [B,H,1,128*ceil(S/128)]");
   check_blockmax(blockmax, q, q.size(0), q.size(1), q.size(2));
   const DeviceGuard guard(q.device());
-  check_status(spattn_fullattn_maxq_denom_blockmax(o.data_ptr(), o_max_q.data_ptr<float>(), o_denom.data_ptr<float>(),
-                                                   blockmax.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                                                   (int)q.size(0), (int)q.size(1), (int)q.size(2), (int)q.size(3),
-                                                   checked_kv_len(kv_len, q), (float)scale, cur_stream()),
+  check_status(spattn_fullattn_maxq_denom_blockmax_of(o.data_ptr(), o_max_q.data_ptr<float>(), o_denom.data_ptr<float>(),
+                                                      blockmax.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                                                      (int)q.size(0), (int)q.size(1), (int)q.size(2), (int)q.size(3),
+                                                      checked_kv_len(kv_len, q), (float)scale, checked_of_heads(of_heads, q),
+                                                      cur_stream()),
                "fullattn_maxq_denom_blockmax");
 }
 
-void maxq_denom_blockmax(torch::Tensor o_max_q, torch::Tensor o_denom, torch::Tensor blockmax, torch::Tensor q,
-                         torch::Tensor k, double scale, int64_t kv_len) {
+void fullattn_maxq_denom_blockmax(torch::Tensor o, torch::Tensor o_max_q, torch::Tensor o_denom, torch::Tensor blockmax,
+                                  torch::Tensor q, torch::Tensor k, torch::Tensor v, double scale, int64_t kv_len) {
+  fullattn_maxq_denom_blockmax_of(o, o_max_q, o_denom, blockmax, q, k, v, scale, kv_len, 0);
+}
+
+void maxq_denom_blockmax_of(torch::Tensor o_max_q, torch::Tensor o_denom, torch::Tensor blockmax, torch::Tensor q,
+                            torch::Tensor k, double scale, int64_t kv_len, int64_t of_heads) {
   check_bhsd(q, "q", q);
   check_bhsd(k, "k", q);
   check_aux(o_max_q, "o_max_q", at::kFloat, q);
@@ -409,10 +422,16 @@ void maxq_denom_blockmax(torch::Tensor o_max_q, torch::Tensor o_denom, torch::Te
   TORCH_CHECK(o_max_q.numel() == need && o_denom.numel() == need, "o_max_q / o_denom must be [B,H,1,128*ceil(S/128)]");
   check_blockmax(blockmax, q, q.size(0), q.size(1), q.size(2));
   const DeviceGuard guard(q.device());
-  check_status(spattn_maxq_denom_blockmax(o_max_q.data_ptr<float>(), o_denom.data_ptr<float>(), blockmax.data_ptr(),
-                                          q.data_ptr(), k.data_ptr(), (int)q.size(0), (int)q.size(1), (int)q.size(2),
-                                          (int)q.size(3), checked_kv_len(kv_len, q), (float)scale, cur_stream()),
+  check_status(spattn_maxq_denom_blockmax_of(o_max_q.data_ptr<float>(), o_denom.data_ptr<float>(), blockmax.data_ptr(),
+                                             q.data_ptr(), k.data_ptr(), (int)q.size(0), (int)q.size(1), (int)q.size(2),
+                                             (int)q.size(3), checked_kv_len(kv_len, q), (float)scale,
+                                             checked_of_heads(of_heads, q), cur_stream()),
                "maxq_denom_blockmax");
+}
+
+void maxq_denom_blockmax(torch::Tensor o_max_q, torch::Tensor o_denom, torch::Tensor blockmax, torch::Tensor q,
+                         torch::Tensor k, double scale, int64_t kv_len) {
+  maxq_denom_blockmax_of(o_max_q, o_denom, blockmax, q, k, scale, kv_len, 0);
 }
 
 // blk_idx int32 [B,H,ceil(seq/qblk),max_blocks], blk_cnt int32 with B*H*ceil(seq/qblk) entries,
@@ -742,8 +761,8 @@ void noop_mask_blocks(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor
 void noop_mask_packed_blocks(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
                              double, int64_t, double, int64_t) {}
 void noop_fmd_bm(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, double,
-                 int64_t) {}
-void noop_md_bm(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, double, int64_t) {}
+                 int64_t, int64_t) {}
+void noop_md_bm(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, double, int64_t, int64_t) {}
 void noop_bm_lists(torch::Tensor, torch::Tensor, OptTensor, torch::Tensor, torch::Tensor, torch::Tensor, double, int64_t, int64_t,
                    int64_t, double, int64_t) {}
 
@@ -775,8 +794,8 @@ TORCH_LIBRARY_FRAGMENT(cuda_attn, m) {
   m.def("qblock_schedule(Tensor(a!) order, Tensor counts, int per_head) -> ()");
   m.def("booleanmask_128_blocks(Tensor(a!) booleanmask, Tensor o_max_q, Tensor o_denom, Tensor q, Tensor k, Tensor blk_idx, Tensor blk_cnt, float threshold, float scale, int kv_len) -> ()");
   m.def("booleanmask_packed_blocks(Tensor(a!) packed, Tensor o_max_q, Tensor o_denom, Tensor q, Tensor k, Tensor blk_idx, Tensor blk_cnt, float threshold, int qblk, float scale, int kv_len) -> ()");
-  m.def("fullattn_maxq_denom_blockmax(Tensor(a!) o, Tensor(b!) o_max_q, Tensor(c!) o_denom, Tensor(d!) blockmax, Tensor q, Tensor k, Tensor v, float scale, int kv_len) -> ()");
-  m.def("maxq_denom_blockmax(Tensor(a!) o_max_q, Tensor(b!) o_denom, Tensor(c!) blockmax, Tensor q, Tensor k, float scale, int kv_len) -> ()");
+  m.def("fullattn_maxq_denom_blockmax(Tensor(a!) o, Tensor(b!) o_max_q, Tensor(c!) o_denom, Tensor(d!) blockmax, Tensor q, Tensor k, Tensor v, float scale, int kv_len, int of_heads=0) -> ()");
+  m.def("maxq_denom_blockmax(Tensor(a!) o_max_q, Tensor(b!) o_denom, Tensor(c!) blockmax, Tensor q, Tensor k, float scale, int kv_len, int of_heads=0) -> ()");
   m.def("blockmax_to_blocklists(Tensor(a!) blk_idx, Tensor(b!) blk_cnt, Tensor(c!)? blockmask, Tensor blockmax, Tensor o_max_q, Tensor o_denom, float threshold, int seq, int head_dim, int qblk, float scale, int kv_len) -> ()");
   m.def("blockmax_to_packedmask(Tensor(a!) packed, Tensor blockmax, Tensor o_max_q, Tensor o_denom, Tensor q, Tensor k, float threshold, float scale, int kv_len) -> ()");
   m.def("packedmask_to_indexmask_filled(Tensor(a!) kv_indices, Tensor(b!) kv_numindices, Tensor packed, int seq) -> ()");
@@ -838,8 +857,8 @@ TORCH_LIBRARY_IMPL(cuda_attn, CUDA, m) {
   m.impl("qblock_schedule", qblock_schedule);
   m.impl("booleanmask_128_blocks", booleanmask_128_blocks);
   m.impl("booleanmask_packed_blocks", booleanmask_packed_blocks);
-  m.impl("fullattn_maxq_denom_blockmax", fullattn_maxq_denom_blockmax);
-  m.impl("maxq_denom_blockmax", maxq_denom_blockmax);
+  m.impl("fullattn_maxq_denom_blockmax", fullattn_maxq_denom_blockmax_of);
+  m.impl("maxq_denom_blockmax", maxq_denom_blockmax_of);
   m.impl("blockmax_to_blocklists", blockmax_to_blocklists);
   m.impl("blockmax_to_packedmask", blockmax_to_packedmask);
   m.impl("packedmask_to_indexmask_filled", packedmask_to_indexmask_filled);

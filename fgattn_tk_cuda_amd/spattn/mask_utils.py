@@ -326,7 +326,7 @@ def qk_indexmask_cuda(q, k, thresh, blocksz=128, onepass=None, fill_tail=True, b
         return qk_indexmask_from_maxq_denom_cuda(max_q, denom, q, k, thresh, blocksz)
 
     def sweep(lo, hi, blockmax, q_, k_, max_q_, denom_):
-        spattn_interface.maxq_denom_blockmax(max_q_, denom_, blockmax, q_, k_, 0.0, 0)
+        spattn_interface.maxq_denom_blockmax(max_q_, denom_, blockmax, q_, k_, 0.0, 0, q.shape[0] * q.shape[1])
 
     return packedmask_to_indexmask_cuda(packedmask_by_groups(groups, sweep, q, k, max_q, denom, thresh), q.shape[2], fill_tail)
 

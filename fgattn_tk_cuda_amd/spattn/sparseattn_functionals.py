@@ -128,7 +128,7 @@ def _dense_and_packedmask(query, key, value, groups, thresh, qblk):
     o_, v_ = out.view(1, B * H, S, D), value.view(1, B * H, S, D)
 
     def sweep(lo, hi, blockmax, qs, ks, ms, ds):
-        spattn_interface.fullattn_maxq_denom_blockmax(o_[:, lo:hi], ms, ds, blockmax, qs, ks, v_[:, lo:hi], 0.0, 0)
+        spattn_interface.fullattn_maxq_denom_blockmax(o_[:, lo:hi], ms, ds, blockmax, qs, ks, v_[:, lo:hi], 0.0, 0, B * H)
 
     return out, mask_utils.packedmask_by_groups(groups, sweep, query, key, max_q, denom, thresh, qblk)
 

@@ -182,6 +182,14 @@ int spattn_maxq_denom_blockmax(float* max_q, float* denom, void* blockmax, const
 int spattn_fullattn_maxq_denom_blockmax(void* o, float* max_q, float* denom, void* blockmax, const void* q, const void* k,
                                         const void* v, int batch, int heads, int seq, int D, int kv_len, float scale,
                                         void* stream);
+/* The same sweeps over some of the of_heads (batch x heads) of one computation: the size of the whole decides how the
+ * rows are split, so max_q, denom, blockmax and o are the same bits as in one call over all of its heads.  of_heads = 0:
+ * the call is the whole; otherwise not below batch * heads. */
+int spattn_maxq_denom_blockmax_of(float* max_q, float* denom, void* blockmax, const void* q, const void* k, int batch,
+                                  int heads, int seq, int D, int kv_len, float scale, int of_heads, void* stream);
+int spattn_fullattn_maxq_denom_blockmax_of(void* o, float* max_q, float* denom, void* blockmax, const void* q,
+                                           const void* k, const void* v, int batch, int heads, int seq, int D, int kv_len,
+                                           float scale, int of_heads, void* stream);
 int spattn_blockmax_to_blocklists(int* blk_indices, int* blk_counts, void* blockmask, const void* blockmax,
                                   const float* max_q, const float* denom, float threshold, int qblk, int batch, int heads,
                                   int seq, int D, int kv_len, float scale, int max_blocks, void* stream);

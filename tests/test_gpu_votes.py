@@ -85,3 +85,36 @@ def test_block_refresh_in_groups_of_heads(dev, S, D, qblk):
     for other in got[1:]:
         assert all(torch.equal(a, b) for a, b in zip(got[0], other))
     assert int(got[0][2].sum()) > 0
+
+
+@pytest.mark.parametrize("H,S,D", [(16, 2000, 128), (26, 2000, 64), (40, 1400, 64), (9, 1990, 128)])
+def test_groups_take_the_form_of_the_whole(dev, H, S, D):
+    """Heads whose launch as a whole takes 128-row q-blocks, in groups small enough for 64-row ones: output, statistics and
+    lists are the bits of all heads at once."""
+    from fgattn_tk_cuda_amd.spattn import mask_utils as mu, sparseattn_functionals as fn
+
+    print("case groups of the whole", H, S, D, flush=True)
+    ops = torch.ops.cuda_attn
+    g = torch.Generator(device=dev).manual_seed(S + H)
+    q, k, v = (torch.randn((1, H, S, D), generator=g, device=dev).to(torch.bfloat16) for _ in range(3))
+    per_head = mu.blockmax_bytes(q) // H
+    kw = [dict(onepass=True), dict(onepass=False), dict(blockmax_budget_bytes=4 * per_head)]
+    got = []
+    for route in kw:
+        cache = mu.NaiveMaskCache([0])
+        out = fn.cached_attn_cuda(q, k, v, 0, 0, thresh=8.0 / S, blocksz=128, mask_cache=cache, **route)
+        got.append((out,) + tuple(cache.get_mask_from_cache(0)))
+    for other in got[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(got[0], other))
+    one = [mu.qk_indexmask_cuda(q, k, 8.0 / S, onepass=r.get("onepass"), budget_bytes=r.get("blockmax_budget_bytes")) for r in kw]
+    assert all(torch.equal(a, b) for other in one[1:] for a, b in zip(one[0], other))
+    m, d = mu._stats_buffers(q)
+    ops.maxq_denom_blockmax(m, d, mu.blockmax_buffer(q), q, k, 0.0, 0)
+    some = q[:, 2:4].contiguous(), k[:, 2:4].contiguous()
+    ms, ds = mu._stats_buffers(some[0])
+    ops.maxq_denom_blockmax(ms, ds, mu.blockmax_buffer(some[0]), *some, 0.0, 0, H)
+    assert torch.equal(ms, m[:, 2:4]) and torch.equal(ds, d[:, 2:4])
+    ops.maxq_denom_blockmax(ms, ds, mu.blockmax_buffer(some[0]), *some, 0.0, 0)
+    assert torch.equal(ms, m[:, 2:4]) and not torch.equal(ds, d[:, 2:4])   # a launch of its own: another order of the sums
+    with pytest.raises(RuntimeError):
+        ops.maxq_denom_blockmax(ms, ds, mu.blockmax_buffer(some[0]), *some, 0.0, 0, 1)
