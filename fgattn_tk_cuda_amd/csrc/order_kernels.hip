@@ -8,6 +8,8 @@
 // Lists whose lengths differ by less than a factor of two keep the default order, in which every XCD works on
 // neighbouring q-blocks of one head.  The reference has no counterpart: its grid is fixed
 // to (q-block, head, batch) (include/sparseattn_asyncgatherload_padded.cuh:273).
+#include <type_traits>
+
 #include "common.h"
 #include "dispatch.h"
 
@@ -128,34 +130,42 @@ __global__ __launch_bounds__(kOrderThreads) void qblock_order_kernel(int* __rest
 // XCD's 64 workgroup slots, a late window would end with it alone, and the share is one window (Zipf lists
 // 24 x 20000 x 64, 0.5 of a slot's work: 0.389 instead of 0.417 ms); and where the shares differ by more than
 // kSkew, the sort over everything balances the XCDs (shares within 1.09 of each other still gain by the windows).
-// The kernel takes 7 us for 6144 q-blocks (qblock_order_kernel: 20; classes of a sixteenth of an octave: no gain).
-// One workgroup per XCD, a wave per window; classes of an eighth of an octave over the seven octaves below the
-// longest list, stable, so the order is a function of the counts alone.
+// That is also so where no list is twice as long as another: block lists 32 x 16384 x 128, head densities rising by
+// 1.8 / 1.4: windows and index order 0.981 / 0.780, sorted 0.846 / 0.731 ms; threshold lists 12 x 32760 x 128, largest
+// share 1.28 of the mean: 0.318 and 0.286.  From kCoarse q-blocks on the sort takes quarters of an octave, which keep
+// more neighbours together: 40 x 32760 x 128 1.018 -> 0.984 ms, 40 x 75600 x 128 5.12 -> 4.88; up to 7092 q-blocks no
+// difference.
+// One workgroup per XCD, a wave per window, the sort over everything by one workgroup; classes of an eighth of an
+// octave (a sixteenth: no gain) over the seven octaves below the longest list, stable, so the order is a function of
+// the counts alone.  What bounds it is the chain of loads and LDS updates of a lane's segment: 6.6 us for 6144
+// q-blocks by windows, 16 for 23640, and 15.5 / 42 us for the sort over everything (one wave of one count at a time:
+// 47 / 171; qblock_order_kernel: 20 / 58).
 // ------------------------------------------------------------------------------------
 constexpr int kXcds = 8;
 constexpr int kSlotsPerXcd = 64;
 constexpr int kWindow = 192;
 constexpr float kTail = 0.3f;
 constexpr float kSkew = 1.1f;
+constexpr int kCoarse = 8192;
 constexpr int kSchedSub = 3;
 constexpr int kSchedOctaves = 7;
 constexpr int kSchedClasses = (kSchedOctaves << kSchedSub) + 4;   // a multiple of 4: a lane reads its table entries 16 bytes at a time
 
-// 0 holds the longest lists; top: floor(log2) of the longest of all
-__device__ __forceinline__ int schedule_class(int c, int top) {
+// 0 holds the longest lists; top: floor(log2) of the longest of all; coarse: 1 for quarters of an octave
+__device__ __forceinline__ int schedule_class(int c, int top, int coarse) {
   if (c <= 0) return kSchedClasses - 1;
   const int lg = 31 - __builtin_clz((unsigned)c);
   const int below = lg >= kSchedSub ? ((c >> (lg - kSchedSub)) & ((1 << kSchedSub) - 1))
                                     : ((c << (kSchedSub - lg)) & ((1 << kSchedSub) - 1));
   const int cls = ((top - lg) << kSchedSub) + ((1 << kSchedSub) - 1 - below);
-  return cls < kSchedClasses - 2 ? cls : kSchedClasses - 2;
+  return cls < kSchedClasses - 2 ? cls >> coarse : kSchedClasses - 2;
 }
 
 __global__ __launch_bounds__(256) void qblock_schedule_kernel(int* __restrict__ order, const int* __restrict__ counts, int n,
                                                               int per_head) {
-  __shared__ __attribute__((aligned(16))) int tables[4][kSchedClasses * 64];   // [wave][class][lane]
+  __shared__ __attribute__((aligned(16))) int tables[4][kSchedClasses * 64];   // [wave][class][lane], or all of it [class][thread]
   __shared__ float share_l[kXcds];
-  __shared__ int longest_l[4];
+  __shared__ int longest_l[4], wave_sum[4];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int x = blockIdx.x;
@@ -204,36 +214,61 @@ __global__ __launch_bounds__(256) void qblock_schedule_kernel(int* __restrict__ 
   for (int i = kXcds * per; i < n; ++i) longest_all = counts[i] > longest_all ? counts[i] : longest_all;
   const int top = 31 - __builtin_clz((unsigned)(longest_all > 0 ? longest_all : 1));
   const bool global = most * kXcds > kSkew * total;
+  const int coarse = global && n >= kCoarse ? 1 : 0;
   const bool one_window = (float)longest * kSlotsPerXcd > kTail * share_l[x];
-  int* const table = tables[wave];
 
-  // Stable counting sort of q-blocks a .. b-1 by class, one wave; the entry of rank r goes to
-  // order[first + r * step].  A lane owns a contiguous segment.  A wave's LDS operations execute in order.
-  auto sort = [&](int a, int b, int first, int step) {
+  // Stable counting sort of q-blocks a .. b-1 by class, by one wave or (ALL) by the workgroup; the entry of rank r
+  // goes to order[first + r * step].  A lane owns a contiguous segment and has eight of its counts in flight.  A
+  // wave's LDS operations execute in order.
+  auto sort = [&](auto all, int a, int b, int first, int step) {
+    constexpr bool ALL = decltype(all)::value;
+    constexpr int L = ALL ? 256 : 64, U = 8;
+    const int id = ALL ? (int)threadIdx.x : lane;
+    int* const table = tables[ALL ? 0 : wave];
     auto settle = [] {
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
+      if constexpr (ALL) {
+        __syncthreads();
+      } else {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      }
     };
-    for (int i = 4 * lane; i < kSchedClasses * 64; i += 256) {
+    for (int i = 4 * id; i < kSchedClasses * L; i += 4 * L) {
       const i32x4 z = {0, 0, 0, 0};
       *reinterpret_cast<i32x4*>(table + i) = z;
     }
-    const int seg = (b - a + 63) / 64;
-    const int i0 = a + lane * seg < b ? a + lane * seg : b;
+    const int seg = (b - a + L - 1) / L;
+    const int i0 = a + id * seg < b ? a + id * seg : b;
     const int i1 = i0 + seg < b ? i0 + seg : b;
+    auto walk = [&](auto&& f) {
+      for (int i = i0; i < i1; i += U) {
+        int c[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) c[u] = i + u < i1 ? counts[i + u] : 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (i + u < i1) f(i + u, schedule_class(c[u], top, coarse) * L + id);
+      }
+    };
     settle();
-    for (int i = i0; i < i1; ++i) table[schedule_class(counts[i], top) * 64 + lane] += 1;
+    walk([&](int, int slot) { table[slot] += 1; });
     settle();
     // exclusive prefix sum in storage order (class-major, lane-minor): lane l scans kSchedClasses entries from
     // l * kSchedClasses on
     int sum = 0;
-    i32x4* const own = reinterpret_cast<i32x4*>(table + lane * kSchedClasses);
+    i32x4* const own = reinterpret_cast<i32x4*>(table + id * kSchedClasses);
 #pragma unroll
     for (int j = 0; j < kSchedClasses / 4; ++j) {
       const i32x4 v = own[j];
       sum += v[0] + v[1] + v[2] + v[3];
     }
     int run = (int)lane_scan((uint32_t)sum) - sum;
+    if constexpr (ALL) {
+      if (lane == 63) wave_sum[wave] = run + sum;
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < 3; ++w) run += w < wave ? wave_sum[w] : 0;
+    }
 #pragma unroll
     for (int j = 0; j < kSchedClasses / 4; ++j) {
       const i32x4 v = own[j];
@@ -246,17 +281,16 @@ __global__ __launch_bounds__(256) void qblock_schedule_kernel(int* __restrict__ 
       own[j] = o;
     }
     settle();
-    for (int i = i0; i < i1; ++i) {
-      const int slot = schedule_class(counts[i], top) * 64 + lane;
+    walk([&](int i, int slot) {
       const int r = table[slot];
       order[(size_t)first + (size_t)r * step] = i;
       table[slot] = r + 1;
-    }
+    });
     settle();
   };
 
   if (global) {
-    if (x == 0 && wave == 0) sort(0, n, 0, 1);
+    if (x == 0) sort(std::true_type{}, 0, n, 0, 1);
     return;
   }
   const int end = (x + 1) * per;
@@ -268,7 +302,7 @@ __global__ __launch_bounds__(256) void qblock_schedule_kernel(int* __restrict__ 
       if (b - a < kWindow) b += (kWindow - (b - a) + per_head - 1) / per_head * per_head;
       b = b < end ? b : end;
     }
-    if ((turn & 3) == wave) sort(a, b, (a - x * per) * kXcds + x, kXcds);
+    if ((turn & 3) == wave) sort(std::false_type{}, a, b, (a - x * per) * kXcds + x, kXcds);
     a = b;
   }
   if (x == 0)

@@ -62,3 +62,24 @@ def test_schedule_equals_its_definition(dev, n, per_head, kind):
     got = order.cpu().numpy()
     assert np.array_equal(np.sort(got), np.arange(n))
     assert np.array_equal(got, _schedule(counts, per_head))
+
+
+@pytest.mark.parametrize("n,per_head,densest", [(520, 65, 1.6), (3072, 256, 1.9), (23640, 591, 1.4), (3001, 250, 3.0), (8191, 256, 6.0),
+                                                (8192, 256, 2.5), (23640, 591, 4.0), (23643, 591, 300.0)])
+def test_schedule_of_heads_of_different_density(dev, n, per_head, densest):
+    """Heads of rising density, so that the XCDs' shares differ: sorted over everything by all four waves, from 8192
+    q-blocks on in quarters of an octave."""
+    print("case schedule of uneven heads", n, per_head, densest, flush=True)
+    rng = np.random.default_rng(n)
+    head = np.arange(n) // per_head
+    counts = (500 * (1 + (densest - 1) * head / head.max()) * rng.uniform(1.0, 1.02, size=n)).astype(np.int32)
+    shares = [int(counts[x * (n // 8):(x + 1) * (n // 8)].sum()) for x in range(8)]
+    assert max(shares) * 8 > 1.1 * sum(shares)
+    cls = _classes(counts)
+    if n >= 8192:
+        cls = np.where(cls < (7 << 3) + 2, cls >> 1, cls)
+    want = np.argsort(cls, kind="stable")
+    c = torch.from_numpy(counts).to(dev)
+    order = torch.full((n,), -1, dtype=torch.int32, device=dev)
+    capi.qblock_schedule(order, c, per_head)
+    assert np.array_equal(order.cpu().numpy(), want)
