@@ -15,7 +15,8 @@ The tile loop of the attention kernels waits for its copies with hand-counted vm
 holds only while the compiler puts no vector-memory instruction of its own into the loop.  The
 third check finds the tile loop of every instantiation (one inner loop, closed by a branch back to
 its header) and asserts that it holds no scratch access (a spill) and no s_waitcnt vmcnt outside
-the asm statements (the compiler waiting for a load of its own)."""
+the asm statements (the compiler waiting for a load of its own).  The same holds for the walk of the votes kernel,
+from its first copy to the wait for the last one."""
 import re
 import shutil
 import subprocess
@@ -28,7 +29,8 @@ from fgattn_tk_cuda_amd import build
 
 CSRC = Path(build.__file__).resolve().parent / "csrc"
 UNITS = ["attn_inst_blocks.hip", "attn_inst_tokens.hip", "attn_inst_dense.hip"]
-M0_UNITS = UNITS + ["mask_kernels.hip"]
+VOTES_UNIT = "votes_kernels.hip"
+M0_UNITS = UNITS + ["mask_kernels.hip", VOTES_UNIT]
 
 
 def _regs(text):
@@ -128,6 +130,37 @@ def tile_loop_findings(listing):
     return out
 
 
+def walk_findings(listing, kernel="blockmax_votes_kernel"):
+    """{kernel: (scratch accesses, compiler vmcnt waits)} between the first copy and the last hand-written wait for all
+    copies, of every instantiation; None where no such wait follows the last copy."""
+    out = {}
+    for m in re.finditer(r"^(_ZN6spattn\d+" + kernel + r"\w+):(.*?)^\.Lfunc_end", listing, re.S | re.M):
+        inside, lines = False, []   # (instruction, is inside an asm statement)
+        for l in m.group(2).split("\n"):
+            inside = "#ASMSTART" in l or (inside and "#ASMEND" not in l)
+            lines.append((l.split(";")[0].strip(), inside))
+        copies = [i for i, (t, _) in enumerate(lines) if t.startswith("global_load_lds")]
+        done = [i for i, (t, asm) in enumerate(lines) if asm and t == "s_waitcnt vmcnt(0)"]
+        if not copies or not done or done[-1] < copies[-1]:
+            out[m.group(1)] = None
+            continue
+        walk = lines[copies[0]:done[-1]]
+        out[m.group(1)] = (sum(t.startswith("scratch_") for t, _ in walk),
+                           sum(not asm and t.startswith("s_waitcnt") and "vmcnt" in t for t, asm in walk))
+    return out
+
+
+def test_walk_checker():
+    asm = "\t;;#ASMSTART\n\t%s\n\t;;#ASMEND\n"
+    name = "_ZN6spattn21blockmax_votes_kernelILi64EEEvNS_11VotesParamsE"
+    body = (name + ":\n\ts_waitcnt vmcnt(0)\n" + asm % "global_load_lds_dwordx4 v1, s[0:1]" + "%s" + asm % "s_waitcnt vmcnt(8) lgkmcnt(0)" +
+            asm % "global_load_lds_dwordx4 v1, s[0:1]" + asm % "s_waitcnt vmcnt(0)" + "\ts_waitcnt vmcnt(0)\n\ts_endpgm\n.Lfunc_end0:\n")
+    assert walk_findings(body % "") == {name: (0, 0)}
+    assert walk_findings(body % "\tscratch_load_dword v1, off, off\n\ts_waitcnt vmcnt(0)\n") == {name: (1, 1)}
+    assert walk_findings((body % "").replace(asm % "s_waitcnt vmcnt(0)", "")) == {name: None}
+    assert walk_findings("") == {}
+
+
 def test_tile_loop_checker():
     body = ("_ZN6spattn15attn_fwd_kernelILi64EEEvNS_10AttnParamsE:\n\ts_nop 0\n.LBB0_3:   ; =>This Inner Loop Header: Depth=1\n"
             "\t;;#ASMSTART\n\ts_waitcnt vmcnt(4)\n\t;;#ASMEND\n%s\ts_cbranch_scc1 .LBB0_3\n\ts_endpgm\n.Lfunc_end0:\n")
@@ -166,6 +199,9 @@ def test_no_instruction_touches_a_register_with_a_load_in_flight(tmp_path):
         assert "global_load_lds_dwordx4" in text, unit
         uses = m0_uses_outside_asm(text)
         assert not uses, "%s: the compiler uses m0 next to hand-written copies: %s" % (unit, uses[:3])
+        if unit == VOTES_UNIT:
+            walks = walk_findings(text)
+            assert len(walks) == 2 and all(f == (0, 0) for f in walks.values()), "%s: %s" % (unit, walks)
         if unit not in UNITS:
             continue
         assert "global_load_dword" in text, unit
