@@ -102,6 +102,92 @@ def test_refresh_and_sparse_steps_replay_from_a_graph(dev, S, D):
         assert torch.equal(eager.view(torch.int16), want["o_blk"].view(torch.int16))
 
 
+@pytest.mark.parametrize("H,S,D", [(3, 2000, 64), (14, 1300, 128)])
+def test_one_sweep_refresh_replays_from_a_graph(dev, H, S, D):
+    """The refresh as cached_attn_cuda runs it - votes from the block maxima, lists with their tails filled, the work
+    order by windows of heads - on both sides of the rule for 64-row q-blocks, with inputs that change between replays."""
+    print("case graph one-sweep refresh", H, S, D, flush=True)
+    B, tau = 1, 2e-3
+    q, k, v = (t.to(dev) for t in wl.clustered_qkv(B, H, S, D, seed=S, sigma=0.8))
+    buf = _buffers(dev, B, H, S, D)
+    buf = {n: buf[n] for n in ("mx", "dn", "bmx", "pk", "kvi", "kvn", "order", "o_dense", "o_tok", "lse")}
+
+    def step():
+        capi.fullattn_maxq_denom_blockmax(buf["o_dense"], buf["mx"], buf["dn"], buf["bmx"], q, k, v)
+        capi.blockmax_to_packedmask(buf["pk"], buf["bmx"], buf["mx"], buf["dn"], q, k, tau)
+        capi.packedmask_to_indexmask(buf["kvi"], buf["kvn"], buf["pk"], S, fill_tail=True)
+        capi.qblock_schedule(buf["order"], buf["kvn"], wl.ceil_div(S, 128))
+        capi.sp_attn(buf["o_tok"], q, k, v, buf["kvi"], buf["kvn"], qblk=128, order=buf["order"], lse=buf["lse"])
+
+    capi.init()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(g, stream=side):
+            step()
+    torch.cuda.current_stream().wait_stream(side)
+    for rep in range(3):
+        for t, new in zip((q, k, v), wl.clustered_qkv(B, H, S, D, seed=S + rep, sigma=0.8)):
+            t.copy_(new)
+        _poison(buf)
+        step()
+        torch.cuda.synchronize()
+        want = {name: t.clone() for name, t in buf.items()}
+        assert 0 < int(want["kvn"].sum()) < want["kvn"].numel() * S and torch.isfinite(want["o_tok"].float()).all()
+        _poison(buf)
+        g.replay()
+        torch.cuda.synchronize()
+        for name, t in buf.items():
+            assert torch.equal(t.view(torch.uint8), want[name].view(torch.uint8)), "replay %d: %s differs from the eager run" % (rep, name)
+
+
+def test_functionals_replay_from_a_graph(dev):
+    """A refresh, the steps from its cache and from bits, and the masks of every step recorded as a program calls them
+    (each computes its work order inside the graph): every replay equals the eager calls on the same inputs."""
+    from fgattn_tk_cuda_amd.spattn import mask_utils as mu, sparseattn_functionals as fn
+
+    print("case graph functionals", flush=True)
+    B, H, S, D = 1, 34, 8000, 64          # 2142 q-blocks: lists that are used once are ordered too
+    q, k, v = (torch.empty((B, H, S, D), dtype=torch.bfloat16, device=dev) for _ in range(3))
+    kw = dict(thresh=16.0 / S, blocksz=128)
+
+    def program():
+        cache, bits = mu.NaiveMaskCache([0]), mu.CompressedBitMaskCache([0])
+        outs = [fn.cached_attn_cuda(q, k, v, 0, 0, mask_cache=cache, **kw)]
+        lists, counts = cache.get_mask_from_cache(0)
+        o = torch.empty_like(q)
+        torch.ops.cuda_attn.sp_attn(o, q, k, v, lists, counts)
+        fn.bitmaskcached_attn_cuda(q, k, v, 0, 0, mask_cache=bits, **kw)
+        return outs + [lists, counts, o, fn.cached_attn_cuda(q, k, v, 0, 1, mask_cache=cache, **kw),
+                       fn.bitmaskcached_attn_cuda(q, k, v, 0, 1, mask_cache=bits, **kw), fn.attn_computed_with_sparse_mask_cuda(q, k, v, **kw),
+                       fn.attn_topkmask_cuda(q, k, v, select_k=200, blocksz=128)]
+
+    def load(seed):
+        g = torch.Generator(device=dev).manual_seed(seed)
+        for t in (q, k, v):
+            t.copy_(torch.randn(t.shape, generator=g, device=dev))
+
+    load(0)
+    program()
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(graph, stream=side):
+            got = program()
+    torch.cuda.current_stream().wait_stream(side)
+    for seed in (1, 2, 3):
+        load(seed)
+        want = program()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for i, (a, b) in enumerate(zip(got, want)):
+            assert torch.equal(a, b), "replay with inputs %d: output %d differs from the eager run" % (seed, i)
+
+
 def test_capture_right_after_init_in_a_fresh_process(dev):
     """A process whose first calls on the device are recorded into a graph: after spattn_init() no entry
     point changes a device setting, so the capture needs no eager warm-up of the library."""

@@ -61,8 +61,21 @@ def test_list_attention_reads_no_freed_slot(dev, D, qblk, S, kv_len):
 @pytest.mark.parametrize("D,S,kv_len", [(128, 1300, 0), (64, 1700, 1601)])
 def test_dense_kernels_read_no_freed_slot(dev, D, S, kv_len):
     print("case poison dense", D, S, kv_len, flush=True)
+    _dense(dev, D, S, kv_len, 2)
+
+
+@pytest.mark.parametrize("D,S,kv_len,H", [(128, 1300, 0, 13), (128, 900, 833, 18), (64, 1700, 1601, 29), (64, 700, 0, 24)])
+def test_large_dense_launches_read_no_freed_slot(dev, D, S, kv_len, H):
+    """Launches with more q-blocks than take the 64-row form."""
+    print("case poison large dense", D, S, kv_len, H, flush=True)
+    n64 = H * wl.ceil_div(S, 64)
+    assert n64 > (768 if D == 64 and (kv_len or S) >= 768 else 256)
+    _dense(dev, D, S, kv_len, H)
+
+
+def _dense(dev, D, S, kv_len, H):
     good, bad = capi.load(), _poison_lib()
-    B, H = 1, 2
+    B = 1
     q, k, v = (t.to(dev) for t in wl.randn_qkv(B, H, S, D, seed=21))
     Sp = 128 * wl.ceil_div(S, 128)
     outs = []
