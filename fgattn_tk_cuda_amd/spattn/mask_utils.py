@@ -53,7 +53,7 @@ class NaiveMaskCache:
 
     def update_cache(self, layer, kv_indices, kv_num_indices):
         self.cache[layer] = (kv_indices, kv_num_indices)
-        self.order[layer] = qblock_order_cuda(kv_num_indices) if _is_dev(kv_num_indices) else None
+        self.order[layer] = qblock_order_cuda(kv_num_indices, kv_indices.shape[2]) if _is_dev(kv_num_indices) else None
 
 
 class BlockListCache(NaiveMaskCache):
@@ -71,7 +71,7 @@ class OffloadMaskCache(NaiveMaskCache):
 
     def update_cache(self, layer, kv_indices, kv_num_indices):
         self.cache[layer] = (kv_indices.cpu(), kv_num_indices)
-        self.order[layer] = qblock_order_cuda(kv_num_indices) if _is_dev(kv_num_indices) else None
+        self.order[layer] = qblock_order_cuda(kv_num_indices, kv_indices.shape[2]) if _is_dev(kv_num_indices) else None
 
 
 class CompressMaskCache(NaiveMaskCache):
@@ -103,7 +103,7 @@ class CompressMaskCache(NaiveMaskCache):
         votes = votes[..., :width].contiguous()
         packed = pack_votes_cuda(votes) if votes.is_cuda and width % 128 == 0 else pack(votes > 0)
         self.cache[layer] = (packed, width, kv_num_indices)
-        self.order[layer] = qblock_order_cuda(kv_num_indices) if _is_dev(kv_num_indices) else None
+        self.order[layer] = qblock_order_cuda(kv_num_indices, kv_indices.shape[2]) if _is_dev(kv_num_indices) else None
 
 
 class BitMaskCache:
@@ -331,13 +331,19 @@ def qk_indexmask_cuda(q, k, thresh, blocksz=128, onepass=None, fill_tail=True, b
     return packedmask_to_indexmask_cuda(packedmask_by_groups(groups, sweep, q, k, max_q, denom, thresh), q.shape[2], fill_tail)
 
 
-def qblock_order_cuda(counts):
-    """int32 [counts.numel()]: the schedule of the list-driven attention operators for counts [B,H,SB].  From 512
-    q-blocks on every XCD works through its share by windows of whole heads, longest lists first inside a
-    window (``qblock_schedule``); below, where all q-blocks are resident at once, longest list first with lists
-    within a factor of two of each other in the default order (``qblock_order``)."""
+def qblock_order_cuda(counts, per_head=None):
+    """int32 [counts.numel()]: the schedule of the list-driven attention operators for counts of ``per_head``
+    q-blocks per head (default: the last dimension of counts [B,H,SB]).  From 512 q-blocks on every XCD works
+    through its share by windows of whole heads, longest lists first inside a window (``qblock_schedule``); below,
+    where all q-blocks are resident at once, and for flat counts whose heads are not known, longest list first with
+    lists within a factor of two of each other in the default order (``qblock_order``)."""
     order = torch.empty((counts.numel(),), dtype=torch.int32, device=counts.device)
-    spattn_interface.qblock_schedule(order, counts.contiguous(), counts.shape[-1])
+    if per_head is None and counts.dim() > 1:
+        per_head = counts.shape[-1]
+    if per_head is None:
+        spattn_interface.qblock_order(order, counts.contiguous())
+    else:
+        spattn_interface.qblock_schedule(order, counts.contiguous(), per_head)
     return order
 
 

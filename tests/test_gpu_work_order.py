@@ -83,3 +83,21 @@ def test_lists_used_once_take_their_own_order(dev, monkeypatch, H, ordered):
     seen.clear()
     fn.attn_topkmask_cuda(q, k, v, select_k=100, blocksz=128)
     assert not seen                                       # lists of equal length
+
+
+def test_flat_counts(dev):
+    """Counts without their heads: sorted as a whole, not as one head; a cache that stores them knows the heads from the
+    lists."""
+    from fgattn_tk_cuda_amd.spattn import mask_utils as mu
+
+    print("case flat counts", flush=True)
+    H, SB = 16, 256
+    c = torch.randint(1, 4000, (1, H, SB), generator=torch.Generator().manual_seed(7), dtype=torch.int32).to(dev)
+    by_heads, as_one = _fresh(torch.ops.cuda_attn, c, SB), _fresh(torch.ops.cuda_attn, c, H * SB)
+    whole = torch.empty_like(by_heads)
+    torch.ops.cuda_attn.qblock_order(whole, c)
+    assert not torch.equal(by_heads, as_one) and not torch.equal(whole, as_one)
+    assert torch.equal(mu.qblock_order_cuda(c), by_heads) and torch.equal(mu.qblock_order_cuda(c.view(-1)), whole)
+    cache = mu.NaiveMaskCache([0])
+    cache.update_cache(0, torch.empty((1, H, SB, 128), dtype=torch.int32, device=dev), c.view(-1))
+    assert torch.equal(cache.get_order(0), by_heads)
