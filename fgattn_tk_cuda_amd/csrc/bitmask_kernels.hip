@@ -133,7 +133,7 @@ __global__ __launch_bounds__(256) void packed_to_indexmask_kernel(int* __restric
         do {
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            stage[bits ? at : 2048 + lane] = key0 + __builtin_ctz(bits);
+            stage[bits ? at : 2048 + lane] = key0 + lowest_bit(bits);
             bits &= bits - 1;
             ++at;
           }

@@ -111,6 +111,14 @@ __device__ __forceinline__ uint32_t lane_scan(uint32_t x) {
   return (uint32_t)v;
 }
 
+// The lowest set bit of x, -1 for 0 (the compiler's builtin is undefined there, and a select on its result costs an
+// instruction).
+__device__ __forceinline__ int lowest_bit(uint32_t x) {
+  int r;
+  asm("v_ffbl_b32 %0, %1" : "=v"(r) : "v"(x));
+  return r;
+}
+
 // WGs are dealt to the 8 XCDs round-robin by launch order; give each XCD one
 // contiguous range of logical work ids so that neighbouring q-blocks of a head
 // share that XCD's L2.
