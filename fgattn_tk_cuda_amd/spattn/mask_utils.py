@@ -458,14 +458,16 @@ def packedmask_by_groups(groups, sweep, q, k, max_q, denom, thresh, qblk=BLOCKSZ
     those heads); the bits of the group follow from the maxima, whose buffer the next group reuses."""
     B, H, S, D = q.shape
     # the operators see views over all heads: what they refuse of the whole tensors is refused here
-    torch._check(k.shape == q.shape, lambda: "k must have the shape of q")
+    if k.shape != q.shape:
+        raise RuntimeError("k must have the shape of q")
     n, sp = B * H, max_q.shape[3]
     packed = torch.empty((B, H, (S + qblk - 1) // qblk, sp // 8), dtype=torch.uint8, device=q.device)
     heads = [t.contiguous().view(1, n, *t.shape[2:]) for t in (q, k, max_q, denom, packed)]
     blockmax = torch.empty((1, max(hi - lo for lo, hi in groups), sp // KVBLK, sp), dtype=torch.bfloat16, device=q.device)
     for lo, hi in groups:
-        qs, ks, ms, ds, ps = (t[:, lo:hi] for t in heads)
-        bm = blockmax[:, : hi - lo]
+        # one group: no views, small computations wait for the host
+        qs, ks, ms, ds, ps = heads if hi - lo == n else (t[:, lo:hi] for t in heads)
+        bm = blockmax if hi - lo == n else blockmax[:, : hi - lo]
         sweep(lo, hi, bm, qs, ks, ms, ds)
         _packedmask_from_blockmax(ps, bm, ms, ds, qs, ks, thresh, qblk, 0)
     return packed

@@ -120,7 +120,8 @@ def sparse_attn_from_cache_cuda(query, key, value, *args, **kwargs):
 def _dense_and_packedmask(query, key, value, groups, thresh, qblk):
     """Dense attention that also writes the block maxima, and the bit-packed threshold mask per qblk rows taken
     over what can hold a key only, by groups of heads (``mask_utils.head_groups``)."""
-    torch._check(value.shape == query.shape, lambda: "v must have the shape of q")
+    if value.shape != query.shape:
+        raise RuntimeError("v must have the shape of q")
     query, key, value = _c(query, key, value)
     out = _out_like(query)
     max_q, denom = mask_utils._stats_buffers(query)
@@ -128,7 +129,8 @@ def _dense_and_packedmask(query, key, value, groups, thresh, qblk):
     o_, v_ = out.view(1, B * H, S, D), value.view(1, B * H, S, D)
 
     def sweep(lo, hi, blockmax, qs, ks, ms, ds):
-        spattn_interface.fullattn_maxq_denom_blockmax(o_[:, lo:hi], ms, ds, blockmax, qs, ks, v_[:, lo:hi], 0.0, 0, B * H)
+        os_, vs = (o_, v_) if hi - lo == B * H else (o_[:, lo:hi], v_[:, lo:hi])
+        spattn_interface.fullattn_maxq_denom_blockmax(os_, ms, ds, blockmax, qs, ks, vs, 0.0, 0, B * H)
 
     return out, mask_utils.packedmask_by_groups(groups, sweep, query, key, max_q, denom, thresh, qblk)
 
