@@ -124,8 +124,8 @@ __global__ __launch_bounds__(kOrderThreads) void qblock_order_kernel(int* __rest
 // q-blocks), and inside a window the longest lists go first: one head at a time stays in its L2, lists of like
 // length walk the keys in step, and the last window still ends balanced.  Attention in ms, sorted over
 // everything / in index order / this: threshold lists 12 x 32760 x 128 0.582 / 0.575 / 0.559, 40 heads 2.00 /
-// 1.93 / 1.87, 24 x 32760 x 64 0.696 / 0.685 / 0.671; Zipf lists 8 x 65536 x 128 4.39 / 5.40 / 4.25, 32 x 16384 x
-// 128 0.661 / 0.585 / 0.502, 32 x 4096 x 128 0.101 / 0.081 / 0.074.
+// 1.93 / 1.87, 24 x 32760 x 64 0.696 / 0.685 / 0.671; Zipf lists 32 x 16384 x 128 0.661 / 0.585 / 0.502,
+// 32 x 4096 x 128 0.101 / 0.081 / 0.074; 8 x 65536 x 128 5.4 in index order, 4.3 in both others.
 // Two exceptions, decided on the counts: where the longest list is more than kTail of the work of one of an
 // XCD's 64 workgroup slots, a late window would end with it alone, and the share is one window (Zipf lists
 // 24 x 20000 x 64, 0.5 of a slot's work: 0.389 instead of 0.417 ms); and where the shares differ by more than
