@@ -3,28 +3,32 @@
 //
 // The reference sweeps Q K^T a second time in full (include/mask_utils.cuh:131-243).  A key can pass
 //   exp2((s[r,c] - max_q[r]) sf) / denom[r] > thresh
-// only in a key block whose maximum over the row's group passes it, so a workgroup, which owns a 128-row
-// q-block and a chunk of keys,
-//   1. reads its column of the block maxima (256 bytes per key block) and notes for every 64-key block
-//      which of the four 32-row groups hold a row whose maximum lies above its threshold,
-//   2. multiplies only those (32-row group, 64-key block) pairs and ORs the votes, a ballot per 32 keys,
-//      into a bit row in LDS,
-//   3. writes the bits of its chunk: one bit per (q-block, key), the layout of the mask cache
+// for row r only in a 64-key block whose maximum for that row passes it.  The key block stands still and the rows come
+// to it: a wave holds 64 keys in registers, as the B operand, and takes from a chunk of q-blocks
+//   1. the block's maxima of the chunk's rows (contiguous: the maxima lie block by block), of which it keeps one bit
+//      per row, "may pass";
+//   2. the list of those rows, q-block by q-block, each filled up to a multiple of four;
+//   3. the listed rows of Q, sixteen to a tile, copied through a ring in LDS that it fills itself (whole rows, so that
+//      the copies coalesce; no barrier) and multiplied with the 64 keys.  In the 16x16 accumulator lanes 16 g .. of
+//      register i hold row 4 g + i of the tile, so the ballot of sixteen keys has sixteen bits for each four of rows,
+//      and the fours of a tile may belong to different q-blocks;
+//   4. the 64 bits of every q-block: one bit per (q-block, key), the layout of the mask cache
 //      (python/spattn/mask_utils.py:421-430).
+// A chain of 16x16x32 multiplies gives the same bits as the 32x32x16 chain of the full sweep (compared on 1.6 million
+// elements, with magnitudes spread over e^8 among them): the votes equal those of the sweep.
 //
-// Split of 2.  A wave keeps the Q rows of R groups in registers (all four at d = 64, two at d = 128) and walks
-// its own share of the blocks with an active group among them, 32 keys at a time; it owns a ring of 32-key
-// pieces in LDS that it fills itself, so there is no barrier in the walk, and an LDS operand feeds up to R
-// multiplies.  Chunks of keys are dealt to the workgroups chunk by chunk, all q-blocks of a head for one
-// chunk before the next, so that the K rows that the workgroups of an XCD walk at a time stay near its 4 MB
-// of L2.
-//
-// What bounds it: no one unit.  At 24 x 32760 x 64 with 45 % of the (128-row, 64-key) pairs and 22 % of the
-// (32-row, 64-key) pairs active it takes 0.88 ms; without the multiplies 0.65, without the copies 0.80,
-// without the walk 0.19.  (The sweep over the listed 64-key blocks that it replaces, all 128 rows of each:
-// 1.51 ms behind 0.15 ms for the lists.  6 x 75600 x 128, 29 / 13 %: 1.46 ms; a full sweep takes 8.2 ms.)
-// Measured and not taken: the four waves sharing the tiles of a 128-row q-block with a barrier per tile or
-// per two tiles, 0.87-1.0 ms and 1.68-1.75 ms.
+// Why by rows: at a threshold of 32 mean weights on correlated tokens 45 % of the (q-block, key block) pairs hold an
+// active row, 22 % of the (32-row group, key block) pairs, but 4.5 % of the (row, key block) pairs.  Multiplying
+// (32-row group, key block) pairs with the rows standing still, as this kernel did before, copied all 64 keys of 45 % of
+// the pairs.  What bounds it now: below 5 % of the rows the maxima (5.3 TB/s of them where nothing is active), the
+// copies (keys of every wave, listed rows) and the latency of a wave's chain of them, behind that the multiplies at
+// 1.25 PFLOP/s of the tiles.  Before and after, us, thresholds of 16 / 32 / 64 mean weights:
+//   24 x 32760 x 64    1134 / 842 / 594     599 / 459 / 368
+//   6 x 75600 x 128    2905 / 2093 / 1426   1312 / 1016 / 858
+//   16 x 6000 x 128    73 / 55 / 41         39 / 31 / 25
+//   96 x 732 x 64      16.3 / 15.3 / 13.9   9.0 / 7.6 / 6.4
+// Measured and not taken: fours replaced by sixteens (every tile of one q-block) 6-14 % slower at d = 128, three ring
+// slots 8-30 % slower, the thresholds copied into the list 20 % slower.
 #include <type_traits>
 
 #include "common.h"
@@ -32,15 +36,16 @@
 
 namespace spattn {
 
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
 template <int D>
 struct VotesCfg {
-  static constexpr int kGroups = (D == 64) ? 4 : 2;            // 32-row groups per wave
-  static constexpr int kRowParts = 4 / kGroups;                 // waves along the rows
-  static constexpr int kWalkers = 4 / kRowParts;                // waves that share the list of a row part
-  static constexpr int kPiece = 32 * D * 2;                     // bytes of 32 keys
-  static constexpr int kSlots = (D == 64) ? 4 : 2;              // pieces in a wave's ring: 64 KB per workgroup
-  static constexpr int kChunkBlocks = (D == 64) ? 512 : 320;    // 64-key blocks per chunk (4 / 5 MB of K): fewer, and
-                                                                // a chunk outgrows L2, more, and the prologue weighs (both measured 2-8 % slower)
+  static constexpr int kTile = 16 * D * 2;                 // bytes of 16 rows
+  static constexpr int kSlots = 2;                         // tiles in a wave's ring: a third one costs a workgroup per CU
+  static constexpr int kChunk = (D == 64) ? 32 : 16;       // q-blocks per chunk, at most: longer chunks load the keys less
+                                                           // often and hold more LDS (thresholds); the other way round
+                                                           // measured 11-18 % (d = 64) and 3-8 % (d = 128) slower
+  static constexpr int kCap = 32;                          // tiles that a wave lists before it multiplies them
 };
 
 struct VotesParams {
@@ -50,298 +55,326 @@ struct VotesParams {
   const float* denom;        // [HB,Sp]
   const uint16_t* q;         // [HB,S,D]
   const uint16_t* k;
-  float log2_thresh;         // of the vote
-  float log2_thresh_blk;     // of the block test: a little lower, see run_blockmax_votes
+  float log2_thresh;
+  float blk_slack;           // how far below its vote threshold a row's block maximum still counts, see run_blockmax_votes
   float sf;
   int HB, S, kv_len, Sp, SB, words;
-  int nch, ch_blocks;        // chunks per row, 64-key blocks per chunk
+  int nch, ch_qblocks;       // chunks of rows per head, q-blocks per chunk (a multiple of four)
+  int jgroups;               // groups of four key blocks per head
 };
 
-// v with lane L (or the lane in m0) replaced by the wave-uniform s; the wait states cover a vector-ALU write
-// of s, as by a ballot.
+// Exclusive position of a lane's x items in its row of sixteen lanes; total: up to and with this lane.
+__device__ __forceinline__ int row_scan(int x, int& total) {
+  int v = x;
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);   // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);   // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);   // row_shr:8
+  total = v;
+  return v - x;
+}
+
+// v with lane L replaced by the wave-uniform s; the wait states cover a vector-ALU write of s.
 template <int L>
 __device__ __forceinline__ int write_lane(int s, int v) {
   asm("s_nop 1\n\tv_writelane_b32 %0, %1, %2" : "+v"(v) : "s"(s), "n"(L));
   return v;
 }
-__device__ __forceinline__ int write_lane_at(int s, int lane, int v) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 1\n\tv_writelane_b32 %0, %1, m0" : "+v"(v) : "s"(s), "s"(lane));
-  return v;
-}
-// Lane U of lo / hi receives the ballot of "row 2 lane or 2 lane + 1 above its threshold" for word U of x.
-template <int U, int N>
-__device__ __forceinline__ void collect_ballots(const uint32_t (&x)[N], float t0, float t1, int& lo, int& hi) {
-  if constexpr (U < N) {
-    const float x0 = __builtin_bit_cast(float, x[U] << 16);
-    const float x1 = __builtin_bit_cast(float, x[U] & 0xffff0000u);
-    const unsigned long long m = __ballot(x0 > t0 || x1 > t1);
-    lo = write_lane<U>((int)(unsigned)m, lo);
-    hi = write_lane<U>((int)(unsigned)(m >> 32), hi);
-    collect_ballots<U + 1, N>(x, t0, t1, lo, hi);
-  }
+
+__device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
 template <int D>
-__global__ __launch_bounds__(256, 2) void blockmax_votes_kernel(const VotesParams p) {
+__global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParams p) {
   using Cfg = VotesCfg<D>;
-  constexpr int NT = D / 16;
-  constexpr int CPR = D / 8;
+  constexpr int NT = D / 32;              // k-steps
+  constexpr int CPR = D / 8;              // 16-byte chunks per row
   constexpr int ROWB = D * 2;
-  constexpr int R = Cfg::kGroups;
-  constexpr int RP = Cfg::kRowParts;
-  constexpr int TW = Cfg::kWalkers;
-  constexpr int PIECE = Cfg::kPiece;
+  constexpr int TILE = Cfg::kTile;
   constexpr int NS = Cfg::kSlots;
-  constexpr int LPP = PIECE / 1024;       // 1 KB copies per piece
-  constexpr int RPL = 1024 / ROWB;        // rows per copy
-  constexpr int CB = Cfg::kChunkBlocks;
-  __shared__ __attribute__((aligned(1024))) unsigned char ring_all[4 * NS * PIECE];
-  __shared__ uint32_t bits[2 * CB];
-  __shared__ uint16_t blist[RP][CB];      // block within the chunk | active groups of the row part << 12
-  __shared__ int n_active[RP];
-  static_assert(CB <= 4096, "a block number takes 12 bits");
+  constexpr int LPP = TILE / 1024;        // 1 KB copies per tile
+  constexpr int CAP = Cfg::kCap;
+  constexpr int ROWS = Cfg::kChunk * 128; // rows per chunk, at most
+  constexpr int NB = ROWS / 512;          // batches of four q-blocks
+  static_assert(NS == 2, "the keys arrive in two halves of the ring's length");
+  static_assert(CAP >= 32, "a batch of four q-blocks has up to 32 tiles");
+  static_assert(Cfg::kChunk < 64, "a lane writes the votes of one q-block");
+  __shared__ __attribute__((aligned(1024))) unsigned char ring_all[4 * NS * TILE];
+  __shared__ __attribute__((aligned(16))) float tab[ROWS + 4];             // minus the vote threshold of a row on its raw score
+  __shared__ __attribute__((aligned(16))) uint16_t list_row[4][CAP * 16];  // row within the chunk, ROWS: none
+  __shared__ unsigned long long votes[4][Cfg::kChunk + 1];                  // of a wave's keys, per q-block
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int ln = lane & 31;
-  const int g = lane >> 5;
-  const int rp = wave % RP;
-  const int tw = wave / RP;
-  // head, then chunk, then q-block: see the top of the file
-  const int wg = xcd_remap(blockIdx.x, p.SB * p.nch * p.HB);
-  const int qb = wg % p.SB;
-  const int hc = wg / p.SB;
+  const int g = lane >> 4;
+  // head, then chunk of rows, then key blocks: the Q rows of a chunk (1 MB at d = 128) stay in an XCD's L2
+  const int wg = xcd_remap(blockIdx.x, p.jgroups * p.nch * p.HB);
+  const int jg = wg % p.jgroups;
+  const int hc = wg / p.jgroups;
   const int bh = hc / p.nch;
-  const int J0 = (hc - bh * p.nch) * p.ch_blocks;
+  const int qb0 = (hc - bh * p.nch) * p.ch_qblocks;
+  const int nqb = (p.SB - qb0) < p.ch_qblocks ? (p.SB - qb0) : p.ch_qblocks;
+  const int row0 = qb0 * 128;
+  const int J = 4 * jg + wave;                       // key block
+  const int left = p.kv_len - 64 * J;                // its keys and those behind
   const size_t head_off = (size_t)bh * p.S * D;
-  const uint16_t* qh = p.q + head_off;
+  const unsigned char* qc = reinterpret_cast<const unsigned char*>(p.q + head_off + (size_t)row0 * D);
   const unsigned char* kh = reinterpret_cast<const unsigned char*>(p.k + head_off);
-  const int nblk = (p.kv_len + 63) >> 6;
-  const int nbc = (nblk - J0) < p.ch_blocks ? (nblk - J0) : p.ch_blocks;   // blocks of this chunk, not positive behind the last
 
-  // The first batch of block maxima (32 key blocks per wave, a lane holds two rows) is requested before
-  // anything else: it takes longest to arrive.
-  const uint16_t* bm = p.blockmax + (size_t)bh * (p.Sp >> 6) * p.Sp + qb * 128 + 2 * lane;
-  uint32_t x[32];
-  auto load_maxima = [&](int b) {
+  // The maxima of the whole chunk are requested before anything else: they take longest to arrive.  Lane l holds
+  // rows 512 b + 8 l .. + 7.
+  u32x4 x[NB];
+  {
+    const uint16_t* bm = p.blockmax + ((size_t)bh * (p.Sp >> 6) + (left > 0 ? J : 0)) * p.Sp + row0 + 8 * lane;
 #pragma unroll
-    for (int u = 0; u < 32; ++u) {
-      const int J = J0 + (b + u < nbc ? b + u : nbc - 1);
-      x[u] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(bm + (size_t)J * p.Sp));
-    }
-  };
-  if (32 * wave < nbc) load_maxima(32 * wave);
-
-  // Thresholds on the raw score, through a table that overlays the ring: minus the vote threshold of row r
-  // (the C operand that starts every multiply chain, as in the full sweep: the same bits), and the block
-  // threshold.  Rows past S or without a key never vote.
-  float* tab = reinterpret_cast<float*>(ring_all);
-  if (tid < 128) {
-    const int row = qb * 128 + tid;
-    float tv = -__builtin_huge_valf(), tb = __builtin_huge_valf();
-    if (row < p.S) {
-      const float mq = p.max_q[(size_t)bh * p.Sp + row];
-      const float dn = p.denom[(size_t)bh * p.Sp + row];
-      const float inv_sf = 1.f / p.sf;
-      if (dn > 0.f) {
-        tv = -(p.log2_thresh + (mq * p.sf + __log2f(dn))) * inv_sf;
-        tb = (p.log2_thresh_blk + (mq * p.sf + __log2f(dn))) * inv_sf;
-      }
-    }
-    tab[tid] = tv;
-    tab[128 + tid] = tb;
-  }
-  for (int i = tid; i < 2 * CB; i += 256) bits[i] = 0;
-  if (tid < RP) n_active[tid] = 0;
-  // A operands: row 32 (R rp + m) + ln of the q-block, k-step t at chunk 2t + g
-  u32x4 qa[R][NT];
-#pragma unroll
-  for (int m = 0; m < R; ++m) {
-    const int row = qb * 128 + 32 * (R * rp + m) + ln;
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const u32x4 z = {0, 0, 0, 0};
-      qa[m][t] = (row < p.S) ? *reinterpret_cast<const u32x4*>(qh + (size_t)row * D + 16 * t + 8 * g) : z;
+    for (int b = 0; b < NB; ++b) {
+      const bool in = left > 0 && 512 * b + 8 * lane < 128 * nqb;
+      const u32x4 none = {0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};
+      x[b] = in ? __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(bm + 512 * b)) : none;
     }
   }
-  __syncthreads();
-  const float tb0 = tab[128 + 2 * lane], tb1 = tab[128 + 2 * lane + 1];
-
-  // ---- 1: active (row group, block) pairs; 32 blocks per wave step, all loads in flight ----
-  for (int b = 32 * wave; b < nbc; b += 128) {
-    int lo = 0, hi = 0;   // lane u: the ballot of block b + u, rows 2l and 2l + 1 in bit l
-    collect_ballots<0, 32>(x, tb0, tb1, lo, hi);
-    int act = ((lo & 0xffff) ? 1 : 0) | (((unsigned)lo >> 16) ? 2 : 0) | ((hi & 0xffff) ? 4 : 0) | (((unsigned)hi >> 16) ? 8 : 0);
-    if (lane >= 32 || b + lane >= nbc) act = 0;
+  // Thresholds: -t[r] is the C operand that starts every multiply chain, as in the full sweep.  Rows past S or
+  // without a key never vote.
+  {
+    constexpr int N = ROWS / 256;
+    float mq[N], dn[N];
 #pragma unroll
-    for (int r = 0; r < RP; ++r) {
-      const int mine = (act >> (R * r)) & ((1 << R) - 1);
-      const unsigned long long keep = __ballot(mine != 0);
-      int base = 0;
-      if (lane == 0) base = atomicAdd(&n_active[r], __popcll(keep));   // the order of a list does not matter
-      base = __builtin_amdgcn_readfirstlane(base);
-      if (mine) blist[r][base + __builtin_amdgcn_mbcnt_lo((unsigned)keep, 0)] = (uint16_t)((b + lane) | (mine << 12));
+    for (int i = 0; i < N; ++i) {
+      const int r = row0 + 256 * i + tid;
+      const size_t so = (size_t)bh * p.Sp + (r < p.S ? r : row0);
+      mq[i] = p.max_q[so];
+      dn[i] = p.denom[so];
     }
-    if (b + 128 < nbc) load_maxima(b + 128);
-  }
-  // The compiler waits for its loads of qa here: inside the walk that wait would be one for every copy.
 #pragma unroll
-  for (int m = 0; m < R; ++m)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) asm volatile("" : "+v"(qa[m][t]));
-  f32x16 nthr[R];   // register 4j+i of group m: row 32 (R rp + m) + 8j + 4g + i
-#pragma unroll
-  for (int m = 0; m < R; ++m)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) nthr[m][4 * j + i] = tab[32 * (R * rp + m) + 8 * j + 4 * g + i];
-#pragma unroll
-  for (int m = 0; m < R; ++m) asm volatile("" : "+v"(nthr[m]));
-  __syncthreads();
-
-  // ---- 2: votes of the active pairs ----
-  // Piece u of this wave: keys 32 (u & 1) .. of block entry u >> 1 of its share (every TW-th entry of the list
-  // of its row part, from tw).  The copies of a piece go out NS pieces ahead; its operands are read from
-  // the ring while the piece before it is multiplied.
-  const int n = __builtin_amdgcn_readfirstlane(n_active[rp]);
-  const int ne = (n - tw + TW - 1) / TW;   // not positive: nothing to do
-  const int nu = 2 * ne;
-  if (nu > 0) {
-    auto swz = [](int r) -> int {
-      return D == 128 ? (((r & 3) << 2) | ((r >> 2) & 3)) : ((((r >> 1) & 1) << 2) | ((r >> 2) & 3));
-    };
-    const uint32_t ring = (uint32_t)(uintptr_t)(lds_cptr)ring_all + wave * (NS * PIECE);
-    uint32_t kread[NT];     // operand of k-step t in slot 0
-#pragma unroll
-    for (int t = 0; t < NT; ++t) kread[t] = ring + ln * ROWB + (((2 * t + g) ^ swz(ln)) << 4);
-    uint32_t goff[LPP];     // copy i: lane offset within a piece
-#pragma unroll
-    for (int i = 0; i < LPP; ++i) {
-      const int r = RPL * i + lane / CPR;
-      goff[i] = (r < p.kv_len ? r : p.kv_len - 1) * ROWB + (((lane % CPR) ^ swz(r)) << 4);
+    for (int i = 0; i < N; ++i) {
+      const bool ok = row0 + 256 * i + tid < p.S && dn[i] > 0.f;
+      const float tv = -(p.log2_thresh + (mq[i] * p.sf + __log2f(dn[i]))) * (1.f / p.sf);
+      tab[256 * i + tid] = ok ? tv : -__builtin_huge_valf();
     }
-    // entry u >> 1 for the 64 pieces of a group: lane l holds that of piece u0 + l (past the end: the last one)
-    auto entries = [&](int u0) -> int {
-      int e = (u0 + lane) >> 1;
-      e = e < ne ? e : ne - 1;
-      return blist[rp][tw + TW * e];
-    };
-    int ev = entries(0), ev_next = entries(64);
-    auto entry = [&](int i) -> int {   // of piece i of the current group (or of the next)
-      return i < 64 ? __builtin_amdgcn_readlane(ev, i) : __builtin_amdgcn_readlane(ev_next, i - 64);
-    };
-    // Piece i into a slot.  A piece that runs past the last key is copied as the last 32 rows of the sequence
-    // (a shorter sequence: from row 0, goff clamps the rows) and its votes are shifted down by what it
-    // was moved; what that leaves behind the last key is masked off at the end.
-    const int r0_max = p.kv_len > 32 ? p.kv_len - 32 : 0;
-    auto first_row = [&](int i) -> int { return (J0 + (entry(i) & 0xfff)) * 64 + 32 * (i & 1); };
-    struct PieceLoad {
-      const unsigned char* base;
-      uint32_t dst;
-    };
-    auto prepare = [&](int i, int slot) -> PieceLoad {
-      const int row0 = first_row(i);
-      return PieceLoad{kh + (size_t)(row0 < r0_max ? row0 : r0_max) * ROWB, ring + slot * PIECE};
-    };
-    auto issue = [&](const PieceLoad& l, int c) { dma16(l.base, goff[c], __builtin_amdgcn_readfirstlane(l.dst + c * 1024)); };
-    u32x4 kf[2][NT];
-    auto read_piece = [&](int slot, u32x4 (&kd)[NT]) {
-#pragma unroll
-      for (int t = 0; t < NT; ++t) kd[t] = *(SPATTN_LDS const u32x4*)((lds_cptr)(uintptr_t)kread[t] + slot * PIECE);
-    };
-#pragma unroll
-    for (int j = 0; j < NS; ++j) {
-      const PieceLoad l = prepare(j, j);
-#pragma unroll
-      for (int c = 0; c < LPP; ++c) issue(l, c);
-    }
-    // pieces past the end repeat the last: the wait counts stay the same
-    wait_vmcnt<(NS - 1) * LPP>();
-    read_piece(0, kf[0]);
-
-    int words = 0;
-    auto piece = [&](auto sc, int i) {   // piece i of the group, in slot S, operands in kf[S & 1]
-      constexpr int S = decltype(sc)::value;
-      u32x4(&kc)[NT] = kf[S & 1];
-      // piece i+1 has landed; the operands of this piece, requested a piece ago, have left its slot
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NS - 2) * LPP) : "memory");
-      const PieceLoad next = prepare(i + NS, S);
-      read_piece((S + 1) % NS, kf[(S + 1) & 1]);
-      const int act = entry(i) >> 12;
-      f32x16 acc[2];
-      typedef __attribute__((ext_vector_type(16))) int i32x16;
-      int top0 = 0, top1 = 0;   // a float is > 0 exactly when its bits are, as an integer
-      auto chain = [&](int m) {
-#pragma unroll
-        for (int t = 0; t < NT; ++t) acc[m & 1] = mfma32(qa[m][t], kc[t], t == 0 ? nthr[m] : acc[m & 1]);
-      };
-      auto reduce = [&](int m) {
-        const i32x16 x = __builtin_bit_cast(i32x16, acc[m & 1]);
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-          top0 = top0 > x[r] ? top0 : x[r];
-          top1 = top1 > x[r + 8] ? top1 : x[r + 8];
-        }
-      };
-      // The maxima of a chain are taken behind the next chain; the copies go out between the chains (in one
-      // burst they queue behind those of the other waves).
-#pragma unroll
-      for (int m = 0; m < R + 1; ++m) {
-        if (m < R && (act & (1 << m))) chain(m);
-        if (m < R) {
-#pragma unroll
-          for (int c = 0; c < LPP / R; ++c) issue(next, m * (LPP / R) + c);
-        }
-        if (m > 0 && (act & (1 << (m - 1)))) reduce(m - 1);
-      }
-      const unsigned long long v = __ballot((top0 > top1 ? top0 : top1) > 0);
-      const int row0 = first_row(i);
-      const uint32_t w = ((uint32_t)v | (uint32_t)(v >> 32)) >> ((row0 < r0_max ? 0 : row0 - r0_max) & 31);
-      words = write_lane_at((int)w, i, words);
-    };
-    for (int u0 = 0; u0 < nu; u0 += 64) {
-      const int lim = nu - u0 < 64 ? nu - u0 : 64;   // even
-      int i = 0;
-      for (; i + NS <= lim; i += NS) {
-        piece(std::integral_constant<int, 0>{}, i);
-        piece(std::integral_constant<int, 1>{}, i + 1);
-        if constexpr (NS == 4) {
-          piece(std::integral_constant<int, 2>{}, i + 2);
-          piece(std::integral_constant<int, 3>{}, i + 3);
-        }
-      }
-      if (NS == 4 && i < lim) {
-        piece(std::integral_constant<int, 0>{}, i);
-        piece(std::integral_constant<int, 1>{}, i + 1);
-      }
-      // lane l: the votes of piece u0 + l
-      if (words) atomicOr(&bits[2 * (ev & 0xfff) + (lane & 1)], (uint32_t)words);
-      words = 0;
-      ev = ev_next;
-      ev_next = entries(u0 + 128);
-    }
-    wait_vmcnt<0>();   // no copy may land after the workgroup has given up its LDS
+    if (tid < 4) tab[ROWS + tid] = -__builtin_huge_valf();
   }
   __syncthreads();
 
-  // ---- 3: the bits of this chunk; the last chunk also writes the words behind the last key ----
-  const bool tail = hc - bh * p.nch == p.nch - 1;
-  const int w_end = tail ? p.words - 2 * J0 : 2 * p.ch_blocks;
-  const int lim = p.kv_len - J0 * 64;   // keys of this chunk and behind
-  uint32_t* dst = p.bits + ((size_t)bh * p.SB + qb) * p.words + 2 * J0;
-  for (int w = tid; w < w_end; w += 256) {
-    uint32_t x = w < 2 * nbc ? bits[w] : 0u;
-    const int left = lim - w * 32;
-    if (left < 32) x = left <= 0 ? 0u : (x & ((1u << left) - 1u));
-    dst[w] = x;
+  // ---- 1: one bit per row ----
+  constexpr int FW = NB / 4;
+  uint32_t flags[FW] = {};   // byte b % 4 of word b / 4: rows 512 b + 8 lane + 0..7
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    if (512 * b < 128 * nqb) {
+      const f32x4* t = reinterpret_cast<const f32x4*>(tab + 512 * b + 8 * lane);
+      const f32x4 t0 = t[0], t1 = t[1];
+      uint32_t f = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float lo = __builtin_bit_cast(float, x[b][i] << 16);
+        const float hi = __builtin_bit_cast(float, x[b][i] & 0xffff0000u);
+        const float a = i < 2 ? t0[2 * (i & 1)] : t1[2 * (i & 1)];
+        const float c = i < 2 ? t0[2 * (i & 1) + 1] : t1[2 * (i & 1) + 1];
+        f |= (lo + a > p.blk_slack) ? (1u << (2 * i)) : 0u;
+        f |= (hi + c > p.blk_slack) ? (2u << (2 * i)) : 0u;
+      }
+      flags[b / 4] |= f << (8 * (b % 4));
+    }
+  }
+  uint32_t any = 0;
+#pragma unroll
+  for (int w = 0; w < FW; ++w) any |= flags[w];
+
+  SPATTN_LDS unsigned long long* vw = (SPATTN_LDS unsigned long long*)votes[wave];
+  if (lane <= Cfg::kChunk) vw[lane] = 0;
+  if (__ballot(any != 0) != 0) {
+    // A copy of a tile: lane h * CPR + pos of copy c fetches chunk pos ^ swz of row LPP h + c, so that the operand
+    // reads below (sixteen lanes, one chunk of sixteen rows) cover all sixteen 16-byte bank groups.
+    auto swz = [](int r) -> int { return D == 128 ? r : ((r & 1) | ((r >> 2) << 1)); };
+    const uint32_t ring = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_cptr)ring_all + wave * (NS * TILE));
+    const int h = lane / CPR;
+    uint32_t goff[LPP];
+#pragma unroll
+    for (int c = 0; c < LPP; ++c) goff[c] = (uint32_t)(((lane % CPR) ^ swz(LPP * h + c)) << 4);
+    // operand of k-step t in slot 0: this ^ (t << 6)
+    const int m = lane & 15;
+    const uint32_t rd0 = ring + (m % LPP) * 1024 + (m / LPP) * ROWB + ((g ^ swz(m)) << 4);
+    auto read_tile = [&](uint32_t slot, u32x4 (&d)[NT]) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) d[t] = *(SPATTN_LDS const u32x4*)((lds_cptr)(uintptr_t)((rd0 + slot) ^ (uint32_t)(t << 6)));
+    };
+    auto copy = [&](const unsigned char* base, uint32_t off, uint32_t slot, int c) {
+      dma16(base, off, __builtin_amdgcn_readfirstlane(ring + slot + c * 1024));
+    };
+    // The keys, sixteen at a time like a tile of rows; rows past the last key repeat it, their votes are masked off.
+    auto copy_keys = [&](int n, int slot) {
+#pragma unroll
+      for (int c = 0; c < LPP; ++c) {
+        int r = 64 * J + 16 * n + LPP * h + c;
+        r = r < p.kv_len ? r : p.kv_len - 1;
+        copy(kh, (uint32_t)r * ROWB + goff[c], slot * TILE, c);
+      }
+    };
+#pragma unroll
+    for (int n = 0; n < NS; ++n) copy_keys(n, n);
+
+    const SPATTN_LDS float* ltab = (const SPATTN_LDS float*)tab;
+    SPATTN_LDS uint16_t* lrow = (SPATTN_LDS uint16_t*)list_row[wave];
+    const int myq = lane >> 4;   // q-block of the batch that this lane's rows belong to
+    u32x4 kf[4][NT];
+    bool keys_left = true;
+    int b = 0;
+    for (;;) {
+      // ---- 2: list rows until the list is full or the chunk has ended; the keys arrive meanwhile ----
+      int ng = 0;   // listed rows, in fours
+      bool more = false;
+      while (512 * b < 128 * nqb) {
+        uint32_t fw = flags[0];
+#pragma unroll
+        for (int w = 1; w < FW; ++w) fw = (b >> 2) == w ? flags[w] : fw;
+        const uint32_t f = (fw >> (8 * (b & 3))) & 0xffu;
+        int total;
+        const int before = row_scan(__popc(f), total);
+        const int n0 = (__builtin_amdgcn_readlane(total, 15) + 3) >> 2;
+        const int n1 = (__builtin_amdgcn_readlane(total, 31) + 3) >> 2;
+        const int n2 = (__builtin_amdgcn_readlane(total, 47) + 3) >> 2;
+        const int n3 = (__builtin_amdgcn_readlane(total, 63) + 3) >> 2;
+        const int e0 = ng + n0, e1 = e0 + n1, e2 = e1 + n2, e3 = e2 + n3;
+        if (e3 > 4 * CAP) {
+          more = true;
+          break;
+        }
+        const int start = myq == 0 ? ng : myq == 1 ? e0 : myq == 2 ? e1 : e2;
+        const int end = myq == 0 ? e0 : myq == 1 ? e1 : myq == 2 ? e2 : e3;
+        if (e3 > ng) {
+          // the last four of a q-block are filled up with a row that never votes
+          if (end > start) lrow[4 * end - 4 + (lane & 3)] = (uint16_t)ROWS;
+          int pos = 4 * start + before;
+#pragma unroll
+          for (int i = 0; i < 8; ++i)
+            if (f & (1u << i)) lrow[pos++] = (uint16_t)(512 * b + 8 * lane + i);
+        }
+        ng = e3;
+        if (b == 0) {
+          wait_vmcnt<0>();
+#pragma unroll
+          for (int n = 0; n < NS; ++n) read_tile(n * TILE, kf[n]);
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+          for (int n = NS; n < 4; ++n) copy_keys(n, n - NS);
+        }
+        ++b;
+      }
+      const int nt = (ng + 3) >> 2;
+      if (lane < 16 * nt - 4 * ng) lrow[4 * ng + lane] = (uint16_t)ROWS;
+      if (keys_left) {
+        keys_left = false;
+        wait_vmcnt<0>();
+#pragma unroll
+        for (int n = NS; n < 4; ++n) read_tile((n - NS) * TILE, kf[n]);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      }
+      // ---- 3: multiply the listed tiles ----
+      if (nt > 0) {
+        // the row lists are written and read by this wave alone, in order
+        struct Load {
+          uint32_t off[LPP];
+        };
+        const int last = p.S - 1 - row0;
+        auto prepare = [&](int i) -> Load {
+          i = i < nt ? i : nt - 1;
+          Load l;
+          uint32_t r[LPP];
+          if constexpr (LPP == 4) {
+            const u32x2 e = *(const SPATTN_LDS u32x2*)(lrow + 16 * i + 4 * h);
+            r[0] = e[0] & 0xffffu, r[1] = e[0] >> 16, r[2] = e[1] & 0xffffu, r[3] = e[1] >> 16;
+          } else {
+            const uint32_t e = *(const SPATTN_LDS uint32_t*)(lrow + 16 * i + 2 * h);
+            r[0] = e & 0xffffu, r[1] = e >> 16;
+          }
+          // "none" copies some row of the chunk
+#pragma unroll
+          for (int c = 0; c < LPP; ++c) l.off[c] = (r[c] < (uint32_t)last ? r[c] : (uint32_t)last) * ROWB + goff[c];
+          return l;
+        };
+#pragma unroll
+        for (int j = 0; j < NS; ++j) {
+          const Load l = prepare(j);
+#pragma unroll
+          for (int c = 0; c < LPP; ++c) copy(qc, l.off[c], j * TILE, c);
+        }
+        wait_vmcnt<(NS - 1) * LPP>();
+        u32x4 qa[2][NT];
+        read_tile(0, qa[0]);
+        // the C operand of tile i: rows 4 g .. 4 g + 3
+        auto read_thr = [&](int i) -> f32x4 {
+          i = i < nt ? i : nt - 1;
+          const u32x2 e = *(const SPATTN_LDS u32x2*)(lrow + 16 * i + 4 * g);
+          return f32x4{ltab[e[0] & 0xffffu], ltab[e[0] >> 16], ltab[e[1] & 0xffffu], ltab[e[1] >> 16]};
+        };
+        f32x4 thr_next = read_thr(0);
+        uint32_t slot = 0;
+        auto tile = [&](auto par, int i) {   // tile i, its operands in qa[P]
+          constexpr int P = decltype(par)::value;
+          const uint32_t next = slot + TILE == NS * TILE ? 0 : slot + TILE;
+          // tile i+1 has landed; the operands of this tile have left its slot
+          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NS - 2) * LPP) : "memory");
+          const Load l = prepare(i + NS);
+          const int qb = (int)lrow[16 * i + 4 * (lane & 3)] >> 7;   // lanes 0..3: q-block of the tile's fours
+          const f32x4 thr = thr_next;
+          thr_next = read_thr(i + 1);
+          read_tile(next, qa[P ^ 1]);
+#pragma unroll
+          for (int c = 0; c < LPP; ++c) copy(qc, l.off[c], slot, c);
+          f32x4 acc[4];
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int n = 0; n < 4; ++n) acc[n] = mfma16(qa[P][t], kf[n][t], t == 0 ? thr : acc[n]);
+          // bit 16 g + j of a ballot: some row of the tile's four g passes for key j of the sixteen
+          unsigned long long w[4];
+#pragma unroll
+          for (int n = 0; n < 4; ++n) {
+            const i32x4 v = __builtin_bit_cast(i32x4, acc[n]);   // a float is > 0 exactly when its bits are, as an integer
+            const int a = v[0] > v[1] ? v[0] : v[1], c = v[2] > v[3] ? v[2] : v[3];
+            w[n] = __ballot((a > c ? a : c) > 0);
+          }
+          int lo = 0, hi = 0;
+          auto four = [&](auto fc) {
+            constexpr int f = decltype(fc)::value;
+            lo = write_lane<f>((int)((w[0] >> (16 * f)) & 0xffffu) | ((int)((w[1] >> (16 * f)) & 0xffffu) << 16), lo);
+            hi = write_lane<f>((int)((w[2] >> (16 * f)) & 0xffffu) | ((int)((w[3] >> (16 * f)) & 0xffffu) << 16), hi);
+          };
+          four(std::integral_constant<int, 0>{});
+          four(std::integral_constant<int, 1>{});
+          four(std::integral_constant<int, 2>{});
+          four(std::integral_constant<int, 3>{});
+          if (lane < 4) {
+            const unsigned long long v = ((unsigned long long)(uint32_t)hi << 32) | (uint32_t)lo;
+            __hip_atomic_fetch_or(vw + qb, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          }
+          slot = next;
+        };
+        int i = 0;
+        for (; i + 2 <= nt; i += 2) {
+          tile(std::integral_constant<int, 0>{}, i);
+          tile(std::integral_constant<int, 1>{}, i + 1);
+        }
+        if (i < nt) tile(std::integral_constant<int, 0>{}, i);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      }
+      wait_vmcnt<0>();   // no copy may land in a slot that the next list uses, or after the workgroup has given up its LDS
+      if (!more) break;
+    }
+    wait_vmcnt<0>();
+  }
+  // ---- 4: the 64 bits of every q-block; keys past the last have none ----
+  if (64 * J < 32 * p.words && lane < nqb) {
+    const unsigned long long v = left >= 64 ? vw[lane] : left <= 0 ? 0ull : vw[lane] & ((1ull << left) - 1ull);
+    *reinterpret_cast<u32x2*>(p.bits + ((size_t)bh * p.SB + qb0 + lane) * p.words + 2 * J) = __builtin_bit_cast(u32x2, v);
   }
 }
 
 // The block test runs a little below the vote threshold, tau (1 - 1e-3): the statistics sweep rounds a
 // score and compares, the vote accumulates s - t in the matrix unit, so a key whose margin is below fp32
-// rounding could otherwise sit in a block the (rounded up) maxima leave out.  The blocks this adds
+// rounding could otherwise sit in a block the (rounded up) maxima leave out.  The rows this adds
 // contribute no votes: the bits equal those of a full threshold sweep.
 hipError_t run_blockmax_votes(uint32_t* bits, const uint16_t* blockmax, const float* max_q, const float* denom,
                               const uint16_t* q, const uint16_t* k, float thresh, int mask_stride, int HB, int S, int D,
@@ -356,7 +389,7 @@ hipError_t run_blockmax_votes(uint32_t* bits, const uint16_t* blockmax, const fl
   p.q = q;
   p.k = k;
   p.log2_thresh = thresh > 0.f ? log2f(thresh) : -__builtin_huge_valf();
-  p.log2_thresh_blk = thresh > 0.f ? log2f((float)((double)thresh * (1.0 - 1e-3))) : -__builtin_huge_valf();
+  p.blk_slack = thresh > 0.f ? log2f((float)(1.0 - 1e-3)) / sf : 0.f;
   p.sf = sf;
   p.HB = HB;
   p.S = S;
@@ -364,12 +397,14 @@ hipError_t run_blockmax_votes(uint32_t* bits, const uint16_t* blockmax, const fl
   p.Sp = SB * 128;
   p.SB = SB;
   p.words = mask_stride / 32;
-  const int nblk = (kv_len + 63) / 64;
-  const int most = D == 128 ? VotesCfg<128>::kChunkBlocks : VotesCfg<64>::kChunkBlocks;
-  p.nch = (nblk + most - 1) / most;
-  p.ch_blocks = (nblk + p.nch - 1) / p.nch;
-  p.nch = (nblk + p.ch_blocks - 1) / p.ch_blocks;   // every chunk holds a key
-  const dim3 grid(SB * HB * p.nch);
+  p.jgroups = (p.words / 2 + 3) / 4;
+  const int most = D == 128 ? VotesCfg<128>::kChunk : VotesCfg<64>::kChunk;
+  int nch = (SB + most - 1) / most;
+  // short sequences: chunks down to four q-blocks (one batch of the list) until there are four workgroups per CU
+  while (nch < (SB + 3) / 4 && (long long)nch * p.jgroups * HB < 1024) ++nch;
+  p.ch_qblocks = ((SB + nch - 1) / nch + 3) / 4 * 4;
+  p.nch = (SB + p.ch_qblocks - 1) / p.ch_qblocks;
+  const dim3 grid(p.jgroups * p.nch * HB);
   if (D == 128) hipLaunchKernelGGL(blockmax_votes_kernel<128>, grid, dim3(256), 0, stream, p);
   else hipLaunchKernelGGL(blockmax_votes_kernel<64>, grid, dim3(256), 0, stream, p);
   return hipGetLastError();

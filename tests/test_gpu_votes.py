@@ -118,3 +118,30 @@ def test_groups_take_the_form_of_the_whole(dev, H, S, D):
     assert torch.equal(ms, m[:, 2:4]) and not torch.equal(ds, d[:, 2:4])   # a launch of its own: another order of the sums
     with pytest.raises(RuntimeError):
         ops.maxq_denom_blockmax(ms, ds, mu.blockmax_buffer(some[0]), *some, 0.0, 0, 1)
+
+
+@pytest.mark.parametrize("D,S,kv_len,stride,x", [
+    (128, 2048, 0, 2048, 16), (128, 2049, 2040, 2304, 16), (64, 4096, 0, 4096, 32), (64, 4225, 4225, 4480, 1e-6), (128, 1535, 0, 1536, 1e-6),
+    (64, 15, 0, 128, 0.5), (128, 17, 16, 256, 0.5), (64, 6000, 127, 6016, 1e-6), (128, 2200, 0, 2304, 1e9),
+])
+def test_votes_by_rows(dev, D, S, kv_len, stride, x):
+    """The tiles of sixteen listed rows: chunks of 16 (d = 128) and 32 (d = 64) q-blocks and their remainders, lists that
+    are full before the chunk has ended (every row active), q-blocks and chunks without an active row, rows filled up
+    to four, rows of bits longer than the sequence - the bits of the full sweep, whose rows of bits are as long."""
+    from fgattn_tk_cuda_amd.spattn import mask_utils as mu
+
+    print("case votes by rows", D, S, kv_len, stride, x, flush=True)
+    ops = torch.ops.cuda_attn
+    H = 3
+    g = torch.Generator(device=dev).manual_seed(S + D)
+    q, k = (torch.randn((1, H, S, D), generator=g, device=dev).to(torch.bfloat16) for _ in range(2))
+    q[:, 1, : S // 2] = 0                                     # equal weights: no row of these passes at x > 1
+    max_q, denom = mu._stats_buffers(q)
+    blockmax = mu.blockmax_buffer(q).fill_(float("nan"))
+    ops.maxq_denom_blockmax(max_q, denom, blockmax, q, k, 0.0, kv_len)
+    got = torch.full((1, H, (S + 127) // 128, stride // 8), 0x5a, dtype=torch.uint8, device=dev)
+    want = torch.full_like(got, 0xa5)
+    thresh = x / (kv_len or S)
+    ops.booleanmask_packed(want, max_q, denom, q, k, thresh, 128, 0.0, kv_len)
+    ops.blockmax_to_packedmask(got, blockmax, max_q, denom, q, k, thresh, 0.0, kv_len)
+    assert torch.equal(got, want) and bool(got.any()) == (x < 1e6)
