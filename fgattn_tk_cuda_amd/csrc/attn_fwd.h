@@ -861,7 +861,6 @@ void attn_fwd_kernel(const AttnParams p) {
     // per row half: three rows of 64 floats (reference, sum, true max), then the accumulators
     // four registers at a time, 16 bytes per lane
     float* mg = reinterpret_cast<float*>(smem) + qsub * ((HAS_V ? D / 2 : 0) + 3) * 64;
-    typedef __attribute__((ext_vector_type(4))) float f32x4;
     f32x4* mg4 = reinterpret_cast<f32x4*>(mg + 3 * 64);
     if (ksub == 1) {
       mg[lane] = mr_sf;

@@ -43,13 +43,16 @@ __global__ __launch_bounds__(256) void qblock_mean_kernel(uint16_t* __restrict__
   const int rows = (S - r0) < blk ? (S - r0) : blk;
   const uint16_t* src = q + ((size_t)bh * S + r0) * D + 8 * c;
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  constexpr int U = 4;   // loads in flight
+  // Loads in flight: a q-block of 128 rows at d = 64, half of one at d = 128; past the caches, which hold nothing that
+  // comes back to these rows before the attention and make room for them slowly (32 x 67660 x 64 103 -> 47 us, 40 x 35226
+  // x 128 90 -> 57 us; the number in flight alone changed nothing).
+  constexpr int U = 16;
   for (int r = j; r < rows; r += P * U) {
     u32x4 x[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const u32x4 z = {0, 0, 0, 0};
-      x[u] = (r + P * u < rows) ? *reinterpret_cast<const u32x4*>(src + (size_t)(r + P * u) * D) : z;
+      x[u] = (r + P * u < rows) ? __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src + (size_t)(r + P * u) * D)) : z;
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
@@ -82,103 +85,131 @@ __global__ __launch_bounds__(256) void qblock_mean_kernel(uint16_t* __restrict__
 }
 
 // ------------------------------------------------------------------------------------
-// score = qmean K^T.  A workgroup takes 64 q-blocks of one head (two 32-row A operands per
-// k-step, in registers, the same in every wave) and a chunk of kKeysPerWg keys, 256 keys at
-// a time: wave w multiplies the 64 keys 64w .. 64w+63 of those (two 32-key B operands, loaded
-// HBM -> registers a few blocks ahead through rotating register sets; the product is tiny,
-// what has to be covered is the latency of the loads).  Accumulator register 4j+i of block
-// mb in lane (n, g) is q-block 32mb + 8j + 4g + i against key n.  The bf16 scores of the
-// 64 x 256 piece are collected in LDS and leave row-wise, 512 contiguous bytes of a score row
-// per half wave: stores in which every lane writes to a different row (rows are a power of
-// two apart) ran an order of magnitude slower.
-// Columns from kv_len to the next multiple of 8 receive unspecified values.
+// score = qmean K^T.  A workgroup takes 64 q-blocks of one head (their means as B operands in registers, the same in
+// every wave) and a chunk of keys, 64 keys per wave and step.  The product is tiny; what counts is how the bytes move:
+//   keys come in as whole rows (a wave-wide load of one 16-byte chunk of 32 rows is served at a quarter of the rate:
+//   9.7 against 38 TB/s from L2), 32 of them at a time, a step of the loop ahead in registers, and go through a
+//   wave-private piece of LDS, swizzled, into A operands;
+//   scores leave through another one as whole 128-byte lines: accumulator register i of lane (n, g) is key 4 g + i
+//   against q-block n, four neighbouring keys of a score row.
+// Nothing is shared behind the prologue: no barrier.  Columns from kv_len to the next multiple of 8 receive
+// unspecified values.
+// What bounds it: its stores next to the keys (24 x 32760 x 64: 107 us for 403 MB of scores; 68 us = 5.9 TB/s with the
+// keys from L1), the latency of one step in short launches.  With keys loaded operand by operand, the scores collected by
+// a workgroup and 2048 keys to every workgroup: 40 x 35226 x 128 406 us, now 256; 24 x 32760 x 64 119 us, now 107;
+// 32 x 2000 x 128 20 us, now 5.  Non-temporal stores 137 us (24 x 32760 x 64).
 // ------------------------------------------------------------------------------------
-constexpr int kKeysPerWg = 2048;
-constexpr int kScorePitch = 512 + 16;   // bytes per staged row; rows 4 apart land 16 banks apart
+constexpr int kMaxSteps = 8;             // 64-key steps per wave, at most
+constexpr int kScorePitch = 128 + 16;    // bytes per staged row of 64 scores; 32 lanes' 8-byte stores cover all banks
 
 template <int D>
 __global__ __launch_bounds__(256, 2) void qmean_scores_kernel(uint16_t* __restrict__ score,
                                                             const uint16_t* __restrict__ qmean,
                                                             const uint16_t* __restrict__ k, int S, int SB, int kv_len,
-                                                            int score_stride) {
-  constexpr int NT = D / 16;
-  __shared__ __attribute__((aligned(16))) unsigned char tile[64 * kScorePitch];
+                                                            int score_stride, int steps, int chunks, int total) {
+  constexpr int NT = D / 32;              // k-steps
+  constexpr int CPR = D / 8;              // 16-byte chunks per row
+  constexpr int ROWB = D * 2;
+  constexpr int LPH = 32 * ROWB / 1024;   // wave-wide loads per 32 keys
+  __shared__ __attribute__((aligned(1024))) unsigned char keys_all[4 * 32 * ROWB];
+  __shared__ __attribute__((aligned(16))) unsigned char stage_all[4 * 64 * kScorePitch];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int ln = lane & 31;
-  const int g = lane >> 5;
-  const int bh = blockIdx.z;
-  const int m0 = blockIdx.y * 64;
-  const int key0 = blockIdx.x * kKeysPerWg;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15;
+  const int g = lane >> 4;
+  // the 64-row groups of a head follow each other on a chunk of keys: it stays in the XCD's L2
+  const int groups = (SB + 63) / 64;
+  const int wg = xcd_remap(blockIdx.x, total);
+  const int m0 = (wg % groups) * 64;
+  const int hc = wg / groups;
+  const int bh = hc / chunks;
+  const int first = (hc - bh * chunks) * steps * 4 + wave;   // this wave's steps: first, first + 4, ...
   const uint16_t* qh = qmean + (size_t)bh * SB * D;
-  const uint16_t* kh = k + (size_t)bh * S * D;
-
-  u32x4 qa[2][NT];
-#pragma unroll
-  for (int mb = 0; mb < 2; ++mb) {
-    const int row = m0 + 32 * mb + ln;
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const u32x4 z = {0, 0, 0, 0};
-      qa[mb][t] = (row < SB) ? *reinterpret_cast<const u32x4*>(qh + (size_t)row * D + 16 * t + 8 * g) : z;
-    }
-  }
-  auto load_keys = [&](int kb, u32x4 (&kf)[NT]) {
-    int key = key0 + kb * 32 + ln;
-    key = key < kv_len ? key : kv_len - 1;   // keys past the end re-read the last one
-#pragma unroll
-    for (int t = 0; t < NT; ++t) kf[t] = *reinterpret_cast<const u32x4*>(kh + (size_t)key * D + 16 * t + 8 * g);
+  const unsigned char* kh = reinterpret_cast<const unsigned char*>(k + (size_t)bh * S * D);
+  // 16-byte chunk c of row r lies at position c ^ swz(r): one chunk of sixteen rows covers all bank groups
+  auto swz = [](int r) -> int { return D == 128 ? (r & 15) : ((r >> 1) & 7); };
+  auto frag = [&](const unsigned char* base, int row, int t) -> u32x4 {
+    return *reinterpret_cast<const u32x4*>(base + row * ROWB + (((4 * t + g) ^ swz(row)) << 4));
   };
-  const int left = kv_len - key0;
-  const int npiece_all = (left + 255) >> 8;
-  const int npiece = npiece_all < kKeysPerWg / 256 ? npiece_all : kKeysPerWg / 256;
 
-  // Step i of a wave is half (i & 1) of its 64 keys of piece i >> 1.
-  constexpr int PF = (D == 64) ? 4 : 2;
-  auto block_of = [&](int i) -> int { return 8 * (i >> 1) + 2 * wave + (i & 1); };
-  u32x4 kf[PF][NT];
+  // Means: 64 rows through LDS.  Rows past the last q-block repeat it and are not stored.
+  static_assert(4 * 32 * ROWB >= 64 * ROWB, "the means fit the key buffers");
 #pragma unroll
-  for (int u = 0; u < PF - 1; ++u) load_keys(block_of(u), kf[u]);
-  for (int i0 = 0; i0 < 2 * npiece; i0 += PF) {
+  for (int i = 0; i < 64 * CPR / 256; ++i) {
+    const int r = (256 * i + tid) / CPR, c = tid % CPR;
+    const int row = m0 + r < SB ? m0 + r : SB - 1;
+    *reinterpret_cast<u32x4*>(keys_all + r * ROWB + ((c ^ swz(r)) << 4)) =
+        *reinterpret_cast<const u32x4*>(qh + (size_t)row * D + 8 * c);
+  }
+  // 32 keys: load i covers rows 64 / CPR * i + lane / CPR; keys past the last repeat it
+  auto load_keys = [&](int key0, u32x4 (&x)[LPH]) {
 #pragma unroll
-    for (int u = 0; u < PF; ++u) {
-      const int i = i0 + u;
-      if (i < 2 * npiece) {   // wave-uniform and the same in every wave; a piece is never split (PF is even)
-        const int half = u & 1;
-        const int piece = i >> 1;
-        load_keys(block_of(i + PF - 1), kf[(u + PF - 1) % PF]);
-        f32x16 acc[2];
+    for (int i = 0; i < LPH; ++i) {
+      int key = key0 + (64 / CPR) * i + lane / CPR;
+      key = key < kv_len ? key : kv_len - 1;
+      x[i] = *reinterpret_cast<const u32x4*>(kh + (size_t)key * ROWB + (lane % CPR) * 16);
+    }
+  };
+  unsigned char* const kbuf = keys_all + wave * 32 * ROWB;
+  unsigned char* const stage = stage_all + wave * 64 * kScorePitch;
+  const int nsteps = (kv_len + 63) >> 6;
+  // A step ahead at d = 64, half a step at d = 128 (24 x 32760 x 64 116 -> 107 us; 40 x 35226 x 128 253 -> 268).
+  constexpr int PF = (D == 64) ? 2 : 1;
+  u32x4 x[PF][LPH];
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb) {
-          const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-          acc[mb] = zero;
+  for (int i = 0; i < PF; ++i) load_keys(first * 64 + 32 * i, x[i]);
+  __syncthreads();
+  u32x4 qf[4][NT];
 #pragma unroll
-          for (int t = 0; t < NT; ++t) acc[mb] = mfma32(qa[mb][t], kf[u][t], acc[mb]);
-        }
+  for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
+    for (int t = 0; t < NT; ++t) qf[mt][t] = frag(keys_all, 16 * mt + n, t);
+  __syncthreads();
+
+  for (int s = 0; s < steps; ++s) {
+    const int key0 = (first + 4 * s) * 64;
+    if (first + 4 * s >= nsteps) break;
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int row = 32 * mb + 8 * (r >> 2) + 4 * g + (r & 3);
-            *reinterpret_cast<uint16_t*>(tile + row * kScorePitch + (64 * wave + 32 * half + ln) * 2) =
-                f32_to_bf16(acc[mb][r]);
+    for (int half = 0; half < 2; ++half) {
+#pragma unroll
+      for (int i = 0; i < LPH; ++i) {
+        const int r = (64 / CPR) * i + lane / CPR;
+        *reinterpret_cast<u32x4*>(kbuf + r * ROWB + (((lane % CPR) ^ swz(r)) << 4)) = x[half % PF][i];
+      }
+      load_keys(PF == 1 && half == 0 ? key0 + 32 : key0 + 256 + (PF == 2 ? 32 * half : 0), x[half % PF]);
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+        u32x4 a[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) a[t] = frag(kbuf, 16 * kt + n, t);
+        f32x4 acc[4];
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int mt = 0; mt < 4; ++mt) {
+            const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+            acc[mt] = mfma16(a[t], qf[mt][t], t == 0 ? zero : acc[mt]);
           }
-        if (half == 1) {
-          __syncthreads();
-          // 32 lanes per row: 16 bytes each, rows tid / 32 + 8 j
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const int row = (tid >> 5) + 8 * j;
-            const int col = 8 * (tid & 31);          // key within the piece
-            const u32x4 v = *reinterpret_cast<const u32x4*>(tile + row * kScorePitch + 2 * col);
-            if (m0 + row < SB && 256 * piece + col < left)
-              *reinterpret_cast<u32x4*>(score + ((size_t)bh * SB + m0 + row) * score_stride + key0 + 256 * piece + col) = v;
-          }
-          __syncthreads();
+        for (int mt = 0; mt < 4; ++mt) {
+          const u32x2 w = {pack_bf16(acc[mt][0], acc[mt][1]), pack_bf16(acc[mt][2], acc[mt][3])};
+          *reinterpret_cast<u32x2*>(stage + (16 * mt + n) * kScorePitch + (32 * half + 16 * kt + 4 * g) * 2) = w;
         }
       }
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     }
+    // 8 lanes per row: 16 bytes each
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int row = 8 * j + (lane >> 3);
+      const int col = 8 * (lane & 7);
+      const u32x4 v = *reinterpret_cast<const u32x4*>(stage + row * kScorePitch + 2 * col);
+      if (m0 + row < SB && key0 + col < kv_len)
+        *reinterpret_cast<u32x4*>(score + ((size_t)bh * SB + m0 + row) * score_stride + key0 + col) = v;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   }
 }
 
@@ -354,7 +385,7 @@ __global__ __launch_bounds__(256) void topk_select_kernel(int* __restrict__ kv_i
 }
 
 // ------------------------------------------------------------------------------------
-// The same selection with the row held in registers: one workgroup of 512 lanes per row, every
+// The same selection with the row held in registers: one workgroup of THREADS lanes per row, every
 // lane keeps VPL 16-byte vectors (8 keys each) of the row as packed 16-bit keys from the one HBM
 // read to the emit.  Wave w owns the vectors [64 VPL w, 64 VPL (w + 1)), lane l of it the
 // vectors 64 VPL w + 64 u + l: a wave-wide load is 1 KB contiguous, and (wave, u, lane, element)
@@ -365,14 +396,14 @@ __global__ __launch_bounds__(256) void topk_select_kernel(int* __restrict__ kv_i
 // above / equal flags of the emit, which one dot product per register turns into a bit mask),
 // and the lane prefix sums of the emit run on counts packed two to a register.
 // ------------------------------------------------------------------------------------
-constexpr int kRegThreads = 512;
 constexpr int kRegSlots = 32;
 constexpr int kRegSlotShift = 5;
-// The longest rows that the register form takes.  The library's longest sequence, 75600 keys, needs 19 vectors per
-// lane (191 registers, no spills): 12 x 75600 x 128 with 8 % of the keys 1619 -> 1121 us for means, scores (496) and
-// selection against the select that reads its row three times.
-constexpr int kRegMaxVpl = 19;
-constexpr int kRegMaxKeys = kRegThreads * kRegMaxVpl * 8;   // 77824
+// 512 lanes per row up to 12 vectors per lane (49152 keys), behind that 1024 with up to 10.  A workgroup takes one row:
+// as a loop over rows the kernel held 80 to 191 registers, three workgroups down to one per CU, and now 38 to 80, four
+// (1024 lanes: two).  Before and after, us: 24 x 32760 x 64 144 -> 118, 40 x 35226 x 128 414 -> 268, 32 x 67660 x 64
+// 1368 -> 836, 16 x 75600 x 128 845 -> 512.  The steps between the instantiations are small so that few slots stay empty
+// (35226 keys: 12 vectors of 512 lanes 412, 9 of them 378, 5 of 1024 lanes 517, all three with the loop).
+constexpr int kRegMaxKeys = 1024 * 10 * 8;
 
 __device__ __forceinline__ uint32_t pk_sub_sat_u16(uint32_t a, uint32_t b) {
   uint32_t d;
@@ -423,40 +454,39 @@ __device__ __forceinline__ void find_bin_top_down(const unsigned* tot, int lane,
   above = __builtin_amdgcn_readlane(a, L);
 }
 
-// Sums the 32 partial counts of every bin into tot[256], clears what it read (and the overflow
-// bin when asked), and finds the bin that holds the need-th largest key.  Two barriers inside;
-// the caller has put one behind the last add.
-template <bool CLEAR_OVERFLOW>
+// Sums the 32 partial counts of every bin into tot[256], clears what it read if another pass follows, and finds the
+// bin that holds the need-th largest key.  Barriers inside; the caller has put one behind the last add.
+template <int THREADS, bool AGAIN>
 __device__ __forceinline__ void reduce_and_find(unsigned* hist, unsigned* tot, int tid, int lane, int need, int& bin,
                                                 int& above) {
-  u32x4* p = reinterpret_cast<u32x4*>(hist + (tid >> 1) * kRegSlots + (tid & 1) * (kRegSlots / 2));
-  const u32x4 zero = {0, 0, 0, 0};
-  unsigned s = 0;
-  // a lane's 64 bytes start 16 banks from its neighbour's: neighbouring pairs of lanes take their
-  // four 16-byte pieces in rotated order, so that 16 lanes cover all banks in every step
+  if (THREADS == 512 || tid < 512) {   // two lanes per bin
+    u32x4* p = reinterpret_cast<u32x4*>(hist + (tid >> 1) * kRegSlots + (tid & 1) * (kRegSlots / 2));
+    const u32x4 zero = {0, 0, 0, 0};
+    unsigned s = 0;
+    // a lane's 64 bytes start 16 banks from its neighbour's: neighbouring pairs of lanes take their
+    // four 16-byte pieces in rotated order, so that 16 lanes cover all banks in every step
 #pragma unroll
-  for (int j = 0; j < kRegSlots / 8; ++j) {
-    const int jj = (j + (tid >> 1)) & (kRegSlots / 8 - 1);
-    const u32x4 c = p[jj];
-    p[jj] = zero;
-    s += c[0] + c[1] + c[2] + c[3];
+    for (int j = 0; j < kRegSlots / 8; ++j) {
+      const int jj = (j + (tid >> 1)) & (kRegSlots / 8 - 1);
+      const u32x4 c = p[jj];
+      if (AGAIN) p[jj] = zero;
+      s += c[0] + c[1] + c[2] + c[3];
+    }
+    s += __shfl_xor(s, 1, 64);
+    if (!(tid & 1)) tot[tid >> 1] = s;
   }
-  s += __shfl_xor(s, 1, 64);
-  if (!(tid & 1)) tot[tid >> 1] = s;
-  if (CLEAR_OVERFLOW && tid < kRegSlots) hist[256 * kRegSlots + tid] = 0;
   __syncthreads();
   find_bin_top_down(tot, lane, need, bin, above);
-  __syncthreads();   // tot is rewritten by the next reduction
+  if (AGAIN) __syncthreads();   // tot is rewritten by the next reduction
 }
 
-template <int VPL>
-__global__ __launch_bounds__(kRegThreads) __attribute__((amdgpu_waves_per_eu(VPL <= 8 ? 6 : (VPL <= 12 ? 4 : 2)))) void topk_select_reg_kernel(int* __restrict__ kv_indices, int* __restrict__ kv_num,
-                                                                     const uint16_t* __restrict__ score, int rows,
-                                                                     int score_stride, int kv_len, int select_k,
-                                                                     int idx_stride) {
+template <int VPL, int THREADS>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(THREADS == 1024 || VPL <= 8 ? 8 : 6)))
+void topk_select_reg_kernel(int* __restrict__ kv_indices, int* __restrict__ kv_num, const uint16_t* __restrict__ score,
+                            int score_stride, int kv_len, int select_k, int idx_stride) {
   __shared__ __attribute__((aligned(16))) unsigned hist[257 * kRegSlots];   // bin 256: pass-2 keys outside the pass-1 bin
   __shared__ __attribute__((aligned(16))) unsigned tot[256];
-  __shared__ unsigned wave_cnt[kRegThreads / 64];
+  __shared__ unsigned wave_cnt[THREADS / 64];
   constexpr int NP = (VPL + 1) / 2;   // registers of counts packed two to a register
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -473,21 +503,17 @@ __global__ __launch_bounds__(kRegThreads) __attribute__((amdgpu_waves_per_eu(VPL
   SPATTN_LDS unsigned* const my_hist_lds = (SPATTN_LDS unsigned*)my_hist;
   const uint32_t one2 = 0x00010001u;
 
-  {
-    const u32x4 zero = {0, 0, 0, 0};
-    for (int i = tid; i < 257 * kRegSlots / 4; i += kRegThreads) reinterpret_cast<u32x4*>(hist)[i] = zero;
+  const int row = blockIdx.x;
+  if (want <= 0) {
+    if (tid == 0) kv_num[row] = 0;
+    return;
   }
-  for (int row = blockIdx.x; row < rows; row += gridDim.x) {
+  // Vectors behind the row hold the bit pattern whose key is 0, the smallest; so do the up to 7
+  // elements behind kv_len in the last vector.  They count as keys: with the largest indices of
+  // the row they are the last candidates among equal keys, and want <= kv_len never reaches them.
+  u32x4 y[VPL];
+  {
     const u32x4* __restrict__ src = reinterpret_cast<const u32x4*>(score + (size_t)row * score_stride);
-    int* __restrict__ dst = kv_indices + (size_t)row * idx_stride;
-    if (want <= 0) {
-      if (tid == 0) kv_num[row] = 0;
-      continue;
-    }
-    // Vectors behind the row hold the bit pattern whose key is 0, the smallest; so do the up to 7
-    // elements behind kv_len in the last vector.  They count as keys: with the largest indices of
-    // the row they are the last candidates among equal keys, and want <= kv_len never reaches them.
-    u32x4 y[VPL];
     if ((wave + 1) * (VPL * 64) <= nvec) {
 #pragma unroll
       for (int u = 0; u < VPL; ++u) y[u] = __builtin_nontemporal_load(src + vbase + 64 * u);
@@ -499,161 +525,164 @@ __global__ __launch_bounds__(kRegThreads) __attribute__((amdgpu_waves_per_eu(VPL
         y[u] = v < nvec ? __builtin_nontemporal_load(src + v) : lowest;
       }
     }
+  }
+  {   // while the row is on its way
+    const u32x4 zero = {0, 0, 0, 0};
+    for (int i = tid; i < 257 * kRegSlots / 4; i += THREADS) reinterpret_cast<u32x4*>(hist)[i] = zero;
+  }
+  int* __restrict__ dst = kv_indices + (size_t)row * idx_stride;
+#pragma unroll
+  for (int u = 0; u < VPL; ++u)
+#pragma unroll
+    for (int h = 0; h < 4; ++h) y[u][h] = order_key2(y[u][h]);
+  if (wave == tail_wave) {
+    const int left = kv_len & 7;   // elements of the vector that are keys
 #pragma unroll
     for (int u = 0; u < VPL; ++u)
+      if (u == tail_u) {
 #pragma unroll
-      for (int h = 0; h < 4; ++h) y[u][h] = order_key2(y[u][h]);
-    if (wave == tail_wave) {
-      const int left = kv_len & 7;   // elements of the vector that are keys
-#pragma unroll
-      for (int u = 0; u < VPL; ++u)
-        if (u == tail_u) {
-#pragma unroll
-          for (int h = 0; h < 4; ++h) {
-            const uint32_t keep = 2 * h + 1 < left ? ~0u : (2 * h < left ? 0x0000ffffu : 0u);
-            y[u][h] &= lane == tail_lane ? keep : ~0u;
-          }
+        for (int h = 0; h < 4; ++h) {
+          const uint32_t keep = 2 * h + 1 < left ? ~0u : (2 * h < left ? 0x0000ffffu : 0u);
+          y[u][h] &= lane == tail_lane ? keep : ~0u;
         }
+      }
+  }
+  __syncthreads();   // the histogram is clear
+  // pass 1: high bytes
+#pragma unroll
+  for (int u = 0; u < VPL; ++u)
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      const uint32_t w = y[u][h];
+      atomicAdd(my_hist + ((w >> 24) << kRegSlotShift), 1u);
+      atomicAdd(my_hist + (((w >> 8) & 0xffu) << kRegSlotShift), 1u);
     }
-    __syncthreads();   // the histogram is clear
-    // pass 1: high bytes
+  __syncthreads();
+  int b1, gt1;
+  reduce_and_find<THREADS, true>(hist, tot, tid, lane, want, b1, gt1);
+  // pass 2: low bytes under high byte b1; every other key goes to bin 256
+  {
+    const uint32_t base2 = (uint32_t)b1 * 0x01000100u;
+    const uint32_t cap2 = 0x01000100u;
+    const uint32_t stride2 = (4u * kRegSlots) * 0x00010001u;                       // bytes per bin
+    const uint32_t slot2 = (uint32_t)(uintptr_t)my_hist_lds * 0x00010001u;          // this lane's count of bin 0
 #pragma unroll
     for (int u = 0; u < VPL; ++u)
 #pragma unroll
       for (int h = 0; h < 4; ++h) {
-        const uint32_t w = y[u][h];
-        atomicAdd(my_hist + ((w >> 24) << kRegSlotShift), 1u);
-        atomicAdd(my_hist + (((w >> 8) & 0xffu) << kRegSlotShift), 1u);
+        // both LDS addresses of the register's two keys in one packed multiply-add (all below 64 KB)
+        const uint32_t a2 = pk_mad_u16(pk_min_u16(pk_sub_u16(y[u][h], base2), cap2), stride2, slot2);
+        lds_add_one(a2 & 0xffffu);
+        lds_add_one(a2 >> 16);
       }
-    __syncthreads();
-    int b1, gt1;
-    reduce_and_find<false>(hist, tot, tid, lane, want, b1, gt1);
-    // pass 2: low bytes under high byte b1; every other key goes to bin 256
-    {
-      const uint32_t base2 = (uint32_t)b1 * 0x01000100u;
-      const uint32_t cap2 = 0x01000100u;
-      const uint32_t stride2 = (4u * kRegSlots) * 0x00010001u;                       // bytes per bin
-      const uint32_t slot2 = (uint32_t)(uintptr_t)my_hist_lds * 0x00010001u;          // this lane's count of bin 0
-#pragma unroll
-      for (int u = 0; u < VPL; ++u)
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          // both LDS addresses of the register's two keys in one packed multiply-add (all below 64 KB)
-          const uint32_t a2 = pk_mad_u16(pk_min_u16(pk_sub_u16(y[u][h], base2), cap2), stride2, slot2);
-          lds_add_one(a2 & 0xffffu);
-          lds_add_one(a2 >> 16);
-        }
-    }
-    __syncthreads();
-    int b2, gt2;
-    reduce_and_find<true>(hist, tot, tid, lane, want - gt1, b2, gt2);
-    const uint32_t T = ((uint32_t)b1 << 8) | (uint32_t)b2;
-    const int r = want - gt1 - gt2;   // keys equal to T that are still needed, in key order
+  }
+  __syncthreads();
+  int b2, gt2;
+  reduce_and_find<THREADS, false>(hist, tot, tid, lane, want - gt1, b2, gt2);
+  const uint32_t T = ((uint32_t)b1 << 8) | (uint32_t)b2;
+  const int r = want - gt1 - gt2;   // keys equal to T that are still needed, in key order
 
-    // per vector: bit 2e of gtm / eqm says that element e lies above / at the threshold.  Both come
-    // from one 2-bit field per element, min(key - (T - 1), 2) with the difference saturating at 0:
-    // 0 below T, 1 at T, 2 above; one dot product per register puts its two fields in place.
-    uint32_t gtm[VPL], eqm[VPL];
-    {
-      const uint32_t Tu = (uint32_t)__builtin_amdgcn_readfirstlane((int)T);
-      const uint32_t two2 = 0x00020002u;
-      const uint32_t below2 = (Tu - 1u) * 0x00010001u;
-      if (Tu) {
-#pragma unroll
-        for (int u = 0; u < VPL; ++u) {
-          uint32_t f = 0;
-#pragma unroll
-          for (int h = 0; h < 4; ++h)
-            f = dot2_u16(pk_min_u16(pk_sub_sat_u16(y[u][h], below2), two2), (1u << (4 * h)) | (4u << (4 * h + 16)), f);
-          gtm[u] = (f >> 1) & 0x5555u;
-          eqm[u] = f & 0x5555u;
-        }
-      } else {   // every key is at or above a threshold of 0
-#pragma unroll
-        for (int u = 0; u < VPL; ++u) {
-          uint32_t f = 0;
-#pragma unroll
-          for (int h = 0; h < 4; ++h)
-            f = dot2_u16(pk_min_u16(y[u][h], one2) + one2, (1u << (4 * h)) | (4u << (4 * h + 16)), f);
-          gtm[u] = (f >> 1) & 0x5555u;
-          eqm[u] = f & 0x5555u;
-        }
-      }
-    }
-    // where this wave's part of the list starts: counts of the waves before it
-    uint32_t mine = 0;
-#pragma unroll
-    for (int u = 0; u < VPL; ++u) mine += (uint32_t)__popc(gtm[u]) + ((uint32_t)__popc(eqm[u]) << 16);
-    const uint32_t wave_total = (uint32_t)__builtin_amdgcn_readlane((int)lane_scan(mine), 63);
-    if (lane == 0) wave_cnt[wave] = wave_total;
-    __syncthreads();
-    int out_pos = 0, eq_seen = 0;
-    {
-      // added up apart: seven waves of 19 vectors per lane hold more than 65535 keys
-#pragma unroll
-      for (int u = 0; u < kRegThreads / 64 - 1; ++u) {
-        const uint32_t c = u < wave ? wave_cnt[u] : 0u;
-        out_pos += (int)(c & 0xffffu);
-        eq_seen += (int)(c >> 16);
-      }
-    }
-    out_pos += eq_seen < r ? eq_seen : r;
-    if (wave_total >> 16) {
-      // keys equal to T in this wave: keep those whose rank among all such keys of the row is below r
-      uint32_t ec[NP];
-#pragma unroll
-      for (int j = 0; j < NP; ++j) {
-        ec[j] = (uint32_t)__popc(eqm[2 * j]);
-        if (2 * j + 1 < VPL) ec[j] += (uint32_t)__popc(eqm[2 * j + 1]) << 16;
-        ec[j] = lane_scan(ec[j]);
-      }
+  // per vector: bit 2e of gtm / eqm says that element e lies above / at the threshold.  Both come
+  // from one 2-bit field per element, min(key - (T - 1), 2) with the difference saturating at 0:
+  // 0 below T, 1 at T, 2 above; one dot product per register puts its two fields in place.
+  uint32_t gtm[VPL], eqm[VPL];
+  {
+    const uint32_t Tu = (uint32_t)__builtin_amdgcn_readfirstlane((int)T);
+    const uint32_t two2 = 0x00020002u;
+    const uint32_t below2 = (Tu - 1u) * 0x00010001u;
+    if (Tu) {
 #pragma unroll
       for (int u = 0; u < VPL; ++u) {
-        const uint32_t incl = (ec[u >> 1] >> (16 * (u & 1))) & 0xffffu;
-        const uint32_t total = ((uint32_t)__builtin_amdgcn_readlane((int)ec[u >> 1], 63) >> (16 * (u & 1))) & 0xffffu;
-        uint32_t e = eqm[u];
-        int keep = r - (eq_seen + (int)incl - __popc(e));
-        uint32_t kept = 0;
-        while (e && keep > 0) {
-          kept |= e & (0u - e);
-          e &= e - 1;
-          --keep;
-        }
-        gtm[u] |= kept;
-        eq_seen += (int)total;
+        uint32_t f = 0;
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+          f = dot2_u16(pk_min_u16(pk_sub_sat_u16(y[u][h], below2), two2), (1u << (4 * h)) | (4u << (4 * h + 16)), f);
+        gtm[u] = (f >> 1) & 0x5555u;
+        eqm[u] = f & 0x5555u;
+      }
+    } else {   // every key is at or above a threshold of 0
+#pragma unroll
+      for (int u = 0; u < VPL; ++u) {
+        uint32_t f = 0;
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+          f = dot2_u16(pk_min_u16(y[u][h], one2) + one2, (1u << (4 * h)) | (4u << (4 * h + 16)), f);
+        gtm[u] = (f >> 1) & 0x5555u;
+        eqm[u] = f & 0x5555u;
       }
     }
-    // ordered emit
-    uint32_t sc[NP];
+  }
+  // where this wave's part of the list starts: counts of the waves before it
+  uint32_t mine = 0;
+#pragma unroll
+  for (int u = 0; u < VPL; ++u) mine += (uint32_t)__popc(gtm[u]) + ((uint32_t)__popc(eqm[u]) << 16);
+  const uint32_t wave_total = (uint32_t)__builtin_amdgcn_readlane((int)lane_scan(mine), 63);
+  if (lane == 0) wave_cnt[wave] = wave_total;
+  __syncthreads();
+  int out_pos = 0, eq_seen = 0;
+  {
+    // added up apart: seven waves of 19 vectors per lane hold more than 65535 keys
+#pragma unroll
+    for (int u = 0; u < THREADS / 64 - 1; ++u) {
+      const uint32_t c = u < wave ? wave_cnt[u] : 0u;
+      out_pos += (int)(c & 0xffffu);
+      eq_seen += (int)(c >> 16);
+    }
+  }
+  out_pos += eq_seen < r ? eq_seen : r;
+  if (wave_total >> 16) {
+    // keys equal to T in this wave: keep those whose rank among all such keys of the row is below r
+    uint32_t ec[NP];
 #pragma unroll
     for (int j = 0; j < NP; ++j) {
-      sc[j] = (uint32_t)__popc(gtm[2 * j]);
-      if (2 * j + 1 < VPL) sc[j] += (uint32_t)__popc(gtm[2 * j + 1]) << 16;
-      sc[j] = lane_scan(sc[j]);
+      ec[j] = (uint32_t)__popc(eqm[2 * j]);
+      if (2 * j + 1 < VPL) ec[j] += (uint32_t)__popc(eqm[2 * j + 1]) << 16;
+      ec[j] = lane_scan(ec[j]);
     }
 #pragma unroll
     for (int u = 0; u < VPL; ++u) {
-      const uint32_t incl = (sc[u >> 1] >> (16 * (u & 1))) & 0xffffu;
-      const uint32_t total = ((uint32_t)__builtin_amdgcn_readlane((int)sc[u >> 1], 63) >> (16 * (u & 1))) & 0xffffu;
-      uint32_t sel = gtm[u];
-      int pos = out_pos + (int)incl - __popc(sel);
-      const int key0 = 8 * (vbase + 64 * u);
-      while (sel) {
-        dst[pos++] = key0 + (__builtin_ctz(sel) >> 1);
-        sel &= sel - 1;
+      const uint32_t incl = (ec[u >> 1] >> (16 * (u & 1))) & 0xffffu;
+      const uint32_t total = ((uint32_t)__builtin_amdgcn_readlane((int)ec[u >> 1], 63) >> (16 * (u & 1))) & 0xffffu;
+      uint32_t e = eqm[u];
+      int keep = r - (eq_seen + (int)incl - __popc(e));
+      uint32_t kept = 0;
+      while (e && keep > 0) {
+        kept |= e & (0u - e);
+        e &= e - 1;
+        --keep;
       }
-      out_pos += (int)total;
+      gtm[u] |= kept;
+      eq_seen += (int)total;
     }
-    if (tid == 0) kv_num[row] = want;
-    // wave_cnt is rewritten only behind the barriers of the next row's passes
   }
+  // ordered emit
+  uint32_t sc[NP];
+#pragma unroll
+  for (int j = 0; j < NP; ++j) {
+    sc[j] = (uint32_t)__popc(gtm[2 * j]);
+    if (2 * j + 1 < VPL) sc[j] += (uint32_t)__popc(gtm[2 * j + 1]) << 16;
+    sc[j] = lane_scan(sc[j]);
+  }
+#pragma unroll
+  for (int u = 0; u < VPL; ++u) {
+    const uint32_t incl = (sc[u >> 1] >> (16 * (u & 1))) & 0xffffu;
+    const uint32_t total = ((uint32_t)__builtin_amdgcn_readlane((int)sc[u >> 1], 63) >> (16 * (u & 1))) & 0xffffu;
+    uint32_t sel = gtm[u];
+    int pos = out_pos + (int)incl - __popc(sel);
+    const int key0 = 8 * (vbase + 64 * u);
+    while (sel) {
+      dst[pos++] = key0 + (__builtin_ctz(sel) >> 1);
+      sel &= sel - 1;
+    }
+    out_pos += (int)total;
+  }
+  if (tid == 0) kv_num[row] = want;
 }
 
-template <int VPL>
+template <int VPL, int THREADS>
 static hipError_t launch_topk_select_reg(int* kv_indices, int* kv_num, const uint16_t* score, int rows, int score_stride,
                                          int kv_len, int select_k, int idx_stride, hipStream_t stream) {
-  const int grid = rows < 16384 ? rows : 16384;
-  hipLaunchKernelGGL(topk_select_reg_kernel<VPL>, dim3(grid), dim3(kRegThreads), 0, stream, kv_indices, kv_num, score, rows,
+  hipLaunchKernelGGL((topk_select_reg_kernel<VPL, THREADS>), dim3(rows), dim3(THREADS), 0, stream, kv_indices, kv_num, score,
                      score_stride, kv_len, select_k, idx_stride);
   return hipGetLastError();
 }
@@ -674,27 +703,37 @@ hipError_t run_topk_mask(int* kv_indices, int* kv_num, uint16_t* score, uint16_t
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (kv_len > 0) {
-    const dim3 grid((kv_len + kKeysPerWg - 1) / kKeysPerWg, (SB + 63) / 64, B * H);
+    // chunks of 2048 keys, shorter ones where that leaves less than four workgroups per CU
+    const int groups = (SB + 63) / 64, nsteps = (kv_len + 63) / 64;
+    int steps = (int)((long long)nsteps * groups * B * H / (4 * 1024));
+    steps = steps < 1 ? 1 : steps > kMaxSteps ? kMaxSteps : steps;
+    const int chunks = (nsteps + 4 * steps - 1) / (4 * steps);
+    const int total = groups * chunks * B * H;
     if (D == 64)
-      hipLaunchKernelGGL(qmean_scores_kernel<64>, grid, dim3(256), 0, stream, score, qmean, k, S, SB, kv_len,
-                         score_stride);
+      hipLaunchKernelGGL(qmean_scores_kernel<64>, dim3(total), dim3(256), 0, stream, score, qmean, k, S, SB, kv_len,
+                         score_stride, steps, chunks, total);
     else
-      hipLaunchKernelGGL(qmean_scores_kernel<128>, grid, dim3(256), 0, stream, score, qmean, k, S, SB, kv_len,
-                         score_stride);
+      hipLaunchKernelGGL(qmean_scores_kernel<128>, dim3(total), dim3(256), 0, stream, score, qmean, k, S, SB, kv_len,
+                         score_stride, steps, chunks, total);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
   if (kv_len <= kRegMaxKeys) {
-    const int vpl = ((kv_len + 7) / 8 + kRegThreads - 1) / kRegThreads;
-#define SPATTN_TOPK_REG(V) \
-  if (vpl <= V) return launch_topk_select_reg<V>(kv_indices, kv_num, score, rows, score_stride, kv_len, select_k, idx_stride, stream)
-    SPATTN_TOPK_REG(1);
-    SPATTN_TOPK_REG(2);
-    SPATTN_TOPK_REG(4);
-    SPATTN_TOPK_REG(8);
-    SPATTN_TOPK_REG(12);
-    SPATTN_TOPK_REG(18);
-    SPATTN_TOPK_REG(19);
+    const int nvec = (kv_len + 7) / 8;
+#define SPATTN_TOPK_REG(V, T) \
+  if (nvec <= V * T) return launch_topk_select_reg<V, T>(kv_indices, kv_num, score, rows, score_stride, kv_len, select_k, idx_stride, stream)
+    SPATTN_TOPK_REG(1, 512);
+    SPATTN_TOPK_REG(2, 512);
+    SPATTN_TOPK_REG(3, 512);
+    SPATTN_TOPK_REG(4, 512);
+    SPATTN_TOPK_REG(6, 512);
+    SPATTN_TOPK_REG(8, 512);
+    SPATTN_TOPK_REG(9, 512);
+    SPATTN_TOPK_REG(10, 512);
+    SPATTN_TOPK_REG(12, 512);
+    SPATTN_TOPK_REG(8, 1024);
+    SPATTN_TOPK_REG(9, 1024);
+    SPATTN_TOPK_REG(10, 1024);
 #undef SPATTN_TOPK_REG
   }
   int grid = (rows + 3) / 4;

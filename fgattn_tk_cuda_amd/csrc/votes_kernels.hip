@@ -36,8 +36,6 @@
 
 namespace spattn {
 
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-
 template <int D>
 struct VotesCfg {
   static constexpr int kTile = 16 * D * 2;                 // bytes of 16 rows
@@ -79,10 +77,6 @@ template <int L>
 __device__ __forceinline__ int write_lane(int s, int v) {
   asm("s_nop 1\n\tv_writelane_b32 %0, %1, %2" : "+v"(v) : "s"(s), "n"(L));
   return v;
-}
-
-__device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
 template <int D>

@@ -163,3 +163,27 @@ def test_topk_argument_errors(dev):
         capi.qk_topkmask_indices(kvi, kvn, score[..., :200].contiguous(), qmean, q, k, 100, blocksz=128)  # score rows too short
     with pytest.raises(capi.SpattnError):
         capi.qk_topkmask_indices(kvi, kvn, score, qmean, q, k, 0, blocksz=128)
+
+
+@pytest.mark.parametrize("H,S,D,select_k,levels", [
+    (40, 4000, 64, 400, 0), (1, 12289, 64, 1500, 9), (2, 24577, 64, 24000, 0), (2, 36864, 128, 3000, 0), (2, 36865, 64, 1, 5),
+    (1, 49152, 64, 5000, 0), (1, 49153, 64, 49152, 3), (1, 65537, 64, 6500, 0), (1, 81920, 64, 81000, 1), (1, 81921, 64, 6000, 7),
+    (3, 8200, 128, 700, 0), (70, 63, 64, 20, 3),
+])
+def test_topk_rows_per_workgroup_and_length_classes(dev, H, S, D, select_k, levels):
+    """Both sides of the steps between 512 and 1024 lanes per row and of their numbers of vectors, more rows than
+    workgroups (the next row is loaded while a list is written), several 64-key steps per wave of the scores and
+    q-blocks behind the last group of 64: every row against a stable sort of the scores the device made."""
+    print("case topk classes", H, S, D, select_k, levels, flush=True)
+    g = torch.Generator().manual_seed(S)
+    q, k = (torch.randn((1, H, S, D), generator=g).bfloat16() for _ in range(2))
+    if levels:                                         # few different keys: ties at every threshold
+        k = k[:, :, torch.randint(0, levels, (S,), generator=g)].contiguous()
+    kvi, kvn, score, qmean, fill = _run(dev, q, k, select_k, 128)
+    want_sc = torch.from_numpy(qmean).to(dev) @ k.to(dev).float().transpose(2, 3)
+    got_sc = torch.from_numpy(score[..., :S]).to(dev)
+    assert bool(((got_sc - want_sc).abs() <= want_sc.abs() * 2.0 ** -7 + 1e-5).all())   # one bf16 step, fp32 sums near zero
+    order = torch.sort(got_sc, dim=-1, descending=True, stable=True).indices[..., :select_k]
+    want = torch.sort(order, dim=-1).values.to(torch.int32).cpu().numpy()
+    assert np.all(kvn == select_k) and np.array_equal(kvi[..., :select_k], want)
+    assert np.all(kvi[..., select_k:] == fill)
