@@ -89,7 +89,7 @@ def attn_topkmask_cuda(query, key, value, current_layer=None, ditrun=None, *args
     """Top-k key lists per q-block, then sparse attention (:39-48).  The lists come from the
     device selector, padded to a multiple of 128 keys as the sparse operator needs."""
     select_k = kwargs.get("select_k") or query.shape[2]
-    kv_indices, kv_num_indices = mask_utils.qk_topkmask_indices_cuda(query, key, select_k, blocksz=kwargs["blocksz"])
+    kv_indices, kv_num_indices = mask_utils.qk_topkmask_indices_cuda(query, key, select_k, blocksz=kwargs["blocksz"], fill_tail=False)
     return _sparse(query, key, value, kv_indices, kv_num_indices, fresh=True)   # lists of equal length: index order
 
 
