@@ -279,10 +279,32 @@ void attn_fwd_kernel(const AttnParams p) {
   // Copies go out in the order K0 K1 V0 K2 | V1 K3 | V2 K4 | ...
   int idw[6] = {0, 0, 0, 0, 0, 0};   // descriptors (key mask, low half) of the tiles in flight, tile j in idw[j % 6]
   int idh[6] = {0, 0, 0, 0, 0, 0};   // token lists: key mask, high half
+  // Q_LDS: the wave's 32 rows of Q come in as whole rows, into the pieces of the slots of K2 and V1 that this wave copies
+  // itself (no other wave writes there, and its own copies into them go out behind the reads).  Loaded operand by
+  // operand, 16 bytes of 32 rows at a time, they are served at a quarter of the rate (9.7 against 38 TB/s from L2) and
+  // hold up the first tiles behind them: 0.3-0.9 us per q-block.  64 x 16384 x 128, 10 % blocks 1.092 -> 1.068 ms, 12 x
+  // 512 x 128 5.6 -> 5.1 us, 48 x 4092 x 128 157 -> 152 us, 4 x 1024 x 64 6.18 -> 5.99 us.  Not with 128-row q-blocks at
+  // d = 64, whose 168 registers it spills, nor without V, where the slots it needs are those of K1 and K2.
+  constexpr bool Q_LDS = HAS_V && (D == 128 || QBLK == 64);
+  constexpr int NQ = 32 / RPL;   // copies
+  static_assert(NQ == 2 * LPT, "the rows of a wave fill its pieces of two slots");
+  auto q_piece = [&](int i) -> uint32_t {   // LDS address of copy i
+    return smem_base + (uint32_t)(i < LPT ? 2 : NK + 1) * TILE + (i % LPT) * 4096 + wave * 1024;
+  };
   if constexpr (MODE == KV_TOKENS) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) ids_load(j, idr[j]);
-    wait_vmcnt<0>();
+  }
+  if constexpr (Q_LDS) {
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      const int r = RPL * i + ld_sub;
+      const int row = q0 + r < p.S ? q0 + r : p.S - 1;
+      dma16(qh, (uint32_t)row * ROWB + ((ld_slot ^ swz(r)) << 4), q_piece(i));
+    }
+  }
+  if constexpr (MODE == KV_TOKENS) {
+    wait_vmcnt<Q_LDS ? NQ : 0>();
 #pragma unroll
     for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(idr[j]));
 #pragma unroll
@@ -306,10 +328,10 @@ void attn_fwd_kernel(const AttnParams p) {
   using G2 = std::integral_constant<int, 2>;
   // The Q loads go out first - their address does not wait for the list - and are counted by
   // hand like the copies (a load the compiler sees makes it wait for every copy issued before
-  // the first use of Q): the wait for K0, issued behind them, covers them.  Rows past the end of
-  // the sequence read the last row and are zeroed.
+  // the first use of Q): the wait for K0, issued behind them, covers them (Q_LDS: a wait of their own, ahead of K2's
+  // copy).  Rows past the end of the sequence read the last row and are zeroed.
   u32x4 qf[NT];
-  {
+  if constexpr (!Q_LDS) {
     const uint16_t* qsrc = qh + (size_t)(qrow_ok ? qrow : p.S - 1) * D + 8 * g;
     load_q_uncounted<0, NT>(qf, qsrc);
   }
@@ -318,6 +340,17 @@ void attn_fwd_kernel(const AttnParams p) {
   if (ntiles > 0) {
     if (1 < ntiles) { issue_tile(head_desc(1), kslot(1), false, G1{}); ++head_pending; }
     if constexpr (HAS_V) { issue_tile(head_desc(0), vslot(0), true, G0{}); ++head_pending; }
+    if constexpr (Q_LDS) {
+      if (head_pending == 2) wait_vmcnt<3 * LPT>(); else wait_vmcnt<2 * LPT>();
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const uint32_t piece = q_piece(0) + ((ln / RPL) % LPT) * 4096 + (ln / RPL >= LPT ? (NK + 1 - 2) * TILE : 0);
+        qf[t] = *(SPATTN_LDS const u32x4*)((lds_cptr)(uintptr_t)(piece + (ln % RPL) * ROWB + (((2 * t + g) ^ swz(ln)) << 4)));
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int t = 0; t < NT; ++t) asm volatile("" : "+v"(qf[t]));
+    }
     if (NK == 3 && 2 < ntiles) { issue_tile(head_desc(2), kslot(2), false, G2{}); ++head_pending; }
   }
 
@@ -849,8 +882,10 @@ void attn_fwd_kernel(const AttnParams p) {
   } else {
     // the Q loads still own their registers
     wait_vmcnt<0>();
+    if constexpr (!Q_LDS) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t) asm volatile("" ::"v"(qf[t]));
+      for (int t = 0; t < NT; ++t) asm volatile("" ::"v"(qf[t]));
+    }
   }
   __syncthreads();   // every wave is done with the ring
   if (ntiles > 0) blockmax_merge(ntiles - 1);
