@@ -49,6 +49,7 @@ _SIGNATURES = {
     "spattn_maxq_denom_blockmax_of": (_c_int, [_c_void_p] * 5 + [_c_int] * 5 + [_c_float, _c_int, _c_void_p]),
     "spattn_fullattn_maxq_denom_blockmax_of": (_c_int, [_c_void_p] * 7 + [_c_int] * 5 + [_c_float, _c_int, _c_void_p]),
     "spattn_blockmax_to_blocklists": (_c_int, [_c_void_p] * 6 + [_c_float] + [_c_int] * 6 + [_c_float, _c_int, _c_void_p]),
+    "spattn_blockmax_to_blocklists_filled": (_c_int, [_c_void_p] * 6 + [_c_float] + [_c_int] * 6 + [_c_float, _c_int, _c_void_p]),
     "spattn_blockmax_to_packedmask": (_c_int, [_c_void_p] * 6 + [_c_float] + [_c_int] * 6 + [_c_float, _c_void_p]),
     "spattn_packedmask_to_indexmask_filled": (_c_int, [_c_void_p] * 3 + [_c_int] * 5 + [_c_void_p]),
     "spattn_booleanmask_128_blocks": (_c_int, [_c_void_p, _c_float, _c_int] + [_c_void_p] * 6 + [_c_int] * 6 + [_c_float, _c_void_p]),

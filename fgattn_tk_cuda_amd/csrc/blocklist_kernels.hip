@@ -126,7 +126,7 @@ __global__ __launch_bounds__(256) void blockmax_to_blocklists_kernel(int* __rest
                                                                     const float* __restrict__ max_q,
                                                                     const float* __restrict__ denom, float log2_thresh,
                                                                     float sf, int heads_total, int S, int Sp, int kv_len,
-                                                                    int max_blocks, int bm_stride) {
+                                                                    int max_blocks, int bm_stride, bool fill_tail) {
   constexpr int BPL = 128 / QB;  // key blocks per load instruction (1 or 2)
   constexpr int U = 32 / BPL;    // loads in flight per wave: 32 key blocks per step
   const int lane = threadIdx.x & 63;
@@ -182,6 +182,8 @@ __global__ __launch_bounds__(256) void blockmax_to_blocklists_kernel(int* __rest
       }
       append_blocks((word >> lane) & 1ull, J0 + lane, bm_stride, count, dst, mrow, max_blocks);
     }
+    if (fill_tail)
+      for (int i = count + lane; i < max_blocks; i += 64) dst[i] = -1;
     // block-mask entries behind the last key block of the head
     if (mrow != nullptr)
       for (int J = ((nblk + 63) & ~63) + lane; J < bm_stride; J += 64) mrow[J] = 0;
@@ -212,7 +214,8 @@ hipError_t run_votes_to_blocklists(int* blk_indices, int* blk_counts, unsigned c
 
 hipError_t run_blockmax_to_blocklists(int* blk_indices, int* blk_counts, unsigned char* blockmask, const uint16_t* blockmax,
                                       const float* max_q, const float* denom, float thresh, float sf, int qblk,
-                                      int heads_total, int S, int kv_len, int max_blocks, hipStream_t stream) {
+                                      int heads_total, int S, int kv_len, int max_blocks, bool fill_tail,
+                                      hipStream_t stream) {
   const int nqb = (S + qblk - 1) / qblk;
   const int rows = heads_total * nqb;
   if (rows <= 0) return hipSuccess;
@@ -221,10 +224,10 @@ hipError_t run_blockmax_to_blocklists(int* blk_indices, int* blk_counts, unsigne
   const int grid = blocklist_grid(rows);
   if (qblk == 128)
     hipLaunchKernelGGL(blockmax_to_blocklists_kernel<128>, dim3(grid), dim3(256), 0, stream, blk_indices, blk_counts, blockmask,
-                       blockmax, max_q, denom, lt, sf, heads_total, S, Sp, kv_len, max_blocks, Sp >> 6);
+                       blockmax, max_q, denom, lt, sf, heads_total, S, Sp, kv_len, max_blocks, Sp >> 6, fill_tail);
   else
     hipLaunchKernelGGL(blockmax_to_blocklists_kernel<64>, dim3(grid), dim3(256), 0, stream, blk_indices, blk_counts, blockmask,
-                       blockmax, max_q, denom, lt, sf, heads_total, S, Sp, kv_len, max_blocks, Sp >> 6);
+                       blockmax, max_q, denom, lt, sf, heads_total, S, Sp, kv_len, max_blocks, Sp >> 6, fill_tail);
   return hipGetLastError();
 }
 

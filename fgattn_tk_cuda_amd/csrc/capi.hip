@@ -160,9 +160,9 @@ int spattn_maxq_denom_blockmax_of(float* max_q, float* denom, void* blockmax, co
   return from_hip(spattn::run_attn_dense(p, D, false, true, as_stream(stream), of_heads));
 }
 
-int spattn_blockmax_to_blocklists(int* blk_indices, int* blk_counts, void* blockmask, const void* blockmax,
+static int blockmax_to_blocklists(int* blk_indices, int* blk_counts, void* blockmask, const void* blockmax,
                                   const float* max_q, const float* denom, float threshold, int qblk, int B, int H, int S,
-                                  int D, int kv_len, float scale, int max_blocks, void* stream) {
+                                  int D, int kv_len, float scale, int max_blocks, bool fill_tail, void* stream) {
   if (!blk_indices || !blk_counts || !blockmax || !max_q || !denom) return done(SPATTN_ERR_NULL);
   if (misaligned(blockmax)) return done(SPATTN_ERR_ALIGN);
   if (D != 64 && D != 128) return done(SPATTN_ERR_HEAD_DIM);
@@ -173,7 +173,21 @@ int spattn_blockmax_to_blocklists(int* blk_indices, int* blk_counts, void* block
   return from_hip(spattn::run_blockmax_to_blocklists(blk_indices, blk_counts, static_cast<unsigned char*>(blockmask),
                                                      static_cast<const uint16_t*>(blockmax),
                                                      max_q, denom, threshold, spattn::kLog2e * sc, qblk, B * H, S, kv,
-                                                     max_blocks, as_stream(stream)));
+                                                     max_blocks, fill_tail, as_stream(stream)));
+}
+
+int spattn_blockmax_to_blocklists(int* blk_indices, int* blk_counts, void* blockmask, const void* blockmax,
+                                  const float* max_q, const float* denom, float threshold, int qblk, int B, int H, int S,
+                                  int D, int kv_len, float scale, int max_blocks, void* stream) {
+  return blockmax_to_blocklists(blk_indices, blk_counts, blockmask, blockmax, max_q, denom, threshold, qblk, B, H, S, D,
+                                kv_len, scale, max_blocks, false, stream);
+}
+
+int spattn_blockmax_to_blocklists_filled(int* blk_indices, int* blk_counts, void* blockmask, const void* blockmax,
+                                         const float* max_q, const float* denom, float threshold, int qblk, int B, int H,
+                                         int S, int D, int kv_len, float scale, int max_blocks, void* stream) {
+  return blockmax_to_blocklists(blk_indices, blk_counts, blockmask, blockmax, max_q, denom, threshold, qblk, B, H, S, D,
+                                kv_len, scale, max_blocks, true, stream);
 }
 
 int spattn_blockmax_to_packedmask(void* packed, const void* blockmax, const float* max_q, const float* denom, const void* q,

@@ -36,7 +36,8 @@ hipError_t run_votes_to_blocklists(int* blk_indices, int* blk_counts, unsigned c
 
 hipError_t run_blockmax_to_blocklists(int* blk_indices, int* blk_counts, unsigned char* blockmask, const uint16_t* blockmax,
                                       const float* max_q, const float* denom, float thresh, float sf, int qblk,
-                                      int heads_total, int S, int kv_len, int max_blocks, hipStream_t stream);
+                                      int heads_total, int S, int kv_len, int max_blocks, bool fill_tail,
+                                      hipStream_t stream);
 
 // votes_kernels.hip
 hipError_t run_blockmax_votes(uint32_t* bits, const uint16_t* blockmax, const float* max_q, const float* denom,

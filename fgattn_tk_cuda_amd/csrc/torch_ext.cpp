@@ -736,6 +736,74 @@ void qk_topkmask_indices(torch::Tensor kv_indices, torch::Tensor kv_numindices, 
   counts_written(kv_numindices);
 }
 
+// A refresh whose block maxima all fit at once, from q, k (and v) to its mask in one operator: with o and v dense
+// attention with statistics, else the statistics alone, then the threshold on what the block maxima leave.  Statistics
+// and block maxima are the operator's own, from the caching allocator.
+namespace {
+struct OnePass {
+  torch::Tensor max_q, denom, blockmax;
+  int B, H, S, D;
+};
+OnePass onepass_sweep(const OptTensor& o, const torch::Tensor& q, const torch::Tensor& k, const OptTensor& v) {
+  check_bhsd(q, "q", q);
+  check_bhsd(k, "k", q);
+  const bool dense = o.has_value() && o->defined();
+  TORCH_CHECK(dense == (v.has_value() && v->defined()), "o and v come together");
+  if (dense) {
+    check_bhsd(*v, "v", q);
+    check_bhsd(*o, "o", q);
+  }
+  const int64_t B = q.size(0), H = q.size(1), S = q.size(2), sp = padded128(S);
+  OnePass p{torch::empty({B, H, 1, sp}, q.options().dtype(at::kFloat)), torch::empty({B, H, 1, sp}, q.options().dtype(at::kFloat)),
+            torch::empty({B, H, sp / 64, sp}, q.options()), (int)B, (int)H, (int)S, (int)q.size(3)};
+  float* const m = p.max_q.data_ptr<float>();
+  float* const d = p.denom.data_ptr<float>();
+  check_status(dense ? spattn_fullattn_maxq_denom_blockmax(o->data_ptr(), m, d, p.blockmax.data_ptr(), q.data_ptr(), k.data_ptr(),
+                                                           v->data_ptr(), p.B, p.H, p.S, p.D, 0, 0.f, cur_stream())
+                     : spattn_maxq_denom_blockmax(m, d, p.blockmax.data_ptr(), q.data_ptr(), k.data_ptr(), p.B, p.H, p.S, p.D, 0,
+                                                  0.f, cur_stream()),
+               "statistics with block maxima");
+  return p;
+}
+}  // namespace
+
+// packed uint8 [B,H,ceil(S/128),Sp/8]
+void onepass_packedmask(torch::Tensor packed, OptTensor o, torch::Tensor q, torch::Tensor k, OptTensor v, double threshold) {
+  TORCH_CHECK(q.is_cuda() && q.dim() == 4, "q must be a device tensor [B,H,S,D]");
+  check_aux(packed, "packed", at::kByte, q);
+  const int64_t sp = padded128(q.size(2));
+  TORCH_CHECK(packed.dim() == 4 && packed.size(0) == q.size(0) && packed.size(1) == q.size(1) && packed.size(2) == sp / 128 &&
+                  packed.size(3) == sp / 8,
+              "packed must be [B,H,ceil(S/128),Sp/8]");
+  const DeviceGuard guard(q.device());
+  const OnePass p = onepass_sweep(o, q, k, v);
+  check_status(spattn_blockmax_to_packedmask(packed.data_ptr(), p.blockmax.data_ptr(), p.max_q.data_ptr<float>(),
+                                             p.denom.data_ptr<float>(), q.data_ptr(), k.data_ptr(), (float)threshold, (int)sp,
+                                             p.B, p.H, p.S, p.D, 0, 0.f, cur_stream()),
+               "onepass_packedmask");
+}
+
+// blk_idx int32 [B,H,ceil(S/qblk),max_blocks], -1 behind the counts; blk_cnt int32 with B*H*ceil(S/qblk) entries
+void onepass_blocklists(torch::Tensor blk_idx, torch::Tensor blk_cnt, OptTensor o, torch::Tensor q, torch::Tensor k, OptTensor v,
+                        double threshold, int64_t qblk) {
+  TORCH_CHECK(q.is_cuda() && q.dim() == 4, "q must be a device tensor [B,H,S,D]");
+  TORCH_CHECK(qblk == 64 || qblk == 128, "qblk must be 64 or 128");
+  check_aux(blk_idx, "blk_idx", at::kInt, q);
+  check_aux(blk_cnt, "blk_cnt", at::kInt, q);
+  const int64_t SB = (q.size(2) + qblk - 1) / qblk;
+  TORCH_CHECK(blk_idx.dim() == 4 && blk_idx.size(0) == q.size(0) && blk_idx.size(1) == q.size(1) && blk_idx.size(2) == SB &&
+                  blk_idx.size(3) > 0,
+              "blk_idx must be [B,H,ceil(S/qblk),max_blocks]");
+  TORCH_CHECK(blk_cnt.numel() == q.size(0) * q.size(1) * SB, "blk_cnt must have B*H*ceil(S/qblk) entries");
+  const DeviceGuard guard(q.device());
+  const OnePass p = onepass_sweep(o, q, k, v);
+  check_status(spattn_blockmax_to_blocklists_filled(blk_idx.data_ptr<int>(), blk_cnt.data_ptr<int>(), nullptr, p.blockmax.data_ptr(),
+                                                    p.max_q.data_ptr<float>(), p.denom.data_ptr<float>(), (float)threshold,
+                                                    (int)qblk, p.B, p.H, p.S, p.D, 0, 0.f, (int)blk_idx.size(3), cur_stream()),
+               "onepass_blocklists");
+  counts_written(blk_cnt);
+}
+
 // Meta kernels: shapes only, nothing to compute (all ops mutate their arguments in place).
 void noop4(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor) {}
 void noop_all_index(torch::Tensor, torch::Tensor, int64_t, int64_t, int64_t, int64_t) {}
@@ -766,6 +834,8 @@ void noop_md_bm(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torc
 void noop_bm_lists(torch::Tensor, torch::Tensor, OptTensor, torch::Tensor, torch::Tensor, torch::Tensor, double, int64_t, int64_t,
                    int64_t, double, int64_t) {}
 
+void noop_onepass_packed(torch::Tensor, OptTensor, torch::Tensor, torch::Tensor, OptTensor, double) {}
+void noop_onepass_lists(torch::Tensor, torch::Tensor, OptTensor, torch::Tensor, torch::Tensor, OptTensor, double, int64_t) {}
 void noop_bm_packed(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, double, double,
                     int64_t) {}
 
@@ -799,6 +869,8 @@ TORCH_LIBRARY_FRAGMENT(cuda_attn, m) {
   m.def("blockmax_to_blocklists(Tensor(a!) blk_idx, Tensor(b!) blk_cnt, Tensor(c!)? blockmask, Tensor blockmax, Tensor o_max_q, Tensor o_denom, float threshold, int seq, int head_dim, int qblk, float scale, int kv_len) -> ()");
   m.def("blockmax_to_packedmask(Tensor(a!) packed, Tensor blockmax, Tensor o_max_q, Tensor o_denom, Tensor q, Tensor k, float threshold, float scale, int kv_len) -> ()");
   m.def("packedmask_to_indexmask_filled(Tensor(a!) kv_indices, Tensor(b!) kv_numindices, Tensor packed, int seq) -> ()");
+  m.def("onepass_packedmask(Tensor(a!) packed, Tensor(b!)? o, Tensor q, Tensor k, Tensor? v, float threshold) -> ()");
+  m.def("onepass_blocklists(Tensor(a!) blk_idx, Tensor(b!) blk_cnt, Tensor(c!)? o, Tensor q, Tensor k, Tensor? v, float threshold, int qblk) -> ()");
 }
 
 TORCH_LIBRARY_IMPL(cuda_attn, Meta, m) {
@@ -830,6 +902,8 @@ TORCH_LIBRARY_IMPL(cuda_attn, Meta, m) {
   m.impl("blockmax_to_blocklists", noop_bm_lists);
   m.impl("blockmax_to_packedmask", noop_bm_packed);
   m.impl("packedmask_to_indexmask_filled", noop_b2i);
+  m.impl("onepass_packedmask", noop_onepass_packed);
+  m.impl("onepass_blocklists", noop_onepass_lists);
 }
 
 // The CUDA dispatch key serves HIP tensors on PyTorch-ROCm.
@@ -862,6 +936,8 @@ TORCH_LIBRARY_IMPL(cuda_attn, CUDA, m) {
   m.impl("blockmax_to_blocklists", blockmax_to_blocklists);
   m.impl("blockmax_to_packedmask", blockmax_to_packedmask);
   m.impl("packedmask_to_indexmask_filled", packedmask_to_indexmask_filled);
+  m.impl("onepass_packedmask", onepass_packedmask);
+  m.impl("onepass_blocklists", onepass_blocklists);
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -894,4 +970,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("blockmax_to_blocklists", &blockmax_to_blocklists, "block maxima -> KV-block lists");
   m.def("blockmax_to_packedmask", &blockmax_to_packedmask, "threshold sweep over what the block maxima leave, bit-packed");
   m.def("packedmask_to_indexmask_filled", &packedmask_to_indexmask_filled, "packedmask_to_indexmask with the tail filled");
+  m.def("onepass_packedmask", &onepass_packedmask, "statistics (and dense attention) and the bit-packed threshold mask");
+  m.def("onepass_blocklists", &onepass_blocklists, "statistics (and dense attention) and KV-block lists");
 }

@@ -320,15 +320,15 @@ def qk_indexmask_cuda(q, k, thresh, blocksz=128, onepass=None, fill_tail=True, b
     ``sp_attn`` and drops them)."""
     assert blocksz == BLOCKSZ
     groups = head_groups(q, onepass, budget_bytes)
-    max_q, denom = _stats_buffers(q)
     if groups is None:
+        max_q, denom = _stats_buffers(q)
         spattn_interface.maxq_denom(max_q, denom, q.contiguous(), k.contiguous())
         return qk_indexmask_from_maxq_denom_cuda(max_q, denom, q, k, thresh, blocksz)
 
     def sweep(lo, hi, blockmax, q_, k_, max_q_, denom_):
         spattn_interface.maxq_denom_blockmax(max_q_, denom_, blockmax, q_, k_, 0.0, 0, q.shape[0] * q.shape[1])
 
-    return packedmask_to_indexmask_cuda(packedmask_by_groups(groups, sweep, q, k, max_q, denom, thresh), q.shape[2], fill_tail)
+    return packedmask_to_indexmask_cuda(packedmask_by_groups(groups, sweep, q, k, None, None, thresh), q.shape[2], fill_tail)
 
 
 def qblock_order_cuda(counts, per_head=None):
@@ -452,16 +452,24 @@ def head_groups(q, onepass=None, budget_bytes=None):
     return [(B * H * i // n, B * H * (i + 1) // n) for i in range(n)]
 
 
-def packedmask_by_groups(groups, sweep, q, k, max_q, denom, thresh, qblk=BLOCKSZ):
+def packedmask_by_groups(groups, sweep, q, k, max_q, denom, thresh, qblk=BLOCKSZ, out=None, value=None):
     """The bit-packed threshold mask (per qblk rows) of a one-sweep refresh.  ``sweep(lo, hi, blockmax, q, k,
     max_q, denom)`` runs the statistics sweep with block maxima over heads lo..hi-1 (its tensors are views of
-    those heads); the bits of the group follow from the maxima, whose buffer the next group reuses."""
+    those heads); the bits of the group follow from the maxima, whose buffer the next group reuses.  max_q, denom
+    None: the statistics are dropped; all heads at once with bits per 128 rows is then one operator, which is told what
+    else the sweep writes (``out`` from ``value``: dense attention)."""
     B, H, S, D = q.shape
     # the operators see views over all heads: what they refuse of the whole tensors is refused here
     if k.shape != q.shape:
         raise RuntimeError("k must have the shape of q")
-    n, sp = B * H, max_q.shape[3]
+    n, sp = B * H, _padded(S)
     packed = torch.empty((B, H, (S + qblk - 1) // qblk, sp // 8), dtype=torch.uint8, device=q.device)
+    if max_q is None:
+        if len(groups) == 1 and qblk == BLOCKSZ:
+            # small computations wait for the host: 32 x 380 x 64 x 4 44 -> 31 us a call against the operators one by one
+            spattn_interface.onepass_packedmask(packed, out, q.contiguous(), k.contiguous(), value, thresh)
+            return packed
+        max_q, denom = _stats_buffers(q)
     heads = [t.contiguous().view(1, n, *t.shape[2:]) for t in (q, k, max_q, denom, packed)]
     blockmax = torch.empty((1, max(hi - lo for lo, hi in groups), sp // KVBLK, sp), dtype=torch.bfloat16, device=q.device)
     for lo, hi in groups:

@@ -124,7 +124,6 @@ def _dense_and_packedmask(query, key, value, groups, thresh, qblk):
         raise RuntimeError("v must have the shape of q")
     query, key, value = _c(query, key, value)
     out = _out_like(query)
-    max_q, denom = mask_utils._stats_buffers(query)
     B, H, S, D = query.shape
     o_, v_ = out.view(1, B * H, S, D), value.view(1, B * H, S, D)
 
@@ -132,7 +131,7 @@ def _dense_and_packedmask(query, key, value, groups, thresh, qblk):
         os_, vs = (o_, v_) if hi - lo == B * H else (o_[:, lo:hi], v_[:, lo:hi])
         spattn_interface.fullattn_maxq_denom_blockmax(os_, ms, ds, blockmax, qs, ks, vs, 0.0, 0, B * H)
 
-    return out, mask_utils.packedmask_by_groups(groups, sweep, query, key, max_q, denom, thresh, qblk)
+    return out, mask_utils.packedmask_by_groups(groups, sweep, query, key, None, None, thresh, qblk, out, value)
 
 
 def cached_attn_cuda(query, key, value, current_layer, ditrun, *args, **kwargs):
@@ -192,11 +191,12 @@ def blockcached_attn_cuda(query, key, value, current_layer, ditrun, *args, **kwa
             # the dense pass also writes the per-(row, key block) score maxima: the lists come from
             # thresholding those, without a second sweep over Q K^T
             out = _out_like(query)
-            max_q, denom = mask_utils._stats_buffers(query)
-            blockmax = mask_utils.blockmax_buffer(query)
-            spattn_interface.fullattn_maxq_denom_blockmax(out, max_q, denom, blockmax, *_c(query, key, value), 0.0, 0)
-            blk_idx, blk_cnt = mask_utils.blockmax_to_blocklists_cuda(blockmax, max_q, denom, kwargs["thresh"], query.shape[2],
-                                                                    query.shape[3], qblk)
+            B, H, S, _ = query.shape
+            shape = (B, H, (S + qblk - 1) // qblk, mask_utils._padded(S) // mask_utils.KVBLK)
+            blk_idx = torch.empty(shape, dtype=torch.int32, device=query.device)
+            blk_cnt = torch.empty(shape[:3], dtype=torch.int32, device=query.device)
+            query, key, value = _c(query, key, value)
+            spattn_interface.onepass_blocklists(blk_idx, blk_cnt, out, query, key, value, kwargs["thresh"], qblk)
         elif groups is not None:
             out, packed = _dense_and_packedmask(query, key, value, groups, kwargs["thresh"], qblk)
             blk_idx, blk_cnt = mask_utils.packedmask_to_blocklists_cuda(packed, query.shape[2])

@@ -193,6 +193,10 @@ int spattn_fullattn_maxq_denom_blockmax_of(void* o, float* max_q, float* denom, 
 int spattn_blockmax_to_blocklists(int* blk_indices, int* blk_counts, void* blockmask, const void* blockmax,
                                   const float* max_q, const float* denom, float threshold, int qblk, int batch, int heads,
                                   int seq, int D, int kv_len, float scale, int max_blocks, void* stream);
+/* The same with the entries behind a count written as -1. */
+int spattn_blockmax_to_blocklists_filled(int* blk_indices, int* blk_counts, void* blockmask, const void* blockmax,
+                                         const float* max_q, const float* denom, float threshold, int qblk, int batch,
+                                         int heads, int seq, int D, int kv_len, float scale, int max_blocks, void* stream);
 
 /* The threshold sweep restricted to listed key blocks.  blk_indices int32
  * [batch,heads,ceil(seq/128),max_blocks] holds, per 128-row q-block, ascending ids of 64-key

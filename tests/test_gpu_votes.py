@@ -145,3 +145,38 @@ def test_votes_by_rows(dev, D, S, kv_len, stride, x):
     ops.booleanmask_packed(want, max_q, denom, q, k, thresh, 128, 0.0, kv_len)
     ops.blockmax_to_packedmask(got, blockmax, max_q, denom, q, k, thresh, 0.0, kv_len)
     assert torch.equal(got, want) and bool(got.any()) == (x < 1e6)
+
+
+@pytest.mark.parametrize("S,D,dense", [(1, 64, True), (65, 128, False), (300, 64, True), (1300, 128, True), (2049, 64, False)])
+def test_onepass_operators_are_the_operators_one_by_one(dev, S, D, dense):
+    """onepass_packedmask and onepass_blocklists: output, bits, lists with their tails and counts are those of the
+    statistics with block maxima and the threshold on them; what those refuse stays refused."""
+    from fgattn_tk_cuda_amd.spattn import mask_utils as mu
+
+    print("case onepass", S, D, dense, flush=True)
+    ops = torch.ops.cuda_attn
+    g = torch.Generator(device=dev).manual_seed(S)
+    q, k, v = (torch.randn((2, 3, S, D), generator=g, device=dev).to(torch.bfloat16) for _ in range(3))
+    thresh, o = 4.0 / S, torch.empty_like(q)
+    m, d = mu._stats_buffers(q)
+    blockmax = mu.blockmax_buffer(q)
+    if dense:
+        ops.fullattn_maxq_denom_blockmax(o, m, d, blockmax, q, k, v, 0.0, 0)
+    else:
+        ops.maxq_denom_blockmax(m, d, blockmax, q, k, 0.0, 0)
+    packed = mu.qk_packedmask_from_blockmax_cuda(blockmax, m, d, q, k, thresh)
+    extra = lambda: (torch.zeros_like(q), q, k, v) if dense else (None, q, k, None)
+    got, a = torch.full_like(packed, 0x5a), extra()
+    ops.onepass_packedmask(got, *a, thresh)
+    assert torch.equal(got, packed) and (not dense or torch.equal(a[0], o))
+    for qblk in (64, 128):
+        idx, cnt = mu.blockmax_to_blocklists_cuda(blockmax, m, d, thresh, S, D, qblk)
+        gi, gc, a = torch.full_like(idx, 7), torch.full_like(cnt, 7), extra()
+        ops.onepass_blocklists(gi, gc, *a, thresh, qblk)
+        assert torch.equal(gi, idx) and torch.equal(gc, cnt) and (not dense or torch.equal(a[0], o))
+    for bad in ((got[..., :-1].contiguous(), *extra(), thresh), (got, None, q, k, v, thresh), (got, None, q, k[:, :, :-1].contiguous(), None, thresh),
+                (got, None, q.float(), k, None, thresh)):
+        with pytest.raises(RuntimeError):
+            ops.onepass_packedmask(*bad)
+    with pytest.raises(RuntimeError):
+        ops.onepass_blocklists(gi, gc, *extra(), thresh, 96)
