@@ -70,13 +70,13 @@ constexpr int attn_lds_bytes() {
 }
 
 // Waves per SIMD the register allocation aims at.  Two (256 registers), except at d = 64 with 128-row q-blocks,
-// where 168 registers are enough for dense attention and block lists with a handful of spills outside the tile
-// loop: the 40 KB ring lets three workgroups share a CU, and these kernels are bound by the vector ALU, which a
-// third wave keeps fed (side by side: block lists -7 %, dense 16 x 16384 1.203 -> 1.178 ms, with statistics 1.253 ->
-// 1.222 ms).  Token lists of that shape need 184 registers and spill in the loop for it (0.72 -> 0.83 ms).
+// where 168 registers are enough with a handful of spills outside the tile loop: the 40 KB ring lets three workgroups
+// share a CU, and these kernels are bound by the vector ALU, which a third wave keeps fed (side by side: block lists
+// -7 %, dense 16 x 16384 1.203 -> 1.178 ms, with statistics 1.253 -> 1.222 ms; token lists, without SPLIT_SM, 24 x 32760
+// 671 -> 643 us, 40 x 12468 319 -> 308 us; with it they spill in the loop and gain 1 % or lose 4).
 template <int D, int QBLK, int MODE>
 constexpr int attn_waves_per_simd() {
-  return (D == 64 && QBLK == 128 && MODE != KV_TOKENS) ? 3 : 2;
+  return (D == 64 && QBLK == 128) ? 3 : 2;
 }
 
 template <int D, int QBLK, int MODE, bool HAS_V, bool STATS>
@@ -388,8 +388,10 @@ void attn_fwd_kernel(const AttnParams p) {
   // block under the P V multiplies of the tile before, registers 8-15 under the QK^T multiplies
   // of the tile after, so that every multiply has the same vector-ALU work next to it (all of
   // it under QK^T leaves the vector ALU the bottleneck there and idle under P V).  Needs the
-  // reference fixed before the tile's scores exist, which LAZY_MAX gives.
-  constexpr bool SPLIT_SM = LAZY_MAX && HAS_V;
+  // reference fixed before the tile's scores exist, which LAZY_MAX gives.  Not with token lists of 128-row q-blocks at
+  // d = 64, whose third wave needs the 16 registers of the second set of operands (dense attention and block lists of
+  // that shape fit with both and lose 1 % without).
+  constexpr bool SPLIT_SM = LAZY_MAX && HAS_V && !(MODE == KV_TOKENS && D == 64 && QBLK == 128);
   u32x4 pb[SPLIT_SM ? 2 : 1][HAS_V ? 2 * NMB : 1];   // P^T operands, k-step 2mb + h; SPLIT_SM: by tile parity
 
   // Per-lane LDS addresses inside slot 0; slot, score block and k-step offsets are added
@@ -397,7 +399,7 @@ void attn_fwd_kernel(const AttnParams p) {
   // A operand of QK^T, k-step t, score block 0.  K_XOR (the forms held to 168 registers): only the address of
   // k-step 0 is kept, that of k-step t is the same with t XORed into chunk bits 1-3 (at d = 128, where the
   // registers reach, keeping all of them is 1 % faster).
-  constexpr bool K_XOR = (QBLK == 128 && HAS_V && D == 64 && MODE != KV_TOKENS);
+  constexpr bool K_XOR = (QBLK == 128 && HAS_V && D == 64);
   lds_cptr k_lo[K_XOR ? 1 : NT];
   {
     const int krow = ksub * KW + ln;
@@ -575,7 +577,7 @@ void attn_fwd_kernel(const AttnParams p) {
   // group as soon as its multiply of this group has been issued (two buffers: at d = 128 sixteen registers
   // more and 0.2-0.6 % slower, at d = 64 spills in the loop and 0.8 % slower).
   constexpr int NG = 2 * NMB;
-  constexpr int VB = (QBLK == 128 && (D == 128 || (LAZY_MAX && MODE != KV_TOKENS))) ? 1 : 2;
+  constexpr int VB = (QBLK == 128 && (D == 128 || LAZY_MAX)) ? 1 : 2;
   u32x2 va[HAS_V ? VB : 1][HAS_V ? NDB : 1][2];
   auto v_read_db = [&](uint32_t vofs, int gi, int db) {
     if constexpr (HAS_V) {
