@@ -64,9 +64,9 @@ struct AttnCfg {
 
 // LDS of one workgroup.  Statistics over 64-row q-blocks: the two waves that share the rows of a tile also exchange
 // its row maxima, for the block maxima (two tiles x 64 rows, behind the ring).
-template <int D, int QBLK, int MODE, bool HAS_V, bool STATS>
+template <int D, int QBLK, int MODE, bool HAS_V, bool STATS, int NGRP>
 constexpr int attn_lds_bytes() {
-  return AttnCfg<D, MODE, HAS_V>::kTotal + ((STATS && QBLK == 64) ? 2 * 64 * 4 : 0);
+  return NGRP * (AttnCfg<D, MODE, HAS_V>::kTotal + ((STATS && QBLK == 64) ? 2 * 64 * 4 : 0));
 }
 
 // Waves per SIMD the register allocation aims at.  Two (256 registers), except at d = 64 with 128-row q-blocks,
@@ -74,14 +74,18 @@ constexpr int attn_lds_bytes() {
 // share a CU, and these kernels are bound by the vector ALU, which a third wave keeps fed (side by side: block lists
 // -7 %, dense 16 x 16384 1.203 -> 1.178 ms, with statistics 1.253 -> 1.222 ms; token lists, without SPLIT_SM, 24 x 32760
 // 671 -> 643 us, 40 x 12468 319 -> 308 us; with it they spill in the loop and gain 1 % or lose 4).
-template <int D, int QBLK, int MODE>
+template <int D, int QBLK, int NGRP>
 constexpr int attn_waves_per_simd() {
-  return (D == 64 && QBLK == 128) ? 3 : 2;
+  return (D == 64 && QBLK == 128 && NGRP == 1) ? 3 : 2;
 }
 
-template <int D, int QBLK, int MODE, bool HAS_V, bool STATS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(attn_waves_per_simd<D, QBLK, MODE>())))
+// NGRP = 2 (dense attention and statistics of launches that leave the chip idle): two groups of four waves share a
+// q-block, each with a ring of its own and half of the tiles; both meet at the same barriers and finish half of the
+// columns each.
+template <int D, int QBLK, int MODE, bool HAS_V, bool STATS, int NGRP>
+__global__ __launch_bounds__(256 * NGRP) __attribute__((amdgpu_waves_per_eu(attn_waves_per_simd<D, QBLK, NGRP>())))
 void attn_fwd_kernel(const AttnParams p) {
+  static_assert(NGRP == 1 || MODE == KV_DENSE, "groups share dense tiles");
   static_assert(D == 64 || D == 128, "head dim");
   static_assert(QBLK == 64 || QBLK == 128, "q-block");
   using Cfg = AttnCfg<D, MODE, HAS_V>;
@@ -99,11 +103,13 @@ void attn_fwd_kernel(const AttnParams p) {
   constexpr int NK = Cfg::kKSlots;
   constexpr float kNegInf = -__builtin_huge_valf();
 
-  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem_all[];
+  const int grp = NGRP == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  unsigned char* const smem = smem_all + grp * Cfg::kTotal;   // this group's ring
   const lds_cptr smem_l = (lds_cptr)smem;
   const uint32_t smem_base = (uint32_t)(uintptr_t)smem_l;
 
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x & 255;   // within the group
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 31;
@@ -142,6 +148,10 @@ void attn_fwd_kernel(const AttnParams p) {
     n = n < 0 ? 0 : (n > p.idx_stride ? p.idx_stride : n);
     ntiles = (MODE == KV_TOKENS) ? ((n + 63) >> 6) : n;
   }
+  // Two groups: of an odd number of tiles the second group's last one is behind the sequence, a tile without keys.
+  const int all_tiles = ntiles;
+  if constexpr (NGRP == 2) ntiles = (all_tiles + 1) >> 1;
+  const int t0 = NGRP == 1 ? 0 : grp * ntiles;   // this group's first tile
   const int last_row = p.kv_len - 1;
 
   // ---- loader role: load i of a tile covers rows RPL*(4i + wave) .. +RPL-1 ----------
@@ -182,7 +192,7 @@ void attn_fwd_kernel(const AttnParams p) {
   // past the end of the list may be asked for (prefetch), their descriptors are never used.
   const bool kv_short = p.kv_len < 64;
   auto tile_desc = [&](int t) -> int {
-    int id = t;
+    int id = t0 + t;
     if constexpr (MODE == KV_BLOCKS) id = lst[t < p.idx_stride ? t : p.idx_stride - 1];
     const bool valid = id >= 0 && id <= (last_row >> 6);
     const int r0 = valid ? id * 64 : 0;
@@ -480,19 +490,22 @@ void attn_fwd_kernel(const AttnParams p) {
   // pre-pass, softmax(r, c) > tau, holds for some key of block J exactly when the block's maximum
   // passes it, so these S x S/64 numbers replace the second score sweep for block-level masks.
   constexpr bool BLOCKMAX = STATS && MODE == KV_DENSE;
-  float* const bm_xchg = reinterpret_cast<float*>(smem + Cfg::kTotal);   // KSPLIT == 2
+  float* const bm_xchg = reinterpret_cast<float*>(smem_all + NGRP * Cfg::kTotal) + grp * 128;   // KSPLIT == 2
+  auto blockmax_at = [&](int tile) -> uint16_t& {   // tile of this group
+    return p.blockmax[((size_t)bh * (p.Sp >> 6) + (t0 + tile)) * p.Sp + qrow];
+  };
+  auto tile_exists = [&](int tile) -> bool { return NGRP == 1 || t0 + tile < all_tiles; };
   float bm_own = kNegInf;
   auto blockmax_merge = [&](int tile) {   // behind the barrier that follows the maxima of this tile
     if constexpr (BLOCKMAX && KSPLIT == 2) {
-      if (p.blockmax != nullptr && ksub == 0 && g == 0)
-        p.blockmax[((size_t)bh * (p.Sp >> 6) + tile) * p.Sp + qrow] =
-            bf16_round_up(max_raw(bm_own, bm_xchg[(tile & 1) * 64 + 32 * qsub + ln]));
+      if (p.blockmax != nullptr && ksub == 0 && g == 0 && tile_exists(tile))
+        blockmax_at(tile) = bf16_round_up(max_raw(bm_own, bm_xchg[(tile & 1) * 64 + 32 * qsub + ln]));
     }
   };
   auto stat_finish = [&](float mloc, int tile) -> float {
     mloc = pair_max(mloc);
     if constexpr (BLOCKMAX && KSPLIT == 1) {
-      if (p.blockmax != nullptr && g == 0) p.blockmax[((size_t)bh * (p.Sp >> 6) + tile) * p.Sp + qrow] = bf16_round_up(mloc);
+      if (p.blockmax != nullptr && g == 0 && tile_exists(tile)) blockmax_at(tile) = bf16_round_up(mloc);
     }
     if constexpr (BLOCKMAX && KSPLIT == 2) {
       // the wave with the upper keys hands its maxima over; they are read behind the next barrier, and a slot is
@@ -914,7 +927,7 @@ void attn_fwd_kernel(const AttnParams p) {
       }
     }
     __syncthreads();
-    if (ksub == 1) return;
+    if (NGRP == 1 && ksub == 1) return;
     const float m2 = mg[lane];
     const float l2 = mg[64 + lane];
     m_true = fmaxf(m_true, mg[128 + lane]);
@@ -923,7 +936,7 @@ void attn_fwd_kernel(const AttnParams p) {
     const float a2 = (m2 == kNegInf) ? 0.f : __builtin_amdgcn_exp2f(m2 - new_sf);
     l_tot = l_tot * a1 + l2 * a2;
     mr_sf = new_sf;
-    if constexpr (HAS_V) {
+    if constexpr (HAS_V) if (NGRP == 1 || ksub == 0) {
 #pragma unroll
       for (int db = 0; db < NDB; ++db)
 #pragma unroll
@@ -935,19 +948,75 @@ void attn_fwd_kernel(const AttnParams p) {
     }
   }
 
+  // Two groups: a wave hands the half of the columns that it does not finish to the wave with the same rows in the
+  // other group, as above; blocks 0 .. ODB-1 of the accumulators are its own half from here on.
+  constexpr int ODB = HAS_V ? NDB / NGRP : 0;
+  constexpr int kHand = (ODB * 16 + 3) * 64;                       // floats
+  constexpr int kHandAt = KSPLIT == 2 ? Cfg::kMerge : 0;           // behind what the key halves exchanged
+  if constexpr (NGRP == 2) {
+    static_assert(kHandAt + NQW * kHand * 4 <= Cfg::kTotal, "the exchange must fit the ring");
+    float* mine = reinterpret_cast<float*>(smem + kHandAt) + qsub * kHand;
+    const float* theirs = reinterpret_cast<const float*>(smem_all + (grp ^ 1) * Cfg::kTotal + kHandAt) + qsub * kHand;
+    if (ksub == 0) {
+      mine[lane] = mr_sf;
+      mine[64 + lane] = l_tot;
+      mine[128 + lane] = m_true;
+      auto hand_over = [&](auto first) {
+        constexpr int D0 = decltype(first)::value;
+#pragma unroll
+        for (int db = 0; db < ODB; ++db)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const f32x16& a = oacc[D0 + db];
+            reinterpret_cast<f32x4*>(mine + 192)[(db * 4 + j) * 64 + lane] = f32x4{a[4 * j], a[4 * j + 1], a[4 * j + 2], a[4 * j + 3]};
+          }
+      };
+      if (grp == 0) {
+        hand_over(std::integral_constant<int, ODB>{});
+      } else {
+        hand_over(std::integral_constant<int, 0>{});
+#pragma unroll
+        for (int db = 0; db < ODB; ++db) oacc[db] = oacc[ODB + db];
+      }
+    }
+    __syncthreads();
+    if (ksub == 1) return;
+    const float m2 = theirs[lane];
+    const float l2 = theirs[64 + lane];
+    m_true = fmaxf(m_true, theirs[128 + lane]);
+    const float new_sf = fmaxf(mr_sf, m2);
+    const float a1 = (mr_sf == kNegInf) ? 0.f : __builtin_amdgcn_exp2f(mr_sf - new_sf);
+    const float a2 = (m2 == kNegInf) ? 0.f : __builtin_amdgcn_exp2f(m2 - new_sf);
+    // the same sums in both groups: the first group's part times its factor, plus the second's
+    auto join = [&](float own, float other) -> float {
+      return grp == 0 ? __builtin_fmaf(own, a1, other * a2) : __builtin_fmaf(other, a2, own * a1);
+    };
+    l_tot = join(l_tot, l2);
+    mr_sf = new_sf;
+#pragma unroll
+    for (int db = 0; db < ODB; ++db)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f32x4 x = reinterpret_cast<const f32x4*>(theirs + 192)[(db * 4 + j) * 64 + lane];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) oacc[db][4 * j + i] = join(oacc[db][4 * j + i], x[i]);
+      }
+  }
+
   // ---- epilogue --------------------------------------------------------------------
-  // The wave's 32 x D output tile is one contiguous piece of O.  It is turned from "a lane
-  // holds a row" into "a lane holds 16 consecutive bytes" through a wave-private piece of
+  // The wave's 32 x D output tile is one contiguous piece of O (two groups: 32 x D/2, half rows).  It is turned from
+  // "a lane holds a row" into "a lane holds 16 consecutive bytes" through a wave-private piece of
   // LDS (row pitch + 8 bytes: conflict-free both ways), so that every store instruction
   // writes whole cache lines.
   if constexpr (HAS_V) {
-    constexpr int RS = ROWB + 8;
-    constexpr int EP0 = (KSPLIT == 2) ? Cfg::kMerge : 0;
+    constexpr int OC = CPR / NGRP;      // 16-byte chunks of a row
+    constexpr int RS = OC * 16 + 8;
+    constexpr int EP0 = NGRP == 2 ? kHandAt + NQW * kHand * 4 : (KSPLIT == 2) ? Cfg::kMerge : 0;
     static_assert(EP0 + NQW * 32 * RS <= Cfg::kRing, "output staging must fit the ring");
     unsigned char* ep = smem + EP0 + qsub * 32 * RS;
     const float inv = (l_tot > 0.f) ? 1.f / l_tot : 0.f;
 #pragma unroll
-    for (int db = 0; db < NDB; ++db)
+    for (int db = 0; db < ODB; ++db)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         u32x2 w;
@@ -957,9 +1026,9 @@ void attn_fwd_kernel(const AttnParams p) {
       }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    constexpr int RPI = 64 / CPR;     // rows per store instruction
-    const int er = lane / CPR, ec = lane % CPR;
-    uint16_t* otile = p.o + head_off + (size_t)q0 * D;
+    constexpr int RPI = 64 / OC;      // rows per store instruction
+    const int er = lane / OC, ec = lane % OC;
+    uint16_t* otile = p.o + head_off + (size_t)q0 * D + (NGRP == 2 ? grp * (D / 2) : 0);
 #pragma unroll
     for (int i = 0; i < 32 / RPI; ++i) {
       const int row = i * RPI + er;
@@ -969,7 +1038,7 @@ void attn_fwd_kernel(const AttnParams p) {
       if (q0 + row < p.S) *reinterpret_cast<u32x4*>(otile + (size_t)row * D + ec * 8) = w;
     }
   }
-  if (g == 0) {
+  if (g == 0 && grp == 0) {
     if (p.lse != nullptr && qrow_ok) {
       p.lse[(size_t)bh * p.S + qrow] = (l_tot > 0.f) ? (mr_sf + __log2f(l_tot)) * kLn2 : kNegInf;
     }
@@ -990,23 +1059,23 @@ void attn_fwd_kernel(const AttnParams p) {
 // Raises the dynamic-LDS limit of one instantiation on the current device (once per device; the
 // launcher does it on the first launch, a caller that is about to record launches into a graph
 // does it beforehand through spattn_init).
-template <int D, int QBLK, int MODE, bool HAS_V, bool STATS>
+template <int D, int QBLK, int MODE, bool HAS_V, bool STATS, int NGRP = 1>
 inline hipError_t prepare_attn_fwd() {
   static bool attr_set[kMaxDevices] = {};
-  return raise_lds_limit(reinterpret_cast<const void*>(attn_fwd_kernel<D, QBLK, MODE, HAS_V, STATS>),
-                         attn_lds_bytes<D, QBLK, MODE, HAS_V, STATS>(), attr_set);
+  return raise_lds_limit(reinterpret_cast<const void*>(attn_fwd_kernel<D, QBLK, MODE, HAS_V, STATS, NGRP>),
+                         attn_lds_bytes<D, QBLK, MODE, HAS_V, STATS, NGRP>(), attr_set);
 }
 
 // Host launcher; returns hipError_t of the launch.
-template <int D, int QBLK, int MODE, bool HAS_V, bool STATS>
+template <int D, int QBLK, int MODE, bool HAS_V, bool STATS, int NGRP = 1>
 inline hipError_t launch_attn_fwd(const AttnParams& p, hipStream_t stream) {
-  auto kern = attn_fwd_kernel<D, QBLK, MODE, HAS_V, STATS>;
-  const hipError_t ea = prepare_attn_fwd<D, QBLK, MODE, HAS_V, STATS>();
+  auto kern = attn_fwd_kernel<D, QBLK, MODE, HAS_V, STATS, NGRP>;
+  const hipError_t ea = prepare_attn_fwd<D, QBLK, MODE, HAS_V, STATS, NGRP>();
   if (ea != hipSuccess) return ea;
   const int total = p.nqblk * p.H * p.B;
   if (total <= 0) return hipSuccess;
-  constexpr int kLds = attn_lds_bytes<D, QBLK, MODE, HAS_V, STATS>();
-  hipLaunchKernelGGL(kern, dim3(total), dim3(256), kLds, stream, p);
+  constexpr int kLds = attn_lds_bytes<D, QBLK, MODE, HAS_V, STATS, NGRP>();
+  hipLaunchKernelGGL(kern, dim3(total), dim3(256 * NGRP), kLds, stream, p);
   return hipGetLastError();
 }
 

@@ -1,34 +1,46 @@
-// Dense attention / row-statistics instantiations: q-blocks of 128 rows, of 64 rows for launches that leave
-// the chip idle with 128.
+// Dense attention / row-statistics instantiations: q-blocks of 128 rows, and for launches that leave the chip idle with
+// those, of 64 rows and of either size with two groups of waves per q-block.
 #include "attn_fwd.h"
 #include "dispatch.h"
 
 namespace spattn {
 
-// With 64-row q-blocks two waves share the rows of a tile and take half of its keys each: a q-block is done in
-// 0.65-0.8 of the time, for twice the K / V copies per row.  That pays while the 64-row q-blocks do not queue:
-//   up to one per CU (256), at both head dims: dense 256 keys 1.07-1.13x, 1000 keys 1.25-1.37x, 4096 keys 1.37-1.51x
-//   (16 x 512 x 128 11.1 -> 9.6 us, 4 x 4096 x 128 58.9 -> 42.8 us, 4 x 4096 x 64 46.4 -> 30.8 us); with statistics
-//   1.11-1.42x (8 x 2048 x 128 34.7 -> 25.5 us), statistics only 1.14-1.38x;
-//   at d = 64 from 768 keys on up to three per CU, what its 40 KB ring and registers allow (768): dense 1.04-1.15x
-//   (24 x 1536 27.0 -> 23.5 us), with statistics 1.02-1.07x, statistics only 1.02-1.12x.  At 256 and 512 keys that
-//   is 0.92-1.08x, behind 768 q-blocks 0.88-0.93x (64 x 1000 21.9 -> 24.3 us).  d = 128 loses 0.81-0.99x (with
-//   statistics 0.65-0.83x, its LDS allows one workgroup per CU) from the second q-block per CU on.
-// The two forms add the row sums and outputs of a row in another order: a launch over some heads of a computation
+// The four forms: q-blocks of 128 or 64 rows (64: two waves share the rows of a tile and take half of its keys each),
+// by one group of four waves or two (which take half of the tiles each).  A q-block is done sooner the more waves share
+// it, for more K / V copies per row and a merge; that pays while the q-blocks do not queue.  Measured as time over that
+// of the 128-row form by one group, unless said otherwise:
+//   64-row q-blocks, up to one per CU (256), both head dims: dense 256 keys 0.89-0.93, 1000 keys 0.73-0.80, 4096 keys
+//   0.66-0.73; with statistics 0.70-0.90, statistics only 0.72-0.88;
+//   at d = 64 from 768 keys on up to three per CU, what the 40 KB ring and registers allow (768): dense 0.87-0.96, with
+//   statistics 0.93-0.98, statistics only 0.89-0.98; at 256 and 512 keys that is 0.93-1.09, behind 768 q-blocks 1.08-1.14.
+//   d = 128 is slower (1.02-1.2, with statistics 1.2-1.5: its LDS allows one workgroup per CU) from the second q-block per
+//   CU on, except the statistics alone, whose ring is 48 KB, from 768 keys on: 0.90-0.96 up to three per CU, 1.12-1.2 behind.
+//   Two groups on 64-row q-blocks, up to one per CU, against one group on them: d = 64 from 12 tiles on 0.72-0.95 (8 tiles
+//   1.00-1.02), d = 128 from 15 on 0.75-1.00 (12 tiles 0.99, 8 tiles 1.07-1.13).  Dense with statistics at d = 128 has no LDS
+//   for it.
+//   Two groups on 128-row q-blocks, up to one per CU, against the best of the other forms: d = 128 from 12 tiles on 0.84-0.95
+//   (8 tiles 0.98-1.06); d = 64 from 24 tiles on 0.90-0.98, with statistics from 15 on 0.92-0.96 (below 0.97-1.02).
+// The forms add the row sums and outputs of a row in another order: a launch over some heads of a computation
 // goes by all of its heads, so that a row's denominator, and with it a key at a threshold, does not depend on the split.
-static bool small_launch(const AttnParams& p, int D, int heads) {
-  constexpr int kCus = 256;
-  const long long n64 = (long long)(heads > 0 ? heads : p.B * p.H) * ((p.S + 63) / 64);
-  return n64 <= kCus || (D == 64 && p.kv_len >= 768 && n64 <= 3 * kCus);
-}
-
 template <int D, bool HAS_V, bool STATS>
 static hipError_t run(const AttnParams& p, int heads, hipStream_t stream) {
-  if (!small_launch(p, D, heads)) return launch_attn_fwd<D, 128, KV_DENSE, HAS_V, STATS>(p, stream);
+  constexpr int kCus = 256;
+  const long long hb = heads > 0 ? heads : p.B * p.H;
+  const long long n64 = hb * ((p.S + 63) / 64), n128 = hb * ((p.S + 127) / 128);
+  const int tiles = (p.kv_len + 63) / 64;
   AttnParams p64 = p;
   // the statistics cover the rows up to Sp
   p64.nqblk = (STATS ? p.Sp : p.S + 63) / 64;
-  return launch_attn_fwd<D, 64, KV_DENSE, HAS_V, STATS>(p64, stream);
+  if (n64 <= kCus) {
+    if constexpr (!(D == 128 && HAS_V && STATS)) {
+      if (tiles >= (D == 64 ? 12 : 15)) return launch_attn_fwd<D, 64, KV_DENSE, HAS_V, STATS, 2>(p64, stream);
+    }
+    return launch_attn_fwd<D, 64, KV_DENSE, HAS_V, STATS>(p64, stream);
+  }
+  if (n128 <= kCus && tiles >= (D == 128 ? 12 : STATS ? 15 : 24))
+    return launch_attn_fwd<D, 128, KV_DENSE, HAS_V, STATS, 2>(p, stream);
+  if ((D == 64 || !HAS_V) && p.kv_len >= 768 && n64 <= 3 * kCus) return launch_attn_fwd<D, 64, KV_DENSE, HAS_V, STATS>(p64, stream);
+  return launch_attn_fwd<D, 128, KV_DENSE, HAS_V, STATS>(p, stream);
 }
 
 hipError_t run_attn_dense(const AttnParams& p, int D, bool has_v, bool stats, hipStream_t stream, int heads) {
@@ -49,6 +61,11 @@ static hipError_t prepare() {
   hipError_t e = prepare_attn_fwd<D, QBLK, KV_DENSE, true, false>();
   if (e == hipSuccess) e = prepare_attn_fwd<D, QBLK, KV_DENSE, true, true>();
   if (e == hipSuccess) e = prepare_attn_fwd<D, QBLK, KV_DENSE, false, true>();
+  if (e == hipSuccess) e = prepare_attn_fwd<D, QBLK, KV_DENSE, true, false, 2>();
+  if constexpr (!(D == 128 && QBLK == 64)) {
+    if (e == hipSuccess) e = prepare_attn_fwd<D, QBLK, KV_DENSE, true, true, 2>();
+  }
+  if (e == hipSuccess) e = prepare_attn_fwd<D, QBLK, KV_DENSE, false, true, 2>();
   return e;
 }
 

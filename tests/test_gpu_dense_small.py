@@ -57,3 +57,47 @@ def test_small_launches_match_large_ones(dev, D, S, kv_len):
         assert bool((r["m"][..., S:] == 0).all())
         n = r["m"].shape[1]
         assert torch.equal(r["m"], large["m"][:, :n]) and torch.equal(r["bm"][..., :S], large["bm"][:, :n][..., :S])
+
+
+@pytest.mark.parametrize("D,S,kv_len", [
+    (64, 705, 0), (64, 769, 768), (64, 900, 833), (64, 1472, 1409), (64, 1537, 0), (128, 704, 0), (128, 705, 0), (128, 897, 769),
+    (128, 961, 960), (128, 961, 897), (128, 1100, 1025),
+])
+def test_two_groups_match_one(dev, D, S, kv_len):
+    """Launches on both sides of the rules that let two groups of waves share a q-block, by numbers of heads and of key
+    tiles (odd numbers leave the second group a tile without keys): outputs and statistics against fp32, row and block
+    maxima bit for bit those of the largest launch."""
+    import fgattn_tk_cuda_amd.spattn.cuda_attn  # noqa: F401
+
+    print("case dense two groups", D, S, kv_len, flush=True)
+    ops = torch.ops.cuda_attn
+    n64, n128 = (S + 63) // 64, (S + 127) // 128
+    heads = sorted({max(1, 256 // n64), 256 // n64 + 1, 256 // n128, 256 // n128 + 1, 768 // n64, 768 // n64 + 1})
+    g = torch.Generator(device=dev).manual_seed(S + D)
+    q, k, v = (torch.randn((1, heads[-1], S, D), generator=g, device=dev).to(torch.bfloat16) for _ in range(3))
+    kv, sp = kv_len or S, n128 * 128
+    s = (q[:, :2].float() @ k[:, :2, :kv].float().transpose(2, 3).contiguous()) * D ** -0.5
+    want, want_lse = f32(torch.softmax(s, -1) @ v[:, :2, :kv].float()), f32(torch.logsumexp(s, -1))
+    largest = None
+    for h in reversed(heads):
+        a = [t[:, :h].contiguous() for t in (q, k, v)]
+        nan = lambda *shape: torch.full(shape, float("nan"), device=dev)
+        o, o2, lse = torch.full_like(a[0], float("nan")), torch.full_like(a[0], float("nan")), nan(1, h, S)
+        m, d, m3, d3 = (nan(1, h, 1, sp) for _ in range(4))
+        bm, bm3 = (torch.full((1, h, sp // 64 + 1, sp), 7.0, device=dev, dtype=torch.bfloat16)[:, :, :-1].contiguous() for _ in range(2))
+        ops.full_attn_ex(o, lse, *a, 0.0, kv_len)
+        ops.fullattn_maxq_denom_blockmax(o2, m, d, bm, *a, 0.0, kv_len)
+        ops.maxq_denom_blockmax(m3, d3, bm3, a[0], a[1], 0.0, kv_len)
+        for out in (o, o2):
+            assert_close_o(f32(out[:, :2]), want[:, :h], "o, %d heads" % h)
+        assert_close_stat(f32(lse[:, :2]), want_lse[:, :h], "lse", atol=1e-4)
+        tiles = (kv + 63) // 64
+        assert torch.equal(m, m3) and torch.equal(bm[..., :S], bm3[..., :S])
+        assert bool((bm[:, :, tiles:] == 7).all()) and bool((bm3[:, :, tiles:] == 7).all())   # blocks without a key stay unwritten
+        for den in (d, d3):
+            got = f32(m[:, :2, 0, :S]) * D ** -0.5 + f32(torch.log(den[:, :2, 0, :S]))
+            assert_close_stat(got, want_lse[:, :h], "statistics", atol=1e-4)
+            assert bool((den[..., S:] == float("-inf")).all())
+        if largest is None:
+            largest = m, bm
+        assert torch.equal(m, largest[0][:, :h]) and torch.equal(bm[..., :S], largest[1][:, :h, :, :S])
