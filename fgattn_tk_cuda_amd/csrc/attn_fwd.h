@@ -11,12 +11,12 @@
 // kv_len, row >= kv_len) are masked on every tile, a superset of the reference's "NaN row
 // -> -inf on the last tile" (include/asyncloadutils.cuh:124-142, include/pad_utils.cuh:54-75).
 //
-// Work split.  A workgroup is 4 waves (256 lanes) and owns one q-block of QBLK rows.
+// Work split.  A workgroup is 4 waves (256 lanes; QBLK = 256: 8 waves) and owns one q-block of QBLK rows.
 // Scores are produced transposed, S^T = K Q^T, so that in the 32x32 MFMA accumulator a
 // lane holds ONE query row (n = lane & 31) and 16 keys: every softmax statistic is a
 // per-lane scalar and only lanes l and l^32 ever exchange data.  O is accumulated
 // transposed too, O^T += V^T P^T, with P^T taken straight from the score accumulators.
-//   QBLK = 128: wave w owns query rows 32w..32w+31 and all 64 keys of a tile.
+//   QBLK = 128, 256: wave w owns query rows 32w..32w+31 and all 64 keys of a tile.
 //   QBLK =  64: wave w owns query rows 32(w&1).. and keys 32(w>>1).. of a tile; the two
 //               key halves are merged through LDS at the end.
 //
@@ -59,14 +59,19 @@ struct AttnCfg {
   static constexpr int kMerge = 2 * (D / 2 + 3) * 64 * 4;     // key-split merge, overlays the ring
   static constexpr int kTotal = (kRing > kMerge) ? kRing : kMerge;
   static constexpr int kRowsPerLoad = 1024 / (D * 2);         // rows one wave-wide 1 KB load covers
-  static constexpr int kLoadsPerTile = kTileBytes / 1024 / 4;   // per wave
 };
 
-// LDS of one workgroup.  Statistics over 64-row q-blocks: the two waves that share the rows of a tile also exchange
+// Waves of a group: they share a ring and its copies.
+template <int QBLK>
+constexpr int attn_waves() {
+  return QBLK == 256 ? 8 : 4;
+}
+
+// LDS of one workgroup.  256-row q-blocks hold their Q rows behind the ring until they are in registers.  Statistics over 64-row q-blocks: the two waves that share the rows of a tile also exchange
 // its row maxima, for the block maxima (two tiles x 64 rows, behind the ring).
 template <int D, int QBLK, int MODE, bool HAS_V, bool STATS, int NGRP>
 constexpr int attn_lds_bytes() {
-  return NGRP * (AttnCfg<D, MODE, HAS_V>::kTotal + ((STATS && QBLK == 64) ? 2 * 64 * 4 : 0));
+  return NGRP * (AttnCfg<D, MODE, HAS_V>::kTotal + ((STATS && QBLK == 64) ? 2 * 64 * 4 : 0)) + (QBLK == 256 ? QBLK * D * 2 : 0);
 }
 
 // Waves per SIMD the register allocation aims at.  Two (256 registers), except at d = 64 with 128-row q-blocks,
@@ -83,14 +88,15 @@ constexpr int attn_waves_per_simd() {
 // q-block, each with a ring of its own and half of the tiles; both meet at the same barriers and finish half of the
 // columns each.
 template <int D, int QBLK, int MODE, bool HAS_V, bool STATS, int NGRP>
-__global__ __launch_bounds__(256 * NGRP) __attribute__((amdgpu_waves_per_eu(attn_waves_per_simd<D, QBLK, NGRP>())))
+__global__ __launch_bounds__(64 * attn_waves<QBLK>() * NGRP) __attribute__((amdgpu_waves_per_eu(attn_waves_per_simd<D, QBLK, NGRP>())))
 void attn_fwd_kernel(const AttnParams p) {
   static_assert(NGRP == 1 || MODE == KV_DENSE, "groups share dense tiles");
   static_assert(D == 64 || D == 128, "head dim");
-  static_assert(QBLK == 64 || QBLK == 128, "q-block");
+  static_assert(QBLK == 64 || QBLK == 128 || (QBLK == 256 && MODE == KV_DENSE && HAS_V && D == 128 && NGRP == 1), "q-block");
   using Cfg = AttnCfg<D, MODE, HAS_V>;
   constexpr int NQW = QBLK / 32;     // waves along the query rows
-  constexpr int KSPLIT = 4 / NQW;    // waves along the keys of a tile
+  constexpr int WV = attn_waves<QBLK>();
+  constexpr int KSPLIT = WV / NQW;   // waves along the keys of a tile
   constexpr int KW = 64 / KSPLIT;    // keys of a tile per wave
   constexpr int NMB = KW / 32;       // 32-key score blocks per wave
   constexpr int NT = D / 16;         // k-steps of the QK^T product
@@ -98,18 +104,18 @@ void attn_fwd_kernel(const AttnParams p) {
   constexpr int CPR = D / 8;         // 16-byte chunks per row
   constexpr int ROWB = D * 2;        // bytes per row
   constexpr int TILE = Cfg::kTileBytes;
-  constexpr int LPT = Cfg::kLoadsPerTile;
+  constexpr int LPT = TILE / 1024 / WV;   // copies of a tile per wave
   constexpr int RPL = Cfg::kRowsPerLoad;
   constexpr int NK = Cfg::kKSlots;
   constexpr float kNegInf = -__builtin_huge_valf();
 
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_all[];
-  const int grp = NGRP == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  const int grp = NGRP == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * WV));
   unsigned char* const smem = smem_all + grp * Cfg::kTotal;   // this group's ring
   const lds_cptr smem_l = (lds_cptr)smem;
   const uint32_t smem_base = (uint32_t)(uintptr_t)smem_l;
 
-  const int tid = threadIdx.x & 255;   // within the group
+  const int tid = threadIdx.x & (64 * WV - 1);   // within the group
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 31;
@@ -154,7 +160,7 @@ void attn_fwd_kernel(const AttnParams p) {
   const int t0 = NGRP == 1 ? 0 : grp * ntiles;   // this group's first tile
   const int last_row = p.kv_len - 1;
 
-  // ---- loader role: load i of a tile covers rows RPL*(4i + wave) .. +RPL-1 ----------
+  // ---- loader role: load i of a tile covers rows RPL*(WV i + wave) .. +RPL-1 ----------
   const int ld_sub = lane / CPR;       // row within the load
   const int ld_slot = lane % CPR;      // 16-byte position within the row in LDS
   // Row r of a tile stores its 16-byte chunk c at position c ^ swz(r).  The swizzle has a
@@ -166,12 +172,12 @@ void attn_fwd_kernel(const AttnParams p) {
   auto swz = [](int r) -> int {
     return D == 128 ? (((r & 3) << 2) | ((r >> 2) & 3)) : ((((r >> 1) & 1) << 2) | ((r >> 2) & 3));
   };
-  // The loads of a tile are 4 RPL rows apart, a multiple of the swizzle period: one chunk
+  // The loads of a tile are WV RPL rows apart, a multiple of the swizzle period: one chunk
   // offset serves all of them.
-  static_assert((4 * RPL) % 16 == 0, "loads of one wave must share the swizzle");
+  static_assert((WV * RPL) % 16 == 0, "loads of one wave must share the swizzle");
   const int ld_row0 = RPL * wave + ld_sub;
   const int ld_off0 = (ld_slot ^ swz(ld_row0)) << 4;   // chunk offset within the row
-  auto ld_row = [&](int i) -> int { return ld_row0 + 4 * RPL * i; };
+  auto ld_row = [&](int i) -> int { return ld_row0 + WV * RPL * i; };
   auto ld_off = [&](int) -> int { return ld_off0; };
   uint32_t ld_go[LPT];                 // lane offset within a contiguous 64-row tile
 #pragma unroll
@@ -271,7 +277,7 @@ void attn_fwd_kernel(const AttnParams p) {
     }
     return tl;
   };
-  auto load_part = [&](const TileLoad& tl, int i) { dma16(tl.base, tl.go[i], tl.lds + i * 4096); };
+  auto load_part = [&](const TileLoad& tl, int i) { dma16(tl.base, tl.go[i], tl.lds + i * (WV * 1024)); };
   auto issue_tile = [&](int desc, int slot, bool is_v, auto gic) {
     const TileLoad tl = prepare_tile(desc, slot, is_v, gic);
 #pragma unroll
@@ -297,8 +303,9 @@ void attn_fwd_kernel(const AttnParams p) {
   // d = 64, whose 168 registers it spills, nor without V, where the slots it needs are those of K1 and K2.
   constexpr bool Q_LDS = HAS_V && (D == 128 || QBLK == 64);
   constexpr int NQ = 32 / RPL;   // copies
-  static_assert(NQ == 2 * LPT, "the rows of a wave fill its pieces of two slots");
-  auto q_piece = [&](int i) -> uint32_t {   // LDS address of copy i
+  static_assert(QBLK == 256 || NQ == 2 * LPT, "the rows of a wave fill its pieces of two slots");
+  auto q_piece = [&](int i) -> uint32_t {   // LDS address of copy i; 256-row q-blocks: behind the ring
+    if constexpr (QBLK == 256) return smem_base + Cfg::kTotal + (wave * NQ + i) * 1024;
     return smem_base + (uint32_t)(i < LPT ? 2 : NK + 1) * TILE + (i % LPT) * 4096 + wave * 1024;
   };
   if constexpr (MODE == KV_TOKENS) {
@@ -354,7 +361,8 @@ void attn_fwd_kernel(const AttnParams p) {
       if (head_pending == 2) wait_vmcnt<3 * LPT>(); else wait_vmcnt<2 * LPT>();
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        const uint32_t piece = q_piece(0) + ((ln / RPL) % LPT) * 4096 + (ln / RPL >= LPT ? (NK + 1 - 2) * TILE : 0);
+        const int i = ln / RPL;   // its copy
+        const uint32_t piece = q_piece(0) + (QBLK == 256 ? i * 1024 : (i % LPT) * 4096 + (i >= LPT ? (NK + 1 - 2) * TILE : 0));
         qf[t] = *(SPATTN_LDS const u32x4*)((lds_cptr)(uintptr_t)(piece + (ln % RPL) * ROWB + (((2 * t + g) ^ swz(ln)) << 4)));
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -505,7 +513,7 @@ void attn_fwd_kernel(const AttnParams p) {
   auto stat_finish = [&](float mloc, int tile) -> float {
     mloc = pair_max(mloc);
     if constexpr (BLOCKMAX && KSPLIT == 1) {
-      if (p.blockmax != nullptr && g == 0 && tile_exists(tile)) blockmax_at(tile) = bf16_round_up(mloc);
+      if (p.blockmax != nullptr && g == 0 && tile_exists(tile) && (QBLK != 256 || qrow < p.Sp)) blockmax_at(tile) = bf16_round_up(mloc);
     }
     if constexpr (BLOCKMAX && KSPLIT == 2) {
       // the wave with the upper keys hands its maxima over; they are read behind the next barrier, and a slot is
@@ -788,7 +796,7 @@ void attn_fwd_kernel(const AttnParams p) {
       auto poison = [&](int slot) {
         unsigned char* base = smem + slot * TILE + wave * 1024 + lane * 16;
 #pragma unroll
-        for (int i = 0; i < LPT; ++i) *reinterpret_cast<u32x4*>(base + i * 4096) = nan4;
+        for (int i = 0; i < LPT; ++i) *reinterpret_cast<u32x4*>(base + i * (WV * 1024)) = nan4;
       };
       if constexpr (HAS_V) poison(VN);
       if (has_kn) poison(KN);
@@ -1075,7 +1083,7 @@ inline hipError_t launch_attn_fwd(const AttnParams& p, hipStream_t stream) {
   const int total = p.nqblk * p.H * p.B;
   if (total <= 0) return hipSuccess;
   constexpr int kLds = attn_lds_bytes<D, QBLK, MODE, HAS_V, STATS, NGRP>();
-  hipLaunchKernelGGL(kern, dim3(total), dim3(256 * NGRP), kLds, stream, p);
+  hipLaunchKernelGGL(kern, dim3(total), dim3(64 * attn_waves<QBLK>() * NGRP), kLds, stream, p);
   return hipGetLastError();
 }
 

@@ -1,5 +1,5 @@
 // Dense attention / row-statistics instantiations: q-blocks of 128 rows, and for launches that leave the chip idle with
-// those, of 64 rows and of either size with two groups of waves per q-block.
+// those, of 64 rows and of either size with two groups of waves per q-block; of 256 rows for long launches at d = 128.
 #include "attn_fwd.h"
 #include "dispatch.h"
 
@@ -20,7 +20,14 @@ namespace spattn {
 //   for it.
 //   Two groups on 128-row q-blocks, up to one per CU, against the best of the other forms: d = 128 from 12 tiles on 0.84-0.95
 //   (8 tiles 0.98-1.06); d = 64 from 24 tiles on 0.90-0.98, with statistics from 15 on 0.92-0.96 (below 0.97-1.02).
-// The forms add the row sums and outputs of a row in another order: a launch over some heads of a computation
+// 256-row q-blocks by one group of eight waves (d = 128 with V): half of the K / V copies per row, at the power cap
+// worth 2-5 % of a full round of one q-block per CU (12 x 32768 5.49 -> 5.28 ms; 2048 keys 2 %, 1024 keys -1, 512 keys -5),
+// and a workgroup of its own finishes a CU's last q-block sooner than two do.  A last round that fills up to half of the CUs
+// costs it 0-19 % instead (its other form spreads that round over twice as many).  From 32 tiles on with the last round
+// empty or more than half full 0.91-0.98.  With statistics, whose row maxima keep the waves of a workgroup waiting for
+// each other, that holds up to two rounds (0.94-0.99; 12 x 9000 502 -> 471 us), behind them 1.00-1.04.  Same bits as the
+// 128-row form.
+// The other forms add the row sums and outputs of a row in another order: a launch over some heads of a computation
 // goes by all of its heads, so that a row's denominator, and with it a key at a threshold, does not depend on the split.
 template <int D, bool HAS_V, bool STATS>
 static hipError_t run(const AttnParams& p, int heads, hipStream_t stream) {
@@ -40,6 +47,15 @@ static hipError_t run(const AttnParams& p, int heads, hipStream_t stream) {
   if (n128 <= kCus && tiles >= (D == 128 ? 12 : STATS ? 15 : 24))
     return launch_attn_fwd<D, 128, KV_DENSE, HAS_V, STATS, 2>(p, stream);
   if ((D == 64 || !HAS_V) && p.kv_len >= 768 && n64 <= 3 * kCus) return launch_attn_fwd<D, 64, KV_DENSE, HAS_V, STATS>(p64, stream);
+  if constexpr (D == 128 && HAS_V) {
+    const long long n256 = hb * ((p.S + 255) / 256);
+    const long long last = n256 % kCus;
+    if (tiles >= 32 && (last == 0 || last > kCus / 2) && (!STATS || n256 <= 2 * kCus)) {
+      AttnParams p256 = p;
+      p256.nqblk = (p.S + 255) / 256;
+      return launch_attn_fwd<D, 256, KV_DENSE, HAS_V, STATS>(p256, stream);
+    }
+  }
   return launch_attn_fwd<D, 128, KV_DENSE, HAS_V, STATS>(p, stream);
 }
 
@@ -74,6 +90,8 @@ hipError_t prepare_attn_dense() {
   if (e == hipSuccess) e = prepare<128, 64>();
   if (e == hipSuccess) e = prepare<64, 128>();
   if (e == hipSuccess) e = prepare<64, 64>();
+  if (e == hipSuccess) e = prepare_attn_fwd<128, 256, KV_DENSE, true, false>();
+  if (e == hipSuccess) e = prepare_attn_fwd<128, 256, KV_DENSE, true, true>();
   return e;
 }
 

@@ -101,3 +101,41 @@ def test_two_groups_match_one(dev, D, S, kv_len):
         if largest is None:
             largest = m, bm
         assert torch.equal(m, largest[0][:, :h]) and torch.equal(bm[..., :S], largest[1][:, :h, :, :S])
+
+
+@pytest.mark.parametrize("S,kv_len,heads", [
+    (2049, 0, (50, 40)),          # 9 q-blocks of 256 rows per head, the last with one row, over rows behind Sp: 450 of them, 360
+    (2176, 2060, (50, 40)),       # key tiles behind the kv length, rows up to a multiple of 128
+    (2304, 2304, (57, 60)),       # 513: last round of one q-block, 540: statistics behind two rounds
+    (2303, 1985, (57, 56, 57)),   # 32 tiles
+    (2100, 1984, (57, 56)),       # 31 tiles
+])
+def test_256_row_qblocks_give_the_same_bits(dev, S, kv_len, heads):
+    """d = 128, launches on both sides of the rule for 256-row q-blocks: outputs, statistics and block maxima of the heads
+    they share are the same bits, and right."""
+    import fgattn_tk_cuda_amd.spattn.cuda_attn  # noqa: F401
+
+    print("case dense 256 rows", S, kv_len, heads, flush=True)
+    ops = torch.ops.cuda_attn
+    g = torch.Generator(device=dev).manual_seed(S)
+    q, k, v = (torch.randn((1, max(heads), S, 128), generator=g, device=dev).to(torch.bfloat16) for _ in range(3))
+    kv, sp = kv_len or S, (S + 127) // 128 * 128
+    s = (q[:, :1].float() @ k[:, :1, :kv].float().transpose(2, 3).contiguous()) * 128 ** -0.5
+    want, want_lse = f32(torch.softmax(s, -1) @ v[:, :1, :kv].float()), f32(torch.logsumexp(s, -1))
+    first = None
+    for h in heads:
+        a = [t[:, :h].contiguous() for t in (q, k, v)]
+        o, o2, lse = torch.full_like(a[0], float("nan")), torch.full_like(a[0], float("nan")), torch.empty((1, h, S), device=dev)
+        m, d = (torch.full((1, h, 1, sp), float("nan"), device=dev) for _ in range(2))
+        bm = torch.full((1, h, sp // 64, sp), 7.0, device=dev, dtype=torch.bfloat16)
+        ops.full_attn_ex(o, lse, *a, 0.0, kv_len)
+        ops.fullattn_maxq_denom_blockmax(o2, m, d, bm, *a, 0.0, kv_len)
+        assert_close_o(f32(o[:, :1]), want, "o")
+        assert_close_o(f32(o2[:, :1]), want, "o with statistics")
+        assert_close_stat(f32(lse[:, :1]), want_lse, "lse", atol=1e-4)
+        assert bool((d[..., S:] == float("-inf")).all()) and bool((m[..., S:] == 0).all())
+        got = (o, o2, lse, m, d, bm)
+        if first is None:
+            first = got
+        n = min(h, first[0].shape[1])
+        assert all(torch.equal(x[:, :n], y[:, :n]) for x, y in zip(got, first))
