@@ -465,8 +465,8 @@ void blockmax_to_blocklists(torch::Tensor blk_idx, torch::Tensor blk_cnt, OptTen
                "blockmax_to_blocklists");
 }
 
-// The threshold sweep over the (32-row group, 64-key block) pairs whose block maxima say that they can hold a
-// passing key: packed uint8 [B,H,ceil(S/128),mask_stride/8], bit for bit booleanmask_packed at qblk = 128.
+// The threshold sweep over the rows of each 64-key block whose block maxima say that they can hold a passing key
+// there: packed uint8 [B,H,ceil(S/128),mask_stride/8], bit for bit booleanmask_packed at qblk = 128.
 void blockmax_to_packedmask(torch::Tensor packed, torch::Tensor blockmax, torch::Tensor o_max_q, torch::Tensor o_denom,
                             torch::Tensor q, torch::Tensor k, double threshold, double scale, int64_t kv_len) {
   check_bhsd(q, "q", q);

@@ -222,7 +222,7 @@ int spattn_booleanmask_packed_blocks(void* packed, float threshold, int mask_str
 
 /* The threshold sweep behind a statistics sweep with block maxima: blockmax
  * ([batch,heads,Sp/64,Sp] of spattn_maxq_denom_blockmax / spattn_fullattn_maxq_denom_blockmax) says which
- * pairs of a 32-row group and a 64-key block can hold a passing key; only those are multiplied.  packed as
+ * rows can pass inside a 64-key block; only those are multiplied with it.  packed as
  * in spattn_booleanmask_packed at qblk = 128, bit for bit what that full sweep writes.  max_q, denom, scale
  * and kv_len must be those of the statistics sweep; mask_stride a multiple of 128 not below the kv length. */
 int spattn_blockmax_to_packedmask(void* packed, const void* blockmax, const float* max_q, const float* denom, const void* q,
