@@ -147,6 +147,31 @@ def test_votes_by_rows(dev, D, S, kv_len, stride, x):
     assert torch.equal(got, want) and bool(got.any()) == (x < 1e6)
 
 
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("D,S,bad", [(128, 2500, (2499, 700)), (64, 5000, (4999, 4096)), (128, 2100, (2048, 5)), (64, 300, (299, 31))])
+def test_votes_beside_rows_that_are_not_finite(dev, D, S, bad, value):
+    """A query row without a finite score never votes, in this sweep as in the full one - whichever row it is, also one
+    that fills up lists: the last, the first of the next chunk."""
+    from fgattn_tk_cuda_amd.spattn import mask_utils as mu
+
+    print("case votes beside", value, D, S, bad, flush=True)
+    ops = torch.ops.cuda_attn
+    g = torch.Generator(device=dev).manual_seed(S + D)
+    q, k = (torch.randn((1, 1, S, D), generator=g, device=dev).to(torch.bfloat16) for _ in range(2))
+    bits = []
+    for v in (value, 0.0):                                    # equal weights: no votes at this threshold
+        q[:, :, list(bad)] = v
+        max_q, denom = mu._stats_buffers(q)
+        blockmax = mu.blockmax_buffer(q)
+        ops.maxq_denom_blockmax(max_q, denom, blockmax, q, k, 0.0, 0)
+        want = mu.qk_packedmask_from_maxq_denom_cuda(max_q, denom, q, k, 20.0 / S, 128, 0)
+        got = torch.full_like(want, 0x5a)
+        ops.blockmax_to_packedmask(got, blockmax, max_q, denom, q, k, 20.0 / S, 0.0, 0)
+        assert torch.equal(got, want) and bool(got.any())
+        bits.append(got)
+    assert torch.equal(*bits)
+
+
 @pytest.mark.parametrize("S,D,dense", [(1, 64, True), (65, 128, False), (300, 64, True), (1300, 128, True), (2049, 64, False)])
 def test_onepass_operators_are_the_operators_one_by_one(dev, S, D, dense):
     """onepass_packedmask and onepass_blocklists: output, bits, lists with their tails and counts are those of the
