@@ -267,7 +267,9 @@ __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParam
       }
       // ---- 3: multiply the listed tiles ----
       if (nt > 0) {
-        // the row lists are written and read by this wave alone, in order
+        // The row lists are written and read by this wave alone, in order: the LDS keeps to it, and the compiler does,
+        // as vector types (the entries are read two and four at a time) may alias what was written.
+        asm volatile("" ::: "memory");
         struct Load {
           uint32_t off[LPP];
         };
@@ -280,8 +282,8 @@ __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParam
             const u32x2 e = *(const SPATTN_LDS u32x2*)(lrow + 16 * i + 4 * h);
             r[0] = e[0] & 0xffffu, r[1] = e[0] >> 16, r[2] = e[1] & 0xffffu, r[3] = e[1] >> 16;
           } else {
-            const uint32_t e = *(const SPATTN_LDS uint32_t*)(lrow + 16 * i + 2 * h);
-            r[0] = e & 0xffffu, r[1] = e >> 16;
+            const u16x2 e = *(const SPATTN_LDS u16x2*)(lrow + 16 * i + 2 * h);
+            r[0] = e[0], r[1] = e[1];
           }
           // "none" copies some row of the chunk
 #pragma unroll

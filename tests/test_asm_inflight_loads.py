@@ -16,7 +16,11 @@ holds only while the compiler puts no vector-memory instruction of its own into 
 third check finds the tile loop of every instantiation (one inner loop, closed by a branch back to
 its header) and asserts that it holds no scratch access (a spill) and no s_waitcnt vmcnt outside
 the asm statements (the compiler waiting for a load of its own).  The same holds for the walk of the votes kernel,
-from its first copy to the wait for the last one."""
+from its first copy to the wait for the last one.
+
+The votes kernel lists rows in LDS as 16-bit numbers and reads several entries at a time.  A read through another scalar
+type would be free to move ahead of the stores (type-based aliasing); the last check looks at the types of its LDS
+loads and stores before any optimisation."""
 import re
 import shutil
 import subprocess
@@ -211,3 +215,25 @@ def test_no_instruction_touches_a_register_with_a_load_in_flight(tmp_path):
         assert len(loops) >= 4, "%s: %d attention kernels found" % (unit, len(loops))
         for kernel, f in loops.items():
             assert f == (0, 0), "%s %s: tile loop not found, or scratch accesses / compiler vmcnt waits inside it: %s" % (unit, kernel, f)
+
+
+def scalar_lds_types(ir):
+    """({types loaded}, {types stored}) by scalar integer accesses to LDS in an LLVM listing; vector types alias everything."""
+    found = [set(re.findall(op + r" (?:volatile )?(%s)" % ty, "\n".join(l for l in ir.split("\n") if "ptr addrspace(3) " in l)))
+             for op, ty in (("load", r"i\d+(?=, ptr addrspace)"), ("store", r"i\d+(?= [%\w.-]+, ptr addrspace)"))]
+    return tuple(found)
+
+
+def test_scalar_lds_type_checker():
+    ir = ("  store i16 %a, ptr addrspace(3) %p, align 2, !tbaa !1\n  %b = load i32, ptr addrspace(3) %p, align 4\n"
+          "  %c = load <2 x i16>, ptr addrspace(3) %p, align 4\n  store i16 4096, ptr addrspace(3) %p\n  store i32 %x, ptr %y\n")
+    assert scalar_lds_types(ir) == ({"i32"}, {"i16"})
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None and not Path("/opt/rocm/bin/hipcc").exists(), reason="hipcc not found")
+def test_row_lists_are_read_as_they_were_written(tmp_path):
+    out = tmp_path / "votes.ll"
+    subprocess.run([build._hipcc(), *build.HIPCC_FLAGS, "-S", "-emit-llvm", "-Xclang", "-disable-llvm-passes", "--cuda-device-only", "-o",
+                    str(out), str(CSRC / VOTES_UNIT)], check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+    loaded, stored = scalar_lds_types(out.read_text())
+    assert "i16" in stored and loaded <= stored, (loaded, stored)
