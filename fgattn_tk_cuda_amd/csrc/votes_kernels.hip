@@ -7,7 +7,7 @@
 // to it: a wave holds 64 keys in registers, as the B operand, and takes from a chunk of q-blocks
 //   1. the block's maxima of the chunk's rows (contiguous: the maxima lie block by block), of which it keeps one bit
 //      per row, "may pass";
-//   2. the list of those rows, q-block by q-block, each filled up to a multiple of four;
+//   2. the list of those rows, q-block by q-block, each filled up to a multiple of four with a row of its own;
 //   3. the listed rows of Q, sixteen to a tile, copied through a ring in LDS that it fills itself (whole rows, so that
 //      the copies coalesce; no barrier) and multiplied with the 64 keys.  In the 16x16 accumulator lanes 16 g .. of
 //      register i hold row 4 g + i of the tile, so the ballot of sixteen keys has sixteen bits for each four of rows,
@@ -93,11 +93,11 @@ __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParam
   constexpr int NB = ROWS / 512;          // batches of four q-blocks
   static_assert(NS == 2, "the keys arrive in two halves of the ring's length");
   static_assert(CAP >= 32, "a batch of four q-blocks has up to 32 tiles");
-  static_assert(Cfg::kChunk < 64, "a lane writes the votes of one q-block");
+  static_assert(Cfg::kChunk <= 64, "a lane writes the votes of one q-block");
   __shared__ __attribute__((aligned(1024))) unsigned char ring_all[4 * NS * TILE];
-  __shared__ __attribute__((aligned(16))) float tab[ROWS + 4];             // minus the vote threshold of a row on its raw score
-  __shared__ __attribute__((aligned(16))) uint16_t list_row[4][CAP * 16];  // row within the chunk, ROWS: none
-  __shared__ unsigned long long votes[4][Cfg::kChunk + 1];                  // of a wave's keys, per q-block
+  __shared__ __attribute__((aligned(16))) float tab[ROWS];                 // minus the vote threshold of a row on its raw score
+  __shared__ __attribute__((aligned(16))) uint16_t list_row[4][CAP * 16];  // row within the chunk
+  __shared__ unsigned long long votes[4][Cfg::kChunk];                      // of a wave's keys, per q-block
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -147,7 +147,6 @@ __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParam
       const float tv = -(p.log2_thresh + (mq[i] * p.sf + __log2f(dn[i]))) * (1.f / p.sf);
       tab[256 * i + tid] = ok ? tv : -__builtin_huge_valf();
     }
-    if (tid < 4) tab[ROWS + tid] = -__builtin_huge_valf();
   }
   __syncthreads();
 
@@ -177,7 +176,7 @@ __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParam
   for (int w = 0; w < FW; ++w) any |= flags[w];
 
   SPATTN_LDS unsigned long long* vw = (SPATTN_LDS unsigned long long*)votes[wave];
-  if (lane <= Cfg::kChunk) vw[lane] = 0;
+  if (lane < Cfg::kChunk) vw[lane] = 0;
   if (__ballot(any != 0) != 0) {
     // A copy of a tile: lane h * CPR + pos of copy c fetches chunk pos ^ swz of row LPP h + c, so that the operand
     // reads below (sixteen lanes, one chunk of sixteen rows) cover all sixteen 16-byte bank groups.
@@ -238,8 +237,12 @@ __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParam
         const int start = myq == 0 ? ng : myq == 1 ? e0 : myq == 2 ? e1 : e2;
         const int end = myq == 0 ? e0 : myq == 1 ? e1 : myq == 2 ? e2 : e3;
         if (e3 > ng) {
-          // the last four of a q-block are filled up with a row that never votes
-          if (end > start) lrow[4 * end - 4 + (lane & 3)] = (uint16_t)ROWS;
+          // The last four of a q-block are filled up with one of its listed rows (whichever lane stores last), which only
+          // votes again: no row of another q-block, finite or not, is multiplied for this one.
+          if (f) {
+            const uint16_t first = (uint16_t)(512 * b + 8 * lane + __builtin_ctz(f));
+            *(SPATTN_LDS u16x4*)(lrow + 4 * end - 4) = u16x4{first, first, first, first};
+          }
           int pos = 4 * start + before;
 #pragma unroll
           for (int i = 0; i < 8; ++i)
@@ -257,7 +260,7 @@ __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParam
         ++b;
       }
       const int nt = (ng + 3) >> 2;
-      if (lane < 16 * nt - 4 * ng) lrow[4 * ng + lane] = (uint16_t)ROWS;
+      if (lane < 16 * nt - 4 * ng) lrow[4 * ng + lane] = lrow[4 * ng - 1];   // the last tile: with its last row
       if (keys_left) {
         keys_left = false;
         wait_vmcnt<0>();
@@ -273,7 +276,6 @@ __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParam
         struct Load {
           uint32_t off[LPP];
         };
-        const int last = p.S - 1 - row0;
         auto prepare = [&](int i) -> Load {
           i = i < nt ? i : nt - 1;
           Load l;
@@ -285,9 +287,8 @@ __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParam
             const u16x2 e = *(const SPATTN_LDS u16x2*)(lrow + 16 * i + 2 * h);
             r[0] = e[0], r[1] = e[1];
           }
-          // "none" copies some row of the chunk
 #pragma unroll
-          for (int c = 0; c < LPP; ++c) l.off[c] = (r[c] < (uint32_t)last ? r[c] : (uint32_t)last) * ROWB + goff[c];
+          for (int c = 0; c < LPP; ++c) l.off[c] = r[c] * ROWB + goff[c];
           return l;
         };
 #pragma unroll
@@ -324,7 +325,9 @@ __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParam
           for (int t = 0; t < NT; ++t)
 #pragma unroll
             for (int n = 0; n < 4; ++n) acc[n] = mfma16(qa[P][t], kf[n][t], t == 0 ? thr : acc[n]);
-          // bit 16 g + j of a ballot: some row of the tile's four g passes for key j of the sixteen
+          // Bit 16 g + j of a ballot: some row of the tile's four g passes for key j of the sixteen.  A listed row has a
+          // finite threshold, hence no score that is a NaN (at a threshold of 0, where every row with a key is listed, a
+          // score of -inf gives one here as in the full sweep).
           unsigned long long w[4];
 #pragma unroll
           for (int n = 0; n < 4; ++n) {

@@ -147,20 +147,20 @@ def test_votes_by_rows(dev, D, S, kv_len, stride, x):
     assert torch.equal(got, want) and bool(got.any()) == (x < 1e6)
 
 
-@pytest.mark.parametrize("value", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("value", [0x7fc0, 0xffc0, 0x7f80, 0xff80])   # NaNs of both signs, infinities
 @pytest.mark.parametrize("D,S,bad", [(128, 2500, (2499, 700)), (64, 5000, (4999, 4096)), (128, 2100, (2048, 5)), (64, 300, (299, 31))])
 def test_votes_beside_rows_that_are_not_finite(dev, D, S, bad, value):
-    """A query row without a finite score never votes, in this sweep as in the full one - whichever row it is, also one
-    that fills up lists: the last, the first of the next chunk."""
+    """A query row without a finite score never votes, in this sweep as in the full one, and no row votes for another
+    q-block than its own - whichever row it is: the last, the first of the next chunk."""
     from fgattn_tk_cuda_amd.spattn import mask_utils as mu
 
-    print("case votes beside", value, D, S, bad, flush=True)
+    print("case votes beside", hex(value), D, S, bad, flush=True)
     ops = torch.ops.cuda_attn
     g = torch.Generator(device=dev).manual_seed(S + D)
     q, k = (torch.randn((1, 1, S, D), generator=g, device=dev).to(torch.bfloat16) for _ in range(2))
     bits = []
-    for v in (value, 0.0):                                    # equal weights: no votes at this threshold
-        q[:, :, list(bad)] = v
+    for v in (value, 0):                                      # zeros: equal weights, no votes at this threshold
+        q.view(torch.int16)[:, :, list(bad)] = v if v < 0x8000 else v - 0x10000
         max_q, denom = mu._stats_buffers(q)
         blockmax = mu.blockmax_buffer(q)
         ops.maxq_denom_blockmax(max_q, denom, blockmax, q, k, 0.0, 0)
