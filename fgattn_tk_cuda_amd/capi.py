@@ -57,6 +57,7 @@ _SIGNATURES = {
     "spattn_pack_mask": (_c_int, [_c_void_p] * 2 + [_c_int] * 4 + [_c_void_p]),
     "spattn_packedmask_to_indexmask": (_c_int, [_c_void_p] * 3 + [_c_int] * 5 + [_c_void_p]),
     "spattn_qk_topkmask_indices": (_c_int, [_c_void_p] * 6 + [_c_int] * 9 + [_c_void_p]),
+    "spattn_dense_form": (_c_int, [_c_int] * 7),
     "spattn_last_status": (_c_int, []),
     "spattn_status_string": (ctypes.c_char_p, [_c_int]),
     "spattn_version": (_c_int, []),

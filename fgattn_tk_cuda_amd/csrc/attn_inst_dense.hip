@@ -29,32 +29,38 @@ namespace spattn {
 // 128-row form.
 // The other forms add the row sums and outputs of a row in another order: a launch over some heads of a computation
 // goes by all of its heads, so that a row's denominator, and with it a key at a threshold, does not depend on the split.
+// Between 128 and 256 rows, where no bit changes, it goes by its own q-blocks (3 of 12 heads x 9000 with statistics 142 us
+// by its own, 210 by all; 3 of 24 x 5000 77 and 120; 5 of 50 x 2049 36 and 52).
+DenseForm dense_form(int D, bool has_v, bool stats, int S, int kv_len, long long launched, long long of_heads) {
+  constexpr int kCus = 256;
+  const long long heads = of_heads > 0 ? of_heads : launched;
+  const long long n64 = heads * ((S + 63) / 64), n128 = heads * ((S + 127) / 128);
+  const int tiles = (kv_len + 63) / 64;
+  if (n64 <= kCus) return {64, !(D == 128 && has_v && stats) && tiles >= (D == 64 ? 12 : 15) ? 2 : 1};
+  if (n128 <= kCus && tiles >= (D == 128 ? 12 : stats ? 15 : 24)) return {128, 2};
+  if ((D == 64 || !has_v) && kv_len >= 768 && n64 <= 3 * kCus) return {64, 1};
+  if (D == 128 && has_v) {
+    const long long n256 = launched * ((S + 255) / 256);
+    const long long last = n256 % kCus;
+    if (tiles >= 32 && (last == 0 || last > kCus / 2) && (!stats || n256 <= 2 * kCus)) return {256, 1};
+  }
+  return {128, 1};
+}
+
 template <int D, bool HAS_V, bool STATS>
 static hipError_t run(const AttnParams& p, int heads, hipStream_t stream) {
-  constexpr int kCus = 256;
-  const long long hb = heads > 0 ? heads : p.B * p.H;
-  const long long n64 = hb * ((p.S + 63) / 64), n128 = hb * ((p.S + 127) / 128);
-  const int tiles = (p.kv_len + 63) / 64;
-  AttnParams p64 = p;
+  const DenseForm f = dense_form(D, HAS_V, STATS, p.S, p.kv_len, (long long)p.B * p.H, heads);
+  AttnParams pf = p;
   // the statistics cover the rows up to Sp
-  p64.nqblk = (STATS ? p.Sp : p.S + 63) / 64;
-  if (n64 <= kCus) {
-    if constexpr (!(D == 128 && HAS_V && STATS)) {
-      if (tiles >= (D == 64 ? 12 : 15)) return launch_attn_fwd<D, 64, KV_DENSE, HAS_V, STATS, 2>(p64, stream);
-    }
-    return launch_attn_fwd<D, 64, KV_DENSE, HAS_V, STATS>(p64, stream);
+  if (f.rows == 64) pf.nqblk = (STATS ? p.Sp : p.S + 63) / 64;
+  if (f.rows == 256) pf.nqblk = (p.S + 255) / 256;
+  if (f.rows == 64 && f.groups == 2) {
+    if constexpr (!(D == 128 && HAS_V && STATS)) return launch_attn_fwd<D, 64, KV_DENSE, HAS_V, STATS, 2>(pf, stream);
   }
-  if (n128 <= kCus && tiles >= (D == 128 ? 12 : STATS ? 15 : 24))
-    return launch_attn_fwd<D, 128, KV_DENSE, HAS_V, STATS, 2>(p, stream);
-  if ((D == 64 || !HAS_V) && p.kv_len >= 768 && n64 <= 3 * kCus) return launch_attn_fwd<D, 64, KV_DENSE, HAS_V, STATS>(p64, stream);
-  if constexpr (D == 128 && HAS_V) {
-    const long long n256 = hb * ((p.S + 255) / 256);
-    const long long last = n256 % kCus;
-    if (tiles >= 32 && (last == 0 || last > kCus / 2) && (!STATS || n256 <= 2 * kCus)) {
-      AttnParams p256 = p;
-      p256.nqblk = (p.S + 255) / 256;
-      return launch_attn_fwd<D, 256, KV_DENSE, HAS_V, STATS>(p256, stream);
-    }
+  if (f.rows == 64) return launch_attn_fwd<D, 64, KV_DENSE, HAS_V, STATS>(pf, stream);
+  if (f.rows == 128 && f.groups == 2) return launch_attn_fwd<D, 128, KV_DENSE, HAS_V, STATS, 2>(pf, stream);
+  if (f.rows == 256) {
+    if constexpr (D == 128 && HAS_V) return launch_attn_fwd<D, 256, KV_DENSE, HAS_V, STATS>(pf, stream);
   }
   return launch_attn_fwd<D, 128, KV_DENSE, HAS_V, STATS>(p, stream);
 }

@@ -143,6 +143,15 @@ int spattn_fullattn_maxq_denom_blockmax_of(void* o, float* max_q, float* denom, 
   return from_hip(spattn::run_attn_dense(p, D, true, true, as_stream(stream), of_heads));
 }
 
+int spattn_dense_form(int D, int has_v, int stats, int heads, int S, int kv_len, int of_heads) {
+  if (D != 64 && D != 128) return done(SPATTN_ERR_HEAD_DIM);
+  if ((!has_v && !stats) || heads <= 0 || S <= 0 || S >= (1 << 24) || (of_heads != 0 && of_heads < heads)) return done(SPATTN_ERR_SHAPE);
+  const int kv = kv_len > 0 && kv_len < S ? kv_len : S;
+  const spattn::DenseForm f = spattn::dense_form(D, has_v != 0, stats != 0, S, kv, heads, of_heads);
+  done(SPATTN_OK);
+  return 10 * f.rows + f.groups;
+}
+
 int spattn_maxq_denom_blockmax(float* max_q, float* denom, void* blockmax, const void* q, const void* k, int B, int H,
                                int S, int D, int kv_len, float scale, void* stream) {
   return spattn_maxq_denom_blockmax_of(max_q, denom, blockmax, q, k, B, H, S, D, kv_len, scale, 0, stream);

@@ -9,6 +9,11 @@ hipError_t run_attn_tokens(const AttnParams& p, int D, int qblk, hipStream_t str
 hipError_t run_attn_blocks(const AttnParams& p, int D, int qblk, hipStream_t stream);
 // heads: of the whole computation where the launch is a part of one, 0: those of the launch
 hipError_t run_attn_dense(const AttnParams& p, int D, bool has_v, bool stats, hipStream_t stream, int heads = 0);
+// The form that such a launch takes: rows per q-block, groups of waves that share one.
+struct DenseForm {
+  int rows, groups;
+};
+DenseForm dense_form(int D, bool has_v, bool stats, int S, int kv_len, long long launched, long long of_heads);   // heads
 // every instantiation's dynamic-LDS limit on the current device (idempotent)
 hipError_t prepare_attn_tokens();
 hipError_t prepare_attn_blocks();

@@ -183,7 +183,7 @@ int spattn_fullattn_maxq_denom_blockmax(void* o, float* max_q, float* denom, voi
                                         const void* v, int batch, int heads, int seq, int D, int kv_len, float scale,
                                         void* stream);
 /* The same sweeps over some of the of_heads (batch x heads) of one computation: the size of the whole decides how the
- * rows are split, so max_q, denom, blockmax and o are the same bits as in one call over all of its heads.  of_heads = 0:
+ * sums of a row are split, so max_q, denom, blockmax and o are the same bits as in one call over all of its heads.  of_heads = 0:
  * the call is the whole; otherwise not below batch * heads. */
 int spattn_maxq_denom_blockmax_of(float* max_q, float* denom, void* blockmax, const void* q, const void* k, int batch,
                                   int heads, int seq, int D, int kv_len, float scale, int of_heads, void* stream);
@@ -289,6 +289,11 @@ int spattn_init(void);
 int spattn_sp_attn_blocks_balanced(void* o, float* lse, const void* q, const void* k, const void* v,
                                    const int* blk_indices, const int* blk_counts, int max_blocks, int qblk, int batch,
                                    int heads, int seq, int D, int kv_len, float scale, void* stream);
+
+/* How dense attention (has_v, without stats), dense attention with statistics or the statistics alone (stats, without has_v)
+ * of `heads` (batch x heads) of a computation of of_heads (0: all of it) is split: rows of a q-block (64, 128 or 256) times
+ * ten, plus the groups of waves that share one (1 or 2); an error status for sizes that the calls refuse.  Host only. */
+int spattn_dense_form(int D, int has_v, int stats, int heads, int seq, int kv_len, int of_heads);
 
 /* Status of the most recent call on this host thread, and its text. */
 int spattn_last_status(void);

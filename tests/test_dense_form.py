@@ -1,0 +1,30 @@
+"""Host: how a dense launch is split (rows of a q-block, groups of waves that share one), by its size and by that of the
+computation that its heads are a part of."""
+import pytest
+
+from fgattn_tk_cuda_amd import capi
+
+
+def form(D, has_v, stats, heads, S, kv_len=0, of_heads=0):
+    return capi.load().spattn_dense_form(D, has_v, stats, heads, S, kv_len, of_heads)
+
+
+@pytest.mark.parametrize("heads,S,of_heads,whole", [(3, 9000, 12, 2561), (6, 9000, 12, 2561), (5, 2049, 50, 2561), (3, 5000, 24, 2561)])
+def test_some_heads_take_256_row_qblocks_by_their_own_number(heads, S, of_heads, whole):
+    """128- and 256-row q-blocks give the same bits: a part of a computation that 256-row ones would leave idle (216, 72
+    and 108, 45, 60 of them for 256 CUs) takes 128-row ones, also where the whole does not."""
+    assert form(128, 1, 1, of_heads, S) == whole
+    last = heads * -(-S // 256) % 256
+    assert form(128, 1, 1, heads, S, 0, of_heads) == (2561 if last == 0 or last > 128 else 1281)
+
+
+def test_forms_that_add_in_another_order_go_by_the_whole():
+    assert form(128, 1, 1, 4, 2000, 0, 16) == form(128, 1, 1, 16, 2000) == 1282 and form(128, 1, 1, 4, 2000) == 641
+    assert form(64, 1, 1, 4, 2000, 0, 26) == form(64, 1, 1, 26, 2000) != form(64, 1, 1, 4, 2000)
+    assert form(128, 0, 1, 2, 9000, 0, 12) == form(128, 0, 1, 12, 9000) == 1281
+
+
+def test_what_the_calls_refuse_has_no_form():
+    assert form(96, 1, 0, 1, 128) == -2
+    for bad in ((64, 0, 0, 1, 128), (64, 1, 0, 0, 128), (64, 1, 0, 1, 0), (64, 1, 0, 1, 1 << 24), (64, 1, 0, 2, 128, 0, 1)):
+        assert form(*bad) == -6

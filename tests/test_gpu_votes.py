@@ -87,10 +87,10 @@ def test_block_refresh_in_groups_of_heads(dev, S, D, qblk):
     assert int(got[0][2].sum()) > 0
 
 
-@pytest.mark.parametrize("H,S,D", [(16, 2000, 128), (26, 2000, 64), (40, 1400, 64), (9, 1990, 128)])
+@pytest.mark.parametrize("H,S,D", [(16, 2000, 128), (26, 2000, 64), (40, 1400, 64), (9, 1990, 128), (50, 2049, 128)])
 def test_groups_take_the_form_of_the_whole(dev, H, S, D):
-    """Heads whose launch as a whole takes 128-row q-blocks, in groups small enough for 64-row ones: output, statistics and
-    lists are the bits of all heads at once."""
+    """Heads whose launch as a whole takes 128-row q-blocks (the last: 256-row ones), in groups small enough for 64-row
+    ones: output, statistics and lists are the bits of all heads at once."""
     from fgattn_tk_cuda_amd.spattn import mask_utils as mu, sparseattn_functionals as fn
 
     print("case groups of the whole", H, S, D, flush=True)
