@@ -11,7 +11,8 @@
 //   3. the listed rows of Q, sixteen to a tile, copied through a ring in LDS that it fills itself (whole rows, so that
 //      the copies coalesce; no barrier) and multiplied with the 64 keys.  In the 16x16 accumulator lanes 16 g .. of
 //      register i hold row 4 g + i of the tile, so the ballot of sixteen keys has sixteen bits for each four of rows,
-//      and the fours of a tile may belong to different q-blocks;
+//      and the fours of a tile may belong to different q-blocks (lanes 0..3 shift theirs out of the four ballots: writing
+//      them lane by lane took 20 wait states and 40 scalar instructions a tile, 2-5 % of the time);
 //   4. the 64 bits of every q-block: one bit per (q-block, key), the layout of the mask cache
 //      (python/spattn/mask_utils.py:421-430).
 // A chain of 16x16x32 multiplies gives the same bits as the 32x32x16 chain of the full sweep (compared on 1.6 million
@@ -21,12 +22,16 @@
 // active row, 22 % of the (32-row group, key block) pairs, but 4.5 % of the (row, key block) pairs.  Multiplying
 // (32-row group, key block) pairs with the rows standing still, as this kernel did before, copied all 64 keys of 45 % of
 // the pairs.  What bounds it now: below 5 % of the rows the maxima (5.3 TB/s of them where nothing is active), the
-// copies (keys of every wave, listed rows) and the latency of a wave's chain of them, behind that the multiplies at
-// 1.25 PFLOP/s of the tiles.  Before and after, us, thresholds of 16 / 32 / 64 mean weights:
-//   24 x 32760 x 64    1134 / 842 / 594     599 / 459 / 368
-//   6 x 75600 x 128    2905 / 2093 / 1426   1312 / 1016 / 858
-//   16 x 6000 x 128    73 / 55 / 41         39 / 31 / 25
-//   96 x 732 x 64      16.3 / 15.3 / 13.9   9.0 / 7.6 / 6.4
+// copies (keys of every wave, listed rows) and the latency of a wave's chain of them, behind that the multiplies next to the
+// vector ALU: where every row is listed 0.93 (d = 64) and 1.02 PFLOP/s (d = 128).  Before and after, us, thresholds of
+// 1/4, 2, 4, 16, 32, 64 mean weights (67, 31, 22, 8, 4.5, 2.3 % of the rows):
+//   24 x 32760 x 64    2576 / 2127 / 1855 / 1200 / 882 / 625    2692 / 1437 / 1085 / 591 / 444 / 353
+//   6 x 75600 x 128    7284 / 5925 / 5016 / 3047 / 2172 / 1489  6228 / 3304 / 2456 / 1327 / 1021 / 843
+//   16 x 6000 x 128    138 / 122 / 108 / 75 / 56 / 42           117 / 68 / 54 / 34 / 27 / 23
+//   96 x 732 x 64      18.3 / 17.7 / 17.4 / 16.2 / 15.3 / 13.9  12.9 / 10.3 / 9.0 / 7.2 / 6.4 / 5.3
+//   16 x 400 x 64      7.5 / 7.5 / 7.5 / 7.4 / 7.2 / 6.4        5.2 / 5.0 / 4.9 / 4.6 / 4.7 / 4.6
+// Rows that nearly all pass are multiplied faster standing still: below 1/4 of a mean weight the kernel before was ahead on
+// long sequences, with every row listed 2485 to 3382 us (24 x 32760 x 64) and 7070 to 7742 (6 x 75600 x 128).
 // Measured and not taken: fours replaced by sixteens (every tile of one q-block) 6-14 % slower at d = 128, three ring
 // slots 8-30 % slower, the thresholds copied into the list 20 % slower.
 #include <type_traits>
@@ -57,7 +62,7 @@ struct VotesParams {
   float blk_slack;           // how far below its vote threshold a row's block maximum still counts, see run_blockmax_votes
   float sf;
   int HB, S, kv_len, Sp, SB, words;
-  int nch, ch_qblocks;       // chunks of rows per head, q-blocks per chunk (a multiple of four)
+  int nch, ch_qblocks;       // chunks of rows per head, q-blocks per chunk
   int jgroups;               // groups of four key blocks per head
 };
 
@@ -72,14 +77,7 @@ __device__ __forceinline__ int row_scan(int x, int& total) {
   return v - x;
 }
 
-// v with lane L replaced by the wave-uniform s; the wait states cover a vector-ALU write of s.
-template <int L>
-__device__ __forceinline__ int write_lane(int s, int v) {
-  asm("s_nop 1\n\tv_writelane_b32 %0, %1, %2" : "+v"(v) : "s"(s), "n"(L));
-  return v;
-}
-
-template <int D>
+template <int D, int CHUNK>
 __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParams p) {
   using Cfg = VotesCfg<D>;
   constexpr int NT = D / 32;              // k-steps
@@ -89,15 +87,15 @@ __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParam
   constexpr int NS = Cfg::kSlots;
   constexpr int LPP = TILE / 1024;        // 1 KB copies per tile
   constexpr int CAP = Cfg::kCap;
-  constexpr int ROWS = Cfg::kChunk * 128; // rows per chunk, at most
+  constexpr int ROWS = CHUNK * 128;       // rows per chunk, at most
   constexpr int NB = ROWS / 512;          // batches of four q-blocks
   static_assert(NS == 2, "the keys arrive in two halves of the ring's length");
   static_assert(CAP >= 32, "a batch of four q-blocks has up to 32 tiles");
-  static_assert(Cfg::kChunk <= 64, "a lane writes the votes of one q-block");
+  static_assert(CHUNK <= 64, "a lane writes the votes of one q-block");
   __shared__ __attribute__((aligned(1024))) unsigned char ring_all[4 * NS * TILE];
   __shared__ __attribute__((aligned(16))) float tab[ROWS];                 // minus the vote threshold of a row on its raw score
   __shared__ __attribute__((aligned(16))) uint16_t list_row[4][CAP * 16];  // row within the chunk
-  __shared__ unsigned long long votes[4][Cfg::kChunk];                      // of a wave's keys, per q-block
+  __shared__ unsigned long long votes[4][CHUNK];                           // of a wave's keys, per q-block
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -151,7 +149,7 @@ __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParam
   __syncthreads();
 
   // ---- 1: one bit per row ----
-  constexpr int FW = NB / 4;
+  constexpr int FW = (NB + 3) / 4;
   uint32_t flags[FW] = {};   // byte b % 4 of word b / 4: rows 512 b + 8 lane + 0..7
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
@@ -176,7 +174,7 @@ __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParam
   for (int w = 0; w < FW; ++w) any |= flags[w];
 
   SPATTN_LDS unsigned long long* vw = (SPATTN_LDS unsigned long long*)votes[wave];
-  if (lane < Cfg::kChunk) vw[lane] = 0;
+  if (lane < CHUNK) vw[lane] = 0;
   if (__ballot(any != 0) != 0) {
     // A copy of a tile: lane h * CPR + pos of copy c fetches chunk pos ^ swz of row LPP h + c, so that the operand
     // reads below (sixteen lanes, one chunk of sixteen rows) cover all sixteen 16-byte bank groups.
@@ -335,18 +333,12 @@ __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParam
             const int a = v[0] > v[1] ? v[0] : v[1], c = v[2] > v[3] ? v[2] : v[3];
             w[n] = __ballot((a > c ? a : c) > 0);
           }
-          int lo = 0, hi = 0;
-          auto four = [&](auto fc) {
-            constexpr int f = decltype(fc)::value;
-            lo = write_lane<f>((int)((w[0] >> (16 * f)) & 0xffffu) | ((int)((w[1] >> (16 * f)) & 0xffffu) << 16), lo);
-            hi = write_lane<f>((int)((w[2] >> (16 * f)) & 0xffffu) | ((int)((w[3] >> (16 * f)) & 0xffffu) << 16), hi);
-          };
-          four(std::integral_constant<int, 0>{});
-          four(std::integral_constant<int, 1>{});
-          four(std::integral_constant<int, 2>{});
-          four(std::integral_constant<int, 3>{});
+          // lanes 0..3: the 64 bits of one four
+          const int sh = 16 * (lane & 3);
+          const uint32_t lo = __builtin_amdgcn_perm((uint32_t)(w[1] >> sh), (uint32_t)(w[0] >> sh), 0x05040100u);
+          const uint32_t hi = __builtin_amdgcn_perm((uint32_t)(w[3] >> sh), (uint32_t)(w[2] >> sh), 0x05040100u);
           if (lane < 4) {
-            const unsigned long long v = ((unsigned long long)(uint32_t)hi << 32) | (uint32_t)lo;
+            const unsigned long long v = ((unsigned long long)hi << 32) | lo;
             __hip_atomic_fetch_or(vw + qb, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
           }
           slot = next;
@@ -369,6 +361,24 @@ __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParam
     const unsigned long long v = left >= 64 ? vw[lane] : left <= 0 ? 0ull : vw[lane] & ((1ull << left) - 1ull);
     *reinterpret_cast<u32x2*>(p.bits + ((size_t)bh * p.SB + qb0 + lane) * p.words + 2 * J) = __builtin_bit_cast(u32x2, v);
   }
+}
+
+// q-blocks per chunk.  A wave's tiles are a serial chain, so where the longest chunks leave the chip idle, or in their second
+// round, they are cut to what fills the round; `resident` workgroups are on the chip at a time (three per CU at d = 128, by
+// registers, four at d = 64, by LDS).  per_chunk: workgroups per chunk of rows.  Longer launches keep whole batches of four
+// q-blocks (16 x 12743 x 64 in chunks of 25 instead of 28: 73 -> 82 us).  With chunks of no less than four q-blocks, cut until
+// there were four workgroups per CU, and now, us at 1/4, 1, 4, 16, 32 mean weights:
+//   16 x 400 x 64      10.6 / 10.2 / 8.7 / 6.6 / 5.5      5.2 / 5.0 / 4.9 / 4.6 / 4.7
+//   16 x 512 x 128     14.7 / 14.3 / 12.8 / 9.5 / 7.9     6.1 / 5.9 / 5.7 / 5.2 / 4.9
+//   24 x 1000 x 128    13.7 / 12.4 / 10.4 / 7.8 / 6.7     10.4 / 9.4 / 8.4 / 7.0 / 6.4
+//   16 x 4096 x 128    66 / 50 / 34 / 22 / 18             58 / 43 / 30 / 18 / 15
+//   12 x 7000 x 64     88 / 65 / 42 / 28 / 23             75 / 56 / 38 / 23 / 19
+static int votes_chunk(int SB, int most, int resident, long long per_chunk) {
+  const int nch = (SB + most - 1) / most;
+  const long long rounds = (nch * per_chunk + resident - 1) / resident;
+  if (rounds > 2) return ((SB + nch - 1) / nch + 3) / 4 * 4;
+  const long long fit = rounds * resident / per_chunk;   // chunks, not fewer than nch
+  return fit < SB ? (SB + (int)fit - 1) / (int)fit : 1;
 }
 
 // The block test runs a little below the vote threshold, tau (1 - 1e-3): the statistics sweep rounds a
@@ -397,15 +407,17 @@ hipError_t run_blockmax_votes(uint32_t* bits, const uint16_t* blockmax, const fl
   p.SB = SB;
   p.words = mask_stride / 32;
   p.jgroups = (p.words / 2 + 3) / 4;
-  const int most = D == 128 ? VotesCfg<128>::kChunk : VotesCfg<64>::kChunk;
-  int nch = (SB + most - 1) / most;
-  // short sequences: chunks down to four q-blocks (one batch of the list) until there are four workgroups per CU
-  while (nch < (SB + 3) / 4 && (long long)nch * p.jgroups * HB < 1024) ++nch;
-  p.ch_qblocks = ((SB + nch - 1) / nch + 3) / 4 * 4;
+  p.ch_qblocks = votes_chunk(SB, D == 128 ? VotesCfg<128>::kChunk : VotesCfg<64>::kChunk, (D == 128 ? 3 : 4) * 256,
+                             (long long)p.jgroups * HB);
   p.nch = (SB + p.ch_qblocks - 1) / p.ch_qblocks;
   const dim3 grid(p.jgroups * p.nch * HB);
-  if (D == 128) hipLaunchKernelGGL(blockmax_votes_kernel<128>, grid, dim3(256), 0, stream, p);
-  else hipLaunchKernelGGL(blockmax_votes_kernel<64>, grid, dim3(256), 0, stream, p);
+  // short chunks: a quarter to an eighth of the thresholds to make, LDS and maxima to hold (96 x 732 x 64 8.9 -> 7.3 us at 16
+  // mean weights, 24 x 1000 x 128 7.5 -> 7.0; a bound read in the one kernel took 2-3 % from the long launches)
+  const bool small = p.ch_qblocks <= 4;
+  if (D == 128 && small) hipLaunchKernelGGL((blockmax_votes_kernel<128, 4>), grid, dim3(256), 0, stream, p);
+  else if (D == 128) hipLaunchKernelGGL((blockmax_votes_kernel<128, VotesCfg<128>::kChunk>), grid, dim3(256), 0, stream, p);
+  else if (small) hipLaunchKernelGGL((blockmax_votes_kernel<64, 4>), grid, dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL((blockmax_votes_kernel<64, VotesCfg<64>::kChunk>), grid, dim3(256), 0, stream, p);
   return hipGetLastError();
 }
 

@@ -205,7 +205,7 @@ def test_no_instruction_touches_a_register_with_a_load_in_flight(tmp_path):
         assert not uses, "%s: the compiler uses m0 next to hand-written copies: %s" % (unit, uses[:3])
         if unit == VOTES_UNIT:
             walks = walk_findings(text)
-            assert len(walks) == 2 and all(f == (0, 0) for f in walks.values()), "%s: %s" % (unit, walks)
+            assert len(walks) == 4 and all(f == (0, 0) for f in walks.values()), "%s: %s" % (unit, walks)
         if unit not in UNITS:
             continue
         assert "global_load_dword" in text, unit

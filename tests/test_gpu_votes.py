@@ -147,6 +147,29 @@ def test_votes_by_rows(dev, D, S, kv_len, stride, x):
     assert torch.equal(got, want) and bool(got.any()) == (x < 1e6)
 
 
+@pytest.mark.parametrize("D,S,H,kv_len", [
+    (64, 640, 100, 0), (128, 1000, 60, 999), (128, 1000, 90, 0), (128, 2300, 20, 0), (64, 1500, 60, 1473), (128, 1500, 64, 0),
+    (64, 900, 170, 897), (128, 2100, 180, 2049),
+])
+def test_votes_by_length_of_the_chunks(dev, D, S, H, kv_len):
+    """Chunks of 2, 3, 4 (the instantiation for short ones), 5, 6, 6, 8 and 12 q-blocks, the last of a head shorter: every row
+    active, and some - the bits of the full sweep."""
+    from fgattn_tk_cuda_amd.spattn import mask_utils as mu
+
+    print("case votes by chunks", D, S, H, kv_len, flush=True)
+    ops = torch.ops.cuda_attn
+    g = torch.Generator(device=dev).manual_seed(S + H)
+    q, k = (torch.randn((1, H, S, D), generator=g, device=dev).to(torch.bfloat16) for _ in range(2))
+    max_q, denom = mu._stats_buffers(q)
+    blockmax = mu.blockmax_buffer(q)
+    ops.maxq_denom_blockmax(max_q, denom, blockmax, q, k, 0.0, kv_len)
+    for x in (1e-6, 16):
+        want = mu.qk_packedmask_from_maxq_denom_cuda(max_q, denom, q, k, x / (kv_len or S), 128, kv_len)
+        got = torch.full_like(want, 0x5a)
+        ops.blockmax_to_packedmask(got, blockmax, max_q, denom, q, k, x / (kv_len or S), 0.0, kv_len)
+        assert torch.equal(got, want) and bool(got.any())
+
+
 @pytest.mark.parametrize("value", [0x7fc0, 0xffc0, 0x7f80, 0xff80])   # NaNs of both signs, infinities
 @pytest.mark.parametrize("D,S,bad", [(128, 2500, (2499, 700)), (64, 5000, (4999, 4096)), (128, 2100, (2048, 5)), (64, 300, (299, 31))])
 def test_votes_beside_rows_that_are_not_finite(dev, D, S, bad, value):
