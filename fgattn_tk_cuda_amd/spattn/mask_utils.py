@@ -324,11 +324,7 @@ def qk_indexmask_cuda(q, k, thresh, blocksz=128, onepass=None, fill_tail=True, b
         max_q, denom = _stats_buffers(q)
         spattn_interface.maxq_denom(max_q, denom, q.contiguous(), k.contiguous())
         return qk_indexmask_from_maxq_denom_cuda(max_q, denom, q, k, thresh, blocksz)
-
-    def sweep(lo, hi, blockmax, q_, k_, max_q_, denom_):
-        spattn_interface.maxq_denom_blockmax(max_q_, denom_, blockmax, q_, k_, 0.0, 0, q.shape[0] * q.shape[1])
-
-    return packedmask_to_indexmask_cuda(packedmask_by_groups(groups, sweep, q, k, None, None, thresh), q.shape[2], fill_tail)
+    return packedmask_to_indexmask_cuda(packedmask_by_groups(groups, None, q, k, None, None, thresh), q.shape[2], fill_tail)
 
 
 def qblock_order_cuda(counts, per_head=None):
@@ -455,9 +451,9 @@ def head_groups(q, onepass=None, budget_bytes=None):
 def packedmask_by_groups(groups, sweep, q, k, max_q, denom, thresh, qblk=BLOCKSZ, out=None, value=None):
     """The bit-packed threshold mask (per qblk rows) of a one-sweep refresh.  ``sweep(lo, hi, blockmax, q, k,
     max_q, denom)`` runs the statistics sweep with block maxima over heads lo..hi-1 (its tensors are views of
-    those heads); the bits of the group follow from the maxima, whose buffer the next group reuses.  max_q, denom
-    None: the statistics are dropped; all heads at once with bits per 128 rows is then one operator, which is told what
-    else the sweep writes (``out`` from ``value``: dense attention)."""
+    those heads); the bits of the group follow from the maxima, whose buffer the next group reuses.  None: the sweep of
+    the operators, over all keys at their own scale - the statistics alone, or with ``out`` dense attention from
+    ``value`` too.  max_q, denom None: the statistics are dropped."""
     B, H, S, D = q.shape
     # the operators see views over all heads: what they refuse of the whole tensors is refused here
     if k.shape != q.shape:
@@ -465,11 +461,20 @@ def packedmask_by_groups(groups, sweep, q, k, max_q, denom, thresh, qblk=BLOCKSZ
     n, sp = B * H, _padded(S)
     packed = torch.empty((B, H, (S + qblk - 1) // qblk, sp // 8), dtype=torch.uint8, device=q.device)
     if max_q is None:
-        if len(groups) == 1 and qblk == BLOCKSZ:
-            # small computations wait for the host: 32 x 380 x 64 x 4 44 -> 31 us a call against the operators one by one
+        if sweep is None and len(groups) == 1 and qblk == BLOCKSZ:
+            # one operator: small computations wait for the host (32 x 380 x 64 x 4 44 -> 31 us a call)
             spattn_interface.onepass_packedmask(packed, out, q.contiguous(), k.contiguous(), value, thresh)
             return packed
         max_q, denom = _stats_buffers(q)
+    if sweep is None:
+        o_, v_ = (None, None) if out is None else (out.view(1, n, S, D), value.view(1, n, S, D))
+
+        def sweep(lo, hi, blockmax, qs, ks, ms, ds):
+            if out is None:
+                spattn_interface.maxq_denom_blockmax(ms, ds, blockmax, qs, ks, 0.0, 0, n)
+            else:
+                os_, vs = (o_, v_) if hi - lo == n else (o_[:, lo:hi], v_[:, lo:hi])
+                spattn_interface.fullattn_maxq_denom_blockmax(os_, ms, ds, blockmax, qs, ks, vs, 0.0, 0, n)
     heads = [t.contiguous().view(1, n, *t.shape[2:]) for t in (q, k, max_q, denom, packed)]
     blockmax = torch.empty((1, max(hi - lo for lo, hi in groups), sp // KVBLK, sp), dtype=torch.bfloat16, device=q.device)
     for lo, hi in groups:

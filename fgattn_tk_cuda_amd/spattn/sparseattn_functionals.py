@@ -124,14 +124,7 @@ def _dense_and_packedmask(query, key, value, groups, thresh, qblk):
         raise RuntimeError("v must have the shape of q")
     query, key, value = _c(query, key, value)
     out = _out_like(query)
-    B, H, S, D = query.shape
-    o_, v_ = out.view(1, B * H, S, D), value.view(1, B * H, S, D)
-
-    def sweep(lo, hi, blockmax, qs, ks, ms, ds):
-        os_, vs = (o_, v_) if hi - lo == B * H else (o_[:, lo:hi], v_[:, lo:hi])
-        spattn_interface.fullattn_maxq_denom_blockmax(os_, ms, ds, blockmax, qs, ks, vs, 0.0, 0, B * H)
-
-    return out, mask_utils.packedmask_by_groups(groups, sweep, query, key, None, None, thresh, qblk, out, value)
+    return out, mask_utils.packedmask_by_groups(groups, None, query, key, None, None, thresh, qblk, out, value)
 
 
 def cached_attn_cuda(query, key, value, current_layer, ditrun, *args, **kwargs):

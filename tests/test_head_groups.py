@@ -50,3 +50,17 @@ def test_masks_of_every_step_keep_to_the_callers_route_and_budget(monkeypatch):
     assert groups() == groups(onepass=True) == groups(blockmax_budget_bytes=6 * per_head) == [[(0, 6)]]
     assert groups(blockmax_budget_bytes=4 * per_head) == [[(0, 2), (2, 4), (4, 6)]]
     assert groups(onepass=False) == groups(blockmax_budget_bytes=per_head) == []
+
+
+@pytest.mark.parametrize("groups", [[(0, 6)], [(0, 2), (2, 6)]])
+@pytest.mark.parametrize("buffers", [True, False])
+def test_a_callers_sweep_runs_over_every_group(groups, buffers):
+    """Also where all heads go at once and the caller has no use for the statistics."""
+    from fgattn_tk_cuda_amd.spattn import mask_utils as mu
+
+    q = torch.empty((2, 3, 300, 64), dtype=torch.bfloat16, device="meta")
+    seen = []
+    max_q, denom = mu._stats_buffers(q) if buffers else (None, None)
+    packed = mu.packedmask_by_groups(groups, lambda lo, hi, blockmax, *t: seen.append((lo, hi, blockmax.shape[1], t[0].shape[1])), q, q,
+                                     max_q, denom, 0.01)
+    assert seen == [(lo, hi, hi - lo, hi - lo) for lo, hi in groups] and packed.shape == (2, 3, 3, 48)
