@@ -60,16 +60,21 @@ def test_list_attention_reads_no_freed_slot(dev, D, qblk, S, kv_len):
 
 @pytest.mark.parametrize("D,S,kv_len", [(128, 1300, 0), (64, 1700, 1601)])
 def test_dense_kernels_read_no_freed_slot(dev, D, S, kv_len):
+    """Small launches: 64-row q-blocks."""
     print("case poison dense", D, S, kv_len, flush=True)
     _dense(dev, D, S, kv_len, 2)
 
 
-@pytest.mark.parametrize("D,S,kv_len,H", [(128, 1300, 0, 13), (128, 900, 833, 18), (64, 1700, 1601, 29), (64, 700, 0, 24)])
-def test_large_dense_launches_read_no_freed_slot(dev, D, S, kv_len, H):
-    """Launches with more q-blocks than take the 64-row form."""
+@pytest.mark.parametrize("D,S,kv_len,H,forms", [
+    (128, 1300, 0, 13, (1282, 1282, 1282)), (128, 900, 833, 18, (1282, 1282, 1282)), (64, 1700, 1601, 29, (1281, 1281, 1281)),
+    (64, 700, 0, 24, (1281, 1281, 1281)), (128, 1300, 0, 40, (1281, 1281, 1281)), (128, 1300, 0, 24, (1281, 1281, 641)),
+    (128, 2049, 2047, 50, (2561, 2561, 1281)), (64, 1700, 0, 18, (1282, 1282, 1282)),
+])
+def test_large_dense_launches_read_no_freed_slot(dev, D, S, kv_len, H, forms):
+    """Launches with more q-blocks than take the 64-row form, in every form that they take: two groups of waves per q-block,
+    one, q-blocks of 256 rows.  forms: of dense attention, of that with statistics, of the statistics alone."""
     print("case poison large dense", D, S, kv_len, H, flush=True)
-    n64 = H * wl.ceil_div(S, 64)
-    assert n64 > (768 if D == 64 and (kv_len or S) >= 768 else 256)
+    assert tuple(capi.load().spattn_dense_form(D, v, st, H, S, kv_len, 0) for v, st in ((1, 0), (1, 1), (0, 1))) == forms
     _dense(dev, D, S, kv_len, H)
 
 
