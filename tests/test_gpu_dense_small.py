@@ -103,19 +103,25 @@ def test_two_groups_match_one(dev, D, S, kv_len):
         assert torch.equal(m, largest[0][:, :h]) and torch.equal(bm[..., :S], largest[1][:, :h, :, :S])
 
 
-@pytest.mark.parametrize("S,kv_len,heads", [
-    (2049, 0, (50, 40)),          # 9 q-blocks of 256 rows per head, the last with one row, over rows behind Sp: 450 of them, 360
-    (2176, 2060, (50, 40)),       # key tiles behind the kv length, rows up to a multiple of 128
-    (2304, 2304, (57, 60)),       # 513: last round of one q-block, 540: statistics behind two rounds
-    (2303, 1985, (57, 56, 57)),   # 32 tiles
-    (2100, 1984, (57, 56)),       # 31 tiles
+@pytest.mark.parametrize("S,kv_len,heads,dense,stats", [
+    # 9 q-blocks of 256 rows per head, the last with one row, over rows behind Sp: 450 of them, 360
+    (2049, 0, (50, 40), (256, 128), (256, 128)),
+    (2176, 2060, (50, 40), (256, 128), (256, 128)),            # key tiles behind the kv length, rows up to a multiple of 128
+    (2304, 2304, (57, 60), (128, 128), (128, 128)),            # 513, 540: last round of one, of 28
+    (2304, 0, (72, 57), (256, 128), (128, 128)),               # 648: a third round, more than half full
+    (2048, 0, (64, 66), (256, 128), (256, 128)),               # 512: rounds that are full, 32 tiles
+    (2303, 1985, (57, 56, 57), (128, 256, 128), (128, 256, 128)),   # 32 tiles
+    (2100, 1984, (57, 56), (128, 128), (128, 128)),            # 31 tiles
 ])
-def test_256_row_qblocks_give_the_same_bits(dev, S, kv_len, heads):
-    """d = 128, launches on both sides of the rule for 256-row q-blocks: outputs, statistics and block maxima of the heads
-    they share are the same bits, and right."""
+def test_256_row_qblocks_give_the_same_bits(dev, S, kv_len, heads, dense, stats):
+    """d = 128, launches on both sides of the rule for 256-row q-blocks (dense, stats: rows per q-block of the calls without
+    and with statistics): outputs, statistics and block maxima of the heads they share are the same bits, and right."""
     import fgattn_tk_cuda_amd.spattn.cuda_attn  # noqa: F401
+    from fgattn_tk_cuda_amd import capi
 
     print("case dense 256 rows", S, kv_len, heads, flush=True)
+    for st, rows in ((0, dense), (1, stats)):
+        assert tuple(capi.load().spattn_dense_form(128, 1, st, h, S, kv_len, 0) for h in heads) == tuple(10 * r + 1 for r in rows)
     ops = torch.ops.cuda_attn
     g = torch.Generator(device=dev).manual_seed(S)
     q, k, v = (torch.randn((1, max(heads), S, 128), generator=g, device=dev).to(torch.bfloat16) for _ in range(3))
