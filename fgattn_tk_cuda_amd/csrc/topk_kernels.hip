@@ -621,7 +621,7 @@ void topk_select_reg_kernel(int* __restrict__ kv_indices, int* __restrict__ kv_n
   __syncthreads();
   int out_pos = 0, eq_seen = 0;
   {
-    // added up apart: seven waves of 19 vectors per lane hold more than 65535 keys
+    // added up apart: fifteen waves of 10 vectors per lane hold 76800 keys, more than 16 bits count
 #pragma unroll
     for (int u = 0; u < THREADS / 64 - 1; ++u) {
       const uint32_t c = u < wave ? wave_cnt[u] : 0u;

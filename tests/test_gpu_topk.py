@@ -56,7 +56,7 @@ def test_topk_generator_matches_oracle(dev, D, blk, S, select_k, kv_len):
 @pytest.mark.parametrize("S,select_k", [(4096, 300), (8200, 8100), (16001, 1300), (32757, 2621), (32768, 32768), (45003, 900),
                                         (72001, 6000), (73728, 73000)])
 def test_topk_select_row_lengths_with_many_ties(dev, S, select_k):
-    """Every row length class of the in-register select (1, 2, 4, 8, 12 and 18 vectors per lane), row
+    """Row lengths over the classes of the in-register select (1 to 12 vectors per lane of 512, 8 to 10 of 1024), row
     ends inside a 16-byte vector, and keys on a coarse grid so that many scores are equal - also at
     the threshold, where the lower key wins."""
     print("case topk row lengths", S, select_k, flush=True)
@@ -86,23 +86,24 @@ def test_topk_select_row_lengths_with_many_ties(dev, S, select_k):
 
 
 def test_topk_rows_longer_than_the_register_path(dev):
-    """More than 73728 keys per row: the select that re-reads its row from memory."""
+    """More than 81920 keys per row: the select that re-reads its row from memory."""
     print("case topk long rows", flush=True)
-    B, H, S, D, blk, select_k = 1, 1, 81000, 64, 128, 700
+    B, H, S, D, blk, select_k = 1, 1, 82001, 64, 128, 700
     q, k, _ = wl.randn_qkv(B, H, S, D, seed=5)
     kvi, kvn, score, qmean, fill = _run(dev, q, k, select_k, blk)
     want_qm, _ = orc.qblock_mean_scores(f32(q)[:, :, :256], f32(k)[:, :, :256], blk)
     assert np.array_equal(qmean[:, :, :2], want_qm[:, :, :2])
-    rows = [0, 1, 317, 632]
+    rows = [0, 1, 317, 632, 640]
     want_sel = orc.topk_select(score[0, 0, rows, :S], select_k)
     assert np.all(kvn == select_k)
     assert np.array_equal(kvi[0, 0, rows, :select_k], want_sel)
 
 
 @pytest.mark.parametrize("S,select_k,ties", [(73729, 5900, False), (75600, 6048, False), (77824, 77000, False), (77823, 77822, True),
-                                             (77825, 300, False)])
+                                             (77825, 300, False), (81920, 81000, False), (81919, 81918, True), (81920, 81919, True),
+                                             (81921, 300, False), (81921, 81000, False)])
 def test_topk_longest_rows_of_the_register_path(dev, S, select_k, ties):
-    """19 vectors per lane, more keys ahead of the last wave than 16 bits count: above the threshold, and all of
+    """10 vectors per lane of 1024, more keys ahead of the last wave than 16 bits count: above the threshold, and all of
     them equal (the lowest keys win); one key more takes the select that re-reads its row."""
     print("case topk longest register rows", S, select_k, ties, flush=True)
     q, k, _ = wl.randn_qkv(1, 1, S, 64, seed=S)
@@ -171,9 +172,9 @@ def test_topk_argument_errors(dev):
     (3, 8200, 128, 700, 0), (70, 63, 64, 20, 3),
 ])
 def test_topk_rows_per_workgroup_and_length_classes(dev, H, S, D, select_k, levels):
-    """Both sides of the steps between 512 and 1024 lanes per row and of their numbers of vectors, more rows than
-    workgroups (the next row is loaded while a list is written), several 64-key steps per wave of the scores and
-    q-blocks behind the last group of 64: every row against a stable sort of the scores the device made."""
+    """Both sides of the steps between 512 and 1024 lanes per row and of their numbers of vectors, 1280 rows, more than
+    the 1024 that are resident at a time, several 64-key steps per wave of the scores and q-blocks behind the last group of 64:
+    every row against a stable sort of the scores the device made."""
     print("case topk classes", H, S, D, select_k, levels, flush=True)
     g = torch.Generator().manual_seed(S)
     q, k = (torch.randn((1, H, S, D), generator=g).bfloat16() for _ in range(2))
