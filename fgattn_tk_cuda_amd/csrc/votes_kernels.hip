@@ -366,7 +366,7 @@ __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParam
 // q-blocks per chunk.  A wave's tiles are a serial chain, so where the longest chunks leave the chip idle, or in their second
 // round, they are cut to what fills the round; `resident` workgroups are on the chip at a time (three per CU at d = 128, by
 // registers, four at d = 64, by LDS).  per_chunk: workgroups per chunk of rows.  Longer launches keep whole batches of four
-// q-blocks (16 x 12743 x 64 in chunks of 25 instead of 28: 73 -> 82 us).  With chunks of no less than four q-blocks, cut until
+// q-blocks (16 x 12743 x 64 in chunks of 25 instead of 28: 75 -> 82 us).  With chunks of no less than four q-blocks, cut until
 // there were four workgroups per CU, and now, us at 1/4, 1, 4, 16, 32 mean weights:
 //   16 x 400 x 64      10.6 / 10.2 / 8.7 / 6.6 / 5.5      5.2 / 5.0 / 4.9 / 4.6 / 4.7
 //   16 x 512 x 128     14.7 / 14.3 / 12.8 / 9.5 / 7.9     6.1 / 5.9 / 5.7 / 5.2 / 4.9
