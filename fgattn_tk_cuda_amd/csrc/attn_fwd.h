@@ -67,8 +67,9 @@ constexpr int attn_waves() {
   return QBLK == 256 ? 8 : 4;
 }
 
-// LDS of one workgroup.  256-row q-blocks hold their Q rows behind the ring until they are in registers.  Statistics over 64-row q-blocks: the two waves that share the rows of a tile also exchange
-// its row maxima, for the block maxima (two tiles x 64 rows, behind the ring).
+// LDS of one workgroup.  256-row q-blocks hold their Q rows behind the ring until they are in registers.  Statistics over
+// 64-row q-blocks: the two waves that share the rows of a tile also exchange its row maxima, for the block maxima (two tiles
+// x 64 rows, behind the ring).
 template <int D, int QBLK, int MODE, bool HAS_V, bool STATS, int NGRP>
 constexpr int attn_lds_bytes() {
   return NGRP * (AttnCfg<D, MODE, HAS_V>::kTotal + ((STATS && QBLK == 64) ? 2 * 64 * 4 : 0)) + (QBLK == 256 ? QBLK * D * 2 : 0);
@@ -297,7 +298,7 @@ void attn_fwd_kernel(const AttnParams p) {
   int idh[6] = {0, 0, 0, 0, 0, 0};   // token lists: key mask, high half
   // Q_LDS: the wave's 32 rows of Q come in as whole rows, into the pieces of the slots of K2 and V1 that this wave copies
   // itself (no other wave writes there, and its own copies into them go out behind the reads).  Loaded operand by
-  // operand, 16 bytes of 32 rows at a time, they are served at a quarter of the rate (9.7 against 38 TB/s from L2) and
+  // operand, 16 bytes of 32 rows at a time, they are served at a quarter of the rate (9.8 against 38 TB/s) and
   // hold up the first tiles behind them: 0.3-0.9 us per q-block.  64 x 16384 x 128, 10 % blocks 1.092 -> 1.068 ms, 12 x
   // 512 x 128 5.6 -> 5.1 us, 48 x 4092 x 128 157 -> 152 us, 4 x 1024 x 64 6.18 -> 5.99 us.  Not with 128-row q-blocks at
   // d = 64, whose 168 registers it spills, nor without V, where the slots it needs are those of K1 and K2.

@@ -5,7 +5,7 @@
 
 namespace spattn {
 
-// The four forms: q-blocks of 128 or 64 rows (64: two waves share the rows of a tile and take half of its keys each),
+// Four forms with q-blocks of 128 or 64 rows (64: two waves share the rows of a tile and take half of its keys each),
 // by one group of four waves or two (which take half of the tiles each).  A q-block is done sooner the more waves share
 // it, for more K / V copies per row and a merge; that pays while the q-blocks do not queue.  Measured as time over that
 // of the 128-row form by one group, unless said otherwise:

@@ -88,7 +88,7 @@ __global__ __launch_bounds__(256) void qblock_mean_kernel(uint16_t* __restrict__
 // score = qmean K^T.  A workgroup takes 64 q-blocks of one head (their means as B operands in registers, the same in
 // every wave) and a chunk of keys, 64 keys per wave and step.  The product is tiny; what counts is how the bytes move:
 //   keys come in as whole rows (a wave-wide load of one 16-byte chunk of 32 rows is served at a quarter of the rate:
-//   9.7 against 38 TB/s from L2), 32 of them at a time, a step of the loop ahead in registers, and go through a
+//   9.8 against 38 TB/s), 32 of them at a time, a step of the loop ahead in registers, and go through a
 //   wave-private piece of LDS, swizzled, into A operands;
 //   scores leave through another one as whole 128-byte lines: accumulator register i of lane (n, g) is key 4 g + i
 //   against q-block n, four neighbouring keys of a score row.

@@ -556,8 +556,8 @@ def _packedmask_from_blockmax(packed, blockmax, max_q, denom, q, k, thresh, qblk
 
 
 def qk_packedmask_from_blockmax_cuda(blockmax, max_q, denom, q, k, thresh, qblk=128, kv_len=0):
-    """The same votes as bits (qk_packedmask_from_maxq_denom_cuda over what can hold a key: pairs of 32 rows and
-    64 keys for bits per 128 rows, key blocks for bits per 64 rows)."""
+    """The same votes as bits (qk_packedmask_from_maxq_denom_cuda over what can hold a key: the rows that can
+    pass in a 64-key block for bits per 128 rows, key blocks for bits per 64 rows)."""
     B, H, S, D = q.shape
     packed = torch.empty((B, H, (S + qblk - 1) // qblk, max_q.shape[3] // 8), dtype=torch.uint8, device=q.device)
     _packedmask_from_blockmax(packed, blockmax, max_q.contiguous(), denom.contiguous(), q.contiguous(), k.contiguous(), thresh,

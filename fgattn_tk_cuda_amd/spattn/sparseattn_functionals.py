@@ -132,7 +132,7 @@ def cached_attn_cuda(query, key, value, current_layer, ditrun, *args, **kwargs):
     pre-pass; on every other step: sparse attention from the cached lists (:95-114).
     The refresh step sweeps Q K^T once in full instead of twice: the dense pass also writes the score
     maximum of every row over every 64-key block (bf16, S*S/32 bytes per head, freed on return) and the
-    votes are then taken over the pairs of row group and key block that can hold a key only; the lists are
+    votes are then taken, in every key block, over the rows that can pass there only; the lists are
     the same.  ``onepass=True`` / ``False`` forces one route (True: all heads at once; False: the
     reference's two full sweeps, no extra buffer); by default all heads go at once when the buffer is at
     most ``blockmax_budget_bytes`` (default ``mask_utils.BLOCKMAX_BUDGET_BYTES``, 2 GiB), else in groups of
