@@ -131,8 +131,9 @@ void attn_fwd_kernel(const AttnParams p) {
   // an entry of a work order that names no q-block: nothing is addressed (wave-uniform, ahead
   // of every copy and barrier)
   if ((unsigned)wg >= (unsigned)total) return;
-  const int qb = wg % p.nqblk;
-  const int bh = wg / p.nqblk;
+  // The compiler divides on the vector ALU and would keep everything that follows from the quotient there.
+  const int bh = __builtin_amdgcn_readfirstlane(wg / p.nqblk);
+  const int qb = wg - bh * p.nqblk;
 
   const size_t head_off = (size_t)bh * p.S * D;
   const uint16_t* __restrict__ qh = p.q + head_off;

@@ -153,12 +153,21 @@ __device__ __forceinline__ void dma16(const void* gptr, uint32_t lds_base) {
 // Same with a wave-uniform base pointer and a 32-bit per-lane byte offset.
 // The base goes through readfirstlane: under scalar-register pressure the compiler may keep
 // a uniform pointer in vector registers, which the "s" constraint alone does not undo.
+// A scalar register that the vector ALU wrote (readfirstlane among others) may be read by a vector-memory instruction five
+// wait states later; the compiler keeps that distance for its own instructions and does not look into asm.  LATE = false:
+// the base has to be scalar from further up, which tests/test_asm_inflight_loads.py checks on the listing; LATE = true: the
+// wait is in the statement, for copies off the hot path whose base the compiler keeps in vector registers.
+template <bool LATE = false>
 __device__ __forceinline__ void dma16(const void* sbase, uint32_t voff, uint32_t lds_base) {
   const uint64_t b = (uint64_t)(uintptr_t)sbase;
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b);
   const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
   const uint64_t sb = ((uint64_t)hi << 32) | lo;
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voff), "s"(sb) : "memory");
+  if constexpr (LATE) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voff), "s"(sb) : "memory");
+  } else {
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voff), "s"(sb) : "memory");
+  }
 }
 // 16-byte global load that the compiler does not count either: the destination is valid only
 // behind a hand-placed vmcnt wait, after which the caller ties the registers to that point with

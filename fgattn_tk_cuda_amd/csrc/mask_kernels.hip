@@ -202,8 +202,8 @@ __global__ __launch_bounds__(256, 2) void booleanmask_kernel(int* __restrict__ m
         int key = kb * 32 + krow[i];
         key = key < kv_len ? key : kv_len - 1;
         key = key < 0 ? 0 : key;
-        dma16(kh, (uint32_t)key * (D * 2) + kcol[i],
-              __builtin_amdgcn_readfirstlane(ring_base + slot * KBLK + i * 1024));
+        dma16<SPARSE>(kh, (uint32_t)key * (D * 2) + kcol[i],
+                      __builtin_amdgcn_readfirstlane(ring_base + slot * KBLK + i * 1024));
       }
     }
   };

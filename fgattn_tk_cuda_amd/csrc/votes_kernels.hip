@@ -191,16 +191,14 @@ __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParam
 #pragma unroll
       for (int t = 0; t < NT; ++t) d[t] = *(SPATTN_LDS const u32x4*)((lds_cptr)(uintptr_t)((rd0 + slot) ^ (uint32_t)(t << 6)));
     };
-    auto copy = [&](const unsigned char* base, uint32_t off, uint32_t slot, int c) {
-      dma16(base, off, __builtin_amdgcn_readfirstlane(ring + slot + c * 1024));
-    };
+    auto copy = [&](uint32_t off, uint32_t slot, int c) { dma16(qc, off, __builtin_amdgcn_readfirstlane(ring + slot + c * 1024)); };
     // The keys, sixteen at a time like a tile of rows; rows past the last key repeat it, their votes are masked off.
     auto copy_keys = [&](int n, int slot) {
 #pragma unroll
       for (int c = 0; c < LPP; ++c) {
         int r = 64 * J + 16 * n + LPP * h + c;
         r = r < p.kv_len ? r : p.kv_len - 1;
-        copy(kh, (uint32_t)r * ROWB + goff[c], slot * TILE, c);
+        dma16<true>(kh, (uint32_t)r * ROWB + goff[c], __builtin_amdgcn_readfirstlane(ring + (slot * LPP + c) * 1024));
       }
     };
 #pragma unroll
@@ -293,7 +291,7 @@ __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParam
         for (int j = 0; j < NS; ++j) {
           const Load l = prepare(j);
 #pragma unroll
-          for (int c = 0; c < LPP; ++c) copy(qc, l.off[c], j * TILE, c);
+          for (int c = 0; c < LPP; ++c) copy(l.off[c], j * TILE, c);
         }
         wait_vmcnt<(NS - 1) * LPP>();
         u32x4 qa[2][NT];
@@ -317,7 +315,7 @@ __global__ __launch_bounds__(256, 3) void blockmax_votes_kernel(const VotesParam
           thr_next = read_thr(i + 1);
           read_tile(next, qa[P ^ 1]);
 #pragma unroll
-          for (int c = 0; c < LPP; ++c) copy(qc, l.off[c], slot, c);
+          for (int c = 0; c < LPP; ++c) copy(l.off[c], slot, c);
           f32x4 acc[4];
 #pragma unroll
           for (int t = 0; t < NT; ++t)

@@ -18,6 +18,10 @@ its header) and asserts that it holds no scratch access (a spill) and no s_waitc
 the asm statements (the compiler waiting for a load of its own).  The same holds for the walk of the votes kernel,
 from its first copy to the wait for the last one.
 
+The asm statements take base addresses in scalar registers.  A vector-memory instruction may read a scalar register that the
+vector ALU wrote (readfirstlane, readlane) five wait states later; the compiler keeps that distance for its own instructions
+and does not look into asm, so the listing is checked for it.
+
 The votes kernel lists rows in LDS as 16-bit numbers and reads several entries at a time.  A read through another scalar
 type would be free to move ahead of the stores (type-based aliasing); the last check looks at the types of its LDS
 loads and stores before any optimisation."""
@@ -98,6 +102,30 @@ def m0_uses_outside_asm(listing):
     return found
 
 
+def scalar_bases_too_close(listing, states=5):
+    """[(vector-ALU write, vector-memory instruction, wait states between them)] where an instruction reads a scalar register
+    fewer than `states` wait states after the vector ALU wrote it, in the order of the listing."""
+    def sregs(text):
+        out = {int(m) for m in re.findall(r"\bs(\d+)\b", text)}
+        for lo, hi in re.findall(r"\bs\[(\d+):(\d+)\]", text):
+            out.update(range(int(lo), int(hi) + 1))
+        return out
+
+    found, recent = [], []   # recent: (wait states since, registers, instruction)
+    for raw in listing.split("\n"):
+        t = raw.split(";")[0].strip()
+        if not t or t.startswith(".") or t.endswith(":"):
+            continue
+        op, args = t.split()[0], t.split(None, 1)[1] if " " in t else ""
+        if _is_vmem(op):
+            found += [(w, t, age) for age, regs, w in recent if age < states and regs & sregs(args)]
+        passed = 1 + (int(args, 0) if op == "s_nop" else 0)
+        recent = [(age + passed, regs, w) for age, regs, w in recent if age + passed < states]
+        if op.startswith("v_") and re.match(r"s\[?\d", args):
+            recent.append((0, sregs(args.split(",")[0]), t))
+    return found
+
+
 def tile_loop_findings(listing):
     """{kernel: (scratch accesses, compiler vmcnt waits)} inside the tile loop of every attn_fwd_kernel
     instantiation of a listing; a kernel whose loop is not found maps to None."""
@@ -173,6 +201,14 @@ def test_tile_loop_checker():
     assert list(tile_loop_findings(body.replace("s_cbranch_scc1 .LBB0_3", "s_nop 1") % "").values()) == [None]
 
 
+def test_scalar_base_checker():
+    late = "\tv_readfirstlane_b32 s21, v9\n\tv_readfirstlane_b32 s20, v8\n%s\ts_mov_b32 m0, s3\n\tglobal_load_lds_dwordx4 v7, s[20:21]\n"
+    assert len(scalar_bases_too_close(late % "")) == 2
+    assert len(scalar_bases_too_close(late % "\ts_nop 2\n")) == 1
+    assert scalar_bases_too_close(late % "\ts_nop 3\n") == []
+    assert scalar_bases_too_close((late % "").replace("s[20:21]", "s[22:23]")) == []
+
+
 def test_m0_checker_sees_a_compiler_use():
     ok = "\t;;#ASMSTART\n\ts_mov_b32 m0, s3\n\tglobal_load_lds_dwordx4 v1, s[0:1]\n\t;;#ASMEND\n\tv_mov_b32_e32 v2, v3\n"
     bad = ok + "\ts_mov_b32 m0, -1\n"
@@ -203,6 +239,8 @@ def test_no_instruction_touches_a_register_with_a_load_in_flight(tmp_path):
         assert "global_load_lds_dwordx4" in text, unit
         uses = m0_uses_outside_asm(text)
         assert not uses, "%s: the compiler uses m0 next to hand-written copies: %s" % (unit, uses[:3])
+        close = scalar_bases_too_close(text)
+        assert not close, "%s: %d bases written too late, e.g. %s" % (unit, len(close), close[0])
         if unit == VOTES_UNIT:
             walks = walk_findings(text)
             assert len(walks) == 4 and all(f == (0, 0) for f in walks.values()), "%s: %s" % (unit, walks)
