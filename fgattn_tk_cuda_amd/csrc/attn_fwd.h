@@ -47,6 +47,9 @@ namespace spattn {
 
 typedef __attribute__((ext_vector_type(4))) short s16x4;
 
+// The pieces of the kernel that hold its register arrays by reference: one that is not inlined puts them into memory.
+#define SPATTN_INLINE __attribute__((always_inline))
+
 template <int D, int MODE, bool HAS_V>
 struct AttnCfg {
   static constexpr int kTileBytes = 64 * D * 2;
@@ -407,11 +410,13 @@ void attn_fwd_kernel(const AttnParams p) {
   // SPLIT_SM: the exponentials of a tile are taken in two halves, score registers 0-7 of every
   // block under the P V multiplies of the tile before, registers 8-15 under the QK^T multiplies
   // of the tile after, so that every multiply has the same vector-ALU work next to it (all of
-  // it under QK^T leaves the vector ALU the bottleneck there and idle under P V).  Needs the
-  // reference fixed before the tile's scores exist, which LAZY_MAX gives.  Not with token lists of 128-row q-blocks at
+  // it under QK^T leaves the vector ALU the bottleneck there and idle under P V).  LAZY_MAX fixes the reference before the
+  // tile's scores exist; with statistics the maxima are reduced under the multiplies of the first 16-key step of P V, ahead of
+  // the exponentials (all exponentials under QK^T: 12 x 9000 x 128 with statistics 494 us, now 477; 24 x 1000 x 64 14.5, now
+  // 13.8; 12 x 9000 x 64 321, now 316).  Not with token lists of 128-row q-blocks at
   // d = 64, whose third wave needs the 16 registers of the second set of operands (dense attention and block lists of
   // that shape fit with both and lose 1 % without).
-  constexpr bool SPLIT_SM = LAZY_MAX && HAS_V && !(MODE == KV_TOKENS && D == 64 && QBLK == 128);
+  constexpr bool SPLIT_SM = HAS_V && !(MODE == KV_TOKENS && D == 64 && QBLK == 128);
   u32x4 pb[SPLIT_SM ? 2 : 1][HAS_V ? 2 * NMB : 1];   // P^T operands, k-step 2mb + h; SPLIT_SM: by tile parity
 
   // Per-lane LDS addresses inside slot 0; slot, score block and k-step offsets are added
@@ -458,7 +463,7 @@ void attn_fwd_kernel(const AttnParams p) {
   // ---- building blocks --------------------------------------------------------------
   // Keys of tile `it` that do not exist get -inf.  Accumulator register 4j+i of block mb
   // is key ksub*KW + 32mb + 8j + 4g + i of the tile.
-  auto mask_tile = [&](int desc, int desc_hi, f32x16 (&s)[NMB]) {
+  auto mask_tile = [&](int desc, int desc_hi, f32x16 (&s)[NMB]) SPATTN_INLINE {
     bool some;                 // wave-uniform: some key of the tile does not exist
     unsigned long long m;      // bit c: key c of the tile exists
     if constexpr (MODE == KV_TOKENS) {
@@ -489,7 +494,7 @@ void attn_fwd_kernel(const AttnParams p) {
   // Row max of a score tile in NP pieces (so that they can be placed between multiplies),
   // then the exchange between the two 32-lane halves; returns max * sf.
   constexpr int NP = 4 * NMB;
-  auto stat_piece = [&](const f32x16 (&s)[NMB], int k, float& mloc) {
+  auto stat_piece = [&](const f32x16 (&s)[NMB], int k, float& mloc) SPATTN_INLINE {
     const int mb = k >> 2, r = 4 * (k & 3);
     if (k == 0) mloc = s[0][0];
     mloc = max3_raw(mloc, s[mb][r], s[mb][r + 1]);
@@ -512,7 +517,7 @@ void attn_fwd_kernel(const AttnParams p) {
         blockmax_at(tile) = bf16_round_up(max_raw(bm_own, bm_xchg[(tile & 1) * 64 + 32 * qsub + ln]));
     }
   };
-  auto stat_finish = [&](float mloc, int tile) -> float {
+  auto stat_finish = [&](float mloc, int tile) SPATTN_INLINE -> float {
     mloc = pair_max(mloc);
     if constexpr (BLOCKMAX && KSPLIT == 1) {
       if (p.blockmax != nullptr && g == 0 && tile_exists(tile) && (QBLK != 256 || qrow < p.Sp)) blockmax_at(tile) = bf16_round_up(mloc);
@@ -526,32 +531,38 @@ void attn_fwd_kernel(const AttnParams p) {
     m_true = max_raw(m_true, mloc);
     return mloc * p.sf;
   };
-  auto row_stats = [&](const f32x16 (&s)[NMB], int tile) -> float {
+  auto row_stats = [&](const f32x16 (&s)[NMB], int tile) SPATTN_INLINE -> float {
     float mloc;
 #pragma unroll
     for (int k = 0; k < NP; ++k) stat_piece(s, k, mloc);
     return stat_finish(mloc, tile);
   };
-  // Move the exponent reference if some row of the wave outgrew it; rescales O and l.
-  auto maybe_rescale = [&](float mloc_sf) {
-    if (__any(mloc_sf > mr_sf + kSlack)) {
+  // Moves the exponent reference if some row of the wave outgrew it; what was accumulated against the old one is then to be
+  // multiplied by alpha, in rescale().
+  float alpha = 1.f;
+  auto move_reference = [&](float mloc_sf) SPATTN_INLINE -> bool {
+    const bool moved = __any(mloc_sf > mr_sf + kSlack);
+    if (moved) {
       const float new_sf = max_raw(mr_sf, mloc_sf);
-      const float alpha = (new_sf == kNegInf) ? 1.f : __builtin_amdgcn_exp2f(mr_sf - new_sf);
+      alpha = (new_sf == kNegInf) ? 1.f : __builtin_amdgcn_exp2f(mr_sf - new_sf);
       mr_sf = new_sf;
       base_eff = (new_sf == kNegInf) ? kNoRef : new_sf;
-      l_run *= alpha;
-      if constexpr (HAS_V) {
+    }
+    return moved;
+  };
+  auto rescale = [&]() SPATTN_INLINE {
+    l_run *= alpha;
+    if constexpr (HAS_V) {
 #pragma unroll
-        for (int db = 0; db < NDB; ++db)
+      for (int db = 0; db < NDB; ++db)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
-      }
+        for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
     }
   };
   // p = exp2(s*sf - reference) for registers r0..r0+cnt-1 of block mb; adds to the row sum
   // and leaves P^T as bf16 MFMA operands (k-step 2mb+h takes registers 8h..8h+7 of block
   // mb, i.e. keys 32mb + 16h + {4g..4g+3} and 32mb + 16h + 8 + {4g..4g+3}).
-  auto softmax_chunk = [&](const f32x16 (&s)[NMB], float base, int mb, int r0, int cnt, int par) {
+  auto softmax_chunk = [&](const f32x16 (&s)[NMB], float base, int mb, int r0, int cnt, int par) SPATTN_INLINE {
 #pragma unroll
     for (int r = r0; r < r0 + cnt; r += 2) {
       const float e0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[mb][r], p.sf, -base));
@@ -564,7 +575,7 @@ void attn_fwd_kernel(const AttnParams p) {
   // Pin the softmax results where they are produced; otherwise the compiler sinks the
   // whole softmax to the first use of P and nothing overlaps the MFMAs.
   // half: 0 = the operands of registers 0-7, 1 = of registers 8-15, 2 = both
-  auto pin_softmax = [&](int par, int half) {
+  auto pin_softmax = [&](int par, int half) SPATTN_INLINE {
     asm volatile("" : "+v"(l_tile));
     if constexpr (HAS_V) {
 #pragma unroll
@@ -574,20 +585,20 @@ void attn_fwd_kernel(const AttnParams p) {
           if (half == 2 || (ks & 1) == half) asm volatile("" : "+v"(pb[SPLIT_SM ? par : 0][ks][i]));
     }
   };
-  auto softmax_only = [&](const f32x16 (&s)[NMB], int par, float base) {
+  auto softmax_only = [&](const f32x16 (&s)[NMB], int par, float base) SPATTN_INLINE {
 #pragma unroll
-    for (int mb = 0; mb < NMB; ++mb) softmax_chunk(s, base, mb, 0, 16, par);
+    for (int i = 0; i < 2 * NMB; ++i) softmax_chunk(s, base, i % NMB, 8 * (i / NMB), 8, par);
   };
-  auto softmax_half = [&](const f32x16 (&s)[NMB], int par, int half) {
+  auto softmax_half = [&](const f32x16 (&s)[NMB], int par, int half) SPATTN_INLINE {
 #pragma unroll
     for (int mb = 0; mb < NMB; ++mb) softmax_chunk(s, base_eff, mb, 8 * half, 8, par);
   };
   // Closes the softmax of a tile: adds its sum to the denominator.  LAZY_MAX: first redoes
   // the tile against a new reference if some row of the wave outgrew the old one.
-  auto softmax_close = [&](const f32x16 (&s)[NMB], int par) {
+  auto softmax_close = [&](const f32x16 (&s)[NMB], int par) SPATTN_INLINE {
     if constexpr (LAZY_MAX) {
       if (__any(!(l_tile <= kTrigger))) {
-        maybe_rescale(row_stats(s, 0));
+        if (move_reference(row_stats(s, 0))) rescale();
         // a row that still has no reference has seen masked keys only: p = exp2(-inf - 0) = 0
         softmax_only(s, par, mr_sf == kNegInf ? 0.f : mr_sf);
       }
@@ -600,9 +611,9 @@ void attn_fwd_kernel(const AttnParams p) {
   // group as soon as its multiply of this group has been issued (two buffers: at d = 128 sixteen registers
   // more and 0.2-0.6 % slower, at d = 64 spills in the loop and 0.8 % slower).
   constexpr int NG = 2 * NMB;
-  constexpr int VB = (QBLK == 128 && (D == 128 || LAZY_MAX)) ? 1 : 2;
+  constexpr int VB = QBLK == 128 ? 1 : 2;
   u32x2 va[HAS_V ? VB : 1][HAS_V ? NDB : 1][2];
-  auto v_read_db = [&](uint32_t vofs, int gi, int db) {
+  auto v_read_db = [&](uint32_t vofs, int gi, int db) SPATTN_INLINE {
     if constexpr (HAS_V) {
       const uint32_t x1 = v_cur ^ (uint32_t)(db << 6);
       const uint32_t x2 = x1 ^ 32u;
@@ -612,7 +623,7 @@ void attn_fwd_kernel(const AttnParams p) {
       va[gi % VB][db][1] = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((SPATTN_LDS s16x4*)a2));
     }
   };
-  auto v_reads = [&](uint32_t vofs, int gi) {
+  auto v_reads = [&](uint32_t vofs, int gi) SPATTN_INLINE {
 #pragma unroll
     for (int db = 0; db < (HAS_V ? NDB : 0); ++db) v_read_db(vofs, gi, db);
   };
@@ -627,7 +638,7 @@ void attn_fwd_kernel(const AttnParams p) {
   // so that PV does not start by waiting for LDS.
   constexpr int kEarly = 1;
   auto qk_tile = [&](auto with_sm, auto early_v, uint32_t kofs, uint32_t vofs, f32x16 (&s_out)[NMB], f32x16 (&s_in)[NMB],
-                     int par_in, const TileLoad* tl, bool live) {
+                     int par_in, const TileLoad* tl, bool live) SPATTN_INLINE {
     constexpr bool WITH_SM = decltype(with_sm)::value;
     constexpr bool EARLY_V = decltype(early_v)::value;
     constexpr int EPM = 16 / NT;
@@ -658,7 +669,9 @@ void attn_fwd_kernel(const AttnParams p) {
         if constexpr (WITH_SM && SPLIT_SM) {
           if (m % MPP == 0) softmax_chunk(s_in, base, (m / MPP) / 4, 8 + 2 * ((m / MPP) % 4), 2, par_in);
         } else if constexpr (WITH_SM) {
-          softmax_chunk(s_in, base, m / NT, (m % NT) * EPM, EPM, par_in);
+          // in the order of the two halves: a row's denominator has the same bits with and without V
+          constexpr int HM = NM / 2;
+          softmax_chunk(s_in, base, (m % HM) / (NT / 2), 8 * (m / HM) + (m % (NT / 2)) * EPM, EPM, par_in);
         }
         if (tl != nullptr && live) {
           constexpr int STEP = NM / LPT;
@@ -698,17 +711,21 @@ void attn_fwd_kernel(const AttnParams p) {
   };
   // O^T += V^T P^T from the V tile at offset vofs from the first V slot, one 16-key step (NDB multiplies) at
   // a time; the operands of step 0 are in flight or here already (FIRST_LOADED), those of
-  // step gi+1 are requested before step gi is multiplied.  STAT: the row maxima of s_next
-  // are reduced between the multiplies; returns them (times sf).
+  // step gi+1 are requested before step gi is multiplied.  STAT: the row maxima of s_next (tile tile_next)
+  // are reduced between the multiplies and the reference follows them.
   // EARLY_SM: the exponentials of registers 0-7 of s_next (the tile after, parity par ^ 1) are
-  // taken between the multiplies.
+  // taken between the multiplies; with STAT between those behind the first step, which has the maxima.
   auto pv_tile = [&](auto first_loaded, auto stat_c, uint32_t vofs, const TileLoad* tl, bool live, const f32x16 (&s_next)[NMB],
-                     int par, auto early_sm, int tile_next = 0) -> float {
+                     int par, auto early_sm, int tile_next = 0) SPATTN_INLINE {
     constexpr bool STAT = decltype(stat_c)::value;
     constexpr bool EARLY_SM = decltype(early_sm)::value;
-    constexpr int MPP = NDB / 2;   // EARLY_SM: multiplies per pair of score registers
-    const float base = base_eff;
+    constexpr int NM = NG * NDB;
+    constexpr int PAIRS = 4 * NMB;                      // of score registers 0-7
+    constexpr int M0 = (STAT && EARLY_SM) ? NDB : 0;    // first multiply with exponentials
+    constexpr int MS = EARLY_SM ? NDB : NM;             // STAT: multiplies with maxima
+    float base = base_eff;
     float mloc = 0.f;
+    bool moved = false;
     if constexpr (HAS_V) {
       if constexpr (!decltype(first_loaded)::value) v_reads(vofs, 0);
 #pragma unroll
@@ -722,15 +739,17 @@ void attn_fwd_kernel(const AttnParams p) {
           if (VB == 1 && gi + 1 < NG) v_read_db(vofs, gi + 1, db);
           const int m = gi * NDB + db;
           if constexpr (EARLY_SM) {
-            if (m % MPP == 0) softmax_chunk(s_next, base, (m / MPP) / 4, 2 * ((m / MPP) % 4), 2, par ^ 1);
+#pragma unroll
+            for (int j = 0; j < PAIRS; ++j)
+              if (m == M0 + j * (NM - M0) / PAIRS) softmax_chunk(s_next, base, j / 4, 2 * (j % 4), 2, par ^ 1);
           }
           if constexpr (STAT) {
-            constexpr int PPM = (NP + NG * NDB - 1) / (NG * NDB);   // pieces per multiply
+            constexpr int PPM = (NP + MS - 1) / MS;   // pieces per multiply
 #pragma unroll
             for (int k = m * PPM; k < (m + 1) * PPM && k < NP; ++k) stat_piece(s_next, k, mloc);
           }
           if (tl != nullptr && live) {   // a tile copy, spread over the multiplies
-            constexpr int STEP = (NG * NDB) / LPT;
+            constexpr int STEP = NM / LPT;
             if (m % STEP == STEP - 1) load_part(*tl, m / STEP);
           }
         }
@@ -738,20 +757,31 @@ void attn_fwd_kernel(const AttnParams p) {
 #pragma unroll
           for (int db = 0; db < NDB; ++db) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if constexpr (MPP == 1) __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
+            // seven instructions per pair, two per piece of the maxima
+            if (gi * NDB + db < M0) __builtin_amdgcn_sched_group_barrier(0x002, (2 * NP + NDB - 1) / NDB, 0);
+            else if constexpr (M0 > 0) __builtin_amdgcn_sched_group_barrier(0x002, (7 * PAIRS + NM - M0 - 1) / (NM - M0), 0);
+            else if constexpr (NM == PAIRS) __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
             else if (db % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
             else __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
           }
         }
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (STAT && EARLY_SM) {
+          if (gi == 0) {
+            moved = move_reference(stat_finish(mloc, tile_next));
+            base = base_eff;
+          }
+        }
       }
       if constexpr (EARLY_SM) pin_softmax(par ^ 1, 0);
     } else if constexpr (STAT) {
 #pragma unroll
       for (int k = 0; k < NP; ++k) stat_piece(s_next, k, mloc);
     }
-    if constexpr (STAT) return stat_finish(mloc, tile_next);
-    return 0.f;
+    if constexpr (STAT && !EARLY_SM) moved = move_reference(stat_finish(mloc, tile_next));
+    if constexpr (STAT) {
+      if (moved) rescale();
+    }
   };
 
   f32x16 s_e[NMB], s_o[NMB];   // scores of even / odd tiles
@@ -761,7 +791,7 @@ void attn_fwd_kernel(const AttnParams p) {
   // tile it (V slot NK + it % 2) is multiplied while the row maxima of tile it+1 are
   // reduced.  The barrier frees the slots of K(it) and V(it-1): V(it+1) and, if it exists,
   // K(it+NK) are copied into them.  KC = it % 6 fixes every slot at compile time.
-  auto tile_body = [&](auto kc, int it) {
+  auto tile_body = [&](auto kc, int it) SPATTN_INLINE {
     constexpr int KC = decltype(kc)::value;
     // KS, KN: ring slots of K(it+1), K(it+NK); VS: V slot of tile it counted from the first
     // V slot; VN: ring slot of V(it+1)
@@ -815,16 +845,14 @@ void attn_fwd_kernel(const AttnParams p) {
     softmax_close(s_a, PAR);
     mask_tile(m_lo, m_hi, s_b);
     if constexpr (MODE != KV_TOKENS) idw[(KC + NK + 1) % 6] = tile_desc(it + NK + 1);
-    float mloc_sf;
-    using stat_t = std::integral_constant<bool, !LAZY_MAX>;
+    using stat_t = std::integral_constant<bool, STATS>;
     if constexpr (HAS_V) {
       const TileLoad tl_second = K_FIRST ? prepare_tile(d_v, VN, true, GV{}) : prepare_tile(d_k, KN, false, GK{});
-      mloc_sf = pv_tile(std::true_type{}, stat_t{}, VS * TILE, &tl_second, K_FIRST ? true : has_kn, s_b, PAR,
-                        std::integral_constant<bool, SPLIT_SM>{}, it + 1);
+      pv_tile(std::true_type{}, stat_t{}, VS * TILE, &tl_second, K_FIRST ? true : has_kn, s_b, PAR,
+              std::integral_constant<bool, SPLIT_SM>{}, it + 1);
     } else {
-      mloc_sf = pv_tile(std::true_type{}, stat_t{}, 0, nullptr, false, s_b, PAR, std::false_type{}, it + 1);
+      pv_tile(std::true_type{}, stat_t{}, 0, nullptr, false, s_b, PAR, std::false_type{}, it + 1);
     }
-    if constexpr (!LAZY_MAX) maybe_rescale(mloc_sf);
   };
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
@@ -849,7 +877,7 @@ void attn_fwd_kernel(const AttnParams p) {
     qk_tile(std::false_type{}, std::false_type{}, 0, 0, s_e, s_e, 0, nullptr, false);
     if constexpr (MODE == KV_TOKENS) mask_tile(idw[0], idh[0], s_e);
     else mask_tile(hd[0], 0, s_e);
-    maybe_rescale(row_stats(s_e, 0));
+    move_reference(row_stats(s_e, 0));   // nothing is accumulated yet
     if constexpr (SPLIT_SM) softmax_half(s_e, 0, 0);   // nothing to hide these under
 
     int it = 0;

@@ -25,8 +25,9 @@ namespace spattn {
 // and a workgroup of its own finishes a CU's last q-block sooner than two do.  A last round that fills up to half of the CUs
 // costs it 0-19 % instead (its other form spreads that round over twice as many).  From 32 tiles on with the last round
 // empty or more than half full 0.91-0.98.  With statistics, whose row maxima keep the waves of a workgroup waiting for
-// each other, that holds up to two rounds (0.94-0.99; 12 x 9000 502 -> 471 us), behind them 1.00-1.04.  Same bits as the
-// 128-row form.
+// each other, that holds up to two rounds (0.94-0.99; 12 x 9000 502 -> 471 us) and from 64 tiles on up to five (68 tiles
+// 0.99, 90 and more 0.95-0.98: 12 x 14000 1163 -> 1105, 12 x 20000 2243 -> 2165, 16 x 20400 2968 -> 2905; 36 tiles in three
+// rounds 0.98, left to the 128-row form), behind them 0.98-1.03.  Same bits as the 128-row form.
 // The other forms add the row sums and outputs of a row in another order: a launch over some heads of a computation
 // goes by all of its heads, so that a row's denominator, and with it a key at a threshold, does not depend on the split.
 // Between 128 and 256 rows, where no bit changes, it goes by its own q-blocks (3 of 12 heads x 9000 with statistics 142 us
@@ -42,7 +43,8 @@ DenseForm dense_form(int D, bool has_v, bool stats, int S, int kv_len, long long
   if (D == 128 && has_v) {
     const long long n256 = launched * ((S + 255) / 256);
     const long long last = n256 % kCus;
-    if (tiles >= 32 && (last == 0 || last > kCus / 2) && (!stats || n256 <= 2 * kCus)) return {256, 1};
+    const bool few = n256 <= 2 * kCus || (tiles >= 64 && n256 <= 5 * kCus);
+    if (tiles >= 32 && (last == 0 || last > kCus / 2) && (!stats || few)) return {256, 1};
   }
   return {128, 1};
 }

@@ -18,6 +18,13 @@ def test_some_heads_take_256_row_qblocks_by_their_own_number(heads, S, of_heads,
     assert form(128, 1, 1, heads, S, 0, of_heads) == (2561 if last == 0 or last > 128 else 1281)
 
 
+def test_256_row_qblocks_with_statistics_by_rounds():
+    """648 q-blocks of 256 rows of 36 key tiles and 660 of 219: behind two rounds from 64 tiles on; five rounds and six."""
+    assert form(128, 1, 1, 72, 2304) == 1281 and form(128, 1, 1, 12, 14000) == 2561
+    assert form(128, 1, 1, 44, 4033) == 2561 and form(128, 1, 1, 44, 4032) == 1281   # 64 and 63 tiles, 704 q-blocks
+    assert form(128, 1, 1, 16, 20480) == 2561 and form(128, 1, 1, 24, 16384) == 1281
+
+
 def test_forms_that_add_in_another_order_go_by_the_whole():
     assert form(128, 1, 1, 4, 2000, 0, 16) == form(128, 1, 1, 16, 2000) == 1282 and form(128, 1, 1, 4, 2000) == 641
     assert form(64, 1, 1, 4, 2000, 0, 26) == form(64, 1, 1, 26, 2000) != form(64, 1, 1, 4, 2000)
