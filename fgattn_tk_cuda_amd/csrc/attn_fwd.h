@@ -562,15 +562,42 @@ void attn_fwd_kernel(const AttnParams p) {
   // p = exp2(s*sf - reference) for registers r0..r0+cnt-1 of block mb; adds to the row sum
   // and leaves P^T as bf16 MFMA operands (k-step 2mb+h takes registers 8h..8h+7 of block
   // mb, i.e. keys 32mb + 16h + {4g..4g+3} and 32mb + 16h + 8 + {4g..4g+3}).
-  auto softmax_chunk = [&](const f32x16 (&s)[NMB], float base, int mb, int r0, int cnt, int par) SPATTN_INLINE {
+  // LAG: the sum and the conversion of a pair are issued behind the exponentials of the next one, so that they do not wait for
+  // their own; at d = 128 the order is pinned, the compiler sorts it back otherwise.  Dense d = 128 0.98-0.99 of the time (12 x
+  // 20000 2131 -> 2104 us), with statistics 0.99, statistics alone 0.97-0.985 (12 x 32760 3342 -> 3299), lists 0.985-1.0
+  // (128-row tokens 12 x 16000 147.7 -> 145.6); dense d = 64 0.98-1.0.  Pinned d = 64 forms lose 1-2 %, and their block lists
+  // 0.7 % by the lag alone.  A lag of two pairs and pinned arguments measured the same.
+  constexpr bool LAG = D == 128 || MODE == KV_DENSE;
+  struct Pair {
+    float e0, e1;
+    int mb, r;   // block and first register; r < 0: none
+  };
+  constexpr Pair kNoPair = {0.f, 0.f, 0, -1};
+  auto softmax_add = [&](const Pair& x, int par) SPATTN_INLINE {
+    if (x.r < 0) return;
+    l_tile = (x.mb == 0 && x.r == 0) ? x.e0 : l_tile + x.e0;
+    l_tile += x.e1;
+    if constexpr (HAS_V) pb[SPLIT_SM ? par : 0][2 * x.mb + (x.r >> 3)][(x.r & 7) >> 1] = pack_bf16(x.e0, x.e1);
+  };
+  // last: the pair that is still to be added, here or behind the last chunk
+  auto softmax_lag = [&](const f32x16 (&s)[NMB], float base, int mb, int r0, int cnt, int par, Pair& last) SPATTN_INLINE {
 #pragma unroll
     for (int r = r0; r < r0 + cnt; r += 2) {
-      const float e0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[mb][r], p.sf, -base));
-      const float e1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[mb][r + 1], p.sf, -base));
-      l_tile = (mb == 0 && r == 0) ? e0 : l_tile + e0;
-      l_tile += e1;
-      if constexpr (HAS_V) pb[SPLIT_SM ? par : 0][2 * mb + (r >> 3)][(r & 7) >> 1] = pack_bf16(e0, e1);
+      Pair now = {__builtin_amdgcn_exp2f(__builtin_fmaf(s[mb][r], p.sf, -base)),
+                  __builtin_amdgcn_exp2f(__builtin_fmaf(s[mb][r + 1], p.sf, -base)), mb, r};
+      if constexpr (!LAG) {
+        softmax_add(now, par);
+      } else {
+        if constexpr (D == 128) asm volatile("" : "+v"(now.e0), "+v"(now.e1));
+        softmax_add(last, par);
+        last = now;
+      }
     }
+  };
+  auto softmax_chunk = [&](const f32x16 (&s)[NMB], float base, int mb, int r0, int cnt, int par) SPATTN_INLINE {
+    Pair last = kNoPair;
+    softmax_lag(s, base, mb, r0, cnt, par, last);
+    softmax_add(last, par);
   };
   // Pin the softmax results where they are produced; otherwise the compiler sinks the
   // whole softmax to the first use of P and nothing overlaps the MFMAs.
@@ -646,6 +673,7 @@ void attn_fwd_kernel(const AttnParams p) {
     const float base = base_eff;
     // Multiply m: k-step m / NMB of score block m % NMB - neighbours share their Q operand.
     constexpr int NM = NMB * NT;
+    Pair last = kNoPair;
     u32x4 ka[NT];
     auto k_reads = [&](int m0, int m1) {
 #pragma unroll
@@ -667,11 +695,11 @@ void attn_fwd_kernel(const AttnParams p) {
         const int t = m / NMB, mb = m % NMB;
         s_out[mb] = mfma32(ka[m % NT], qf[t], t == 0 ? zero : s_out[mb]);
         if constexpr (WITH_SM && SPLIT_SM) {
-          if (m % MPP == 0) softmax_chunk(s_in, base, (m / MPP) / 4, 8 + 2 * ((m / MPP) % 4), 2, par_in);
+          if (m % MPP == 0) softmax_lag(s_in, base, (m / MPP) / 4, 8 + 2 * ((m / MPP) % 4), 2, par_in, last);
         } else if constexpr (WITH_SM) {
           // in the order of the two halves: a row's denominator has the same bits with and without V
           constexpr int HM = NM / 2;
-          softmax_chunk(s_in, base, (m % HM) / (NT / 2), 8 * (m / HM) + (m % (NT / 2)) * EPM, EPM, par_in);
+          softmax_lag(s_in, base, (m % HM) / (NT / 2), 8 * (m / HM) + (m % (NT / 2)) * EPM, EPM, par_in, last);
         }
         if (tl != nullptr && live) {
           constexpr int STEP = NM / LPT;
@@ -707,7 +735,10 @@ void attn_fwd_kernel(const AttnParams p) {
         steps(m0, m1);
       }
     }
-    if constexpr (WITH_SM) pin_softmax(par_in, SPLIT_SM ? 1 : 2);
+    if constexpr (WITH_SM) {
+      softmax_add(last, par_in);
+      pin_softmax(par_in, SPLIT_SM ? 1 : 2);
+    }
   };
   // O^T += V^T P^T from the V tile at offset vofs from the first V slot, one 16-key step (NDB multiplies) at
   // a time; the operands of step 0 are in flight or here already (FIRST_LOADED), those of
@@ -726,6 +757,7 @@ void attn_fwd_kernel(const AttnParams p) {
     float base = base_eff;
     float mloc = 0.f;
     bool moved = false;
+    Pair last = kNoPair;
     if constexpr (HAS_V) {
       if constexpr (!decltype(first_loaded)::value) v_reads(vofs, 0);
 #pragma unroll
@@ -741,7 +773,7 @@ void attn_fwd_kernel(const AttnParams p) {
           if constexpr (EARLY_SM) {
 #pragma unroll
             for (int j = 0; j < PAIRS; ++j)
-              if (m == M0 + j * (NM - M0) / PAIRS) softmax_chunk(s_next, base, j / 4, 2 * (j % 4), 2, par ^ 1);
+              if (m == M0 + j * (NM - M0) / PAIRS) softmax_lag(s_next, base, j / 4, 2 * (j % 4), 2, par ^ 1, last);
           }
           if constexpr (STAT) {
             constexpr int PPM = (NP + MS - 1) / MS;   // pieces per multiply
@@ -773,7 +805,10 @@ void attn_fwd_kernel(const AttnParams p) {
           }
         }
       }
-      if constexpr (EARLY_SM) pin_softmax(par ^ 1, 0);
+      if constexpr (EARLY_SM) {
+        softmax_add(last, par ^ 1);
+        pin_softmax(par ^ 1, 0);
+      }
     } else if constexpr (STAT) {
 #pragma unroll
       for (int k = 0; k < NP; ++k) stat_piece(s_next, k, mloc);
