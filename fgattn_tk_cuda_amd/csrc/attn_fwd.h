@@ -91,10 +91,12 @@ constexpr int attn_waves_per_simd() {
 // NGRP = 2 (dense attention and statistics of launches that leave the chip idle): two groups of four waves share a
 // q-block, each with a ring of its own and half of the tiles; both meet at the same barriers and finish half of the
 // columns each.
-template <int D, int QBLK, int MODE, bool HAS_V, bool STATS, int NGRP>
+// HALVES (lists of 128-row q-blocks in launches that leave the chip idle): a workgroup takes 64 rows, two share a list.
+template <int D, int QBLK, int MODE, bool HAS_V, bool STATS, int NGRP, bool HALVES>
 __global__ __launch_bounds__(64 * attn_waves<QBLK>() * NGRP) __attribute__((amdgpu_waves_per_eu(attn_waves_per_simd<D, QBLK, NGRP>())))
 void attn_fwd_kernel(const AttnParams p) {
   static_assert(NGRP == 1 || MODE == KV_DENSE, "groups share dense tiles");
+  static_assert(!HALVES || (MODE != KV_DENSE && QBLK == 64), "halves of a list's q-block");
   static_assert(D == 64 || D == 128, "head dim");
   static_assert(QBLK == 64 || QBLK == 128 || (QBLK == 256 && MODE == KV_DENSE && HAS_V && D == 128 && NGRP == 1), "q-block");
   using Cfg = AttnCfg<D, MODE, HAS_V>;
@@ -128,15 +130,32 @@ void attn_fwd_kernel(const AttnParams p) {
   const int ksub = wave / NQW;
 
   const int total = p.nqblk * p.H * p.B;
+  int half = 0;
+  unsigned at = blockIdx.x;
+  if constexpr (HALVES) {
+    if (p.order) {
+      // eight entries at a time, their first halves and then their second ones: both halves of a list on one XCD, for its L2
+      const int e0 = (int)(at >> 4) * 8, j = (int)(at & 15);
+      const int n8 = total - e0 < 8 ? total - e0 : 8;
+      half = j >= n8;
+      at = e0 + (half ? j - n8 : j);
+    } else {
+      at = xcd_remap(at, 2 * total);
+      half = (int)(at & 1);
+      at >>= 1;
+    }
+  }
   // a caller-given work order (longest lists first) replaces the XCD-contiguous default
-  const int wg = p.order ? ((const __attribute__((address_space(4))) int*)p.order)[blockIdx.x]
-                         : xcd_remap(blockIdx.x, total);
+  const int wg = p.order ? ((const __attribute__((address_space(4))) int*)p.order)[at]
+                         : HALVES ? (int)at : xcd_remap(at, total);
   // an entry of a work order that names no q-block: nothing is addressed (wave-uniform, ahead
   // of every copy and barrier)
   if ((unsigned)wg >= (unsigned)total) return;
   // The compiler divides on the vector ALU and would keep everything that follows from the quotient there.
   const int bh = __builtin_amdgcn_readfirstlane(wg / p.nqblk);
-  const int qb = wg - bh * p.nqblk;
+  const int lb = wg - bh * p.nqblk;                  // list
+  const int qb = HALVES ? 2 * lb + half : lb;        // rows
+  if (HALVES && qb * QBLK >= p.S) return;            // the last q-block may end in its first half
 
   const size_t head_off = (size_t)bh * p.S * D;
   const uint16_t* __restrict__ qh = p.q + head_off;
@@ -153,7 +172,7 @@ void attn_fwd_kernel(const AttnParams p) {
   if constexpr (MODE == KV_DENSE) {
     ntiles = (p.kv_len + 63) >> 6;
   } else {
-    const size_t lrow = (size_t)bh * p.nqblk + qb;
+    const size_t lrow = (size_t)bh * p.nqblk + lb;
     lst = (cint_p)(p.idx + lrow * p.idx_stride);
     n = ((cint_p)p.cnt)[lrow];
     n = n < 0 ? 0 : (n > p.idx_stride ? p.idx_stride : n);
@@ -223,7 +242,7 @@ void attn_fwd_kernel(const AttnParams p) {
   int idr[6] = {};   // used with token lists only
   uint64_t lst_addr = 0;
   if constexpr (MODE == KV_TOKENS) {
-    const uint64_t a = (uint64_t)(uintptr_t)(p.idx + ((size_t)bh * p.nqblk + qb) * p.idx_stride);
+    const uint64_t a = (uint64_t)(uintptr_t)(p.idx + ((size_t)bh * p.nqblk + lb) * p.idx_stride);
     // readfirstlane returns a signed int: without the casts the low word would be sign-extended
     const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a);
     const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
@@ -1132,20 +1151,20 @@ void attn_fwd_kernel(const AttnParams p) {
 // Raises the dynamic-LDS limit of one instantiation on the current device (once per device; the
 // launcher does it on the first launch, a caller that is about to record launches into a graph
 // does it beforehand through spattn_init).
-template <int D, int QBLK, int MODE, bool HAS_V, bool STATS, int NGRP = 1>
+template <int D, int QBLK, int MODE, bool HAS_V, bool STATS, int NGRP = 1, bool HALVES = false>
 inline hipError_t prepare_attn_fwd() {
   static bool attr_set[kMaxDevices] = {};
-  return raise_lds_limit(reinterpret_cast<const void*>(attn_fwd_kernel<D, QBLK, MODE, HAS_V, STATS, NGRP>),
+  return raise_lds_limit(reinterpret_cast<const void*>(attn_fwd_kernel<D, QBLK, MODE, HAS_V, STATS, NGRP, HALVES>),
                          attn_lds_bytes<D, QBLK, MODE, HAS_V, STATS, NGRP>(), attr_set);
 }
 
 // Host launcher; returns hipError_t of the launch.
-template <int D, int QBLK, int MODE, bool HAS_V, bool STATS, int NGRP = 1>
+template <int D, int QBLK, int MODE, bool HAS_V, bool STATS, int NGRP = 1, bool HALVES = false>
 inline hipError_t launch_attn_fwd(const AttnParams& p, hipStream_t stream) {
-  auto kern = attn_fwd_kernel<D, QBLK, MODE, HAS_V, STATS, NGRP>;
-  const hipError_t ea = prepare_attn_fwd<D, QBLK, MODE, HAS_V, STATS, NGRP>();
+  auto kern = attn_fwd_kernel<D, QBLK, MODE, HAS_V, STATS, NGRP, HALVES>;
+  const hipError_t ea = prepare_attn_fwd<D, QBLK, MODE, HAS_V, STATS, NGRP, HALVES>();
   if (ea != hipSuccess) return ea;
-  const int total = p.nqblk * p.H * p.B;
+  const int total = p.nqblk * p.H * p.B * (HALVES ? 2 : 1);
   if (total <= 0) return hipSuccess;
   constexpr int kLds = attn_lds_bytes<D, QBLK, MODE, HAS_V, STATS, NGRP>();
   hipLaunchKernelGGL(kern, dim3(total), dim3(64 * attn_waves<QBLK>() * NGRP), kLds, stream, p);

@@ -83,7 +83,8 @@ int spattn_full_attn(void* o, float* lse, const void* q, const void* k, const vo
                      int D, int kv_len, float scale, void* stream);
 
 /* qblk in {64,128}: rows per q-block = rows sharing one list; kv_indices is
- * [B,H,ceil(S/qblk),mask_stride]. */
+ * [B,H,ceil(S/qblk),mask_stride].  Lists of 128 rows in launches that leave the chip idle run by workgroups of 64
+ * rows, here and in the other list entry points, so low bits of o and lse depend on batch * heads * seq. */
 int spattn_sp_attn(void* o, float* lse, const void* q, const void* k, const void* v, const int* kv_indices,
                    const int* num_kv_indices, int mask_stride, int qblk, int batch, int heads, int seq, int D,
                    int kv_len, float scale, void* stream);
