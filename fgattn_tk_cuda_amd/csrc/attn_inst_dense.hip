@@ -15,17 +15,21 @@ namespace spattn {
 //   statistics 0.93-0.98, statistics only 0.89-0.98; at 256 and 512 keys that is 0.93-1.09, behind 768 q-blocks 1.08-1.14.
 //   d = 128 is slower (1.02-1.2, with statistics 1.2-1.5: its LDS allows one workgroup per CU) from the second q-block per
 //   CU on, except the statistics alone, whose ring is 48 KB, from 768 keys on: 0.90-0.96 up to three per CU, 1.12-1.2 behind.
-//   Two groups on 64-row q-blocks, up to one per CU, against one group on them: d = 64 from 12 tiles on 0.72-0.95 (8 tiles
-//   1.00-1.02), d = 128 from 15 on 0.75-1.00 (12 tiles 0.99, 8 tiles 1.07-1.13).  Dense with statistics at d = 128 has no LDS
-//   for it.
+//   The statistics alone at d = 64 fit five to a CU; that pays again where the 128-row form has a third one on some CUs, from 513
+//   to 640 of its q-blocks: 0.94-0.98 (8 x 8508 146 -> 138 us, 32 x 2050 40.4 -> 38.1), with fewer 1.05-1.09, behind 1.09-1.12.
+//   Two groups on 64-row q-blocks, up to one per CU, against one group on them: d = 64 from 12 tiles on 0.72-0.95, 10 and 11
+//   0.92-0.99 (8 x 588 with statistics 9.0 -> 8.3 us), 8 and 9 0.99-1.04; d = 128 from 15 on 0.75-1.00 (12 tiles 0.99, 8 tiles
+//   1.07-1.13).  Dense with statistics at d = 128 has no LDS for it.
 //   Two groups on 128-row q-blocks, up to one per CU, against the best of the other forms: d = 128 from 12 tiles on 0.84-0.95
 //   (8 tiles 0.98-1.06); d = 64 from 24 tiles on 0.90-0.98, with statistics from 15 on 0.92-0.96 (below 0.97-1.02).
 // 256-row q-blocks by one group of eight waves (d = 128 with V): half of the K / V copies per row, at the power cap
 // worth 2-5 % of a full round of one q-block per CU (12 x 32768 5.49 -> 5.28 ms; 2048 keys 2 %, 1024 keys -1, 512 keys -5),
 // and a workgroup of its own finishes a CU's last q-block sooner than two do.  A last round that fills up to half of the CUs
 // costs it 0-19 % instead (its other form spreads that round over twice as many).  From 32 tiles on with the last round
-// empty or more than half full 0.91-0.98.  With statistics, whose row maxima keep the waves of a workgroup waiting for
-// each other, that holds up to two rounds (0.94-0.99; 12 x 9000 502 -> 471 us) and from 64 tiles on up to five (68 tiles
+// empty or more than half full 0.91-0.98; where that is the only round from 22 tiles on 0.90-0.99 (24 x 1715 46.9 -> 42.1 us, 32 x
+// 1495 44.6 -> 41.6, with statistics 24 x 1626 46.2 -> 44.0), two rounds of 22-31 tiles 0.97-1.02.  With
+// statistics, whose row maxima keep the waves of a workgroup waiting for each other, that holds up to two rounds (0.94-0.99; 12
+// x 9000 502 -> 471 us) and from 64 tiles on up to five (68 tiles
 // 0.99, 90 and more 0.95-0.98: 12 x 14000 1163 -> 1105, 12 x 20000 2243 -> 2165, 16 x 20400 2968 -> 2905; 36 tiles in three
 // rounds 0.98, left to the 128-row form), behind them 0.98-1.03.  Same bits as the 128-row form.
 // The other forms add the row sums and outputs of a row in another order: a launch over some heads of a computation
@@ -37,14 +41,15 @@ DenseForm dense_form(int D, bool has_v, bool stats, int S, int kv_len, long long
   const long long heads = of_heads > 0 ? of_heads : launched;
   const long long n64 = heads * ((S + 63) / 64), n128 = heads * ((S + 127) / 128);
   const int tiles = (kv_len + 63) / 64;
-  if (n64 <= kCus) return {64, !(D == 128 && has_v && stats) && tiles >= (D == 64 ? 12 : 15) ? 2 : 1};
+  if (n64 <= kCus) return {64, !(D == 128 && has_v && stats) && tiles >= (D == 64 ? 10 : 15) ? 2 : 1};
   if (n128 <= kCus && tiles >= (D == 128 ? 12 : stats ? 15 : 24)) return {128, 2};
   if ((D == 64 || !has_v) && kv_len >= 768 && n64 <= 3 * kCus) return {64, 1};
+  if (D == 64 && !has_v && kv_len >= 768 && n128 > 2 * kCus && n64 <= 5 * kCus) return {64, 1};
   if (D == 128 && has_v) {
     const long long n256 = launched * ((S + 255) / 256);
     const long long last = n256 % kCus;
     const bool few = n256 <= 2 * kCus || (tiles >= 64 && n256 <= 5 * kCus);
-    if (tiles >= 32 && (last == 0 || last > kCus / 2) && (!stats || few)) return {256, 1};
+    if (tiles >= (n256 <= kCus ? 22 : 32) && (last == 0 || last > kCus / 2) && (!stats || few)) return {256, 1};
   }
   return {128, 1};
 }

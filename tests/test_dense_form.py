@@ -35,3 +35,19 @@ def test_what_the_calls_refuse_has_no_form():
     assert form(96, 1, 0, 1, 128) == -2
     for bad in ((64, 0, 0, 1, 128), (64, 1, 0, 0, 128), (64, 1, 0, 1, 0), (64, 1, 0, 1, 1 << 24), (64, 1, 0, 2, 128, 0, 1)):
         assert form(*bad) == -6
+
+
+def test_256_row_qblocks_in_one_round():
+    """From 22 key tiles on where they fit one round that is more than half full, 32 otherwise."""
+    assert form(128, 1, 0, 24, 1345) == form(128, 1, 1, 42, 1345) == 2561              # 144 and 252 q-blocks
+    assert form(128, 1, 0, 43, 1345) == form(128, 1, 1, 24, 1345, 1344) == 1281        # 258; 21 tiles
+    assert form(128, 1, 0, 80, 1506) == 1281                                            # 480 of 24 tiles
+
+
+def test_statistics_alone_five_to_a_cu():
+    assert [form(64, 0, 1, h, 1100) for h in (56, 57, 71, 72)] == [1281, 641, 641, 1281]   # 504 and 513 of 128, 1278 and 1296 of 64 rows
+    assert form(64, 1, 1, 57, 1100) == form(64, 0, 1, 90, 767) == 1281
+
+
+def test_two_groups_from_ten_tiles_at_d64():
+    assert [form(64, v, s, 8, S) for v, s in ((1, 0), (1, 1), (0, 1)) for S in (576, 577)] == [641, 642] * 3
