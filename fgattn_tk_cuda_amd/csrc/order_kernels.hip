@@ -15,7 +15,7 @@
 
 namespace spattn {
 
-constexpr int kOrderThreads = 128;
+constexpr int kOrderWaves = 16;
 constexpr int kOrderSub = 2;                              // bits below the leading one that tell classes apart
 constexpr int kOrderClasses = (22 << kOrderSub) + 2;      // 4 per octave up to 2^22 keys, one for longer lists, one for empty ones
 
@@ -29,90 +29,114 @@ __device__ __forceinline__ int length_class(int c) {
   return kOrderClasses - 2 - (fine < kOrderClasses - 2 ? fine : kOrderClasses - 2);
 }
 
-__global__ __launch_bounds__(kOrderThreads) void qblock_order_kernel(int* __restrict__ order,
-                                                                      const int* __restrict__ counts, int n) {
-  constexpr int T = kOrderThreads;
-  __shared__ int cls_cnt[kOrderClasses * T];   // [class][thread]: members in that thread's segment, then offsets
-  __shared__ int part[T];
-  __shared__ int lo_hi[2];
+// One workgroup; wave w owns a contiguous segment of the counts and goes through it 64 at a time, four of those in flight.
+// Lanes of one class find each other by seven ballots, so a class has one LDS add per wave and step, and the place of a count
+// is what the classes ahead and the waves before hold plus its lanes before.  What bounds it is the chain of launch, load, three
+// barriers and store in short calls, of the steps of a wave in long ones (one thread per segment, tables by thread and a
+// serial scan over them: 9.6 us for 36 counts, now 3.5; 511 9.8, now 3.7; 8192 25, now 12.3; 100003 219, now 120).
+__global__ __launch_bounds__(64 * kOrderWaves) void qblock_order_kernel(int* __restrict__ order,
+                                                                         const int* __restrict__ counts, int n) {
+  constexpr int W = kOrderWaves;
+  constexpr int U = 4;
+  static_assert(kOrderClasses <= 128, "two waves scan the classes, seven bits tell them apart");
+  __shared__ int table[kOrderClasses * W];   // [class][wave]: members in that wave's segment, then offsets
+  __shared__ int lo_l[W], hi_l[W], first_half;
   const int tid = threadIdx.x;
-  // A thread owns a contiguous segment (the order inside a class is the index order), a multiple of
-  // four counts long so that it is read with 16-byte loads, sixteen counts in flight at a time: one
-  // count per load, each waiting for the one before, made this kernel 23 us of pure load latency.
-  const int seg = (((n + T - 1) / T) + 3) & ~3;
-  const int i0 = tid * seg < n ? tid * seg : n;
-  const int i1 = (i0 + seg) < n ? (i0 + seg) : n;
-  const bool vec_ok = ((uintptr_t)counts & 15) == 0;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int steps = (n + 64 * W - 1) / (64 * W);
+  const int i0 = wave * steps * 64 + lane;
+
+  // f(index, count, its slot, members of its class in lanes before, and in all lanes; 0 where there is no count)
   auto walk = [&](auto&& f) {
-    for (int b = i0; b < i1; b += 16) {
-      i32x4 v[4];
+    for (int s = 0; s < steps; s += U) {
+      int c[U];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int i = b + 4 * u;
-        if (vec_ok && i + 4 <= i1) {
-          v[u] = *reinterpret_cast<const i32x4*>(counts + i);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[u][e] = (i + e < i1) ? counts[i + e] : 0;
-        }
+      for (int u = 0; u < U; ++u) {
+        const int i = i0 + 64 * (s + u);
+        c[u] = s + u < steps && i < n ? counts[i] : 0;
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
+      for (int u = 0; u < U; ++u) {
+        if (s + u >= steps) break;
+        const int i = i0 + 64 * (s + u);
+        const int cls = length_class(c[u]);
+        unsigned long long same = __ballot(i < n);
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (b + 4 * u + e < i1) f(b + 4 * u + e, v[u][e]);
+        for (int b = 0; b < 7; ++b) {
+          const unsigned long long m = __ballot((cls >> b) & 1);
+          same &= (cls >> b) & 1 ? m : ~m;
+        }
+        if (i < n) {
+          const int before = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(same >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)same, 0));
+          f(i, c[u], cls * W + wave, before, (int)__popcll(same));
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      }
     }
   };
 
-  for (int c = 0; c < kOrderClasses; ++c) cls_cnt[c * T + tid] = 0;
-  if (tid == 0) {
-    lo_hi[0] = 0x7fffffff;
-    lo_hi[1] = 0;
-  }
+  for (int e = tid; e < kOrderClasses * W; e += 64 * W) table[e] = 0;
   __syncthreads();
   int lo = 0x7fffffff, hi = 0;
-  walk([&](int, int c) {
+  walk([&](int, int c, int slot, int before, int all) {
     lo = c < lo ? c : lo;
     hi = c > hi ? c : hi;
-    cls_cnt[length_class(c) * T + tid] += 1;
+    if (before == 0) table[slot] += all;
   });
-  atomicMin(&lo_hi[0], lo);
-  atomicMax(&lo_hi[1], hi);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const int l = __shfl_xor(lo, off, 64), h = __shfl_xor(hi, off, 64);
+    lo = l < lo ? l : lo;
+    hi = h > hi ? h : hi;
+  }
+  if (lane == 0) {
+    lo_l[wave] = lo;
+    hi_l[wave] = hi;
+  }
   __syncthreads();
-  lo = lo_hi[0];
-  hi = lo_hi[1];
+#pragma unroll
+  for (int w = 0; w < W; ++w) {
+    lo = lo_l[w] < lo ? lo_l[w] : lo;
+    hi = hi_l[w] > hi ? hi_l[w] : hi;
+  }
   // the longest list less than twice the shortest: little to balance (measured: sorting such
   // lists costs 2 % through the lost locality), keep neighbours together
   if (hi <= 0 || hi < 2 * lo) {
-    for (int i = i0; i < i1; ++i) order[i] = xcd_remap(i, n);
+    for (int s = 0; s < steps; ++s)
+      if (i0 + 64 * s < n) order[i0 + 64 * s] = xcd_remap(i0 + 64 * s, n);
     return;
   }
-  // exclusive prefix sum over cls_cnt in storage order (class-major, thread-minor)
-  constexpr int PER = kOrderClasses;   // entries per scanning thread
-  int sum = 0;
-  for (int j = 0; j < PER; ++j) sum += cls_cnt[tid * PER + j];
-  part[tid] = sum;
+  // exclusive prefix sum over the table in storage order; a thread of the first two waves has a class
+  int own = 0, upto = 0;
+  if (tid < 128) {
+    if (tid < kOrderClasses)
+#pragma unroll
+      for (int w = 0; w < W; ++w) own += table[tid * W + w];
+    upto = own;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int t = __shfl_up(upto, off, 64);
+      if (lane >= off) upto += t;
+    }
+    if (tid == 63) first_half = upto;
+  }
   __syncthreads();
-  if (tid == 0) {
-    int run = 0;
-    for (int j = 0; j < T; ++j) {
-      const int x = part[j];
-      part[j] = run;
+  if (tid < kOrderClasses) {
+    int run = upto - own + (wave == 1 ? first_half : 0);
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const int x = table[tid * W + w];
+      table[tid * W + w] = run;
       run += x;
     }
   }
   __syncthreads();
-  int run = part[tid];
-  for (int j = 0; j < PER; ++j) {
-    const int x = cls_cnt[tid * PER + j];
-    cls_cnt[tid * PER + j] = run;
-    run += x;
-  }
-  __syncthreads();
-  walk([&](int i, int c) {
-    const int slot = length_class(c) * T + tid;
-    order[cls_cnt[slot]] = i;
-    cls_cnt[slot] += 1;
+  walk([&](int i, int, int slot, int before, int all) {
+    const int at = table[slot];
+    order[at + before] = i;
+    if (before == all - 1) table[slot] = at + all;
   });
 }
 
@@ -139,7 +163,7 @@ __global__ __launch_bounds__(kOrderThreads) void qblock_order_kernel(int* __rest
 // octave (a sixteenth: no gain) over the seven octaves below the longest list, stable, so the order is a function of
 // the counts alone.  What bounds it is the chain of loads and LDS updates of a lane's segment: 6.6 us for 6144
 // q-blocks by windows, 16 for 23640, and 15.5 / 42 us for the sort over everything (one wave of one count at a time:
-// 47 / 171; qblock_order_kernel: 20 / 58).
+// 47 / 171; qblock_order_kernel: 9 / 32).
 // ------------------------------------------------------------------------------------
 constexpr int kXcds = 8;
 constexpr int kSlotsPerXcd = 64;
@@ -317,7 +341,7 @@ hipError_t run_qblock_schedule(int* order, const int* counts, int n, int per_hea
 
 hipError_t run_qblock_order(int* order, const int* counts, int n, hipStream_t stream) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(qblock_order_kernel, dim3(1), dim3(kOrderThreads), 0, stream, order, counts, n);
+  hipLaunchKernelGGL(qblock_order_kernel, dim3(1), dim3(64 * kOrderWaves), 0, stream, order, counts, n);
   return hipGetLastError();
 }
 
