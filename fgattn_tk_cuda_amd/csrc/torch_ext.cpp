@@ -741,7 +741,9 @@ void qk_topkmask_indices(torch::Tensor kv_indices, torch::Tensor kv_numindices, 
 // and block maxima are the operator's own, from the caching allocator.
 namespace {
 struct OnePass {
-  torch::Tensor max_q, denom, blockmax;
+  torch::Tensor held;   // max_q, denom and blockmax in one allocation: three cost the host 1.5 us more
+  float *max_q, *denom;
+  void* blockmax;
   int B, H, S, D;
 };
 OnePass onepass_sweep(const OptTensor& o, const torch::Tensor& q, const torch::Tensor& k, const OptTensor& v) {
@@ -754,13 +756,15 @@ OnePass onepass_sweep(const OptTensor& o, const torch::Tensor& q, const torch::T
     check_bhsd(*o, "o", q);
   }
   const int64_t B = q.size(0), H = q.size(1), S = q.size(2), sp = padded128(S);
-  OnePass p{torch::empty({B, H, 1, sp}, q.options().dtype(at::kFloat)), torch::empty({B, H, 1, sp}, q.options().dtype(at::kFloat)),
-            torch::empty({B, H, sp / 64, sp}, q.options()), (int)B, (int)H, (int)S, (int)q.size(3)};
-  float* const m = p.max_q.data_ptr<float>();
-  float* const d = p.denom.data_ptr<float>();
-  check_status(dense ? spattn_fullattn_maxq_denom_blockmax(o->data_ptr(), m, d, p.blockmax.data_ptr(), q.data_ptr(), k.data_ptr(),
+  const int64_t rows = B * H * sp;   // a multiple of 128: every part is aligned as the allocation is
+  OnePass p{torch::empty({2 * rows * 4 + rows * (sp / 64) * 2}, q.options().dtype(at::kByte)), nullptr, nullptr, nullptr,
+            (int)B, (int)H, (int)S, (int)q.size(3)};
+  p.max_q = static_cast<float*>(p.held.data_ptr());
+  p.denom = p.max_q + rows;
+  p.blockmax = p.denom + rows;
+  check_status(dense ? spattn_fullattn_maxq_denom_blockmax(o->data_ptr(), p.max_q, p.denom, p.blockmax, q.data_ptr(), k.data_ptr(),
                                                            v->data_ptr(), p.B, p.H, p.S, p.D, 0, 0.f, cur_stream())
-                     : spattn_maxq_denom_blockmax(m, d, p.blockmax.data_ptr(), q.data_ptr(), k.data_ptr(), p.B, p.H, p.S, p.D, 0,
+                     : spattn_maxq_denom_blockmax(p.max_q, p.denom, p.blockmax, q.data_ptr(), k.data_ptr(), p.B, p.H, p.S, p.D, 0,
                                                   0.f, cur_stream()),
                "statistics with block maxima");
   return p;
@@ -777,9 +781,8 @@ void onepass_packedmask(torch::Tensor packed, OptTensor o, torch::Tensor q, torc
               "packed must be [B,H,ceil(S/128),Sp/8]");
   const DeviceGuard guard(q.device());
   const OnePass p = onepass_sweep(o, q, k, v);
-  check_status(spattn_blockmax_to_packedmask(packed.data_ptr(), p.blockmax.data_ptr(), p.max_q.data_ptr<float>(),
-                                             p.denom.data_ptr<float>(), q.data_ptr(), k.data_ptr(), (float)threshold, (int)sp,
-                                             p.B, p.H, p.S, p.D, 0, 0.f, cur_stream()),
+  check_status(spattn_blockmax_to_packedmask(packed.data_ptr(), p.blockmax, p.max_q, p.denom, q.data_ptr(), k.data_ptr(),
+                                             (float)threshold, (int)sp, p.B, p.H, p.S, p.D, 0, 0.f, cur_stream()),
                "onepass_packedmask");
 }
 
@@ -797,9 +800,9 @@ void onepass_blocklists(torch::Tensor blk_idx, torch::Tensor blk_cnt, OptTensor 
   TORCH_CHECK(blk_cnt.numel() == q.size(0) * q.size(1) * SB, "blk_cnt must have B*H*ceil(S/qblk) entries");
   const DeviceGuard guard(q.device());
   const OnePass p = onepass_sweep(o, q, k, v);
-  check_status(spattn_blockmax_to_blocklists_filled(blk_idx.data_ptr<int>(), blk_cnt.data_ptr<int>(), nullptr, p.blockmax.data_ptr(),
-                                                    p.max_q.data_ptr<float>(), p.denom.data_ptr<float>(), (float)threshold,
-                                                    (int)qblk, p.B, p.H, p.S, p.D, 0, 0.f, (int)blk_idx.size(3), cur_stream()),
+  check_status(spattn_blockmax_to_blocklists_filled(blk_idx.data_ptr<int>(), blk_cnt.data_ptr<int>(), nullptr, p.blockmax,
+                                                    p.max_q, p.denom, (float)threshold, (int)qblk, p.B, p.H, p.S, p.D, 0, 0.f,
+                                                    (int)blk_idx.size(3), cur_stream()),
                "onepass_blocklists");
   counts_written(blk_cnt);
 }

@@ -16,7 +16,8 @@ spattn_interface = torch.ops.cuda_attn
 
 
 def _out_like(query):
-    return torch.empty(query.shape, device=query.device, dtype=torch.bfloat16)
+    # 1.3 us; torch.empty from shape and device 2.3, and a small step waits for the host
+    return torch.empty_like(query, dtype=torch.bfloat16, memory_format=torch.contiguous_format)
 
 
 def _c(*tensors):
@@ -185,9 +186,9 @@ def blockcached_attn_cuda(query, key, value, current_layer, ditrun, *args, **kwa
             # thresholding those, without a second sweep over Q K^T
             out = _out_like(query)
             B, H, S, _ = query.shape
-            shape = (B, H, (S + qblk - 1) // qblk, mask_utils._padded(S) // mask_utils.KVBLK)
-            blk_idx = torch.empty(shape, dtype=torch.int32, device=query.device)
-            blk_cnt = torch.empty(shape[:3], dtype=torch.int32, device=query.device)
+            nq = (S + qblk - 1) // qblk
+            blk_idx = mask_utils._new(query, torch.int32, B, H, nq, mask_utils._padded(S) // mask_utils.KVBLK)
+            blk_cnt = mask_utils._new(query, torch.int32, B, H, nq)
             query, key, value = _c(query, key, value)
             spattn_interface.onepass_blocklists(blk_idx, blk_cnt, out, query, key, value, kwargs["thresh"], qblk)
         elif groups is not None:
