@@ -174,9 +174,10 @@ void attn_fwd_kernel(const AttnParams p) {
   } else {
     const size_t lrow = (size_t)bh * p.nqblk + lb;
     lst = (cint_p)(p.idx + lrow * p.idx_stride);
-    n = ((cint_p)p.cnt)[lrow];
-    n = n < 0 ? 0 : (n > p.idx_stride ? p.idx_stride : n);
-    ntiles = (MODE == KV_TOKENS) ? ((n + 63) >> 6) : n;
+    if constexpr (MODE == KV_BLOCKS) {
+      n = ((cint_p)p.cnt)[lrow];
+      ntiles = n = n < 0 ? 0 : (n > p.idx_stride ? p.idx_stride : n);
+    }
   }
   // Two groups: of an odd number of tiles the second group's last one is behind the sequence, a tile without keys.
   const int all_tiles = ntiles;
@@ -345,6 +346,13 @@ void attn_fwd_kernel(const AttnParams p) {
     }
   }
   if constexpr (MODE == KV_TOKENS) {
+    // The count is asked for behind the first ids, which do not depend on it: the compiler, left to itself, waits for it ahead
+    // of them, and a q-block starts with two cold reads in a row.
+    uint64_t at = (uint64_t)(uintptr_t)(p.cnt + ((size_t)bh * p.nqblk + lb));
+    asm volatile("" : "+s"(at));
+    n = *(cint_p)at;
+    n = n < 0 ? 0 : (n > p.idx_stride ? p.idx_stride : n);
+    ntiles = (n + 63) >> 6;
     wait_vmcnt<Q_LDS ? NQ : 0>();
 #pragma unroll
     for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(idr[j]));
