@@ -129,6 +129,10 @@ void attn_fwd_kernel(const AttnParams p) {
   const int qsub = wave % NQW;
   const int ksub = wave / NQW;
 
+  // All arguments that the first loads need in one scalar read: the compiler asks for some behind the branches below and waits
+  // a second time (12 x 512 x 128 dense 9.40 -> 9.20 us, 8 x 900 x 128 token lists 7.47 -> 7.31).
+  if constexpr (MODE == KV_DENSE) asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.kv_len));
+  else asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.idx), "s"(p.cnt), "s"(p.idx_stride));
   const int total = p.nqblk * p.H * p.B;
   int half = 0;
   unsigned at = blockIdx.x;
