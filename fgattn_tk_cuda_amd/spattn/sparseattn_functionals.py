@@ -43,7 +43,7 @@ def baseline_attn_maxq_denom(query, key, value, current_layer=None, ditrun=None,
     return _dense_with_stats(query, key, value)[0]
 
 
-# From this many q-blocks on, lists that are used once are worth a work order of their own.  Its kernel takes 5-10 us;
+# From this many q-blocks on, lists that are used once are worth a work order of their own.  Its kernel takes 6-12 us;
 # threshold lists d = 128, heads of equal density / density from 0.4 to 1.4 of the logits' deviation, attention without
 # an order against order and attention: 752 q-blocks 38 / 45 against 44 / 43 us, 1880 q-blocks 87 / 98 against 98 / 93,
 # 3072 q-blocks 338 / 344 against 334 / 287, 10240 q-blocks 2053 / 1959 against 1990 / 1674.
