@@ -147,8 +147,9 @@ typedef SPATTN_LDS const unsigned char* lds_cptr;
 // so the waits are placed by hand.  m0 cannot be named as clobbered (the compiler reserves it and
 // warns that such a clobber is not honoured); tests/test_asm_inflight_loads.py checks on the
 // listing that no compiler-generated instruction reads m0 across these statements.
+// The copy may read m0 one wait state behind the write (the compiler inserts it behind writes of its own only): s_nop 0.
 __device__ __forceinline__ void dma16(const void* gptr, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(gptr) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(gptr) : "memory");
 }
 // Same with a wave-uniform base pointer and a 32-bit per-lane byte offset.
 // The base goes through readfirstlane: under scalar-register pressure the compiler may keep
@@ -166,7 +167,7 @@ __device__ __forceinline__ void dma16(const void* sbase, uint32_t voff, uint32_t
   if constexpr (LATE) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voff), "s"(sb) : "memory");
   } else {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voff), "s"(sb) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voff), "s"(sb) : "memory");
   }
 }
 // 16-byte global load that the compiler does not count either: the destination is valid only

@@ -22,6 +22,8 @@ The asm statements take base addresses in scalar registers.  A vector-memory ins
 vector ALU wrote (readfirstlane, readlane) five wait states later; the compiler keeps that distance for its own instructions
 and does not look into asm, so the listing is checked for it.
 
+A copy into LDS may read m0 one wait state behind a scalar write of it; the compiler puts it there behind its own writes only.
+
 The votes kernel lists rows in LDS as 16-bit numbers and reads several entries at a time.  A read through another scalar
 type would be free to move ahead of the stores (type-based aliasing); the last check looks at the types of its LDS
 loads and stores before any optimisation."""
@@ -126,6 +128,54 @@ def scalar_bases_too_close(listing, states=5):
     return found
 
 
+class Flow:
+    """The instructions of one kernel, [(operation, operands, inside an asm statement)], and what may follow each."""
+
+    def __init__(self, body):
+        self.ins, labels, inside = [], {}, False
+        for raw in body.split("\n"):
+            inside = "#ASMSTART" in raw or (inside and "#ASMEND" not in raw)
+            t = raw.split(";")[0].strip()
+            label = re.match(r"(\.?\w+):", t)
+            if label:
+                labels[label.group(1)] = len(self.ins)
+            elif t and not t.startswith("."):
+                op, _, args = t.partition(" ")
+                self.ins.append((op, args.strip(), inside))
+        self.after = []
+        for i, (op, args, _) in enumerate(self.ins):
+            follow = [] if op in ("s_branch", "s_endpgm", "s_setpc_b64") or i + 1 == len(self.ins) else [i + 1]
+            self.after.append(follow + ([labels[args]] if op == "s_branch" or op.startswith("s_cbranch") else []))
+
+    def within(self, i, states):
+        """{instruction: fewest wait states between it and instruction i} of those that less than `states` lie ahead of."""
+        near, todo = {}, [(j, 0) for j in self.after[i]]
+        while todo:
+            j, passed = todo.pop()
+            if passed >= states or near.get(j, states) <= passed:
+                continue
+            near[j] = passed
+            op, args, _ = self.ins[j]
+            todo += [(n, passed + 1 + (int(args, 0) if op == "s_nop" else 0)) for n in self.after[j]]
+        return near
+
+
+def kernel_flows(listing):
+    for m in re.finditer(r"^(_Z\w+):(.*?)^\.Lfunc_end", listing, re.S | re.M):
+        yield m.group(1), Flow(m.group(2))
+
+
+def m0_too_close(listing):
+    """[(kernel, scalar write of m0, copy)] where a copy into LDS follows a scalar write of m0, which it reads, without a wait
+    state between them, along any path."""
+    found = []
+    for kernel, flow in kernel_flows(listing):
+        for i, (op, args, _) in enumerate(flow.ins):
+            if op.startswith("s_") and args.split(",")[0] == "m0":
+                found += [(kernel, op + " " + args, " ".join(flow.ins[j][:2])) for j in flow.within(i, 1) if "_lds_" in flow.ins[j][0]]
+    return found
+
+
 def tile_loop_findings(listing):
     """{kernel: (scratch accesses, compiler vmcnt waits)} inside the tile loop of every attn_fwd_kernel
     instantiation of a listing; a kernel whose loop is not found maps to None."""
@@ -209,8 +259,17 @@ def test_scalar_base_checker():
     assert scalar_bases_too_close((late % "").replace("s[20:21]", "s[22:23]")) == []
 
 
+def test_m0_distance_checker():
+    def found(*lines):
+        return len(m0_too_close("_ZN6spattn1kE:\n.LBB0_1:\n\t" + "\n\t".join(lines) + "\n\ts_endpgm\n.Lfunc_end0:\n"))
+
+    copy, write = "global_load_lds_dwordx4 v1, s[0:1]", "s_mov_b32 m0, s3"
+    assert found(write, copy) == 1 and found(write, "s_nop 0", copy) == 0 and found(write, "v_mov_b32_e32 v2, v3", copy) == 0
+    assert found(copy, write, "s_cbranch_scc1 .LBB0_1") == 0 and found("global_load_dwordx4 v[0:3], v[4:5], off", write) == 0
+
+
 def test_m0_checker_sees_a_compiler_use():
-    ok = "\t;;#ASMSTART\n\ts_mov_b32 m0, s3\n\tglobal_load_lds_dwordx4 v1, s[0:1]\n\t;;#ASMEND\n\tv_mov_b32_e32 v2, v3\n"
+    ok = "\t;;#ASMSTART\n\ts_mov_b32 m0, s3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 v1, s[0:1]\n\t;;#ASMEND\n\tv_mov_b32_e32 v2, v3\n"
     bad = ok + "\ts_mov_b32 m0, -1\n"
     assert m0_uses_outside_asm(ok) == []
     assert len(m0_uses_outside_asm(bad)) == 1
@@ -239,6 +298,8 @@ def test_no_instruction_touches_a_register_with_a_load_in_flight(tmp_path):
         assert "global_load_lds_dwordx4" in text, unit
         uses = m0_uses_outside_asm(text)
         assert not uses, "%s: the compiler uses m0 next to hand-written copies: %s" % (unit, uses[:3])
+        early = m0_too_close(text)
+        assert not early, "%s: %d copies too close behind their m0, e.g. %s" % (unit, len(early), early[0])
         close = scalar_bases_too_close(text)
         assert not close, "%s: %d bases written too late, e.g. %s" % (unit, len(close), close[0])
         if unit == VOTES_UNIT:
