@@ -909,6 +909,7 @@ void attn_fwd_kernel(const AttnParams p) {
     // counts stay the same on every tile, and the registers are held until the final wait.
     if constexpr (MODE == KV_TOKENS) ids_load(it + NK + 1, idr[(KC + NK + 1) % 6]);
     softmax_close(s_a, PAR);
+    if constexpr (!HAS_V) settle(s_b[NMB - 1]);   // with V multiplies of P V lie between the scores and their maxima
     mask_tile(m_lo, m_hi, s_b);
     if constexpr (MODE != KV_TOKENS) idw[(KC + NK + 1) % 6] = tile_desc(it + NK + 1);
     using stat_t = std::integral_constant<bool, STATS>;
@@ -941,6 +942,7 @@ void attn_fwd_kernel(const AttnParams p) {
     __syncthreads();
     v_addr_refresh();
     qk_tile(std::false_type{}, std::false_type{}, 0, 0, s_e, s_e, 0, nullptr, false);
+    settle(s_e[NMB - 1]);
     if constexpr (MODE == KV_TOKENS) mask_tile(idw[0], idh[0], s_e);
     else mask_tile(hd[0], 0, s_e);
     move_reference(row_stats(s_e, 0));   // nothing is accumulated yet

@@ -74,6 +74,8 @@ __device__ __forceinline__ uint16_t bf16_round_up(float x) {
 // passes every operand it cannot prove free of signalling NaNs (the accumulators of a matrix
 // multiply among them) through a v_max_f32 x, x of its own, three instructions per two scores
 // instead of one per two.  A NaN operand is skipped like in fmaxf.
+// The vector ALU may read what a matrix multiply wrote twelve wait states later; the compiler keeps that distance for its own
+// instructions and does not look into asm: see settle().
 __device__ __forceinline__ float max3_raw(float a, float b, float c) {
   float d;
   asm("v_max3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
@@ -84,6 +86,14 @@ __device__ __forceinline__ float max_raw(float a, float b) {
   float d;
   asm("v_max_f32 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
   return d;
+}
+
+// Reads one register of the last accumulator of a product by a move of the compiler's own: behind it, asm may read all that the
+// product wrote.  In straight line behind the multiply: where two paths from it meet, the compiler has been seen to count the
+// longer one.  (tests/test_asm_inflight_loads.py checks the distances on the listing.)
+__device__ __forceinline__ void settle(const f32x16& acc) {
+  const int b = __builtin_bit_cast(int, acc[15]);
+  asm volatile("" ::"v"(__builtin_amdgcn_update_dpp(b, b, 0xe4, 0xf, 0xf, true)));   // quad_perm 0 1 2 3
 }
 
 // Max / sum of the values held by lanes l and l ^ 32, in both lanes.  v_permlane32_swap

@@ -24,6 +24,10 @@ and does not look into asm, so the listing is checked for it.
 
 A copy into LDS may read m0 one wait state behind a scalar write of it; the compiler puts it there behind its own writes only.
 
+The row maxima read accumulators of matrix multiplies in asm.  The vector ALU may read or write what a multiply writes only some
+wait states later (twelve behind a 32x32x16, eight behind a 16x16x32); the compiler keeps that distance for its own instructions
+and does not look into asm, so the listing is checked for it, along every path.
+
 The votes kernel lists rows in LDS as 16-bit numbers and reads several entries at a time.  A read through another scalar
 type would be free to move ahead of the stores (type-based aliasing); the last check looks at the types of its LDS
 loads and stores before any optimisation."""
@@ -41,6 +45,7 @@ CSRC = Path(build.__file__).resolve().parent / "csrc"
 UNITS = ["attn_inst_blocks.hip", "attn_inst_tokens.hip", "attn_inst_dense.hip"]
 VOTES_UNIT = "votes_kernels.hip"
 M0_UNITS = UNITS + ["mask_kernels.hip", VOTES_UNIT]
+TOPK_UNIT = "topk_kernels.hip"   # asm and matrix multiplies, no copies into LDS
 
 
 def _regs(text):
@@ -165,6 +170,22 @@ def kernel_flows(listing):
         yield m.group(1), Flow(m.group(2))
 
 
+def multiplies_too_close(listing):
+    """[(kernel, multiply, asm instruction, wait states between them)] where a vector-ALU or memory instruction of an asm
+    statement names a register that a matrix multiply writes before it may."""
+    found = []
+    for kernel, flow in kernel_flows(listing):
+        for i, (op, args, _) in enumerate(flow.ins):
+            if not op.startswith("v_mfma"):
+                continue
+            dst = _regs(args.split(",")[0])
+            for j, passed in flow.within(i, 12 if "32x32x16" in op else 8 if "16x16x32" in op else 20).items():
+                op2, args2, asm = flow.ins[j]
+                if asm and (op2.startswith("v_") or _is_vmem(op2)) and _regs(args2) & dst:
+                    found.append((kernel, op + " " + args, op2 + " " + args2, passed))
+    return found
+
+
 def m0_too_close(listing):
     """[(kernel, scalar write of m0, copy)] where a copy into LDS follows a scalar write of m0, which it reads, without a wait
     state between them, along any path."""
@@ -259,6 +280,25 @@ def test_scalar_base_checker():
     assert scalar_bases_too_close((late % "").replace("s[20:21]", "s[22:23]")) == []
 
 
+def test_multiply_checker():
+    asm = "\t;;#ASMSTART\n\tv_max3_f32 v1, v%d, v1, v2\n\t;;#ASMEND\n"
+    multiply = "\tv_mfma_f32_32x32x16_bf16 v[64:79], v[4:7], v[8:11], 0\n"
+
+    def states(*lines):
+        body = "_ZN6spattn15attn_fwd_kernelILi64EEEvNS_10AttnParamsE:\n" + "".join(lines) + "\ts_endpgm\n.Lfunc_end0:\n"
+        return [f[3] for f in multiplies_too_close(body)]
+
+    branch, target = "\ts_cbranch_scc1 .LBB0_2\n", ".LBB0_2:\n"
+    assert states(multiply, asm % 79) == [0] and states(multiply, asm % 80) == []
+    assert states(multiply, "\ts_nop 10\n", asm % 79) == [11] and states(multiply, "\ts_nop 11\n", asm % 79) == []
+    assert states(multiply, branch, "\ts_nop 15\n", target, asm % 64) == [1]                # the way past the wait
+    assert states(target, asm % 64, multiply, branch) == [1]                               # around a loop
+    assert states(target, asm % 64, multiply, "\ts_nop 15\n", branch) == []
+    assert states(multiply, "\ts_branch .LBB0_2\n", asm % 64, "\ts_nop 15\n", target) == []  # not on a path
+    small = multiply.replace("32x32x16", "16x16x32").replace("v[64:79]", "v[64:67]")
+    assert states(small, "\ts_nop 6\n", asm % 64) == [7] and states(small, "\ts_nop 7\n", asm % 64) == []
+
+
 def test_m0_distance_checker():
     def found(*lines):
         return len(m0_too_close("_ZN6spattn1kE:\n.LBB0_1:\n\t" + "\n\t".join(lines) + "\n\ts_endpgm\n.Lfunc_end0:\n"))
@@ -293,7 +333,10 @@ def test_no_instruction_touches_a_register_with_a_load_in_flight(tmp_path):
         return out.read_text()
 
     with ThreadPoolExecutor(max_workers=4) as ex:
-        texts = list(ex.map(listing, M0_UNITS))
+        texts = list(ex.map(listing, M0_UNITS + [TOPK_UNIT]))
+    for unit, text in zip(M0_UNITS + [TOPK_UNIT], texts):
+        near = multiplies_too_close(text)
+        assert not near, "%s: %d asm instructions name a multiply's result too early, e.g. %s" % (unit, len(near), near[0])
     for unit, text in zip(M0_UNITS, texts):
         assert "global_load_lds_dwordx4" in text, unit
         uses = m0_uses_outside_asm(text)
