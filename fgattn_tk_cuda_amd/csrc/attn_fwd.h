@@ -728,7 +728,7 @@ void attn_fwd_kernel(const AttnParams p) {
         if constexpr (WITH_SM && SPLIT_SM) {
           if (m % MPP == 0) softmax_lag(s_in, base, (m / MPP) / 4, 8 + 2 * ((m / MPP) % 4), 2, par_in, last);
         } else if constexpr (WITH_SM) {
-          // in the order of the two halves: a row's denominator has the same bits with and without V
+          // in the order of the two halves: in one form a row's denominator has the same bits with and without V
           constexpr int HM = NM / 2;
           softmax_lag(s_in, base, (m % HM) / (NT / 2), 8 * (m / HM) + (m % (NT / 2)) * EPM, EPM, par_in, last);
         }

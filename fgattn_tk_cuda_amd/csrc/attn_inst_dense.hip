@@ -15,8 +15,8 @@ namespace spattn {
 //   statistics 0.93-0.98, statistics only 0.89-0.98; at 256 and 512 keys that is 0.93-1.09, behind 768 q-blocks 1.08-1.14.
 //   d = 128 is slower (1.02-1.2, with statistics 1.2-1.5: its LDS allows one workgroup per CU) from the second q-block per
 //   CU on, except the statistics alone, whose ring is 48 KB, from 768 keys on: 0.90-0.96 up to three per CU, 1.12-1.2 behind.
-//   The statistics alone at d = 64 fit five to a CU; that pays again where the 128-row form has a third one on some CUs, from 513
-//   to 640 of its q-blocks: 0.94-0.98 (8 x 8508 146 -> 138 us, 32 x 2050 40.4 -> 38.1), with fewer 1.05-1.09, behind 1.09-1.12.
+//   The statistics alone at d = 64 would fit five to a CU and gain 2-6 % from 513 to 640 q-blocks of 128 rows, but a row's
+//   denominator would then not have the bits that attention with statistics gives it, nor its mask the same keys.
 //   Two groups on 64-row q-blocks, up to one per CU, against one group on them: d = 64 from 12 tiles on 0.72-0.95, 10 and 11
 //   0.92-0.99 (8 x 588 with statistics 9.0 -> 8.3 us), 8 and 9 0.99-1.04; d = 128 from 15 on 0.75-1.00 (12 tiles 0.99, 8 tiles
 //   1.07-1.13).  Dense with statistics at d = 128 has no LDS for it.
@@ -44,7 +44,6 @@ DenseForm dense_form(int D, bool has_v, bool stats, int S, int kv_len, long long
   if (n64 <= kCus) return {64, !(D == 128 && has_v && stats) && tiles >= (D == 64 ? 10 : 15) ? 2 : 1};
   if (n128 <= kCus && tiles >= (D == 128 ? 12 : stats ? 15 : 24)) return {128, 2};
   if ((D == 64 || !has_v) && kv_len >= 768 && n64 <= 3 * kCus) return {64, 1};
-  if (D == 64 && !has_v && kv_len >= 768 && n128 > 2 * kCus && n64 <= 5 * kCus) return {64, 1};
   if (D == 128 && has_v) {
     const long long n256 = launched * ((S + 255) / 256);
     const long long last = n256 % kCus;

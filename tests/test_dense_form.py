@@ -44,9 +44,12 @@ def test_256_row_qblocks_in_one_round():
     assert form(128, 1, 0, 80, 1506) == 1281                                            # 480 of 24 tiles
 
 
-def test_statistics_alone_five_to_a_cu():
-    assert [form(64, 0, 1, h, 1100) for h in (56, 57, 71, 72)] == [1281, 641, 641, 1281]   # 504 and 513 of 128, 1278 and 1296 of 64 rows
-    assert form(64, 1, 1, 57, 1100) == form(64, 0, 1, 90, 767) == 1281
+def test_statistics_at_d64_take_the_form_of_attention_with_statistics():
+    """Other forms add a row's sum in another order: a key at its threshold would be in the mask of a call that takes the
+    statistics alone and not in that of a refresh, or the other way round."""
+    for heads in (1, 3, 8, 24, 44, 56, 57, 64, 71, 72, 90, 240):
+        for S, kv_len in ((64, 0), (300, 0), (577, 0), (767, 0), (1100, 0), (1100, 767), (1473, 1408), (2050, 0), (8508, 0), (32760, 0)):
+            assert form(64, 0, 1, heads, S, kv_len) == form(64, 1, 1, heads, S, kv_len), (heads, S, kv_len)
 
 
 def test_two_groups_from_ten_tiles_at_d64():

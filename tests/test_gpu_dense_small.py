@@ -156,13 +156,12 @@ def test_256_row_qblocks_in_one_round(dev, S, kv_len, heads, rows):
     test_256_row_qblocks_give_the_same_bits(dev, S, kv_len, heads, rows, rows)
 
 
-@pytest.mark.parametrize("S,kv_len,heads", [(1100, 0, (57, 56, 71, 72)), (1473, 1408, (45, 44, 53))])
+@pytest.mark.parametrize("S,kv_len,heads", [(1100, 0, (57, 56, 71, 72)), (1473, 1408, (45, 44, 53)), (700, 0, (2, 24, 70))])
 def test_statistics_alone_at_d64_match_those_of_attention(dev, S, kv_len, heads):
-    """Launches of the statistics alone on both sides of the rule for five 64-row q-blocks to a CU: row and block maxima bit for
-    bit those of the sweep with V, denominators to the rounding of fp32 sums in another order."""
+    """Row maxima, denominators and block maxima of the statistics alone: bit for bit those of the sweep with V."""
     import fgattn_tk_cuda_amd.spattn.cuda_attn  # noqa: F401
 
-    print("case statistics five to a CU", S, kv_len, heads, flush=True)
+    print("case statistics alone against attention", S, kv_len, heads, flush=True)
     ops = torch.ops.cuda_attn
     g = torch.Generator(device=dev).manual_seed(S)
     sp = (S + 127) // 128 * 128
@@ -173,5 +172,4 @@ def test_statistics_alone_at_d64_match_those_of_attention(dev, S, kv_len, heads)
         bm, bm2 = (torch.full((1, h, sp // 64, sp), 7.0, device=dev, dtype=torch.bfloat16) for _ in range(2))
         ops.fullattn_maxq_denom_blockmax(o, m, d, bm, q, k, v, 0.0, kv_len)
         ops.maxq_denom_blockmax(m2, d2, bm2, q, k, 0.0, kv_len)
-        assert torch.equal(m, m2) and torch.equal(bm[..., :S], bm2[..., :S])
-        assert torch.allclose(d[..., :S], d2[..., :S], rtol=2e-5, atol=0) and torch.equal(d[..., S:], d2[..., S:])
+        assert torch.equal(m, m2) and torch.equal(d, d2) and torch.equal(bm[..., :S], bm2[..., :S])
