@@ -33,6 +33,8 @@ _SIGNATURES = {
     "spattn_sp_attn_ordered": (_c_int, [_c_void_p] * 8 + [_c_int] * 7 + [_c_float, _c_void_p]),
     "spattn_sp_attn_blocks_ordered": (_c_int, [_c_void_p] * 8 + [_c_int] * 7 + [_c_float, _c_void_p]),
     "spattn_sp_attn_blocks_balanced": (_c_int, [_c_void_p] * 7 + [_c_int] * 7 + [_c_float, _c_void_p]),
+    "spattn_sp_attn_of": (_c_int, [_c_void_p] * 8 + [_c_int] * 7 + [_c_float, _c_int, _c_void_p]),
+    "spattn_sp_attn_blocks_of": (_c_int, [_c_void_p] * 8 + [_c_int] * 7 + [_c_float, _c_int, _c_void_p]),
     "spattn_init": (_c_int, []),
     "spattn_qblock_order": (_c_int, [_c_void_p] * 2 + [_c_int, _c_void_p]),
     "spattn_qblock_schedule": (_c_int, [_c_void_p] * 2 + [_c_int, _c_int, _c_void_p]),
@@ -58,6 +60,7 @@ _SIGNATURES = {
     "spattn_packedmask_to_indexmask": (_c_int, [_c_void_p] * 3 + [_c_int] * 5 + [_c_void_p]),
     "spattn_qk_topkmask_indices": (_c_int, [_c_void_p] * 6 + [_c_int] * 9 + [_c_void_p]),
     "spattn_dense_form": (_c_int, [_c_int] * 7),
+    "spattn_list_form": (_c_int, [_c_int] * 8),
     "spattn_last_status": (_c_int, []),
     "spattn_status_string": (ctypes.c_char_p, [_c_int]),
     "spattn_version": (_c_int, []),
@@ -133,10 +136,11 @@ def full_attn(o, q, k, v, *, lse=None, kv_len=0, scale=0.0, stream=None):
 
 
 def sp_attn(o, q, k, v, kv_indices, kv_num_indices, *, lse=None, qblk=None, kv_len=0, scale=0.0, order=None,
-            stream=None):
+            of_heads=0, stream=None):
     """Token-list sparse attention.  qblk defaults to the value implied by kv_indices.shape[2].
     order: optional int32 [B*H*SB] work order from qblock_order (same results, better balance
-    when the lists differ much in length)."""
+    when the lists differ much in length).  of_heads: B*H of the computation that the call is a part of (0: the call is the
+    whole); the results are then the bits of one call over all of it."""
     B, H, S, D = _bhsd(q)
     if kv_indices.dim() != 4:
         raise ValueError("kv_indices must be [B,H,SB,mask_stride]")
@@ -144,21 +148,16 @@ def sp_attn(o, q, k, v, kv_indices, kv_num_indices, *, lse=None, qblk=None, kv_l
         qblk = infer_qblk(S, int(kv_indices.shape[2]))
     if kv_num_indices.numel() != B * H * int(kv_indices.shape[2]):
         raise ValueError("kv_num_indices must have B*H*SB entries")
-    if order is None:
-        _check(load().spattn_sp_attn(_ptr(o, bf16), _ptr(lse, f32), _ptr(q, bf16), _ptr(k, bf16), _ptr(v, bf16),
-                                     _ptr(kv_indices, i32), _ptr(kv_num_indices, i32), int(kv_indices.shape[3]), qblk,
-                                     B, H, S, D, kv_len, scale, _stream(stream)))
-        return
-    if order.numel() != kv_num_indices.numel():
+    if order is not None and order.numel() != kv_num_indices.numel():
         raise ValueError("order must have B*H*SB entries")
-    _check(load().spattn_sp_attn_ordered(_ptr(o, bf16), _ptr(lse, f32), _ptr(q, bf16), _ptr(k, bf16), _ptr(v, bf16),
-                                         _ptr(kv_indices, i32), _ptr(kv_num_indices, i32), _ptr(order, i32),
-                                         int(kv_indices.shape[3]), qblk, B, H, S, D, kv_len, scale, _stream(stream)))
+    _check(load().spattn_sp_attn_of(_ptr(o, bf16), _ptr(lse, f32), _ptr(q, bf16), _ptr(k, bf16), _ptr(v, bf16),
+                                    _ptr(kv_indices, i32), _ptr(kv_num_indices, i32), _ptr(order, i32),
+                                    int(kv_indices.shape[3]), qblk, B, H, S, D, kv_len, scale, int(of_heads), _stream(stream)))
 
 
 def sp_attn_blocks(o, q, k, v, blk_indices, blk_counts, *, lse=None, qblk=None, kv_len=0, scale=0.0, order=None,
-                   stream=None):
-    """Block-list sparse attention over 64-key blocks.  order: as for sp_attn."""
+                   of_heads=0, stream=None):
+    """Block-list sparse attention over 64-key blocks.  order, of_heads: as for sp_attn."""
     B, H, S, D = _bhsd(q)
     if blk_indices.dim() != 4:
         raise ValueError("blk_indices must be [B,H,SB,max_blocks]")
@@ -166,17 +165,11 @@ def sp_attn_blocks(o, q, k, v, blk_indices, blk_counts, *, lse=None, qblk=None, 
         qblk = infer_qblk(S, int(blk_indices.shape[2]))
     if blk_counts.numel() != B * H * int(blk_indices.shape[2]):
         raise ValueError("blk_counts must have B*H*SB entries")
-    if order is None:
-        _check(load().spattn_sp_attn_blocks(_ptr(o, bf16), _ptr(lse, f32), _ptr(q, bf16), _ptr(k, bf16), _ptr(v, bf16),
-                                            _ptr(blk_indices, i32), _ptr(blk_counts, i32), int(blk_indices.shape[3]),
-                                            qblk, B, H, S, D, kv_len, scale, _stream(stream)))
-        return
-    if order.numel() != blk_counts.numel():
+    if order is not None and order.numel() != blk_counts.numel():
         raise ValueError("order must have B*H*SB entries")
-    _check(load().spattn_sp_attn_blocks_ordered(_ptr(o, bf16), _ptr(lse, f32), _ptr(q, bf16), _ptr(k, bf16),
-                                                _ptr(v, bf16), _ptr(blk_indices, i32), _ptr(blk_counts, i32),
-                                                _ptr(order, i32), int(blk_indices.shape[3]), qblk, B, H, S, D, kv_len,
-                                                scale, _stream(stream)))
+    _check(load().spattn_sp_attn_blocks_of(_ptr(o, bf16), _ptr(lse, f32), _ptr(q, bf16), _ptr(k, bf16), _ptr(v, bf16),
+                                           _ptr(blk_indices, i32), _ptr(blk_counts, i32), _ptr(order, i32),
+                                           int(blk_indices.shape[3]), qblk, B, H, S, D, kv_len, scale, int(of_heads), _stream(stream)))
 
 
 BALANCED_MAX_QBLOCKS = 1 << 20

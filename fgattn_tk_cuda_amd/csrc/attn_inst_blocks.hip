@@ -4,8 +4,8 @@
 
 namespace spattn {
 
-hipError_t run_attn_blocks(const AttnParams& p, int D, int qblk, hipStream_t stream) {
-  if (lists_by_halves(D, qblk, p, false)) {
+hipError_t run_attn_blocks(const AttnParams& p, int D, int qblk, hipStream_t stream, int heads) {
+  if (lists_by_halves(D, qblk, false, heads > 0 ? heads : (long long)p.B * p.H, p.S, p.kv_len, p.idx_stride)) {
     if (D == 128) return launch_attn_fwd<128, 64, KV_BLOCKS, true, false, 1, true>(p, stream);
     return launch_attn_fwd<64, 64, KV_BLOCKS, true, false, 1, true>(p, stream);
   }

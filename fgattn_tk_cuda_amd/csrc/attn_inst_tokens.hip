@@ -13,17 +13,17 @@ namespace spattn {
 //   d = 128 up to one per CU 0.77-0.97 (8 x 2000 16.8 -> 12.9 us with 10 tiles), lists of one tile 1.01-1.05, which sequences
 //   below 768 keys have; from the second per CU on 0.98-1.23.
 // The rule looks at the launch alone, not at the counts, which are on the device.  The halves add a row's keys in another
-// order, so low bits of the outputs depend on how many heads share a call, as those of dense attention do.
-bool lists_by_halves(int D, int qblk, const AttnParams& p, bool tokens) {
+// order: a launch over some heads of a computation goes by all of its heads, so that no bit depends on the split.
+bool lists_by_halves(int D, int qblk, bool tokens, long long heads, int S, int kv_len, int idx_stride) {
   if (qblk != 128) return false;
   constexpr long long kCus = 256;
-  const long long n64 = (long long)p.B * p.H * ((p.S + 63) / 64);
-  if (D == 128) return n64 <= kCus && p.kv_len >= 768 && p.idx_stride >= (tokens ? 256 : 2);
-  return n64 <= kCus || (n64 <= 3 * kCus && p.kv_len >= 1024 && (tokens || p.idx_stride >= 5));
+  const long long n64 = heads * ((S + 63) / 64);
+  if (D == 128) return n64 <= kCus && kv_len >= 768 && idx_stride >= (tokens ? 256 : 2);
+  return n64 <= kCus || (n64 <= 3 * kCus && kv_len >= 1024 && (tokens || idx_stride >= 5));
 }
 
-hipError_t run_attn_tokens(const AttnParams& p, int D, int qblk, hipStream_t stream) {
-  if (lists_by_halves(D, qblk, p, true)) {
+hipError_t run_attn_tokens(const AttnParams& p, int D, int qblk, hipStream_t stream, int heads) {
+  if (lists_by_halves(D, qblk, true, heads > 0 ? heads : (long long)p.B * p.H, p.S, p.kv_len, p.idx_stride)) {
     if (D == 128) return launch_attn_fwd<128, 64, KV_TOKENS, true, false, 1, true>(p, stream);
     return launch_attn_fwd<64, 64, KV_TOKENS, true, false, 1, true>(p, stream);
   }

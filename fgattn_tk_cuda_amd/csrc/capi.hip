@@ -61,10 +61,11 @@ int spattn_full_attn(void* o, float* lse, const void* q, const void* k, const vo
   return from_hip(spattn::run_attn_dense(p, D, true, false, as_stream(stream)));
 }
 
-int spattn_sp_attn(void* o, float* lse, const void* q, const void* k, const void* v, const int* kv_indices,
-                   const int* num_kv_indices, int mask_stride, int qblk, int B, int H, int S, int D, int kv_len,
-                   float scale, void* stream) {
+int spattn_sp_attn_of(void* o, float* lse, const void* q, const void* k, const void* v, const int* kv_indices,
+                      const int* num_kv_indices, const int* order, int mask_stride, int qblk, int B, int H, int S, int D,
+                      int kv_len, float scale, int of_heads, void* stream) {
   if (int st = check_qkv(q, k, B, H, S, D)) return done(st);
+  if (of_heads != 0 && of_heads < B * H) return done(SPATTN_ERR_SHAPE);
   if (!o || !v || !kv_indices || !num_kv_indices) return done(SPATTN_ERR_NULL);
   if (misaligned(o) || misaligned(v) || misaligned(kv_indices)) return done(SPATTN_ERR_ALIGN);
   if (qblk != 64 && qblk != 128) return done(SPATTN_ERR_QBLK);
@@ -75,13 +76,22 @@ int spattn_sp_attn(void* o, float* lse, const void* q, const void* k, const void
   p.idx = kv_indices;
   p.cnt = num_kv_indices;
   p.idx_stride = mask_stride;
-  return from_hip(spattn::run_attn_tokens(p, D, qblk, as_stream(stream)));
+  p.order = order;
+  return from_hip(spattn::run_attn_tokens(p, D, qblk, as_stream(stream), of_heads));
 }
 
-int spattn_sp_attn_blocks(void* o, float* lse, const void* q, const void* k, const void* v, const int* blk_indices,
-                          const int* blk_counts, int max_blocks, int qblk, int B, int H, int S, int D, int kv_len,
-                          float scale, void* stream) {
+int spattn_sp_attn(void* o, float* lse, const void* q, const void* k, const void* v, const int* kv_indices,
+                   const int* num_kv_indices, int mask_stride, int qblk, int B, int H, int S, int D, int kv_len,
+                   float scale, void* stream) {
+  return spattn_sp_attn_of(o, lse, q, k, v, kv_indices, num_kv_indices, nullptr, mask_stride, qblk, B, H, S, D, kv_len, scale, 0,
+                           stream);
+}
+
+int spattn_sp_attn_blocks_of(void* o, float* lse, const void* q, const void* k, const void* v, const int* blk_indices,
+                             const int* blk_counts, const int* order, int max_blocks, int qblk, int B, int H, int S, int D,
+                             int kv_len, float scale, int of_heads, void* stream) {
   if (int st = check_qkv(q, k, B, H, S, D)) return done(st);
+  if (of_heads != 0 && of_heads < B * H) return done(SPATTN_ERR_SHAPE);
   if (!o || !v || !blk_indices || !blk_counts) return done(SPATTN_ERR_NULL);
   if (misaligned(o) || misaligned(v)) return done(SPATTN_ERR_ALIGN);
   if (qblk != 64 && qblk != 128) return done(SPATTN_ERR_QBLK);
@@ -91,7 +101,15 @@ int spattn_sp_attn_blocks(void* o, float* lse, const void* q, const void* k, con
   p.idx = blk_indices;
   p.cnt = blk_counts;
   p.idx_stride = max_blocks;
-  return from_hip(spattn::run_attn_blocks(p, D, qblk, as_stream(stream)));
+  p.order = order;
+  return from_hip(spattn::run_attn_blocks(p, D, qblk, as_stream(stream), of_heads));
+}
+
+int spattn_sp_attn_blocks(void* o, float* lse, const void* q, const void* k, const void* v, const int* blk_indices,
+                          const int* blk_counts, int max_blocks, int qblk, int B, int H, int S, int D, int kv_len,
+                          float scale, void* stream) {
+  return spattn_sp_attn_blocks_of(o, lse, q, k, v, blk_indices, blk_counts, nullptr, max_blocks, qblk, B, H, S, D, kv_len, scale, 0,
+                                  stream);
 }
 
 int spattn_all_index_mask(int* kv_indices, int* num_kv_indices, int B, int H, int seqblocks, int seq, int mask_stride,
@@ -150,6 +168,16 @@ int spattn_dense_form(int D, int has_v, int stats, int heads, int S, int kv_len,
   const spattn::DenseForm f = spattn::dense_form(D, has_v != 0, stats != 0, S, kv, heads, of_heads);
   done(SPATTN_OK);
   return 10 * f.rows + f.groups;
+}
+
+int spattn_list_form(int D, int qblk, int tokens, int heads, int S, int kv_len, int stride, int of_heads) {
+  if (D != 64 && D != 128) return done(SPATTN_ERR_HEAD_DIM);
+  if (qblk != 64 && qblk != 128) return done(SPATTN_ERR_QBLK);
+  if (heads <= 0 || S <= 0 || S >= (1 << 24) || stride <= 0 || (of_heads != 0 && of_heads < heads)) return done(SPATTN_ERR_SHAPE);
+  if (tokens && stride % 128 != 0) return done(SPATTN_ERR_STRIDE);
+  const int kv = kv_len > 0 && kv_len < S ? kv_len : S;
+  done(SPATTN_OK);
+  return spattn::lists_by_halves(D, qblk, tokens != 0, of_heads > 0 ? of_heads : heads, S, kv, stride) ? 64 : qblk;
 }
 
 int spattn_maxq_denom_blockmax(float* max_q, float* denom, void* blockmax, const void* q, const void* k, int B, int H,
@@ -372,34 +400,17 @@ int spattn_sp_attn_ordered(void* o, float* lse, const void* q, const void* k, co
                            const int* num_kv_indices, const int* order, int mask_stride, int qblk, int B, int H, int S,
                            int D, int kv_len, float scale, void* stream) {
   if (int st = check_qkv(q, k, B, H, S, D)) return done(st);
-  if (!o || !v || !kv_indices || !num_kv_indices || !order) return done(SPATTN_ERR_NULL);
-  if (misaligned(o) || misaligned(v) || misaligned(kv_indices)) return done(SPATTN_ERR_ALIGN);
-  if (qblk != 64 && qblk != 128) return done(SPATTN_ERR_QBLK);
-  if (mask_stride <= 0 || mask_stride % 128 != 0) return done(SPATTN_ERR_STRIDE);
-  spattn::AttnParams p = base_params(q, k, v, o, B, H, S, D, kv_len, scale, qblk);
-  p.lse = lse;
-  p.idx = kv_indices;
-  p.cnt = num_kv_indices;
-  p.idx_stride = mask_stride;
-  p.order = order;
-  return from_hip(spattn::run_attn_tokens(p, D, qblk, as_stream(stream)));
+  if (!order) return done(SPATTN_ERR_NULL);
+  return spattn_sp_attn_of(o, lse, q, k, v, kv_indices, num_kv_indices, order, mask_stride, qblk, B, H, S, D, kv_len, scale, 0, stream);
 }
 
 int spattn_sp_attn_blocks_ordered(void* o, float* lse, const void* q, const void* k, const void* v,
                                   const int* blk_indices, const int* blk_counts, const int* order, int max_blocks,
                                   int qblk, int B, int H, int S, int D, int kv_len, float scale, void* stream) {
   if (int st = check_qkv(q, k, B, H, S, D)) return done(st);
-  if (!o || !v || !blk_indices || !blk_counts || !order) return done(SPATTN_ERR_NULL);
-  if (misaligned(o) || misaligned(v)) return done(SPATTN_ERR_ALIGN);
-  if (qblk != 64 && qblk != 128) return done(SPATTN_ERR_QBLK);
-  if (max_blocks <= 0) return done(SPATTN_ERR_SHAPE);
-  spattn::AttnParams p = base_params(q, k, v, o, B, H, S, D, kv_len, scale, qblk);
-  p.lse = lse;
-  p.idx = blk_indices;
-  p.cnt = blk_counts;
-  p.idx_stride = max_blocks;
-  p.order = order;
-  return from_hip(spattn::run_attn_blocks(p, D, qblk, as_stream(stream)));
+  if (!order) return done(SPATTN_ERR_NULL);
+  return spattn_sp_attn_blocks_of(o, lse, q, k, v, blk_indices, blk_counts, order, max_blocks, qblk, B, H, S, D, kv_len, scale, 0,
+                                  stream);
 }
 
 // ---- block-list attention in balanced order without a caller-provided order buffer -------------

@@ -5,11 +5,11 @@
 namespace spattn {
 
 // attn_inst_tokens.hip / attn_inst_blocks.hip / attn_inst_dense.hip
-hipError_t run_attn_tokens(const AttnParams& p, int D, int qblk, hipStream_t stream);
-hipError_t run_attn_blocks(const AttnParams& p, int D, int qblk, hipStream_t stream);
-// Whether lists of 128-row q-blocks run by workgroups of 64 rows, two to a list (attn_inst_tokens.hip).
-bool lists_by_halves(int D, int qblk, const AttnParams& p, bool tokens);
 // heads: of the whole computation where the launch is a part of one, 0: those of the launch
+hipError_t run_attn_tokens(const AttnParams& p, int D, int qblk, hipStream_t stream, int heads = 0);
+hipError_t run_attn_blocks(const AttnParams& p, int D, int qblk, hipStream_t stream, int heads = 0);
+// Whether lists of 128-row q-blocks run by workgroups of 64 rows, two to a list (attn_inst_tokens.hip).
+bool lists_by_halves(int D, int qblk, bool tokens, long long heads, int S, int kv_len, int idx_stride);
 hipError_t run_attn_dense(const AttnParams& p, int D, bool has_v, bool stats, hipStream_t stream, int heads = 0);
 // The form that such a launch takes: rows per q-block, groups of waves that share one.
 struct DenseForm {

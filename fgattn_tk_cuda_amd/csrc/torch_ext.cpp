@@ -77,6 +77,12 @@ int checked_kv_len(int64_t kv_len, const torch::Tensor& q) {
   return (int)kv_len;
 }
 
+// of_heads: B*H of the computation that these heads are a part of (0: the call is the whole).
+int checked_of_heads(int64_t of_heads, const torch::Tensor& q) {
+  TORCH_CHECK(of_heads == 0 || (of_heads >= q.size(0) * q.size(1) && of_heads <= INT32_MAX), "of_heads must be 0 or at least B*H");
+  return (int)of_heads;
+}
+
 }  // namespace
 
 // Work orders that sp_attn keeps for these counts are computed again (defined with them, below).
@@ -118,21 +124,13 @@ void all_index_mask(torch::Tensor kv_indices, torch::Tensor kv_num_indices, int6
 // Token lists.  order: the work order of spattn_qblock_order for these counts, or none.
 static void sp_attn_impl(torch::Tensor& o, const OptTensor& lse, torch::Tensor& q, torch::Tensor& k, torch::Tensor& v,
                          torch::Tensor& kv_indices, torch::Tensor& kv_num_indices, const int* order, double scale,
-                         int64_t kv_len) {
+                         int64_t kv_len, int64_t of_heads) {
   const int qblk = infer_qblk(q.size(2), kv_indices.size(2));
-  const int B = (int)q.size(0), H = (int)q.size(1), S = (int)q.size(2), D = (int)q.size(3);
-  const int kv = checked_kv_len(kv_len, q);
-  if (order != nullptr) {
-    check_status(spattn_sp_attn_ordered(o.data_ptr(), lse_ptr(lse, q), q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                                        kv_indices.data_ptr<int>(), kv_num_indices.data_ptr<int>(), order,
-                                        (int)kv_indices.size(3), qblk, B, H, S, D, kv, (float)scale, cur_stream()),
-                 "sp_attn");
-  } else {
-    check_status(spattn_sp_attn(o.data_ptr(), lse_ptr(lse, q), q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                                kv_indices.data_ptr<int>(), kv_num_indices.data_ptr<int>(), (int)kv_indices.size(3), qblk,
-                                B, H, S, D, kv, (float)scale, cur_stream()),
-                 "sp_attn");
-  }
+  check_status(spattn_sp_attn_of(o.data_ptr(), lse_ptr(lse, q), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                                 kv_indices.data_ptr<int>(), kv_num_indices.data_ptr<int>(), order, (int)kv_indices.size(3), qblk,
+                                 (int)q.size(0), (int)q.size(1), (int)q.size(2), (int)q.size(3), checked_kv_len(kv_len, q),
+                                 (float)scale, checked_of_heads(of_heads, q), cur_stream()),
+               "sp_attn");
 }
 
 static void check_sp_attn_args(torch::Tensor& o, torch::Tensor& q, torch::Tensor& k, torch::Tensor& v,
@@ -261,23 +259,28 @@ void sp_attn(torch::Tensor o, torch::Tensor q, torch::Tensor k, torch::Tensor v,
   // attention launch alone.
   const OptTensor order = sp_attn_work_order(kv_num_indices, kv_indices.size(2));
   sp_attn_impl(o, c10::nullopt, q, k, v, kv_indices, kv_num_indices, order.has_value() ? order->data_ptr<int>() : nullptr, 0.0,
-               0);
+               0, 0);
 }
 
 // sp_attn with an optional log-sum-exp output, an optional precomputed work order (none: the
 // default order, one launch and no allocation), a softmax scale (0 = 1/sqrt(D)) and a kv length.
-void sp_attn_ex(torch::Tensor o, OptTensor lse, torch::Tensor q, torch::Tensor k, torch::Tensor v,
-                torch::Tensor kv_indices, torch::Tensor kv_num_indices, OptTensor order, double scale, int64_t kv_len) {
+void sp_attn_ex_of(torch::Tensor o, OptTensor lse, torch::Tensor q, torch::Tensor k, torch::Tensor v, torch::Tensor kv_indices,
+                   torch::Tensor kv_num_indices, OptTensor order, double scale, int64_t kv_len, int64_t of_heads) {
   check_sp_attn_args(o, q, k, v, kv_indices, kv_num_indices);
   const DeviceGuard guard(q.device());
-  sp_attn_impl(o, lse, q, k, v, kv_indices, kv_num_indices, order_ptr(order, kv_num_indices), scale, kv_len);
+  sp_attn_impl(o, lse, q, k, v, kv_indices, kv_num_indices, order_ptr(order, kv_num_indices), scale, kv_len, of_heads);
+}
+
+void sp_attn_ex(torch::Tensor o, OptTensor lse, torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                torch::Tensor kv_indices, torch::Tensor kv_num_indices, OptTensor order, double scale, int64_t kv_len) {
+  sp_attn_ex_of(o, lse, q, k, v, kv_indices, kv_num_indices, order, scale, kv_len, 0);
 }
 
 // Sparse attention over lists of 64-key blocks: blk_idx int32 [B,H,ceil(S/qblk),max_blocks],
 // blk_cnt int32 with B*H*ceil(S/qblk) entries, qblk 64 or 128 (0 = implied by blk_idx.size(2)).
-void sp_attn_block(torch::Tensor o, OptTensor lse, torch::Tensor q, torch::Tensor k, torch::Tensor v,
-                   torch::Tensor blk_idx, torch::Tensor blk_cnt, OptTensor order, int64_t qblk, double scale,
-                   int64_t kv_len) {
+void sp_attn_block_of(torch::Tensor o, OptTensor lse, torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                      torch::Tensor blk_idx, torch::Tensor blk_cnt, OptTensor order, int64_t qblk, double scale,
+                      int64_t kv_len, int64_t of_heads) {
   check_bhsd(q, "q", q);
   check_bhsd(k, "k", q);
   check_bhsd(v, "v", q);
@@ -291,21 +294,17 @@ void sp_attn_block(torch::Tensor o, OptTensor lse, torch::Tensor q, torch::Tenso
   TORCH_CHECK(blk_idx.size(2) == (q.size(2) + qblk - 1) / qblk, "blk_idx must hold ceil(S/qblk) lists per head");
   TORCH_CHECK(blk_cnt.numel() == q.size(0) * q.size(1) * blk_idx.size(2), "blk_cnt must have B*H*SB entries");
   const DeviceGuard guard(q.device());
-  const int B = (int)q.size(0), H = (int)q.size(1), S = (int)q.size(2), D = (int)q.size(3);
-  const int kv = checked_kv_len(kv_len, q);
-  const int* ord = order_ptr(order, blk_cnt);
-  if (ord != nullptr) {
-    check_status(spattn_sp_attn_blocks_ordered(o.data_ptr(), lse_ptr(lse, q), q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                                               blk_idx.data_ptr<int>(), blk_cnt.data_ptr<int>(), ord,
-                                               (int)blk_idx.size(3), (int)qblk, B, H, S, D, kv, (float)scale,
-                                               cur_stream()),
-                 "sp_attn_block");
-  } else {
-    check_status(spattn_sp_attn_blocks(o.data_ptr(), lse_ptr(lse, q), q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                                       blk_idx.data_ptr<int>(), blk_cnt.data_ptr<int>(), (int)blk_idx.size(3), (int)qblk,
-                                       B, H, S, D, kv, (float)scale, cur_stream()),
-                 "sp_attn_block");
-  }
+  check_status(spattn_sp_attn_blocks_of(o.data_ptr(), lse_ptr(lse, q), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                                        blk_idx.data_ptr<int>(), blk_cnt.data_ptr<int>(), order_ptr(order, blk_cnt),
+                                        (int)blk_idx.size(3), (int)qblk, (int)q.size(0), (int)q.size(1), (int)q.size(2),
+                                        (int)q.size(3), checked_kv_len(kv_len, q), (float)scale, checked_of_heads(of_heads, q),
+                                        cur_stream()),
+               "sp_attn_block");
+}
+
+void sp_attn_block(torch::Tensor o, OptTensor lse, torch::Tensor q, torch::Tensor k, torch::Tensor v, torch::Tensor blk_idx,
+                   torch::Tensor blk_cnt, OptTensor order, int64_t qblk, double scale, int64_t kv_len) {
+  sp_attn_block_of(o, lse, q, k, v, blk_idx, blk_cnt, order, qblk, scale, kv_len, 0);
 }
 
 // order int32 [n] <- the q-blocks of counts (int32, n entries) longest list first.
@@ -378,12 +377,6 @@ void check_blockmax(const torch::Tensor& blockmax, const torch::Tensor& q_like, 
   check_aux(blockmax, "blockmax", at::kBFloat16, q_like);
   const int64_t sp = padded128(S);
   TORCH_CHECK(blockmax.numel() == B * H * (sp / 64) * sp, "blockmax must be bf16 [B,H,Sp/64,Sp] with Sp = 128*ceil(S/128)");
-}
-
-// of_heads: B*H of the computation that these heads are a part of (0: the call is the whole).
-int checked_of_heads(int64_t of_heads, const torch::Tensor& q) {
-  TORCH_CHECK(of_heads == 0 || (of_heads >= q.size(0) * q.size(1) && of_heads <= INT32_MAX), "of_heads must be 0 or at least B*H");
-  return (int)of_heads;
 }
 
 void fullattn_maxq_denom_blockmax_of(torch::Tensor o, torch::Tensor o_max_q, torch::Tensor o_denom, torch::Tensor blockmax,
@@ -818,9 +811,9 @@ void noop_schedule(torch::Tensor, torch::Tensor, int64_t) {}
 void noop_topk(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, int64_t, int64_t) {}
 void noop_full_ex(torch::Tensor, OptTensor, torch::Tensor, torch::Tensor, torch::Tensor, double, int64_t) {}
 void noop_sp_ex(torch::Tensor, OptTensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, OptTensor,
-                double, int64_t) {}
+                double, int64_t, int64_t) {}
 void noop_sp_block(torch::Tensor, OptTensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
-                   OptTensor, int64_t, double, int64_t) {}
+                   OptTensor, int64_t, double, int64_t, int64_t) {}
 void noop_fmd_ex(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, double, int64_t) {}
 void noop_md_ex(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, double, int64_t) {}
 void noop_mask_ex(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, double, double, int64_t) {}
@@ -855,8 +848,8 @@ TORCH_LIBRARY_FRAGMENT(cuda_attn, m) {
   m.def("qk_topkmask_indices(Tensor(a!) kv_indices, Tensor(b!) kv_numindices, Tensor(c!) score, Tensor(d!) qmean, Tensor q, Tensor k, int select_k, int blocksz) -> ()");
   // scale 0 = 1/sqrt(D); kv_len 0 = S
   m.def("full_attn_ex(Tensor(a!) o, Tensor(b!)? lse, Tensor q, Tensor k, Tensor v, float scale, int kv_len) -> ()");
-  m.def("sp_attn_ex(Tensor(a!) o, Tensor(b!)? lse, Tensor q, Tensor k, Tensor v, Tensor kv_indices, Tensor kv_num_indices, Tensor? order, float scale, int kv_len) -> ()");
-  m.def("sp_attn_block(Tensor(a!) o, Tensor(b!)? lse, Tensor q, Tensor k, Tensor v, Tensor blk_idx, Tensor blk_cnt, Tensor? order, int qblk, float scale, int kv_len) -> ()");
+  m.def("sp_attn_ex(Tensor(a!) o, Tensor(b!)? lse, Tensor q, Tensor k, Tensor v, Tensor kv_indices, Tensor kv_num_indices, Tensor? order, float scale, int kv_len, int of_heads=0) -> ()");
+  m.def("sp_attn_block(Tensor(a!) o, Tensor(b!)? lse, Tensor q, Tensor k, Tensor v, Tensor blk_idx, Tensor blk_cnt, Tensor? order, int qblk, float scale, int kv_len, int of_heads=0) -> ()");
   m.def("fullattn_maxq_denom_ex(Tensor(a!) o, Tensor(b!) o_max_q, Tensor(c!) o_denom, Tensor q, Tensor k, Tensor v, float scale, int kv_len) -> ()");
   m.def("maxq_denom_ex(Tensor(a!) o_max_q, Tensor(b!) o_denom, Tensor q, Tensor k, float scale, int kv_len) -> ()");
   m.def("booleanmask_128_ex(Tensor(a!) booleanmask, Tensor o_max_q, Tensor o_denom, Tensor q, Tensor k, float threshold, float scale, int kv_len) -> ()");
@@ -922,8 +915,8 @@ TORCH_LIBRARY_IMPL(cuda_attn, CUDA, m) {
   m.impl("packedmask_to_indexmask", packedmask_to_indexmask);
   m.impl("qk_topkmask_indices", qk_topkmask_indices);
   m.impl("full_attn_ex", full_attn_ex);
-  m.impl("sp_attn_ex", sp_attn_ex);
-  m.impl("sp_attn_block", sp_attn_block);
+  m.impl("sp_attn_ex", sp_attn_ex_of);
+  m.impl("sp_attn_block", sp_attn_block_of);
   m.impl("fullattn_maxq_denom_ex", fullattn_maxq_denom_ex);
   m.impl("maxq_denom_ex", maxq_denom_ex);
   m.impl("booleanmask_128_ex", booleanmask_128_ex);

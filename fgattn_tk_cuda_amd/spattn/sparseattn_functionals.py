@@ -4,6 +4,10 @@ Each takes ``(query, key, value, current_layer, ditrun, **kwargs)`` with bf16 te
 [B,H,S,D] and returns the bf16 output, like the reference
 (python/spattn/sparseattn_functionals.py:10-154).  Outputs are allocated on the device
 of ``query``.
+
+``of_heads=``, taken by all that attend over lists: batch x heads of the computation, for a caller who splits its heads over
+calls or devices; attention over the same lists then gives the bits of one call over all of them (without it the low bits can
+depend on how many heads share the call).
 """
 from __future__ import annotations
 
@@ -50,22 +54,26 @@ def baseline_attn_maxq_denom(query, key, value, current_layer=None, ditrun=None,
 _ORDER_MIN_FRESH = 2048
 
 
-def _sparse(query, key, value, kv_indices, kv_num_indices, order=None, fresh=False):
+def _sparse(query, key, value, kv_indices, kv_num_indices, order=None, fresh=False, of_heads=None):
     """order: the work order that a cache computed when it stored these lists; the step is then one launch and
     allocates only the output.  fresh: lists of this call alone run in the order given, or in index order.
     Otherwise ``sp_attn`` keeps an order for the counts tensor."""
     out = _out_like(query)
-    if order is not None or fresh:
+    if of_heads:
+        if order is None and not fresh:
+            order = cuda_attn.work_order_of(kv_num_indices.contiguous(), kv_indices.shape[2])
+        spattn_interface.sp_attn_ex(out, None, *_c(query, key, value, kv_indices, kv_num_indices), order, 0.0, 0, of_heads)
+    elif order is not None or fresh:
         spattn_interface.sp_attn_ex(out, None, *_c(query, key, value, kv_indices, kv_num_indices), order, 0.0, 0)
     else:
         spattn_interface.sp_attn(out, *_c(query, key, value, kv_indices, kv_num_indices))
     return out
 
 
-def _sparse_once(query, key, value, kv_indices, kv_num_indices):
+def _sparse_once(query, key, value, kv_indices, kv_num_indices, of_heads=None):
     """Attention over lists that are dropped with this call, of uneven length."""
     order = mask_utils.qblock_order_cuda(kv_num_indices) if kv_num_indices.numel() >= _ORDER_MIN_FRESH else None
-    return _sparse(query, key, value, kv_indices, kv_num_indices, order, fresh=True)
+    return _sparse(query, key, value, kv_indices, kv_num_indices, order, fresh=True, of_heads=of_heads)
 
 
 def _cached_order(mask_cache, layer):
@@ -76,14 +84,14 @@ def _cached_order(mask_cache, layer):
 def attn_computed_with_sparse_mask_python(query, key, value, current_layer=None, ditrun=None, *args, **kwargs):
     """Index lists from the pure-torch mask definition, then sparse attention (:29-36)."""
     kv_indices, kv_num_indices = mask_utils.qk_indexmask(query, key, kwargs["thresh"], blocksz=kwargs["blocksz"])
-    return _sparse_once(query, key, value, kv_indices, kv_num_indices)
+    return _sparse_once(query, key, value, kv_indices, kv_num_indices, kwargs.get("of_heads"))
 
 
 def attn_lshmask_cuda(query, key, value, current_layer=None, ditrun=None, *args, **kwargs):
     """LSH-selected key lists, then sparse attention (:51-58).  As in the reference the selector is
     not implemented (python/spattn/mask_utils.py:385-386): the call raises NotImplementedError."""
     kv_indices, kv_num_indices = mask_utils.qk_lshmask_indices(query, key, kwargs["thresh"], blocksz=kwargs["blocksz"])
-    return _sparse_once(query, key, value, kv_indices, kv_num_indices)
+    return _sparse_once(query, key, value, kv_indices, kv_num_indices, kwargs.get("of_heads"))
 
 
 def attn_topkmask_cuda(query, key, value, current_layer=None, ditrun=None, *args, **kwargs):
@@ -91,7 +99,8 @@ def attn_topkmask_cuda(query, key, value, current_layer=None, ditrun=None, *args
     device selector, padded to a multiple of 128 keys as the sparse operator needs."""
     select_k = kwargs.get("select_k") or query.shape[2]
     kv_indices, kv_num_indices = mask_utils.qk_topkmask_indices_cuda(query, key, select_k, blocksz=kwargs["blocksz"], fill_tail=False)
-    return _sparse(query, key, value, kv_indices, kv_num_indices, fresh=True)   # lists of equal length: index order
+    # lists of equal length: index order
+    return _sparse(query, key, value, kv_indices, kv_num_indices, fresh=True, of_heads=kwargs.get("of_heads"))
 
 
 def attn_computed_with_sparse_mask_cuda(query, key, value, *args, **kwargs):
@@ -101,7 +110,7 @@ def attn_computed_with_sparse_mask_cuda(query, key, value, *args, **kwargs):
     kv_indices, kv_num_indices = mask_utils.qk_indexmask_cuda(query, key, kwargs["thresh"], blocksz=kwargs["blocksz"],
                                                               onepass=kwargs.get("onepass"), fill_tail=False,
                                                               budget_bytes=kwargs.get("blockmax_budget_bytes"))
-    return _sparse_once(query, key, value, kv_indices, kv_num_indices)
+    return _sparse_once(query, key, value, kv_indices, kv_num_indices, kwargs.get("of_heads"))
 
 
 def compute_cache_and_attn_cuda(query, key, value, *args, **kwargs):
@@ -115,7 +124,8 @@ def compute_cache_and_attn_cuda(query, key, value, *args, **kwargs):
 def sparse_attn_from_cache_cuda(query, key, value, *args, **kwargs):
     """Sparse attention from cached lists (:88-93)."""
     kv_indices, kv_num_indices = kwargs["mask_cache"].get_mask_from_cache(kwargs.get("current_layer"))
-    return _sparse(query, key, value, kv_indices, kv_num_indices, _cached_order(kwargs["mask_cache"], kwargs.get("current_layer")))
+    return _sparse(query, key, value, kv_indices, kv_num_indices, _cached_order(kwargs["mask_cache"], kwargs.get("current_layer")),
+                   False, kwargs.get("of_heads"))
 
 
 def _dense_and_packedmask(query, key, value, groups, thresh, qblk):
@@ -163,7 +173,8 @@ def cached_attn_cuda(query, key, value, current_layer, ditrun, *args, **kwargs):
         mask_cache.update_cache(current_layer, kv_indices, kv_num_indices)
         return out
     kv_indices, kv_num_indices = mask_cache.get_mask_from_cache(current_layer)
-    return _sparse(query, key, value, kv_indices, kv_num_indices, _cached_order(mask_cache, current_layer))
+    return _sparse(query, key, value, kv_indices, kv_num_indices, _cached_order(mask_cache, current_layer),
+                   False, kwargs.get("of_heads"))
 
 
 def blockcached_attn_cuda(query, key, value, current_layer, ditrun, *args, **kwargs):
@@ -202,7 +213,7 @@ def blockcached_attn_cuda(query, key, value, current_layer, ditrun, *args, **kwa
     blk_idx, blk_cnt = mask_cache.get_mask_from_cache(current_layer)
     out = _out_like(query)
     spattn_interface.sp_attn_block(out, None, *_c(query, key, value, blk_idx, blk_cnt), mask_cache.get_order(current_layer),
-                                   qblk, 0.0, 0)
+                                   qblk, 0.0, 0, kwargs.get("of_heads") or 0)
     return out
 
 
@@ -216,7 +227,7 @@ def bitmaskcached_attn_cuda(query, key, value, current_layer, ditrun, *args, **k
         return out
     lists = getattr(mask_cache, "lists_for_attention", mask_cache.get_mask_from_cache)
     kv_indices, kv_num_indices = lists(current_layer)
-    return _sparse_once(query, key, value, kv_indices, kv_num_indices)
+    return _sparse_once(query, key, value, kv_indices, kv_num_indices, kwargs.get("of_heads"))
 
 
 def attn_2xmask_cuda(query, key, value, current_layer=None, ditrun=None, *args, **kwargs):
@@ -229,4 +240,5 @@ def attn_2xmask_cuda(query, key, value, current_layer=None, ditrun=None, *args, 
     row[: S // 2] = 2 * torch.arange(S // 2, dtype=torch.int32, device=query.device)
     kv_indices = row.expand(B, H, nb, stride).contiguous()
     kv_num_indices = torch.full((B, H, nb), S // 2, dtype=torch.int32, device=query.device)
-    return _sparse(query, key, value, kv_indices, kv_num_indices, fresh=True)   # lists of equal length: index order
+    # lists of equal length: index order
+    return _sparse(query, key, value, kv_indices, kv_num_indices, fresh=True, of_heads=kwargs.get("of_heads"))

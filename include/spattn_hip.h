@@ -84,7 +84,8 @@ int spattn_full_attn(void* o, float* lse, const void* q, const void* k, const vo
 
 /* qblk in {64,128}: rows per q-block = rows sharing one list; kv_indices is
  * [B,H,ceil(S/qblk),mask_stride].  Lists of 128 rows in launches that leave the chip idle run by workgroups of 64
- * rows, here and in the other list entry points, so low bits of o and lse depend on batch * heads * seq. */
+ * rows, here and in the other list entry points, so low bits of o and lse depend on batch * heads * seq; a caller who
+ * splits the heads of a computation over calls or devices names them all in the _of forms below. */
 int spattn_sp_attn(void* o, float* lse, const void* q, const void* k, const void* v, const int* kv_indices,
                    const int* num_kv_indices, int mask_stride, int qblk, int batch, int heads, int seq, int D,
                    int kv_len, float scale, void* stream);
@@ -270,6 +271,16 @@ int spattn_sp_attn_blocks_ordered(void* o, float* lse, const void* q, const void
                                   const int* blk_indices, const int* blk_counts, const int* order, int max_blocks,
                                   int qblk, int batch, int heads, int seq, int D, int kv_len, float scale, void* stream);
 
+/* The list-driven entry points over some of the of_heads (batch x heads) of one computation: the size of the whole decides how
+ * a q-block is split, so o and lse are the same bits as in one call over all of its heads.  order: as above, or NULL;
+ * of_heads = 0: the call is the whole, otherwise at least batch x heads, else SPATTN_ERR_SHAPE. */
+int spattn_sp_attn_of(void* o, float* lse, const void* q, const void* k, const void* v, const int* kv_indices,
+                      const int* num_kv_indices, const int* order, int mask_stride, int qblk, int batch, int heads, int seq,
+                      int D, int kv_len, float scale, int of_heads, void* stream);
+int spattn_sp_attn_blocks_of(void* o, float* lse, const void* q, const void* k, const void* v, const int* blk_indices,
+                             const int* blk_counts, const int* order, int max_blocks, int qblk, int batch, int heads,
+                             int seq, int D, int kv_len, float scale, int of_heads, void* stream);
+
 /* Block-list attention in balanced (longest list first) order for callers that cannot
  * allocate: code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.
  * It has no counterpart in the reference.  It is spattn_qblock_order followed by
@@ -295,6 +306,10 @@ int spattn_sp_attn_blocks_balanced(void* o, float* lse, const void* q, const voi
  * of `heads` (batch x heads) of a computation of of_heads (0: all of it) is split: rows of a q-block (64, 128 or 256) times
  * ten, plus the groups of waves that share one (1 or 2); an error status for sizes that the calls refuse.  Host only. */
 int spattn_dense_form(int D, int has_v, int stats, int heads, int seq, int kv_len, int of_heads);
+
+/* Rows per workgroup (64 or 128) of list-driven attention over `heads` (batch x heads) of a computation of of_heads (0: all of
+ * it); stride: mask_stride of token lists (tokens != 0) or max_blocks; an error status for what the calls refuse.  Host only. */
+int spattn_list_form(int D, int qblk, int tokens, int heads, int seq, int kv_len, int stride, int of_heads);
 
 /* Status of the most recent call on this host thread, and its text. */
 int spattn_last_status(void);

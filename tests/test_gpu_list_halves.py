@@ -63,6 +63,45 @@ def test_halves_give_the_bits_of_64_row_lists(dev, D, H, S, kv_len, halved):
             assert float((got[0].view(torch.bfloat16).float() - o).norm()) <= 1e-2 * float(o.norm())
 
 
+@pytest.mark.parametrize("D,H,S,few", [(64, 25, 2048, 3), (64, 24, 2048, 5), (128, 9, 2048, 1), (128, 8, 1050, 3)])
+def test_some_heads_give_the_bits_of_all(dev, D, H, S, few):
+    """Some heads of a computation that runs by whole lists, and of one that runs by halves, through the operators and the
+    functional, in index order and in a work order; without of_heads the former would run by halves."""
+    from fgattn_tk_cuda_amd.spattn import cuda_attn, mask_utils, sparseattn_functionals as fn  # noqa: F401
+
+    print("case some heads", D, H, S, few, flush=True)
+    ops = torch.ops.cuda_attn
+    q, k, v = (t.to(dev) for t in wl.randn_qkv(1, H, S, D, seed=36))
+    lists, order = _lists(dev, H, S)
+
+    def call(kind, heads, order=None, of_heads=0):
+        qh, kh, vh, idx, n = (t[:, heads].contiguous() for t in (q, k, v, *lists[kind]))
+        o, lse = torch.empty_like(qh), torch.empty(qh.shape[:3], device=dev)
+        if kind == "tokens":
+            ops.sp_attn_ex(o, lse, qh, kh, vh, idx, n, order, 0.0, 0, of_heads)
+        else:
+            ops.sp_attn_block(o, lse, qh, kh, vh, idx, n, order, 128, 0.0, 0, of_heads)
+        return o, lse, (qh, kh, vh, idx, n)
+
+    nq = wl.ceil_div(S, 128)
+    for kind in lists:
+        whole = call(kind, slice(0, H), order)
+        for h0 in range(0, H, few):
+            heads = slice(h0, min(H, h0 + few))
+            some = torch.randperm((heads.stop - h0) * nq, generator=torch.Generator().manual_seed(h0)).to(torch.int32).to(dev)
+            for by in (None, some):
+                o, lse, _ = call(kind, heads, by, H)
+                assert torch.equal(o, whole[0][:, heads]) and torch.equal(lse, whole[1][:, heads]), (kind, h0)
+        o, _, part = call(kind, slice(0, few))
+        assert kind != "tokens" or torch.equal(o, whole[0][:, :few]) == (H * wl.ceil_div(S, 64) <= (768 if D == 64 else 256))
+        cache = (mask_utils.NaiveMaskCache if kind == "tokens" else mask_utils.BlockListCache)([0])
+        cache.update_cache(0, *part[3:])
+        step = fn.cached_attn_cuda if kind == "tokens" else fn.blockcached_attn_cuda
+        assert torch.equal(step(*part[:3], 0, 1, blocksz=128, mask_cache=cache, of_heads=H), whole[0][:, :few])
+    with pytest.raises(RuntimeError):
+        call("tokens", slice(0, 2), None, 1)
+
+
 @pytest.mark.parametrize("D,H,S", [(128, 16, 1100), (64, 56, 900)])
 def test_large_list_launches_read_no_freed_slot(dev, D, H, S):
     """Lists of 128-row q-blocks behind the rule, one workgroup to a list, in the NaN-poisoning build."""
