@@ -43,7 +43,7 @@ def _call(lib, kind, qkv, idx, n, qblk, kv_len, order=None):
     (64, 5, 1050, 0, True), (64, 8, 2048, 2000, True),       # the last q-block ends in its first half; one per CU
     (64, 24, 2048, 0, True), (64, 24, 1100, 1023, False),    # three per CU; more than one per CU and too short
     (64, 25, 2048, 0, False),                                # behind three per CU
-    (128, 5, 1050, 0, True), (128, 8, 2048, 0, True), (128, 1, 16384, 0, True),   # up to one per CU
+    (128, 5, 1650, 0, True), (128, 8, 2048, 0, True), (128, 1, 16384, 0, True),   # up to one per CU
     (128, 5, 900, 767, False), (128, 9, 2048, 0, False),     # too short; behind one per CU
 ])
 def test_halves_give_the_bits_of_64_row_lists(dev, D, H, S, kv_len, halved):
@@ -63,7 +63,7 @@ def test_halves_give_the_bits_of_64_row_lists(dev, D, H, S, kv_len, halved):
             assert float((got[0].view(torch.bfloat16).float() - o).norm()) <= 1e-2 * float(o.norm())
 
 
-@pytest.mark.parametrize("D,H,S,few", [(64, 25, 2048, 3), (64, 24, 2048, 5), (128, 9, 2048, 1), (128, 8, 1050, 3)])
+@pytest.mark.parametrize("D,H,S,few", [(64, 25, 2048, 3), (64, 24, 2048, 5), (128, 9, 2048, 1), (128, 8, 1700, 3)])
 def test_some_heads_give_the_bits_of_all(dev, D, H, S, few):
     """Some heads of a computation that runs by whole lists, and of one that runs by halves, through the operators and the
     functional, in index order and in a work order; without of_heads the former would run by halves."""

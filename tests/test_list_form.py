@@ -20,6 +20,26 @@ def test_some_heads_go_by_all_heads(D, S, whole, tokens):
     assert form(D, tokens, 1, S) == 64
 
 
+def test_workgroups_count_and_not_blocks_of_64_rows():
+    """Thirteen and 25 blocks of 64 rows a head: a list's second half may be empty, its workgroup is started all the same."""
+    assert form(128, 0, 18, 800) == 64 and form(128, 0, 19, 800) == 128    # 252 and 266 workgroups
+    assert form(64, 0, 29, 1600) == 64 and form(64, 0, 30, 1600) == 128    # 754 and 780
+
+
+@pytest.mark.parametrize("D,tokens,heads,S,stride,rows", [
+    (128, 0, 4, 4096, 1, 128), (128, 0, 4, 4096, 2, 64),
+    (128, 1, 4, 4096, 128, 128), (128, 1, 4, 4096, 256, 64),          # rows shorter than the sequence
+    (128, 1, 9, 1600, 1664, 128), (128, 1, 9, 1601, 1664, 64),        # 4 % of the keys: one tile, two
+    (64, 0, 4, 4096, 1, 128), (64, 1, 4, 4096, 128, 64), (64, 1, 18, 800, 896, 64),
+    (64, 0, 8, 4096, 6, 128), (64, 0, 8, 4096, 7, 64), (64, 1, 8, 4096, 256, 128), (64, 1, 8, 4096, 384, 64),
+    (64, 1, 10, 3200, 3200, 128), (64, 1, 9, 3201, 3328, 64),
+    (64, 0, 12, 4096, 4, 128), (64, 0, 12, 4096, 5, 64), (64, 1, 12, 4096, 128, 128), (64, 1, 12, 4096, 256, 64),
+    (64, 1, 29, 1600, 1664, 128), (64, 1, 29, 1601, 1664, 64),
+])
+def test_lists_that_lose_by_halves_keep_their_form(D, tokens, heads, S, stride, rows):
+    assert form(D, tokens, heads, S, 0, stride) == rows
+
+
 def test_what_the_rule_does_not_reach():
     assert form(64, 1, 1, 64, qblk=64) == form(128, 0, 400, 9000, qblk=64) == 64
     assert form(128, 1, 400, 9000) == form(64, 0, 400, 9000) == 128
