@@ -20,7 +20,7 @@ from its first copy to the wait for the last one.
 
 The asm statements take base addresses in scalar registers.  A vector-memory instruction may read a scalar register that the
 vector ALU wrote (readfirstlane, readlane) five wait states later; the compiler keeps that distance for its own instructions
-and does not look into asm, so the listing is checked for it.
+and does not look into asm, so the listing is checked for it, along every path.
 
 A copy into LDS may read m0 one wait state behind a scalar write of it; the compiler puts it there behind its own writes only.
 
@@ -109,30 +109,6 @@ def m0_uses_outside_asm(listing):
     return found
 
 
-def scalar_bases_too_close(listing, states=5):
-    """[(vector-ALU write, vector-memory instruction, wait states between them)] where an instruction reads a scalar register
-    fewer than `states` wait states after the vector ALU wrote it, in the order of the listing."""
-    def sregs(text):
-        out = {int(m) for m in re.findall(r"\bs(\d+)\b", text)}
-        for lo, hi in re.findall(r"\bs\[(\d+):(\d+)\]", text):
-            out.update(range(int(lo), int(hi) + 1))
-        return out
-
-    found, recent = [], []   # recent: (wait states since, registers, instruction)
-    for raw in listing.split("\n"):
-        t = raw.split(";")[0].strip()
-        if not t or t.startswith(".") or t.endswith(":"):
-            continue
-        op, args = t.split()[0], t.split(None, 1)[1] if " " in t else ""
-        if _is_vmem(op):
-            found += [(w, t, age) for age, regs, w in recent if age < states and regs & sregs(args)]
-        passed = 1 + (int(args, 0) if op == "s_nop" else 0)
-        recent = [(age + passed, regs, w) for age, regs, w in recent if age + passed < states]
-        if op.startswith("v_") and re.match(r"s\[?\d", args):
-            recent.append((0, sregs(args.split(",")[0]), t))
-    return found
-
-
 class Flow:
     """The instructions of one kernel, [(operation, operands, inside an asm statement)], and what may follow each."""
 
@@ -168,6 +144,27 @@ class Flow:
 def kernel_flows(listing):
     for m in re.finditer(r"^(_Z\w+):(.*?)^\.Lfunc_end", listing, re.S | re.M):
         yield m.group(1), Flow(m.group(2))
+
+
+def scalar_bases_too_close(listing, states=5):
+    """[(vector-ALU write, vector-memory instruction, wait states between them)] where an instruction reads a scalar register
+    fewer than `states` wait states after the vector ALU wrote it, along any path."""
+    def sregs(text):
+        out = {"s" + m for m in re.findall(r"\bs(\d+)\b", text)} | set(re.findall(r"\bvcc\b", text))
+        for lo, hi in re.findall(r"\bs\[(\d+):(\d+)\]", text):
+            out.update("s%d" % r for r in range(int(lo), int(hi) + 1))
+        return out
+
+    found = []
+    for _, flow in kernel_flows(listing):
+        for i, (op, args, _) in enumerate(flow.ins):
+            # the result, or the carry that add, sub and div_scale write beside it
+            written = sregs(",".join(args.split(",")[:2 if "_co_" in op or "div_scale" in op else 1])) if op.startswith("v_") else None
+            for j, passed in flow.within(i, states).items() if written else ():
+                op2, args2, _ = flow.ins[j]
+                if _is_vmem(op2) and written & sregs(args2):
+                    found.append((op + " " + args, op2 + " " + args2, passed))
+    return found
 
 
 def multiplies_too_close(listing):
@@ -273,11 +270,19 @@ def test_tile_loop_checker():
 
 
 def test_scalar_base_checker():
-    late = "\tv_readfirstlane_b32 s21, v9\n\tv_readfirstlane_b32 s20, v8\n%s\ts_mov_b32 m0, s3\n\tglobal_load_lds_dwordx4 v7, s[20:21]\n"
-    assert len(scalar_bases_too_close(late % "")) == 2
-    assert len(scalar_bases_too_close(late % "\ts_nop 2\n")) == 1
-    assert scalar_bases_too_close(late % "\ts_nop 3\n") == []
-    assert scalar_bases_too_close((late % "").replace("s[20:21]", "s[22:23]")) == []
+    def found(*lines):
+        body = "_ZN6spattn1kE:\n" + "".join("\t" * (not l.endswith(":")) + l + "\n" for l in lines) + "\ts_endpgm\n.Lfunc_end0:\n"
+        return sorted(f[2] for f in scalar_bases_too_close(body))
+
+    write = ("v_readfirstlane_b32 s21, v9", "v_readfirstlane_b32 s20, v8")
+    copy = ("s_mov_b32 m0, s3", "global_load_lds_dwordx4 v7, s[20:21]")
+    assert found(*write, *copy) == [1, 2] and found(*write, "s_nop 2", *copy) == [4] and found(*write, "s_nop 3", *copy) == []
+    assert found(*write, copy[0], "global_load_lds_dwordx4 v7, s[22:23]") == []
+    assert found(".LBB0_1:", *copy, write[1], "s_cbranch_scc1 .LBB0_1") == [2]                         # around a loop
+    assert found(write[1], "s_cbranch_scc1 .LBB0_2", "s_nop 15", ".LBB0_2:", *copy) == [2]            # past the wait
+    assert found(write[1], "s_branch .LBB0_2", *copy, ".LBB0_2:") == []                               # not on a path
+    assert found("v_add_co_u32_e32 v1, vcc, v2, v3", "global_load_lds_dwordx4 v7, vcc") == [0]
+    assert found("v_cmp_gt_i32_e64 s[20:21], v1, v2", copy[1]) == [0] and found("v_add_u32_e32 v1, s20, v2", copy[1]) == []
 
 
 def test_multiply_checker():
