@@ -147,9 +147,11 @@ static void check_sp_attn_args(torch::Tensor& o, torch::Tensor& q, torch::Tensor
   TORCH_CHECK(kv_num_indices.numel() == q.size(0) * q.size(1) * kv_indices.size(2), "kv_num_indices must have B*H*SB entries");
 }
 
-// Up to one q-block per CU there is nothing to balance, and every workgroup would only wait for its entry: token
-// lists 8 x 4096 x 128 14.8 us without an order, 15.9 with; 4 x 2048 x 128 9.3 / 9.2 (heads of equal density),
-// 10.1 / 10.6 (very different ones).
+// Up to one list per CU there is little to balance, and every workgroup waits for its entry.  Token lists of masks that keep
+// 8.5 % of the keys, without an order and with one, heads of equal / very different density, us: one workgroup to a list 8 x 4096
+// x 128 13.75 and 13.93 / 16.3 and 17.1, 16 x 2048 x 64 7.2 and 7.3 / 8.4 and 8.5; two to a list 4 x 2048 x 128 7.1 and 7.2 / 8.1 and
+// 8.1, 8 x 2048 x 64 6.0 and 6.1 / 6.5 and 6.5.  Where two to a list are two to a CU (d = 64, 129 to 256 lists) both signs
+// occur, and the counts are not known here: 8 x 4096 x 64 9.3 and 9.8 / 10.3 and 9.7, 4 x 8192 x 64 15.0 and 14.7 / 16.2 and 13.9.
 constexpr int64_t kNoOrder = 256;
 // The work order for counts of per_head q-blocks per head.  Below kScheduleMin q-blocks all of them are resident
 // at once and the plain longest-first order does.
