@@ -18,8 +18,9 @@ namespace spattn {
 //   in the second per CU 1.03-1.06 with one to three tiles, 0.99 with four, 0.93-0.97 with six; 4 % 1.04-1.10 up to 2300 keys, 0.99
 //   at 4000, 0.88 at 8000; in the third 1.00-1.04 with one, 0.95-0.98 with two and three; 4 % 1.03-1.04 up to 1600 keys, 1.015 at
 //   2300, 0.95 at 4000.
-// The counts are on the device.  A row that is shorter than the sequence says how long its lists are; one that holds the
-// sequence is taken to hold 4 % of its keys, the sparsest mask, so denser ones in short sequences keep the 128-row form.
+// The counts are on the device.  A row of token ids that is shorter than the sequence says how long its lists are; one that holds
+// the sequence is taken to hold 4 % of its keys, the sparsest mask, so denser ones in short sequences keep the 128-row form.
+// Block lists are taken to be as long as their rows: masks that fill rows of the whole sequence keep a third of the blocks.
 // The halves add a row's keys in another order: a launch over some heads of a computation goes by all of its heads, so that no
 // bit depends on the split.
 bool lists_by_halves(int D, int qblk, bool tokens, long long heads, int S, int kv_len, int idx_stride) {
